@@ -200,11 +200,11 @@ int mlff_plan_set_cell_grid(mlff_plan* plan, const int32_t* grid_host, int n_str
 
 /* Rebind a bound plan to a new weight blob of the same layout (a training
  * step's updated weights) without the host synchronisation of
- * mlff_plan_bind: the bf16 planes of the filter weights are re-split on
- * `stream`, ordered after the blob's writes when those are on the same
- * stream.  Evaluations on another stream must be ordered after it by the
- * caller.  Drops the plan's captured graphs.  (The reference's modules read
- * their parameters in place, student_model.py:585-605.) */
+ * mlff_plan_bind: what the plan derives from the weights (bf16 planes and
+ * distance tables of the filters) is remade by the next evaluation, on its
+ * stream, which the caller orders after the blob's writes.  Drops the plan's
+ * captured graphs.  (The reference's modules read their parameters in place,
+ * student_model.py:585-605.) */
 int mlff_plan_set_weights(mlff_plan* plan, void* stream, const float* weights_dev);
 
 /* Device pointer to the plan's int32 counts[MLFF_COUNT_SLOTS]. */
@@ -228,8 +228,8 @@ int mlff_energy_forces(mlff_plan* plan, void* stream, const float* pos_dev,
  * mlff_energy_forces with the same config (one stream, bit-identical), but
  * the workspace is a static device array of MLFF_STATIC_SCRATCH_BYTES that
  * each GPU the library runs on holds until the process ends; a batch whose
- * workspace (mlff_plan_workspace_bytes of the same config) exceeds it is
- * rejected with MLFF_ERR_WORKSPACE.  No hipMalloc/hipFree, no stream or event
+ * workspace (mlff_plan_workspace_bytes of the same config, less the filter
+ * tables, which have a static array of their own) exceeds it is rejected with MLFF_ERR_WORKSPACE.  No hipMalloc/hipFree, no stream or event
  * creation, no host synchronisation: everything is enqueued on `stream`.
  *
  * Every call on one GPU shares that GPU's scratch, which keeps the last

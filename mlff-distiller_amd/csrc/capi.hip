@@ -121,9 +121,15 @@ struct mlff_plan {
   int stream_dev;
   hipStream_t aux;
   hipEvent_t ev[2 * 8 + 2];
-  // workspace carve-up (byte offsets)
+  // filter tables: what the host knows of the guard's flag, whether the
+  // weights changed since they were made, and the evaluations since then
+  enum { kTabNone, kTabGood, kTabBad, kTabUnknown } tab_state;
+  bool tab_stale;
+  int tab_runs;
+  // workspace carve-up (byte offsets); core_bytes: without the tables
   struct { int64_t off, bytes; } seg[48];
   int nseg;
+  int64_t core_bytes;
 };
 
 namespace {
@@ -132,6 +138,7 @@ enum Seg {
   S_COUNTS, S_DEG, S_UDEG, S_ROWPTR, S_PAIRPTR, S_COL, S_EPAIR, S_PLO, S_PHI, S_PSHIFT, S_GEOM,
   S_PACC, S_GVEC, S_WF, S_S, S_V, S_SMID, S_VMID, S_AUPD, S_G12, S_GS0, S_GV0, S_GS1, S_GV1,
   S_EPS, S_VIR, S_GRID, S_CELLCNT, S_CELLSTART, S_CELLATOMS, S_ATOMCELL, S_TMPSHIFT, S_WBF,
+  S_TABBAD, S_TAB,   // the tables last: the static entry keeps them elsewhere
   S_COUNT_
 };
 
@@ -178,8 +185,12 @@ void carve(mlff_plan* pl) {
   sz[S_ATOMCELL] = CC ? 4 * N : 0;
   sz[S_TMPSHIFT] = CC ? 12 * E : 0;
   sz[S_WBF] = 2 * wbf_elems((int)H, (int)L);
+  pl->buf.ts = table_shape((int)H, c.num_rbf, (int)L, c.cutoff);
+  sz[S_TABBAD] = pl->buf.ts.bytes ? 4 : 0;
+  sz[S_TAB] = pl->buf.ts.bytes;
   int64_t off = 0;
   for (int k = 0; k < S_COUNT_; ++k) {
+    if (k == S_TAB) pl->core_bytes = off;
     pl->seg[k].off = off;
     pl->seg[k].bytes = sz[k];
     off += (sz[k] + 255) & ~(int64_t)255;
@@ -245,6 +256,57 @@ void set_default_shapes(mlff_plan* pl) {
   pl->buf.unroll_fwd = default_shape(H, 2);
   pl->buf.unroll_bwd = default_shape(H, 3);
   pl->buf.bwd_variant = default_shape(H, 4);
+}
+
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+// How the pair kernels of the next evaluation run, from what is known of the tables.
+void choose_filter_form(mlff_plan* pl) {
+  Buffers& b = pl->buf;
+  b.use_table = pl->tab_state == mlff_plan::kTabGood || pl->tab_state == mlff_plan::kTabUnknown;
+  b.gate = pl->tab_state == mlff_plan::kTabUnknown ? b.tab_bad : nullptr;
+}
+
+// Read the guard's flag on the host (waits for stream s).
+hipError_t resolve_tables(mlff_plan* pl, hipStream_t s) {
+  int32_t bad = 1;
+  hipError_t e = hipMemcpyAsync(&bad, pl->buf.tab_bad, 4, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e != hipSuccess) return e;
+  pl->tab_state = bad ? mlff_plan::kTabBad : mlff_plan::kTabGood;
+  choose_filter_form(pl);
+  return hipSuccess;
+}
+
+// Bring the planes and tables up to the bound weights on stream s.  They are
+// remade by the first evaluation after a weight change (a training loop over
+// changing batch shapes keeps several plans and uses one of them per step).
+// That evaluation launches both forms of the pair kernels behind the flag, so
+// nothing waits for it; when a second one follows on the same weights the
+// host reads the flag once and the idle launches go (never under capture).
+// now: read the flag at once.
+hipError_t refresh_filters(mlff_plan* pl, hipStream_t s, bool now) {
+  const bool known = pl->tab_state != mlff_plan::kTabUnknown;
+  if (!pl->tab_stale && known) return hipSuccess;
+  if (pl->tab_stale) {
+    hipError_t e = prepare_filters(pl->buf, s);
+    if (e != hipSuccess) return e;
+    pl->tab_stale = false;
+    pl->tab_runs = 0;
+    pl->tab_state = pl->buf.tab != nullptr ? mlff_plan::kTabUnknown : mlff_plan::kTabNone;
+    choose_filter_form(pl);
+    if (pl->tab_state == mlff_plan::kTabNone) return hipSuccess;
+  }
+  if ((now || pl->tab_runs > 0) && !capturing(s)) return resolve_tables(pl, s);
+  ++pl->tab_runs;
+  return hipSuccess;
 }
 
 template <typename T>
@@ -435,6 +497,10 @@ int bind_buffers(mlff_plan* pl, const char* who, void* ws, const float* weights_
   b.eps = segp<float>(pl, ws, S_EPS);
   b.vir_atom = segp<float>(pl, ws, S_VIR);
   b.wbf = segp<uint16_t>(pl, ws, S_WBF);
+  b.tab = segp<float>(pl, ws, S_TAB);
+  b.tab_bad = segp<int32_t>(pl, ws, S_TABBAD);
+  b.use_table = false;
+  b.gate = nullptr;
   NLArgs& a = pl->nl;
   memset(&a, 0, sizeof(a));
   a.N = b.N; a.B = b.B; a.mol_ptr = mol_ptr_dev; a.atom_mol = atom_mol_dev;
@@ -479,8 +545,14 @@ int mlff_plan_bind(mlff_plan* pl, void* ws, int64_t ws_bytes, const float* weigh
   if (e != hipSuccess) return hip_fail(e, "mlff_plan_bind");
   e = acquire_streams(pl);
   if (e != hipSuccess) return hip_fail(e, "mlff_plan_bind: filter stream");
-  e = split_filter_weights(b);
-  if (e != hipSuccess) return hip_fail(e, "mlff_plan_bind: bf16 weight planes");
+  // the weights may have just been written on another stream
+  e = hipDeviceSynchronize();
+  if (e == hipSuccess) {
+    pl->tab_stale = true;
+    e = refresh_filters(pl, nullptr, true);
+  }
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  if (e != hipSuccess) return hip_fail(e, "mlff_plan_bind: filter planes and tables");
   pl->bound = true;
   pl->md_bound = false;
   pl->mts_bound = false;
@@ -497,10 +569,9 @@ int mlff_plan_set_weights(mlff_plan* pl, void* stream, const float* weights_dev)
     set_error("mlff_plan_set_weights: weights must be non-null and 16-byte aligned");
     return MLFF_ERR_INVALID;
   }
+  (void)stream;
   pl->buf.w = weights_dev;
-  // the bf16 planes follow the new weights in stream order on the caller's stream
-  hipError_t e = split_filter_weights_async(pl->buf, static_cast<hipStream_t>(stream));
-  if (e != hipSuccess) return hip_fail(e, "mlff_plan_set_weights: bf16 weight planes");
+  pl->tab_stale = true;   // planes and tables follow with the next evaluation, on its stream
   // captured graphs hold the old weights
   if (pl->mts_exec) { (void)hipGraphExecDestroy(pl->mts_exec); pl->mts_exec = nullptr; }
   if (pl->mts_graph) { (void)hipGraphDestroy(pl->mts_graph); pl->mts_graph = nullptr; }
@@ -514,7 +585,9 @@ int32_t* mlff_plan_counts(mlff_plan* pl) { return (pl && pl->bound) ? pl->buf.co
 static int run_ef(mlff_plan* pl, hipStream_t s, const float* pos, double* energy, float* forces,
                   double* virial, float* atom_energy) {
   pl->nl.pos = pos;
-  hipError_t e = launch_neighbor_list(pl->nl, s, true);
+  hipError_t e = refresh_filters(pl, s, false);
+  if (e != hipSuccess) return hip_fail(e, "filter tables");
+  e = launch_neighbor_list(pl->nl, s, true);
   if (e != hipSuccess) return hip_fail(e, "neighbour list");
   e = launch_forward(pl->buf, s);
   if (e != hipSuccess) return hip_fail(e, "forward");
@@ -543,6 +616,8 @@ int mlff_launch_stage(mlff_plan* pl, void* stream, int stage, int layer) {
     if (!pl->nl.pos) { set_error("mlff_launch_stage: no evaluation yet"); return MLFF_ERR_STATE; }
     e = launch_neighbor_list(pl->nl, s, true);
   } else {
+    e = refresh_filters(pl, s, true);
+    if (e != hipSuccess) return hip_fail(e, "mlff_launch_stage: filter tables");
     e = launch_stage(pl->buf, s, stage, layer);
   }
   if (e != hipSuccess) return hip_fail(e, "mlff_launch_stage");
@@ -727,7 +802,9 @@ int mlff_md_graph_run(mlff_plan* pl, void* stream, int steps_per_graph, int n_la
   if (!pl->graph_exec || pl->graph_steps != steps_per_graph) {
     if (pl->graph_exec) { (void)hipGraphExecDestroy(pl->graph_exec); pl->graph_exec = nullptr; }
     if (pl->graph) { (void)hipGraphDestroy(pl->graph); pl->graph = nullptr; }
-    hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+    hipError_t e = refresh_filters(pl, s, true);   // the graph holds one form only
+    if (e != hipSuccess) return hip_fail(e, "mlff_md_graph_run: filter tables");
+    e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
     int rc = MLFF_OK;
     for (int k = 0; k < steps_per_graph && rc == MLFF_OK; ++k) rc = md_step(pl, s);
@@ -753,12 +830,14 @@ int mlff_md_graph_run(mlff_plan* pl, void* stream, int steps_per_graph, int n_la
 // positions, same cutoff, equal capacities).
 static int run_ef_on(mlff_plan* pl, hipStream_t s, double* energy, float* forces,
                      const Buffers& src) {
+  hipError_t e = refresh_filters(pl, s, false);
+  if (e != hipSuccess) return hip_fail(e, "outer filter tables");
   Buffers b = pl->buf;
   b.counts = src.counts;
   b.row_ptr = src.row_ptr; b.col = src.col; b.edge_pair = src.edge_pair;
   b.pair_lo = src.pair_lo; b.pair_hi = src.pair_hi; b.pair_shift = src.pair_shift;
   b.geom = src.geom;
-  hipError_t e = launch_forward(b, s);
+  e = launch_forward(b, s);
   if (e != hipSuccess) return hip_fail(e, "outer forward");
   e = launch_backward(b, s, forces, false);
   if (e != hipSuccess) return hip_fail(e, "outer adjoint");
@@ -870,7 +949,10 @@ int mlff_mts_graph_run(mlff_plan* pl, void* stream, int outer_per_graph, int n_l
   if (!pl->mts_exec || pl->mts_graph_steps != outer_per_graph) {
     if (pl->mts_exec) { (void)hipGraphExecDestroy(pl->mts_exec); pl->mts_exec = nullptr; }
     if (pl->mts_graph) { (void)hipGraphDestroy(pl->mts_graph); pl->mts_graph = nullptr; }
-    hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+    hipError_t e = refresh_filters(pl, s, true);
+    if (e == hipSuccess) e = refresh_filters(pl->mts_inner, s, true);
+    if (e != hipSuccess) return hip_fail(e, "mlff_mts_graph_run: filter tables");
+    e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
     int rc = MLFF_OK;
     for (int k = 0; k < outer_per_graph && rc == MLFF_OK; ++k) rc = mts_outer_step(pl, s, false);
@@ -902,19 +984,24 @@ int mlff_mts_graph_run(mlff_plan* pl, void* stream, int outer_per_graph, int n_l
 namespace {
 
 static __device__ __align__(256) unsigned char scratch[MLFF_STATIC_SCRATCH_BYTES];
+// filter tables of the calls' weights, beside the workspace (kTableMaxBytes
+// bounds them, so every configuration that has tables fits)
+static __device__ __align__(256) unsigned char table_scratch[kTableMaxBytes];
 
 constexpr int kMaxDevices = 64;
 
-// Per device: the device address of `scratch` (the host-side name is only a
-// stand-in and must never reach a kernel) and the CU count.
+// Per device: the device addresses of `scratch` and `table_scratch` (the
+// host-side names are only stand-ins and must never reach a kernel) and the
+// CU count.
 struct StaticScratch {
   std::mutex mu;
   void* ptr[kMaxDevices] = {};
+  void* tab[kMaxDevices] = {};
   int cus[kMaxDevices] = {};
 };
 StaticScratch g_static;
 
-int static_scratch(int* dev_out, void** ptr_out, int* cus_out) {
+int static_scratch(int* dev_out, void** ptr_out, void** tab_out, int* cus_out) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "mlff_energy_forces_static: hipGetDevice");
@@ -925,10 +1012,11 @@ int static_scratch(int* dev_out, void** ptr_out, int* cus_out) {
   }
   std::lock_guard<std::mutex> lock(g_static.mu);
   if (!g_static.ptr[dev]) {
-    void* p = nullptr;
+    void *p = nullptr, *t = nullptr;
     e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+    if (e == hipSuccess) e = hipGetSymbolAddress(&t, HIP_SYMBOL(table_scratch));
     if (e != hipSuccess) return hip_fail(e, "mlff_energy_forces_static: hipGetSymbolAddress");
-    if (!p) {
+    if (!p || !t) {
       set_error("mlff_energy_forces_static: no device address for the scratch array");
       return MLFF_ERR_HIP;
     }
@@ -938,9 +1026,11 @@ int static_scratch(int* dev_out, void** ptr_out, int* cus_out) {
       cus = prop.multiProcessorCount;
     g_static.cus[dev] = cus;
     g_static.ptr[dev] = p;
+    g_static.tab[dev] = t;
   }
   *dev_out = dev;
   *ptr_out = g_static.ptr[dev];
+  *tab_out = g_static.tab[dev];
   *cus_out = g_static.cus[dev];
   return MLFF_OK;
 }
@@ -982,15 +1072,15 @@ extern "C" int mlff_energy_forces_static(void* stream, const mlff_config* cfg,
                         &pl.mw, nullptr, 0, nullptr);
   if (rc != MLFF_OK) return rc;
   carve(&pl);
-  if (pl.ws_bytes > (int64_t)MLFF_STATIC_SCRATCH_BYTES) {
-    set_error("%s: this batch needs %lld bytes of scratch; the static scratch holds %lld "
-              "(use mlff_energy_forces with a workspace)", who, (long long)pl.ws_bytes,
-              (long long)MLFF_STATIC_SCRATCH_BYTES);
+  if (pl.core_bytes > (int64_t)MLFF_STATIC_SCRATCH_BYTES) {
+    set_error("%s: this batch needs %lld bytes of scratch, filter tables included; the static "
+              "scratch holds %lld beside the tables (use mlff_energy_forces with a workspace)",
+              who, (long long)pl.ws_bytes, (long long)MLFF_STATIC_SCRATCH_BYTES);
     return MLFF_ERR_WORKSPACE;
   }
   int dev = 0, cus = 0;
-  void* ws = nullptr;
-  rc = static_scratch(&dev, &ws, &cus);
+  void *ws = nullptr, *tab = nullptr;
+  rc = static_scratch(&dev, &ws, &tab, &cus);
   if (rc != MLFF_OK) return rc;
   pl.buf.blocks = persistent_grid(cfg->persistent_blocks, cus);
   set_default_shapes(&pl);
@@ -1003,13 +1093,13 @@ extern "C" int mlff_energy_forces_static(void* stream, const mlff_config* cfg,
   // a memset node, so the call can be captured into a HIP graph)
   pl.buf.counts = counts_dev;
   pl.nl.counts = counts_dev;
+  pl.buf.tab = pl.buf.ts.bytes ? static_cast<float*>(tab) : nullptr;
   pl.buf.aux = nullptr;
   pl.buf.ev = pl.ev;
   hipStream_t s = static_cast<hipStream_t>(stream);
   fill_i32_kernel<<<1, 64, 0, s>>>(counts_dev, MLFF_COUNT_SLOTS, 0);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, who);
-  e = split_filter_weights_async(pl.buf, s);
-  if (e != hipSuccess) return hip_fail(e, "mlff_energy_forces_static: bf16 weight planes");
+  pl.tab_stale = true;   // planes and tables of this call's weights, made by run_ef
   return run_ef(&pl, s, pos_dev, energy_dev, forces_dev, virial_dev, atom_energy_dev);
 }

@@ -326,6 +326,17 @@ __device__ __forceinline__ void zero_acc(f4 (&acc)[RT][NT]) {
     for (int ct = 0; ct < NT; ++ct) acc[rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
 }
 
+// dE/dvec of a pair from its accumulated (dE/du, dE/dd) in acc, geometry gm:
+// gd vec/d + gu/(d+eps) - vec (vec.gu)/(d (d+eps)^2)
+__device__ __forceinline__ float4 pair_gradient(const float4& gm, const float4& acc) {
+  const float d = gm.w, den = d + kEdgeEps;
+  const float vdot = gm.x * acc.x + gm.y * acc.y + gm.z * acc.z;
+  const float a1 = (d > 0.f) ? acc.w / d : 0.f;
+  const float a2 = (d > 0.f) ? vdot / (d * den * den) : 0.f;
+  return make_float4(a1 * gm.x + acc.x / den - a2 * gm.x, a1 * gm.y + acc.y / den - a2 * gm.y,
+                     a1 * gm.z + acc.z / den - a2 * gm.z, 0.f);
+}
+
 // Work tiles of a persistent block: tiles t0, t0 + step, ... below t1.
 // Workgroups are dispatched round-robin over the 8 XCDs (block b runs on XCD
 // b % 8).  Each XCD owns one contiguous eighth of the tiles, and its blocks

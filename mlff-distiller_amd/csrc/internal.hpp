@@ -46,6 +46,49 @@ struct NLArgs {
 };
 hipError_t launch_neighbor_list(const NLArgs& a, hipStream_t s, bool build_pairs);
 
+// Distance tables of the filter MLP (filter_table.hip): K intervals of width
+// h for W', Kc of width 2h for W, over [0, rc] of every block.
+constexpr int64_t kTableMaxBytes = 64ll << 20;   // per plan; larger: direct product only
+struct TableShape {
+  double h;
+  int K, Kc;
+  int64_t d_off, layer_floats;      // floats: start of the W' part, size of a block's table
+  int64_t bytes;                    // all blocks; 0: no table for this configuration
+};
+TableShape table_shape(int H, int R, int L, float rc);
+
+// One block's table as a kernel reads it.
+struct TableView {
+  const float* w;                   // [Kc+1][2][C]: W, 2h W'
+  const float* d;                   // [K+1][2][C]: W', h W''
+  float inv, inv_c;                 // 1/h, 1/(2h): powers of two
+  int K, Kc;
+};
+__host__ __device__ inline TableView table_view(const TableShape& t, const float* tab, int l,
+                                                int C) {
+  const float* w = tab + l * t.layer_floats;
+  return TableView{w, w + t.d_off, (float)(1.0 / t.h), (float)(0.5 / t.h), t.K, t.Kc};
+}
+// Interval k of distance d and the weights of its cubic Hermite interpolant
+//   f0 + h01 (f1 - f0) + h10 g0 + h11 g1
+// of the knot values f and scaled slopes g.  inv is a power of two, so x, k
+// and t carry no rounding.
+struct TableAt {
+  int k;
+  float h01, h10, h11;
+};
+__device__ __forceinline__ TableAt table_at(float d, float inv, int K) {
+  const float x = d * inv;
+  const int k = min((int)x, K - 1);
+  const float t = x - (float)k, u = 1.f - t;
+  return TableAt{k, t * t * (3.f - 2.f * t), t * u * u, -t * t * u};
+}
+template <typename T>
+__device__ __forceinline__ T hermite(const TableAt& a, const T& f0, const T& g0, const T& f1,
+                                     const T& g1) {
+  return f0 + (a.h01 * (f1 - f0) + (a.h10 * g0 + a.h11 * g1));
+}
+
 // Model launches (painn_fwd.hip / painn_bwd.hip).
 struct Buffers {
   int N, B, H, L, R;
@@ -62,6 +105,14 @@ struct Buffers {
   // bf16 three-plane copies of the filter's second layer, per block l:
   // W2 [3H][H] at wbf + wbf_f2w(l); plane stride 3H^2
   uint16_t* wbf;
+  // filter tables of every block, and the flag their guard raises.  use_table:
+  // the pair kernels read the tables; gate (not null): they were not checked
+  // on the host yet, so both forms are launched and the flag picks one
+  TableShape ts;
+  float* tab;
+  int32_t* tab_bad;
+  bool use_table;
+  const int32_t* gate;
   const int64_t* numbers;
   const int32_t* mol_ptr;
   const int32_t* atom_mol;
@@ -95,10 +146,16 @@ __host__ __device__ inline int64_t wbf_elems(int H, int L) { return (int64_t)L *
 // variant number; every value up to it exists).
 int default_shape(int H, int which);
 int alternative_shape(int H, int which);
-// Split the filter weights into their bf16 planes (once per bind; synchronous).
-hipError_t split_filter_weights(const Buffers& b);
-// The same split enqueued on stream s (no synchronisation).
-hipError_t split_filter_weights_async(const Buffers& b, hipStream_t s);
+// What the pair kernels read beside the weight blob, remade on stream s for
+// new weights: the filters' bf16 planes and their tables with the guard's flag.
+hipError_t prepare_filters(const Buffers& b, hipStream_t s);
+// Fill and check every block's table (tab_bad must be 0 before).
+hipError_t build_tables(const Buffers& b, hipStream_t s);
+template <int H>
+void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l);
+template <int H>
+void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l, const float* gS1,
+                             const float* gV1, int first, int last);
 hipError_t launch_forward(const Buffers& b, hipStream_t s);
 hipError_t launch_backward(const Buffers& b, hipStream_t s, float* forces, bool want_virial);
 // One model stage (mlff_stage 1..8) of block `layer`, on the workspace as the

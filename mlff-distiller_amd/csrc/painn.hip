@@ -92,7 +92,8 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_fwd_kernel(
     const float4* __restrict__ geom, const int32_t* __restrict__ counts, int32_t pcap,
     const float* __restrict__ w, LayerW lw, const float* __restrict__ centers,
     const float* __restrict__ widths, int R, int RP, float rc, float* __restrict__ Wout,
-    const uint16_t* __restrict__ w2bf) {
+    const uint16_t* __restrict__ w2bf, const int32_t* __restrict__ gate) {
+  if (gate != nullptr && *gate == 0) return;
   constexpr int RT = TM / 16;
   constexpr int LDE = kMaxRbf + 4;
   constexpr int LDHB = H + 8;          // bf16 row stride of the split hidden activations
@@ -747,7 +748,8 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_bwd_kernel(
     const float* __restrict__ widths, int R, int RP, float rc, const float* __restrict__ Wf,
     const float* __restrict__ s_in, const float* __restrict__ v_in,
     const float* __restrict__ gs1, const float* __restrict__ gv1, float4* __restrict__ pacc,
-    float4* __restrict__ gvec, int first, int last) {
+    float4* __restrict__ gvec, int first, int last, const int32_t* __restrict__ gate) {
+  if (gate != nullptr && *gate == 0) return;
   constexpr int RT = TM / 16;
   constexpr int LDE = kMaxRbf + 4, LDG = 3 * H + 4, LDA = H + 4;
   constexpr int C4 = H / 4;                    // lanes per pair in the gather (4 channels each)
@@ -914,7 +916,6 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_bwd_kernel(
       const int m = threadIdx.x, p = pbase + m;
       if (p < P) {
         const float4 gm = geom[p];
-        const float d = gm.w;
         const int nparts = (RP > 16) ? 2 * ((H / 16 < 4) ? H / 16 : 4) : ((H / 16 < 8) ? H / 16 : 8);
         float gd = 0.f;
         for (int q = 0; q < nparts; ++q) gd += gd_lds[q * TM + m];
@@ -928,14 +929,7 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_bwd_kernel(
         float4 acc = first ? make_float4(0.f, 0.f, 0.f, 0.f) : pacc[p];
         acc.x += gx; acc.y += gy; acc.z += gz; acc.w += gd;
         if (last) {
-          // dE/dvec = gd vec/d + gu/(d+eps) - vec (vec.gu)/(d (d+eps)^2)
-          const float den = d + kEdgeEps;
-          const float vdot = gm.x * acc.x + gm.y * acc.y + gm.z * acc.z;
-          const float a1 = (d > 0.f) ? acc.w / d : 0.f;
-          const float a2 = (d > 0.f) ? vdot / (d * den * den) : 0.f;
-          gvec[p] = make_float4(a1 * gm.x + acc.x / den - a2 * gm.x,
-                                a1 * gm.y + acc.y / den - a2 * gm.y,
-                                a1 * gm.z + acc.z / den - a2 * gm.z, 0.f);
+          gvec[p] = pair_gradient(gm, acc);
         } else {
           pacc[p] = acc;
         }
@@ -1043,9 +1037,12 @@ __global__ void copy_f32_kernel(int n, const float* __restrict__ src, float* __r
   if (i < n) dst[i] = src[i];
 }
 
-// bf16 planes of W2 [3H][H] of every block (dense in the blob)
+// bf16 planes of W2 [3H][H] of every block (dense in the blob); also clears the
+// flag that the table kernels behind it raise
 __global__ void split_filter_weights_kernel(const float* __restrict__ w, ModelW mw,
-                                            uint16_t* __restrict__ wbf) {
+                                            uint16_t* __restrict__ wbf,
+                                            int32_t* __restrict__ tab_bad) {
+  if (tab_bad != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *tab_bad = 0;
   const int H = mw.H;
   const int64_t S = wbf_plane(H);
   const int64_t total = (int64_t)mw.L * S;
@@ -1068,6 +1065,10 @@ inline size_t nh(const Buffers& b) { return (size_t)b.N * b.H; }
 // unroll_fwd, unroll_bwd; each is the default or its alternative).
 template <int H>
 void launch_filter_fwd(const Buffers& b, hipStream_t st, int l) {
+  if (b.use_table) {
+    launch_filter_table_fwd<H>(b, st, l);
+    if (b.gate == nullptr) return;
+  }
   const ModelW& mw = *b.mw;
   const float* centers = b.w + mw.centers;
   const float* widths = b.w + mw.widths;
@@ -1076,17 +1077,23 @@ void launch_filter_fwd(const Buffers& b, hipStream_t st, int l) {
   if (b.tile_fwd == kFwdPairsAlt<H>) {
     constexpr int TM = kFwdPairsAlt<H>;
     filter_fwd_kernel<H, TM><<<pair_grid(b, TM), kPairBlock, 0, st>>>(
-        b.geom, b.counts, b.pcap, b.w, mw.layer[l], centers, widths, b.R, mw.RP, b.rc, Wl, w2);
+        b.geom, b.counts, b.pcap, b.w, mw.layer[l], centers, widths, b.R, mw.RP, b.rc, Wl, w2,
+        b.gate);
   } else {
     constexpr int TM = kFwdPairs<H>;
     filter_fwd_kernel<H, TM><<<pair_grid(b, TM), kPairBlock, 0, st>>>(
-        b.geom, b.counts, b.pcap, b.w, mw.layer[l], centers, widths, b.R, mw.RP, b.rc, Wl, w2);
+        b.geom, b.counts, b.pcap, b.w, mw.layer[l], centers, widths, b.R, mw.RP, b.rc, Wl, w2,
+        b.gate);
   }
 }
 
 template <int H>
 void launch_filter_bwd(const Buffers& b, hipStream_t st, int l, const float* gS1,
                        const float* gV1, int first, int last) {
+  if (b.use_table) {
+    launch_filter_table_bwd<H>(b, st, l, gS1, gV1, first, last);
+    if (b.gate == nullptr) return;
+  }
   const ModelW& mw = *b.mw;
   const float* centers = b.w + mw.centers;
   const float* widths = b.w + mw.widths;
@@ -1097,17 +1104,17 @@ void launch_filter_bwd(const Buffers& b, hipStream_t st, int l, const float* gS1
     constexpr int TM = kBwdPairsAlt<H>;
     filter_bwd_kernel<H, TM, false><<<pair_grid(b, TM), kPairBlock, 0, st>>>(
         b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, b.w, mw.layer[l], centers, widths, b.R,
-        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, b.pacc, b.gvec, first, last);
+        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, b.pacc, b.gvec, first, last, b.gate);
   } else if (b.bwd_variant == 1) {
     constexpr int TM = kBwdPairs<H>;
     filter_bwd_kernel<H, TM, true><<<pair_grid(b, TM), kPairBlock, 0, st>>>(
         b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, b.w, mw.layer[l], centers, widths, b.R,
-        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, b.pacc, b.gvec, first, last);
+        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, b.pacc, b.gvec, first, last, b.gate);
   } else {
     constexpr int TM = kBwdPairs<H>;
     filter_bwd_kernel<H, TM, false><<<pair_grid(b, TM), kPairBlock, 0, st>>>(
         b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, b.w, mw.layer[l], centers, widths, b.R,
-        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, b.pacc, b.gvec, first, last);
+        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, b.pacc, b.gvec, first, last, b.gate);
   }
 }
 
@@ -1305,21 +1312,12 @@ int alternative_shape(int H, int which) {
   }
 }
 
-hipError_t split_filter_weights(const Buffers& b) {
+hipError_t prepare_filters(const Buffers& b, hipStream_t s) {
   if (b.wbf == nullptr || b.L < 1) return hipSuccess;
-  // the weights may have just been written on another stream
-  hipError_t e = hipDeviceSynchronize();
-  if (e != hipSuccess) return e;
-  split_filter_weights_kernel<<<256, 256, 0, nullptr>>>(b.w, *b.mw, b.wbf);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return hipDeviceSynchronize();
-}
-
-hipError_t split_filter_weights_async(const Buffers& b, hipStream_t s) {
-  if (b.wbf == nullptr || b.L < 1) return hipSuccess;
-  split_filter_weights_kernel<<<256, 256, 0, s>>>(b.w, *b.mw, b.wbf);
-  return hipGetLastError();
+  split_filter_weights_kernel<<<256, 256, 0, s>>>(b.w, *b.mw, b.wbf, b.tab_bad);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess && b.tab != nullptr) e = build_tables(b, s);
+  return e;
 }
 
 hipError_t launch_stage(const Buffers& b, hipStream_t s, int stage, int layer) {

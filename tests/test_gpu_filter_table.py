@@ -1,0 +1,106 @@
+"""The filter's distance tables (csrc/filter_table.hip) on the GPU: distances
+at and around the knots and the cutoff, weights that the tables cannot follow,
+and the evaluations right after a weight change, against the FP64 oracle."""
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import pkg, pkg_mod
+from oracle import painn_ref as R
+
+pytestmark = pytest.mark.gpu
+
+
+def note(msg):
+    print(f"[case] {msg}", flush=True)
+
+
+def _model(H, L, R_, rc, bias=0.05):
+    torch.manual_seed(0)
+    m = pkg().StudentForceField(hidden_dim=H, num_interactions=L, num_rbf=R_, cutoff=rc)
+    with torch.no_grad():
+        for n, p in m.named_parameters():
+            if n.endswith(".bias"):
+                p.copy_(bias * torch.randn(p.shape))
+    return m.to("cuda:0")
+
+
+def _check(model, Z, P32, sizes, rc):
+    """Energies and forces against FP64: within three times what the same
+    algorithm's float32 on the CPU is off, plus 1e-6 of the largest value (the
+    float32 rounding of sums over a few neighbours)."""
+    e, f, _ = model.evaluate(torch.tensor(Z, device="cuda:0"), torch.tensor(P32, device="cuda:0"),
+                             np.asarray(sizes))
+    sd = {k: v.detach().cpu() for k, v in model.state_dict().items()}
+    b = np.repeat(np.arange(len(sizes)), sizes)
+    E, F = R.energy_and_forces(sd, Z, P32.astype(np.float64), rc, batch=b, n_structures=len(sizes))
+    E32, F32 = R.energy_and_forces(sd, Z, P32, rc, batch=b, n_structures=len(sizes),
+                                   dtype=torch.float32)
+    for got, want, ref in ((e.cpu(), E, E32), (f.cpu().double(), F, F32)):
+        tol = 3.0 * (ref.double() - want).abs().max() + 1e-6 * want.abs().max()
+        assert (got - want).abs().max() <= tol, ((got - want).abs().max(), tol)
+    return e, f
+
+
+@pytest.mark.parametrize("H,R_,rc", [(32, 16, 5.0), (64, 1, 5.0), (128, 20, 4.7), (64, 32, 6.0)])
+def test_dimers_at_knots_and_cutoff(gpu, H, R_, rc):
+    """Dimers along x (the distance is the float32 coordinate itself): at the
+    first and last knots, one ulp either side of knots, in the middle of
+    intervals, nearly coincident and within a few ulp of the cutoff."""
+    note(f"table dimers H{H} R{R_} rc {rc}")
+    h = np.float32(2.0 ** -9)
+    d = [h, 2 * h, 3 * h, np.float32(0.5) * h, np.float32(1e-4)]
+    for k in (0.5, 1.0, 1.25, 2.0, 3.0 + h):
+        x = np.float32(k)
+        d += [x, np.nextafter(x, np.float32(0)), np.nextafter(x, np.float32(9)), x + h / 2]
+    c = np.float32(rc)
+    for _ in range(3):
+        d.append(c)
+        c = np.nextafter(c, np.float32(0))
+    d += [np.float32(rc) - h, np.float32(rc) - h / 2, np.float32(rc) + h]
+    P = np.zeros((2 * len(d), 3), dtype=np.float32)
+    P[1::2, 0] = d
+    Z = np.tile([6, 1], len(d))
+    _check(_model(H, 2, R_, rc), Z, P, [2] * len(d), rc)
+
+
+@pytest.mark.parametrize("what", ["narrow", "steep", "one narrow"])
+def test_weights_beyond_the_tables(gpu, what):
+    """Basis widths below the knot spacing, or a first layer so steep that the
+    filter turns within an interval: the guard keeps the direct product."""
+    note(f"table guard: {what}")
+    m = _model(64, 2, 20, 5.0)
+    with torch.no_grad():
+        if what == "narrow":
+            m.rbf.widths.fill_(2.0 ** -10)
+        elif what == "one narrow":
+            m.rbf.widths[7] = 0.004
+        else:
+            m.interactions[1].message.rbf_to_scalar[0].weight.mul_(3e3)
+    mols = pkg_mod("synth").molecule_set(6, 5, 30, seed=9)
+    Z, P, ptr = pkg_mod("synth").flatten(mols)
+    _check(m, Z, P.astype(np.float32), np.diff(ptr), 5.0)
+
+
+@pytest.mark.parametrize("narrow", [False, True])
+def test_evaluations_after_a_weight_change(gpu, narrow):
+    """The first evaluation after a weight change launches both forms behind
+    the guard's flag, the next one the chosen form: same bits, and those of a
+    plan that was bound to the new weights."""
+    note(f"table refresh, narrow {narrow}")
+    m = _model(32, 2, 16, 5.0)
+    mols = pkg_mod("synth").molecule_set(5, 5, 40, seed=3)
+    Z, P, ptr = pkg_mod("synth").flatten(mols)
+    P32, sizes = P.astype(np.float32), np.diff(ptr)
+    before = _check(m, Z, P32, sizes, 5.0)
+    with torch.no_grad():
+        m.interactions[0].message.rbf_to_scalar[2].weight.mul_(1.1)
+        if narrow:
+            m.rbf.widths.mul_(0.02)
+    runs = [_check(m, Z, P32, sizes, 5.0) for _ in range(3)]
+    m._plans.clear()
+    runs.append(_check(m, Z, P32, sizes, 5.0))
+    assert not torch.equal(before[1], runs[0][1])
+    for e, f in runs[1:]:
+        assert torch.equal(e, runs[0][0]) and torch.equal(f, runs[0][1])
