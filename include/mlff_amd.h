@@ -277,7 +277,7 @@ int mlff_plan_set_blocks(mlff_plan* plan, int blocks);
  * message forward and adjoint.  0 keeps the default; each kind has one
  * pre-instantiated alternative (forward tile 64 or 32 for H >= 64, 128 or 64
  * for H = 32; adjoint tile 32 or 64 for H >= 64, 64 or 32 for H = 32;
- * message 5 or 3 and 4 or 2 edges), anything else is MLFF_ERR_UNSUPPORTED.
+ * message 8 or 4 edges each), anything else is MLFF_ERR_UNSUPPORTED.
  * bwd_variant (default adjoint tile only) picks the filter adjoint's form:
  * 0 as described above; 1 loads the pair indices of the next tile's gather
  * before the current tile's matrix products.

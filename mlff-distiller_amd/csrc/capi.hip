@@ -136,7 +136,7 @@ namespace {
 
 enum Seg {
   S_COUNTS, S_DEG, S_UDEG, S_ROWPTR, S_PAIRPTR, S_COL, S_EPAIR, S_PLO, S_PHI, S_PSHIFT, S_GEOM,
-  S_PACC, S_GVEC, S_WF, S_S, S_V, S_SMID, S_VMID, S_AUPD, S_G12, S_GS0, S_GV0, S_GS1, S_GV1,
+  S_UNIT,  S_PACC, S_GVEC, S_WF, S_S, S_V, S_SMID, S_VMID, S_AUPD, S_G12, S_GS0, S_GV0, S_GS1, S_GV1,
   S_EPS, S_VIR, S_GRID, S_CELLCNT, S_CELLSTART, S_CELLATOMS, S_ATOMCELL, S_TMPSHIFT, S_WBF,
   S_TABBAD, S_TAB,   // the tables last: the static entry keeps them elsewhere
   S_COUNT_
@@ -162,6 +162,7 @@ void carve(mlff_plan* pl) {
   // row 0 of the pair geometry and of the filter outputs
   const int64_t P1 = P > 0 ? P : 1;
   sz[S_GEOM] = 16 * P1;
+  sz[S_UNIT] = 16 * P1;
   sz[S_PACC] = 16 * P;
   sz[S_GVEC] = 16 * P;
   sz[S_WF] = 4 * L * P1 * 3 * H;
@@ -481,6 +482,7 @@ int bind_buffers(mlff_plan* pl, const char* who, void* ws, const float* weights_
   b.pair_hi = segp<int32_t>(pl, ws, S_PHI);
   b.pair_shift = segp<int32_t>(pl, ws, S_PSHIFT);
   b.geom = segp<float4>(pl, ws, S_GEOM);
+  b.unit = segp<float4>(pl, ws, S_UNIT);
   b.pacc = segp<float4>(pl, ws, S_PACC);
   b.gvec = segp<float4>(pl, ws, S_GVEC);
   b.Wf = segp<float>(pl, ws, S_WF);
@@ -512,6 +514,7 @@ int bind_buffers(mlff_plan* pl, const char* who, void* ws, const float* weights_
   a.edge_pair = segp<int32_t>(pl, ws, S_EPAIR); a.ecap = b.ecap;
   a.pair_lo = segp<int32_t>(pl, ws, S_PLO); a.pair_hi = segp<int32_t>(pl, ws, S_PHI);
   a.pair_shift = segp<int32_t>(pl, ws, S_PSHIFT); a.geom = segp<float4>(pl, ws, S_GEOM);
+  a.unit = segp<float4>(pl, ws, S_UNIT);
   a.pcap = b.pcap; a.counts = b.counts;
   a.grid = nullptr;   // brute force until mlff_plan_set_cell_grid
   a.n_cells = 0;
@@ -837,6 +840,7 @@ static int run_ef_on(mlff_plan* pl, hipStream_t s, double* energy, float* forces
   b.row_ptr = src.row_ptr; b.col = src.col; b.edge_pair = src.edge_pair;
   b.pair_lo = src.pair_lo; b.pair_hi = src.pair_hi; b.pair_shift = src.pair_shift;
   b.geom = src.geom;
+  b.unit = src.unit;
   e = launch_forward(b, s);
   if (e != hipSuccess) return hip_fail(e, "outer forward");
   e = launch_backward(b, s, forces, false);

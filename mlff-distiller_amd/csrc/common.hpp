@@ -8,6 +8,11 @@ namespace mlff {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 
+// fused multiply-add of a scalar or of four channels
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ f4 fma_(f4 a, f4 b, f4 c) { return __builtin_elementwise_fma(a, b, c); }
+__device__ __forceinline__ f4 fma_(float a, f4 b, f4 c) { return fma_(f4{a, a, a, a}, b, c); }
+
 constexpr int kWave = 64;
 constexpr float kPi = 3.14159265358979323846f;
 constexpr float kEdgeEps = 1e-8f;   // edge_vector / (d + 1e-8), student_model.py:715
@@ -262,7 +267,7 @@ __device__ __forceinline__ void mma_tile_x6(const uint16_t* __restrict__ A, int 
 
 // mma_tile_k with the k sub-steps of every slab split over two accumulator
 // sets (even and odd), added at the end: twice the independent MFMA chains
-// for tiles with few output blocks per wave.
+// for tiles with few output blocks per wave, and shorter rounding chains.
 template <int RT, int NT, int K, int PF = 2, bool PIN = false>
 __device__ __forceinline__ void mma_tile_k2(const float* __restrict__ A, int lda,
                                             const float* __restrict__ B, int ldb,

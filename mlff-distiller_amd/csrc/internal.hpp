@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "../../include/mlff_amd.h"
+#include "common.hpp"
 
 namespace mlff {
 
@@ -37,7 +38,7 @@ struct NLArgs {
   const float* cells; const uint8_t* pbc; float rc;
   int32_t* deg; int32_t* udeg; int32_t* row_ptr; int32_t* pair_ptr;
   int32_t* col; int32_t* edge_shift; int32_t* edge_pair; int32_t ecap;
-  int32_t* pair_lo; int32_t* pair_hi; int32_t* pair_shift; float4* geom; int32_t pcap;
+  int32_t* pair_lo; int32_t* pair_hi; int32_t* pair_shift; float4* geom; float4* unit; int32_t pcap;
   int32_t* counts;
   // cell list (periodic structures): grid[b] = {nc0, nc1, nc2, base}, nc0 == 0 -> brute force
   const int4* grid; int32_t n_cells;
@@ -83,10 +84,12 @@ __device__ __forceinline__ TableAt table_at(float d, float inv, int K) {
   const float t = x - (float)k, u = 1.f - t;
   return TableAt{k, t * t * (3.f - 2.f * t), t * u * u, -t * t * u};
 }
+// The fused operations are spelled out here and in the message terms, so that
+// every kernel that evaluates them gets the same bits.
 template <typename T>
 __device__ __forceinline__ T hermite(const TableAt& a, const T& f0, const T& g0, const T& f1,
                                      const T& g1) {
-  return f0 + (a.h01 * (f1 - f0) + (a.h10 * g0 + a.h11 * g1));
+  return f0 + fma_(a.h01, f1 - f0, fma_(a.h10, g0, a.h11 * g1));
 }
 
 // Model launches (painn_fwd.hip / painn_bwd.hip).
@@ -120,7 +123,8 @@ struct Buffers {
   int32_t* counts;
   const int32_t* row_ptr; const int32_t* col; const int32_t* edge_pair;
   const int32_t* pair_lo; const int32_t* pair_hi; const int32_t* pair_shift;
-  const float4* geom;
+  const float4* geom;               // {p_hi - p_lo, d}
+  const float4* unit;               // {(p_hi - p_lo) / (d + eps), d}
   float4* pacc;                     // per pair (gu.xyz, gd)
   float4* gvec;                     // per pair dE/dvec
   float* Wf;                        // [L][pcap][3H]

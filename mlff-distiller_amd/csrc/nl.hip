@@ -145,6 +145,17 @@ __device__ __forceinline__ void for_each_cell_candidate(const CellList& cl, int 
   }
 }
 
+// Geometry of pair p: {vec, d}, and {vec / (d + eps), d} for the message
+// kernels (one division per pair instead of one per lane, edge and block)
+__device__ __forceinline__ void store_pair(float4* __restrict__ geom, float4* __restrict__ unit,
+                                           int p, float vx, float vy, float vz, float d) {
+  geom[p] = make_float4(vx, vy, vz, d);
+  if (unit != nullptr) {
+    const float den = d + kEdgeEps;
+    unit[p] = make_float4(vx / den, vy / den, vz / den, d);
+  }
+}
+
 __device__ __forceinline__ int wave_inclusive_scan(int v) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
@@ -465,7 +476,8 @@ __global__ void nl_fill_kernel(const float* __restrict__ pos, int N,
                                int32_t* __restrict__ edge_shift, int32_t* __restrict__ edge_pair,
                                int32_t ecap, int32_t* __restrict__ pair_lo,
                                int32_t* __restrict__ pair_hi, int32_t* __restrict__ pair_shift,
-                               float4* __restrict__ geom, int32_t pcap, CellList cl,
+                               float4* __restrict__ geom, float4* __restrict__ unit,
+                               int32_t pcap, CellList cl,
                                int32_t* __restrict__ tmp_shift) {
   // one wave per atom, as the count pass
   __shared__ int4 hits_lds[(kNlBlock / 64) * kCellRowMax];
@@ -533,7 +545,7 @@ __global__ void nl_fill_kernel(const float* __restrict__ pos, int N,
           if (pair_shift) {
             pair_shift[3 * pk] = s0; pair_shift[3 * pk + 1] = s1; pair_shift[3 * pk + 2] = s2;
           }
-          geom[pk] = make_float4(vx, vy, vz, norm3_exact(vx, vy, vz));
+          store_pair(geom, unit, pk, vx, vy, vz, norm3_exact(vx, vy, vz));
         }
         if (edge_pair != nullptr && e_ok) edge_pair[ek] = (pk < pcap) ? pk : -1;
       }
@@ -591,7 +603,7 @@ __global__ void nl_fill_kernel(const float* __restrict__ pos, int N,
           if (pair_shift) {
             pair_shift[3 * p] = s0; pair_shift[3 * p + 1] = s1; pair_shift[3 * p + 2] = s2;
           }
-          geom[p] = make_float4(vx, vy, vz, norm3_exact(vx, vy, vz));
+          store_pair(geom, unit, p, vx, vy, vz, norm3_exact(vx, vy, vz));
         }
         if (edge_pair != nullptr) edge_pair[k] = (p < pcap) ? p : -1;
         ++p;
@@ -627,7 +639,7 @@ __global__ void nl_fill_kernel(const float* __restrict__ pos, int N,
           if (pair_shift) {
             pair_shift[3 * pk] = s0; pair_shift[3 * pk + 1] = s1; pair_shift[3 * pk + 2] = s2;
           }
-          geom[pk] = make_float4(vx, vy, vz, d);
+          store_pair(geom, unit, pk, vx, vy, vz, d);
         }
         if (edge_pair != nullptr && e_ok) edge_pair[ek] = (pk < pcap) ? pk : -1;
       }
@@ -702,7 +714,7 @@ hipError_t launch_neighbor_list(const NLArgs& a, hipStream_t s, bool build_pairs
                                   a.row_ptr, a.pair_ptr, a.col, a.edge_shift,
                                   build_pairs ? a.edge_pair : nullptr, a.ecap,
                                   build_pairs ? a.pair_lo : nullptr, a.pair_hi, a.pair_shift,
-                                  a.geom, a.pcap, cl, a.edge_tmp_shift);
+                                  a.geom, a.unit, a.pcap, cl, a.edge_tmp_shift);
   if (build_pairs) {
     nl_link_kernel<<<gw, kNlBlock, 0, s>>>(a.N, a.row_ptr, a.pair_ptr, a.col, a.edge_pair,
                                             a.ecap, a.pcap);

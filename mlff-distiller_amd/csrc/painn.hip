@@ -23,6 +23,8 @@
 //   force_gather receiver rows, forces and per-atom virial from dE/dvec
 //   reduce       per structure FP64 sums (energy, virial)
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -44,8 +46,8 @@ constexpr int kBwdPairs = H <= 32 ? 64 : 32;
 constexpr int kUpdWaves = 8;          // update kernels: waves per 32-atom tile
 constexpr int kUpdBlock = 64 * kUpdWaves;
 // edges in flight per row in the message kernels (forward, adjoint)
-constexpr int kMsgUnrollFwd = 5;
-constexpr int kMsgUnrollBwd = 4;
+constexpr int kMsgUnrollFwd = 8;
+constexpr int kMsgUnrollBwd = 8;
 // The other launch shape of each kernel, pre-instantiated so the launch-shape
 // tuner can choose per workload (mlff_plan_set_tiles).  Results are
 // bit-identical across shapes: every output element sums in the same order.
@@ -53,8 +55,8 @@ template <int H>
 constexpr int kFwdPairsAlt = H <= 32 ? 64 : 32;
 template <int H>
 constexpr int kBwdPairsAlt = H <= 32 ? 32 : 64;
-constexpr int kMsgUnrollFwdAlt = 3;
-constexpr int kMsgUnrollBwdAlt = 2;
+constexpr int kMsgUnrollFwdAlt = 4;
+constexpr int kMsgUnrollBwdAlt = 4;
 
 // Grid of a pair kernel: the plan's persistent grid, capped at the number of
 // tiles the pair capacity allows (a multiple of 8 for the XCD-interleaved tile
@@ -210,104 +212,103 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_fwd_kernel(
 // message (forward) and its node-gradient transpose (backward).
 // FWD:  s'_i = s_i + sum_j s_j * Ws_p ;  v'_i = v_i + sum_j v_j * Wv1_p + u_ji (x) Wv2_p
 // BWD:  gs_i = gs'_i + sum_j gs'_j * Ws_p ; gv_i = gv'_i + sum_j gv'_j * Wv1_p
-// One row per H/4 lanes, four channels (one float4) per lane; neighbours in
-// ascending j, a few edges' operands loaded before any is added.
+// One channel per lane, H lanes per row, neighbours in ascending j, added one
+// at a time; the operands of UNROLL edges are requested before any is added.
+// A wave works on one row (H >= 64), so a row's neighbour and pair indices and
+// unit vectors are scalar loads and the loop spends its vector registers on
+// operands in flight only.  Bound by reading every W_p once per direction
+// (HBM) on large batches, by the chain of load rounds per row on small ones.
+// Four channels per lane, five edges in flight, took 209 / 155 us (forward /
+// adjoint) for 256 molecules of 10-100 atoms at H = 128, 55 / 36 us for 1000
+// waters and 32 / 21 us for one molecule of 60 atoms; this form 180 / 144,
+// 47 / 32 and 10 / 7 us.  Twelve edges in flight: 180 / 143, 48 / 33, 12 / 7.
 // ---------------------------------------------------------------------------
 template <int H, bool FWD, int UNROLL>
 __global__ __launch_bounds__(kBlock) void message_kernel(
     int N, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col,
-    const int32_t* __restrict__ edge_pair, int32_t ecap, const float4* __restrict__ geom,
+    const int32_t* __restrict__ edge_pair, int32_t ecap, const float4* __restrict__ unit,
     const float* __restrict__ Wf, const float* __restrict__ s_in, const float* __restrict__ v_in,
     float* __restrict__ s_out, float* __restrict__ v_out) {
-  constexpr int LPR = H / 4;
-  constexpr int RPB = kBlock / LPR;
-  const int sub = threadIdx.x % LPR;
-  const int i = xcd_block() * RPB + threadIdx.x / LPR;
+  constexpr int RPB = kBlock / H;
+  const int c = threadIdx.x % H;
+  int i = xcd_block() * RPB + threadIdx.x / H;
+  if (H >= 64) i = __builtin_amdgcn_readfirstlane(i);   // uniform: indices in scalar registers
   if (i >= N) return;
-  const int c = 4 * sub;
-  f4 as = {0.f, 0.f, 0.f, 0.f}, a0 = as, a1 = as, a2 = as;
+  float as = 0.f, a0 = 0.f, a1 = 0.f, a2 = 0.f;
   const int e0 = min(row_ptr[i], ecap), e1 = min(row_ptr[i + 1], ecap);
-  // operands of one edge; kUnroll edges are loaded before any is accumulated
-  // (more loads in flight per row), and they are accumulated in edge order,
-  // so the sums round exactly as a one-edge-at-a-time loop
-  struct Edge {
-    f4 ws, wv1, wv2, sj, v0, v1, v2;
-    float ux, uy, uz;
-    bool on;
-  };
-  auto load = [&](int j, int p) {
-    Edge q;
-    q.on = p >= 0;
-    const int pc = q.on ? p : 0;
-    const float* wp = Wf + (size_t)pc * 3 * H + c;
-    const float* vj = v_in + (size_t)j * 3 * H + c;
-    q.ws = *reinterpret_cast<const f4*>(wp);
-    q.wv1 = *reinterpret_cast<const f4*>(wp + H);
-    q.sj = *reinterpret_cast<const f4*>(s_in + (size_t)j * H + c);
-    q.v0 = *reinterpret_cast<const f4*>(vj);
-    q.v1 = *reinterpret_cast<const f4*>(vj + H);
-    q.v2 = *reinterpret_cast<const f4*>(vj + 2 * H);
-    if (FWD) {
-      q.wv2 = *reinterpret_cast<const f4*>(wp + 2 * H);
-      const float4 gm = geom[pc];
-      const float den = gm.w + kEdgeEps;
-      // u_ji = (p_j - p_i)/(d + eps): +pair vector when j is the pair's hi atom
-      q.ux = gm.x / den; q.uy = gm.y / den; q.uz = gm.z / den;
-      if (j < i) { q.ux = -q.ux; q.uy = -q.uy; q.uz = -q.uz; }
-    }
-    return q;
-  };
-  auto accumulate = [&](const Edge& q) {
-    if (!q.on) return;
-    as += q.sj * q.ws;
-    a0 += q.v0 * q.wv1;
-    a1 += q.v1 * q.wv1;
-    a2 += q.v2 * q.wv1;
-    if (FWD) {
-      a0 += q.ux * q.wv2;
-      a1 += q.uy * q.wv2;
-      a2 += q.uz * q.wv2;
-    }
-  };
-  constexpr int kUnroll = UNROLL;
-  // The row's lanes load the neighbour and pair indices of a batch of
-  // kBatch edges together (one edge per lane), the next batch's while this
-  // one is processed; each group of kUnroll edges takes its indices from the
-  // row's lanes by shuffle, so its operand loads wait for no index load.
-  // Past the row's end, edges are switched off (p = -1).
-  constexpr int kBatch = (LPR / kUnroll) * kUnroll;
-  static_assert(kBatch >= kUnroll, "a batch holds at least one group");
-  const int rbase = (threadIdx.x & 63) - sub;   // the row's first lane in the wave
-  int jn = i, pn = -1;
-  if (sub < kBatch && e0 + sub < e1) { jn = col[e0 + sub]; pn = edge_pair[e0 + sub]; }
-  for (int bs = e0; bs < e1; bs += kBatch) {
-    const int jc = jn, pcur = pn;
-    jn = i; pn = -1;
-    if (sub < kBatch && bs + kBatch + sub < e1) {
-      jn = col[bs + kBatch + sub];
-      pn = edge_pair[bs + kBatch + sub];
-    }
-    const int nb = min(kBatch, e1 - bs);
-    for (int k = 0; k < nb; k += kUnroll) {
-      Edge q[kUnroll];
+  // neighbour and pair indices of the next step, requested a step ahead (past
+  // the row's end: the last edge's)
+  int jn[UNROLL], pn[UNROLL];
+  auto indices = [&](int e) {
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
-        q[u] = load(__shfl(jc, rbase + k + u, 64), __shfl(pcur, rbase + k + u, 64));
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) accumulate(q[u]);
+    for (int u = 0; u < UNROLL; ++u) {
+      const int ec = min(e + u, e1 - 1);
+      jn[u] = col[ec];
+      pn[u] = edge_pair[ec];
     }
-  }
+  };
+  // UNROLL edges from e on: all their operands are requested before any is
+  // used (the barrier keeps the compiler from moving loads behind the sums).
+  // TAIL: edges past the row's end count with zero weights.
+  auto step = [&](int e, auto tail) {
+    constexpr bool TAIL = decltype(tail)::value;
+    float ws[UNROLL], wv1[UNROLL], wv2[UNROLL], sj[UNROLL], v0[UNROLL], v1[UNROLL], v2[UNROLL];
+    float4 uu[UNROLL];
+    int jc[UNROLL];
+    bool on[UNROLL];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int p = max(pn[u], 0);
+      jc[u] = jn[u];
+      on[u] = (!TAIL || e + u < e1) && pn[u] >= 0;
+      const float* wp = Wf + (size_t)p * 3 * H;
+      const float* vj = v_in + (size_t)jc[u] * 3 * H;
+      ws[u] = wp[c];
+      wv1[u] = wp[H + c];
+      sj[u] = (s_in + (size_t)jc[u] * H)[c];
+      v0[u] = vj[c];
+      v1[u] = vj[H + c];
+      v2[u] = vj[2 * H + c];
+      if (FWD) {
+        wv2[u] = wp[2 * H + c];
+        uu[u] = unit[p];
+      }
+    }
+    if (!TAIL) indices(e + UNROLL);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const float w0 = on[u] ? ws[u] : 0.f, w1 = on[u] ? wv1[u] : 0.f;
+      as = fma_(sj[u], w0, as);
+      a0 = fma_(v0[u], w1, a0);
+      a1 = fma_(v1[u], w1, a1);
+      a2 = fma_(v2[u], w1, a2);
+      if (FWD) {
+        // u_ji = (p_j - p_i)/(d + eps): +pair vector when j is the pair's hi atom
+        const float w2 = on[u] ? (jc[u] < i ? -wv2[u] : wv2[u]) : 0.f;
+        a0 = fma_(uu[u].x, w2, a0);
+        a1 = fma_(uu[u].y, w2, a1);
+        a2 = fma_(uu[u].z, w2, a2);
+      }
+    }
+  };
+  if (e0 < e1) indices(e0);
+  int e = e0;
+  for (; e + UNROLL <= e1; e += UNROLL) step(e, std::false_type{});
+  if (e < e1) step(e, std::true_type{});
   const float* vi = v_in + (size_t)i * 3 * H + c;
   float* vo = v_out + (size_t)i * 3 * H + c;
-  *reinterpret_cast<f4*>(s_out + (size_t)i * H + c) =
-      *reinterpret_cast<const f4*>(s_in + (size_t)i * H + c) + as;
-  *reinterpret_cast<f4*>(vo) = *reinterpret_cast<const f4*>(vi) + a0;
-  *reinterpret_cast<f4*>(vo + H) = *reinterpret_cast<const f4*>(vi + H) + a1;
-  *reinterpret_cast<f4*>(vo + 2 * H) = *reinterpret_cast<const f4*>(vi + 2 * H) + a2;
+  s_out[(size_t)i * H + c] = s_in[(size_t)i * H + c] + as;
+  vo[0] = vi[0] + a0;
+  vo[H] = vi[H] + a1;
+  vo[2 * H] = vi[2 * H] + a2;
 }
 
 // ---------------------------------------------------------------------------
-// update forward, 32 atoms per tile
+// update forward, 32 atoms per tile.  The products run on two accumulator sets
+// (even and odd k sub-steps, mma_tile_k2): the energies of 12 molecules with
+// large biases are off by 3.1e-5 eV/atom rms that way, 4.7e-5 with one set,
+// in the same time.
 // ---------------------------------------------------------------------------
 template <int H>
 __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
@@ -353,7 +354,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
 #pragma unroll
     for (int ct = 0; ct < NT1; ++ct) cb[ct] = (wave * NT1 + ct) * 16;
     zero_acc(acc);
-    mma_tile_k<RT, NT1, 2 * H>(x_lds, LDX, w + lw.u1w, 2 * H, cb, acc);
+    mma_tile_k2<RT, NT1, 2 * H>(x_lds, LDX, w + lw.u1w, 2 * H, cb, acc);
     const float* b1 = w + lw.u1b;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
         }
     }
     zero_acc(acc);
-    mma_tile_k<RT, NT2, H>(h_lds, LDH, w + lw.u2w, H, cb, acc);
+    mma_tile_k2<RT, NT2, H>(h_lds, LDH, w + lw.u2w, H, cb, acc);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -466,7 +467,7 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
     int cb[1] = {wave * 16};
     f4 acc[RT][1];
     zero_acc(acc);
-    mma_tile_k<RT, 1, H>(x_lds, LDX, w + mw.r1w, H, cb, acc);
+    mma_tile_k2<RT, 1, H>(x_lds, LDX, w + mw.r1w, H, cb, acc);
     const int c = cb[0] + r;
     const float bias = w[mw.r1b + c];
 #pragma unroll
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
     int cb[1] = {wave * 16};
     f4 acc[RT][1];
     zero_acc(acc);
-    mma_tile_k<RT, 1, HP2>(h1_lds, LD2, w + mw.r2w, HP2, cb, acc);
+    mma_tile_k2<RT, 1, HP2>(h1_lds, LD2, w + mw.r2w, HP2, cb, acc);
     const int c = cb[0] + r;
     const float bias = w[mw.r2b + c];
 #pragma unroll
@@ -509,7 +510,7 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
     int cb[1] = {wave * 16};
     f4 acc[RT][1];
     zero_acc(acc);
-    mma_tile_k<RT, 1, HP4>(g2_lds, LD4, w + mw.r2t, HP4, cb, acc);
+    mma_tile_k2<RT, 1, HP4>(g2_lds, LD4, w + mw.r2t, HP4, cb, acc);
     const int c = cb[0] + r;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
 #pragma unroll
       for (int ct = 0; ct < NT; ++ct) cb[ct] = (wave * NT + ct) * 16;
       zero_acc(acc);
-      mma_tile_k<RT, NT, HP2>(h1_lds, LD2, w + mw.r1t, HP2, cb, acc);
+      mma_tile_k2<RT, NT, HP2>(h1_lds, LD2, w + mw.r1t, HP2, cb, acc);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -616,7 +617,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_bwd_kernel(
             av[rt][ct][k] = a_upd[(size_t)i * H + cb[ct] + r];
           }
       zero_acc(acc);
-      mma_tile_k<RT, NT, 3 * H, 2, true>(y_lds, LDY, w + lw.u2t, 3 * H, cb, acc);
+      mma_tile_k2<RT, NT, 3 * H, 2, true>(y_lds, LDY, w + lw.u2t, 3 * H, cb, acc);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -639,7 +640,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_bwd_kernel(
 #pragma unroll
       for (int ct = 0; ct < NT; ++ct) cb[ct] = (wave * NT + ct) * 16;
       zero_acc(acc);
-      mma_tile_k<RT, NT, H, 2, true>(a_lds, LDA, w + lw.u1t, H, cb, acc);
+      mma_tile_k2<RT, NT, H, 2, true>(a_lds, LDA, w + lw.u1t, H, cb, acc);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -1125,11 +1126,11 @@ void launch_message(const Buffers& b, hipStream_t st, int grid, const float* Wl,
   constexpr int U1 = FWD ? kMsgUnrollFwdAlt : kMsgUnrollBwdAlt;
   if ((FWD ? b.unroll_fwd : b.unroll_bwd) == U1)
     message_kernel<H, FWD, U1><<<grid, kBlock, 0, st>>>(b.N, b.row_ptr, b.col, b.edge_pair,
-                                                        b.ecap, b.geom, Wl, s_in, v_in, s_out,
+                                                        b.ecap, b.unit, Wl, s_in, v_in, s_out,
                                                         v_out);
   else
     message_kernel<H, FWD, U0><<<grid, kBlock, 0, st>>>(b.N, b.row_ptr, b.col, b.edge_pair,
-                                                        b.ecap, b.geom, Wl, s_in, v_in, s_out,
+                                                        b.ecap, b.unit, Wl, s_in, v_in, s_out,
                                                         v_out);
 }
 
@@ -1169,7 +1170,7 @@ hipError_t forward_impl(const Buffers& b, hipStream_t s) {
     embed_kernel<H><<<(unsigned)((total + kBlock - 1) / kBlock), kBlock, 0, s>>>(
         N, b.numbers, b.w + mw.emb, b.S, b.V);
   }
-  const int rows_per_block = kBlock / (H / 4);
+  const int rows_per_block = kBlock / H;
   const int msg_grid = ((N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
   const int atom_grid = (N + 31) / 32;
   for (int l = 0; l < b.L; ++l) {
@@ -1197,7 +1198,7 @@ hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool wa
   const int N = b.N;
   const float* centers = b.w + mw.centers;
   const float* widths = b.w + mw.widths;
-  const int rows_per_block = kBlock / (H / 4);
+  const int rows_per_block = kBlock / H;
   const int msg_grid = ((N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
   const int atom_grid = (N + 31) / 32;
   Streams st(b, s);
@@ -1237,7 +1238,7 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
   const int N = b.N;
   const float* centers = b.w + mw.centers;
   const float* widths = b.w + mw.widths;
-  const int rows_per_block = kBlock / (H / 4);
+  const int rows_per_block = kBlock / H;
   const int msg_grid = ((N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
   const int atom_grid = (N + 31) / 32;
   const LayerW& lw = mw.layer[l];

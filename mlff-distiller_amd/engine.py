@@ -243,7 +243,7 @@ def launch_shapes(H: int):
     adjoint's variant (0 plain, 1 next-tile index prefetch; default adjoint
     tile only) (mlff_plan_set_tiles)."""
     small = H <= 32
-    return ((128, 64) if small else (64, 32), (64, 32) if small else (32, 64), (5, 3), (4, 2),
+    return ((128, 64) if small else (64, 32), (64, 32) if small else (32, 64), (8, 4), (8, 4),
             (0, 1))
 
 
