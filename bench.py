@@ -562,7 +562,7 @@ def main():
     ap.add_argument("--stage-reps", type=int, default=20)
     ap.add_argument("--blocks", type=int, default=0,
                     help="persistent grid of the pair kernels (0: autotune)")
-    ap.add_argument("--streams", type=int, default=2, choices=[1, 2],
+    ap.add_argument("--streams", type=int, default=1, choices=[1, 2],
                     help="2: pair filter kernels on a second stream beside the atom-side kernels")
     ap.add_argument("--copy-probe", type=int, default=0,
                     help="MiB copied by a plain device copy at the end (byte-counter calibration)")

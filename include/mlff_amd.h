@@ -286,11 +286,12 @@ int mlff_plan_set_blocks(mlff_plan* plan, int blocks);
 int mlff_plan_set_tiles(mlff_plan* plan, int fwd_pairs, int bwd_pairs, int msg_unroll_fwd,
                         int msg_unroll_bwd, int bwd_variant);
 
-/* Number of streams one evaluation uses: 2 (default) runs the pair filter
- * kernels on a stream of the plan's own, forked from and joined back into the
- * caller's stream with events, so they overlap the atom-side kernels; 1 keeps
- * every kernel on the caller's stream.  Results are bit-identical either way.
- * The filter stream is created on the device current at mlff_plan_bind. */
+/* Number of streams one evaluation uses: 1 (default) keeps every kernel on the
+ * caller's stream; 2 runs the pair filter kernels on a stream of the plan's
+ * own, forked from and joined back into the caller's stream with events, so
+ * they overlap the atom-side kernels.  Results are bit-identical either way.
+ * The filter stream is created on the device current at mlff_plan_bind or at
+ * this call. */
 int mlff_plan_set_streams(mlff_plan* plan, int n_streams);
 
 /* ---------------------------------------------------------------------------

@@ -38,7 +38,7 @@ def _key(plan) -> str:
     name = torch.cuda.get_device_name(0) if torch.cuda.is_available() else "cpu"
     counts = plan.read_counts()
     pairs = max(int(counts[C.MLFF_COUNT_PAIRS]), 1)
-    streams = getattr(plan, "streams", 2)
+    streams = getattr(plan, "streams", 1)
     return f"{name}|H{plan.H}|L{plan.L}|S{streams}|P2^{int(math.log2(pairs))}"
 
 

@@ -427,7 +427,11 @@ int mlff_plan_create(mlff_plan** out, const mlff_config* cfg) {
   carve(pl);
   pl->buf.blocks = persistent_grid(cfg->persistent_blocks, -1);
   set_default_shapes(pl);
-  pl->n_streams = 2;
+  // one stream: with the filter tables the pair kernels are short and bound by
+  // memory like the atom-side ones, and the fork and join events cost more than
+  // the overlap gives (256 molecules 2.41 ms on two streams, 2.30 on one; an MD
+  // step of one 60-atom molecule 298 and 245 us)
+  pl->n_streams = 1;
   pl->stream_dev = -1;
   *out = pl;
   return MLFF_OK;

@@ -233,7 +233,7 @@ def edge_capacity_bound(sizes: Sequence[int], periodic: bool, max_neighbors: int
 # ---------------------------------------------------------------------------
 
 # streams per evaluation for new plans (Plan.set_streams)
-DEFAULT_STREAMS = 2
+DEFAULT_STREAMS = 1
 
 
 def launch_shapes(H: int):
@@ -287,7 +287,7 @@ class Plan:
         self.counts = self.workspace[off:off + 4 * C.MLFF_COUNT_SLOTS].view(torch.int32)
         self._apply_cell_grid()
         self.streams = int(streams if streams is not None else DEFAULT_STREAMS)
-        if self.streams != 2:
+        if self.streams != 1:
             self.set_streams(self.streams)
         self.tiles = default_tiles(H)
         if tiles is not None:
@@ -324,7 +324,7 @@ class Plan:
             C.ptr(forces), C.ptr(virial), C.ptr(atom_energy)))
 
     def set_streams(self, n_streams: int):
-        """1: every kernel on the caller's stream; 2 (default): the pair filter
+        """1 (default): every kernel on the caller's stream; 2: the pair filter
         kernels on a second stream of the plan's own, overlapping the
         atom-side kernels.  Bit-identical results either way."""
         C.check("mlff_plan_set_streams", self.lib.mlff_plan_set_streams(self.handle, int(n_streams)))
