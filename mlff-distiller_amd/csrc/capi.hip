@@ -137,7 +137,7 @@ namespace {
 enum Seg {
   S_COUNTS, S_DEG, S_UDEG, S_ROWPTR, S_PAIRPTR, S_COL, S_EPAIR, S_PLO, S_PHI, S_PSHIFT, S_GEOM,
   S_UNIT,  S_PACC, S_GVEC, S_WF, S_S, S_V, S_SMID, S_VMID, S_AUPD, S_G12, S_GS0, S_GV0, S_GS1, S_GV1,
-  S_EPS, S_VIR, S_GRID, S_CELLCNT, S_CELLSTART, S_CELLATOMS, S_ATOMCELL, S_TMPSHIFT, S_WBF,
+  S_GA, S_EPS, S_VIR, S_GRID, S_CELLCNT, S_CELLSTART, S_CELLATOMS, S_ATOMCELL, S_TMPSHIFT, S_WBF,
   S_TABBAD, S_TAB,   // the tables last: the static entry keeps them elsewhere
   S_COUNT_
 };
@@ -176,6 +176,7 @@ void carve(mlff_plan* pl) {
   sz[S_GV0] = 4 * N * 3 * H;
   sz[S_GS1] = 4 * L * N * H;
   sz[S_GV1] = 4 * L * N * 3 * H;
+  sz[S_GA] = 4 * N * H;
   sz[S_EPS] = 4 * N;
   sz[S_VIR] = 4 * 9 * N;
   const int64_t CC = c.cell_capacity > 0 ? c.cell_capacity : 0;
@@ -500,6 +501,7 @@ int bind_buffers(mlff_plan* pl, const char* who, void* ws, const float* weights_
   b.gV0 = segp<float>(pl, ws, S_GV0);
   b.gS1 = segp<float>(pl, ws, S_GS1);
   b.gV1 = segp<float>(pl, ws, S_GV1);
+  b.gA = segp<float>(pl, ws, S_GA);
   b.eps = segp<float>(pl, ws, S_EPS);
   b.vir_atom = segp<float>(pl, ws, S_VIR);
   b.wbf = segp<uint16_t>(pl, ws, S_WBF);

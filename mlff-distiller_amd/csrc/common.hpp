@@ -38,7 +38,7 @@ __device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
 // d/dx [x sigmoid(x)] = s (1 + x (1 - s))
 __device__ __forceinline__ float silu_grad(float x) {
   const float s = 1.0f / (1.0f + expf(-x));
-  return s * (1.0f + x * (1.0f - s));
+  return s * fma_(x, 1.0f - s, 1.0f);
 }
 
 // Gaussian RBF x cosine cutoff (student_model.py:249-253, 285-290, 720-722),
@@ -265,11 +265,42 @@ __device__ __forceinline__ void mma_tile_x6(const uint16_t* __restrict__ A, int 
   }
 }
 
-// mma_tile_k with the k sub-steps of every slab split over two accumulator
-// sets (even and odd), added at the end: twice the independent MFMA chains
-// for tiles with few output blocks per wave, and shorter rounding chains.
+// The four k sub-steps of every slab on accumulators of their own, added
+// pairwise at the end: four independent MFMA chains for tiles with few output
+// blocks per wave, and rounding chains a quarter as long.
+template <int RT, int NT>
+struct Acc4 {
+  f4 v[4][RT][NT];
+  __device__ __forceinline__ Acc4() {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) v[s][rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
+  }
+  __device__ __forceinline__ void slab(const f4 (&a)[RT], const f4 (&b)[NT]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct)
+          v[s][rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][s], b[ct][s], v[s][rt][ct], 0,
+                                                              0, 0);
+  }
+  __device__ __forceinline__ void add_to(f4 (&acc)[RT][NT]) const {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct)
+        acc[rt][ct] += (v[0][rt][ct] + v[1][rt][ct]) + (v[2][rt][ct] + v[3][rt][ct]);
+  }
+};
+
+// mma_tile_k on those accumulators
 template <int RT, int NT, int K, int PF = 2, bool PIN = false>
-__device__ __forceinline__ void mma_tile_k2(const float* __restrict__ A, int lda,
+__device__ __forceinline__ void mma_tile_k4(const float* __restrict__ A, int lda,
                                             const float* __restrict__ B, int ldb,
                                             const int (&cb)[NT], f4 (&acc)[RT][NT]) {
   static_assert(K % 16 == 0, "K must be a multiple of 16");
@@ -281,11 +312,7 @@ __device__ __forceinline__ void mma_tile_k2(const float* __restrict__ A, int lda
   int boff[NT];
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct) boff[ct] = (cb[ct] + r) * ldb + 4 * g;
-  f4 odd[RT][NT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int ct = 0; ct < NT; ++ct) odd[rt][ct] = f4{0.f, 0.f, 0.f, 0.f};
+  Acc4<RT, NT> sum;
   f4 b[PF + 1][NT];
 #pragma unroll
   for (int q = 0; q < PF; ++q)
@@ -304,23 +331,43 @@ __device__ __forceinline__ void mma_tile_k2(const float* __restrict__ A, int lda
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
       a[rt] = *reinterpret_cast<const f4*>(arow + rt * 16 * lda + 16 * sl);
-    const int cur = sl % (PF + 1);
-#pragma unroll
-    for (int s = 0; s < 4; s += 2)
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-          acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][s], b[cur][ct][s], acc[rt][ct],
-                                                             0, 0, 0);
-          odd[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][s + 1], b[cur][ct][s + 1],
-                                                             odd[rt][ct], 0, 0, 0);
-        }
+    sum.slab(a, b[sl % (PF + 1)]);
   }
+  sum.add_to(acc);
+}
+
+// mma_tile_k4 with the whole weight operand in registers: load_weights requests
+// it (long before its use, where a tile's latency is what counts), mma_regs
+// multiplies.  The sums are those of mma_tile_k4, bit for bit.
+template <int NT, int K>
+struct Weights {
+  f4 b[K / 16][NT];
+};
+template <int NT, int K>
+__device__ __forceinline__ void load_weights(const float* __restrict__ B, int ldb,
+                                             const int (&cb)[NT], Weights<NT, K>& w) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
+  for (int q = 0; q < K / 16; ++q)
 #pragma unroll
-    for (int ct = 0; ct < NT; ++ct) acc[rt][ct] += odd[rt][ct];
+    for (int ct = 0; ct < NT; ++ct)
+      w.b[q][ct] = *reinterpret_cast<const f4*>(B + (cb[ct] + r) * ldb + 4 * g + 16 * q);
+}
+template <int RT, int NT, int K>
+__device__ __forceinline__ void mma_regs(const float* __restrict__ A, int lda,
+                                         const Weights<NT, K>& w, f4 (&acc)[RT][NT]) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const float* arow = A + r * lda + 4 * g;
+  Acc4<RT, NT> sum;
+#pragma unroll
+  for (int sl = 0; sl < K / 16; ++sl) {
+    f4 a[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      a[rt] = *reinterpret_cast<const f4*>(arow + rt * 16 * lda + 16 * sl);
+    sum.slab(a, w.b[sl]);
+  }
+  sum.add_to(acc);
 }
 
 template <int RT, int NT>

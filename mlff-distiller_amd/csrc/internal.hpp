@@ -133,6 +133,7 @@ struct Buffers {
   float* Aupd; float* G12;          // [L][N][H], [L][N][2H]
   float* gS0; float* gV0;           // gradient w.r.t. the update outputs of the block below
   float* gS1; float* gV1;           // [L][N][H], [L][N][3][H]: gradient w.r.t. message outputs
+  float* gA;                        // [N][H]: hidden gradient of the split update adjoint
   float* eps;                       // [N]
   float* vir_atom;                  // [N][9]
   // second stream for the filter kernels (overlaps the memory-bound message

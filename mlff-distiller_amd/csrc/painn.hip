@@ -45,6 +45,12 @@ template <int H>
 constexpr int kBwdPairs = H <= 32 ? 64 : 32;
 constexpr int kUpdWaves = 8;          // update kernels: waves per 32-atom tile
 constexpr int kUpdBlock = 64 * kUpdWaves;
+// Atoms up to which the update blocks run split over columns, and the readout on
+// 16-atom tiles.  H = 128, forward + adjoint of a block: 60 atoms 24 us split,
+// 34 us whole (33 with 16-atom tiles); 3000 atoms 42 us split, 41 us whole.
+// Readout: 14 -> 7 us at 60 atoms, 15 -> 9 us at 3000.
+constexpr int kSplitAtoms = 1024;
+constexpr int kReadoutSmallAtoms = 4096;
 // edges in flight per row in the message kernels (forward, adjoint)
 constexpr int kMsgUnrollFwd = 8;
 constexpr int kMsgUnrollBwd = 8;
@@ -212,8 +218,9 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_fwd_kernel(
 // message (forward) and its node-gradient transpose (backward).
 // FWD:  s'_i = s_i + sum_j s_j * Ws_p ;  v'_i = v_i + sum_j v_j * Wv1_p + u_ji (x) Wv2_p
 // BWD:  gs_i = gs'_i + sum_j gs'_j * Ws_p ; gv_i = gv'_i + sum_j gv'_j * Wv1_p
-// One channel per lane, H lanes per row, neighbours in ascending j, added one
-// at a time; the operands of UNROLL edges are requested before any is added.
+// One channel per lane, H lanes per row, neighbours in ascending j; the operands
+// of UNROLL edges are requested before any is added.  Even and odd
+// edges have sums of their own (shorter rounding chains).
 // A wave works on one row (H >= 64), so a row's neighbour and pair indices and
 // unit vectors are scalar loads and the loop spends its vector registers on
 // operands in flight only.  Bound by reading every W_p once per direction
@@ -234,7 +241,7 @@ __global__ __launch_bounds__(kBlock) void message_kernel(
   int i = xcd_block() * RPB + threadIdx.x / H;
   if (H >= 64) i = __builtin_amdgcn_readfirstlane(i);   // uniform: indices in scalar registers
   if (i >= N) return;
-  float as = 0.f, a0 = 0.f, a1 = 0.f, a2 = 0.f;
+  float as[2] = {0.f, 0.f}, a0[2] = {0.f, 0.f}, a1[2] = {0.f, 0.f}, a2[2] = {0.f, 0.f};
   const int e0 = min(row_ptr[i], ecap), e1 = min(row_ptr[i + 1], ecap);
   // neighbour and pair indices of the next step, requested a step ahead (past
   // the row's end: the last edge's)
@@ -279,16 +286,17 @@ __global__ __launch_bounds__(kBlock) void message_kernel(
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       const float w0 = on[u] ? ws[u] : 0.f, w1 = on[u] ? wv1[u] : 0.f;
-      as = fma_(sj[u], w0, as);
-      a0 = fma_(v0[u], w1, a0);
-      a1 = fma_(v1[u], w1, a1);
-      a2 = fma_(v2[u], w1, a2);
+      const int o = u & 1;   // UNROLL is even: the edge's parity in its row
+      as[o] = fma_(sj[u], w0, as[o]);
+      a0[o] = fma_(v0[u], w1, a0[o]);
+      a1[o] = fma_(v1[u], w1, a1[o]);
+      a2[o] = fma_(v2[u], w1, a2[o]);
       if (FWD) {
         // u_ji = (p_j - p_i)/(d + eps): +pair vector when j is the pair's hi atom
         const float w2 = on[u] ? (jc[u] < i ? -wv2[u] : wv2[u]) : 0.f;
-        a0 = fma_(uu[u].x, w2, a0);
-        a1 = fma_(uu[u].y, w2, a1);
-        a2 = fma_(uu[u].z, w2, a2);
+        a0[o] = fma_(uu[u].x, w2, a0[o]);
+        a1[o] = fma_(uu[u].y, w2, a1[o]);
+        a2[o] = fma_(uu[u].z, w2, a2[o]);
       }
     }
   };
@@ -298,17 +306,23 @@ __global__ __launch_bounds__(kBlock) void message_kernel(
   if (e < e1) step(e, std::true_type{});
   const float* vi = v_in + (size_t)i * 3 * H + c;
   float* vo = v_out + (size_t)i * 3 * H + c;
-  s_out[(size_t)i * H + c] = s_in[(size_t)i * H + c] + as;
-  vo[0] = vi[0] + a0;
-  vo[H] = vi[H] + a1;
-  vo[2 * H] = vi[2 * H] + a2;
+  s_out[(size_t)i * H + c] = s_in[(size_t)i * H + c] + (as[0] + as[1]);
+  vo[0] = vi[0] + (a0[0] + a0[1]);
+  vo[H] = vi[H] + (a1[0] + a1[1]);
+  vo[2 * H] = vi[2 * H] + (a2[0] + a2[1]);
+}
+
+// a . b in x order, with the fused operations spelled out: every tile shape of a
+// kernel gets the same bits
+__device__ __forceinline__ float dot3(float a0, float a1, float a2, float b0, float b1, float b2) {
+  return fma_(a2, b2, fma_(a1, b1, a0 * b0));
 }
 
 // ---------------------------------------------------------------------------
-// update forward, 32 atoms per tile.  The products run on two accumulator sets
-// (even and odd k sub-steps, mma_tile_k2): the energies of 12 molecules with
-// large biases are off by 3.1e-5 eV/atom rms that way, 4.7e-5 with one set,
-// in the same time.
+// update forward, 32 atoms per tile.  The products run on four accumulator sets
+// (mma_tile_k4): on one set they are the largest part of an energy's error
+// (molecules with large biases: 4.7e-5 eV/atom rms with one set, 3.1e-5 with
+// two, 2.3e-5 with four, in the same time).
 // ---------------------------------------------------------------------------
 template <int H>
 __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
@@ -354,7 +368,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
 #pragma unroll
     for (int ct = 0; ct < NT1; ++ct) cb[ct] = (wave * NT1 + ct) * 16;
     zero_acc(acc);
-    mma_tile_k2<RT, NT1, 2 * H>(x_lds, LDX, w + lw.u1w, 2 * H, cb, acc);
+    mma_tile_k4<RT, NT1, 2 * H>(x_lds, LDX, w + lw.u1w, 2 * H, cb, acc);
     const float* b1 = w + lw.u1b;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -403,7 +417,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
         }
     }
     zero_acc(acc);
-    mma_tile_k2<RT, NT2, H>(h_lds, LDH, w + lw.u2w, H, cb, acc);
+    mma_tile_k4<RT, NT2, H>(h_lds, LDH, w + lw.u2w, H, cb, acc);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -419,9 +433,9 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
           s_out[(size_t)i * H + c] = x_lds[m * LDX + c] + ds;
           const float x0 = xv[rt][q][k][0], x1 = xv[rt][q][k][1], x2 = xv[rt][q][k][2];
           float* vo = v_out + (size_t)i * 3 * H;
-          vo[c] = x0 * gt1 + (u[0] * x0 + u[1] * x1 + u[2] * x2) * gt2;
-          vo[H + c] = x1 * gt1 + (u[3] * x0 + u[4] * x1 + u[5] * x2) * gt2;
-          vo[2 * H + c] = x2 * gt1 + (u[6] * x0 + u[7] * x1 + u[8] * x2) * gt2;
+          vo[c] = fma_(dot3(u[0], u[1], u[2], x0, x1, x2), gt2, x0 * gt1);
+          vo[H + c] = fma_(dot3(u[3], u[4], u[5], x0, x1, x2), gt2, x1 * gt1);
+          vo[2 * H + c] = fma_(dot3(u[6], u[7], u[8], x0, x1, x2), gt2, x2 * gt1);
           g12[(size_t)i * 2 * H + c] = gt1;
           g12[(size_t)i * 2 * H + H + c] = gt2;
         }
@@ -432,12 +446,13 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
 // ---------------------------------------------------------------------------
 // readout: eps_i = head(s_i) and gs_i = d eps_i / d s_i, 32 atoms per tile
 // ---------------------------------------------------------------------------
-template <int H>
+template <int H, int TM>
 __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __restrict__ w,
                                                          ModelW mw, const float* __restrict__ sL,
                                                          float* __restrict__ eps,
                                                          float* __restrict__ gS) {
-  constexpr int TM = 32, RT = 2;
+  constexpr int RT = TM / 16;
+  constexpr bool kRegs = TM == 16;
   constexpr int HP2 = ((H / 2) + 15) & ~15, HP4 = ((H / 4) + 15) & ~15;
   constexpr int LDX = H + 4, LD2 = HP2 + 4, LD4 = HP4 + 4;
   __shared__ __align__(16) float x_lds[TM * LDX];
@@ -447,6 +462,21 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
   __shared__ __align__(16) float g2_lds[TM * LD4];
   const int base = blockIdx.x * TM;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  // a wave's column tile of the two hidden layers, and its tiles of the input
+  // gradient (waves past the last repeat the first's loads, unused)
+  constexpr int CTG = H / 16, NTG = (CTG + 3) / 4;
+  int c2[1] = {wave < HP2 / 16 ? wave * 16 : 0}, c4[1] = {wave < HP4 / 16 ? wave * 16 : 0},
+      cg[NTG];
+#pragma unroll
+  for (int ct = 0; ct < NTG; ++ct) cg[ct] = (wave < CTG / NTG ? wave * NTG + ct : ct) * 16;
+  Weights<1, H> wr1;
+  Weights<1, HP2> wr2;
+  Weights<1, HP4> wr2t;
+  Weights<NTG, HP2> wr1t;
+  if (kRegs) {
+    load_weights(w + mw.r1w, H, c2, wr1);
+    load_weights(w + mw.r2w, HP2, c4, wr2);
+  }
   {
     constexpr int PER = TM * H / kBlock;
     static_assert(PER * kBlock == TM * H, "tile split");
@@ -456,6 +486,10 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
       const int idx = threadIdx.x + k * kBlock, m = idx / H, c = idx % H;
       xs[k] = sL[(size_t)min(base + m, N - 1) * H + c];
     }
+    if (kRegs) {
+      load_weights(w + mw.r2t, HP4, c2, wr2t);
+      load_weights(w + mw.r1t, HP2, cg, wr1t);
+    }
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int idx = threadIdx.x + k * kBlock, m = idx / H, c = idx % H;
@@ -464,11 +498,11 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
   }
   __syncthreads();
   if (wave < HP2 / 16) {   // Linear(H, H/2) + SiLU, one column tile per wave
-    int cb[1] = {wave * 16};
     f4 acc[RT][1];
     zero_acc(acc);
-    mma_tile_k2<RT, 1, H>(x_lds, LDX, w + mw.r1w, H, cb, acc);
-    const int c = cb[0] + r;
+    if constexpr (kRegs) mma_regs(x_lds, LDX, wr1, acc);
+    else mma_tile_k4<RT, 1, H>(x_lds, LDX, w + mw.r1w, H, c2, acc);
+    const int c = c2[0] + r;
     const float bias = w[mw.r1b + c];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -482,11 +516,11 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
   }
   __syncthreads();
   if (wave < HP4 / 16) {   // Linear(H/2, H/4)
-    int cb[1] = {wave * 16};
     f4 acc[RT][1];
     zero_acc(acc);
-    mma_tile_k2<RT, 1, HP2>(h1_lds, LD2, w + mw.r2w, HP2, cb, acc);
-    const int c = cb[0] + r;
+    if constexpr (kRegs) mma_regs(h1_lds, LD2, wr2, acc);
+    else mma_tile_k4<RT, 1, HP2>(h1_lds, LD2, w + mw.r2w, HP2, c4, acc);
+    const int c = c4[0] + r;
     const float bias = w[mw.r2b + c];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -495,23 +529,28 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
   }
   __syncthreads();
   const float* w3 = w + mw.r3w;
-  if (threadIdx.x < TM) {   // Linear(H/4, 1), its input gradient, and SiLU'
-    const int m = threadIdx.x, i = base + m;
+  // Linear(H/4, 1), its input gradient, and SiLU': eight lanes per atom, a run
+  // of HP4 / 8 channels each
+  if (threadIdx.x < TM * 8) {
+    constexpr int RUN = HP4 / 8;
+    const int m = threadIdx.x / 8, c0 = (threadIdx.x % 8) * RUN, i = base + m;
     float e = 0.f;
-    for (int c = 0; c < HP4; ++c) {
-      const float a = a2_lds[m * LD4 + c];
-      e += silu(a) * w3[c];
-      g2_lds[m * LD4 + c] = w3[c] * silu_grad(a);
+#pragma unroll
+    for (int k = 0; k < RUN; ++k) {
+      const float a = a2_lds[m * LD4 + c0 + k], q = w3[c0 + k];
+      e = fma_(silu(a), q, e);
+      g2_lds[m * LD4 + c0 + k] = q * silu_grad(a);
     }
-    if (i < N) eps[i] = e + w[mw.r3b];
+    e = group_sum<8>(e);
+    if (c0 == 0 && i < N) eps[i] = e + w[mw.r3b];
   }
   __syncthreads();
   if (wave < HP2 / 16) {   // d/dh1 = g2 W2, then SiLU'
-    int cb[1] = {wave * 16};
     f4 acc[RT][1];
     zero_acc(acc);
-    mma_tile_k2<RT, 1, HP4>(g2_lds, LD4, w + mw.r2t, HP4, cb, acc);
-    const int c = cb[0] + r;
+    if constexpr (kRegs) mma_regs(g2_lds, LD4, wr2t, acc);
+    else mma_tile_k4<RT, 1, HP4>(g2_lds, LD4, w + mw.r2t, HP4, c2, acc);
+    const int c = c2[0] + r;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -522,22 +561,19 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
   }
   __syncthreads();
   {   // d/ds = g1 W1 over H output columns
-    constexpr int CT = H / 16, NT = (CT + 3) / 4;
-    if (wave < CT / NT) {
-      int cb[NT];
-      f4 acc[RT][NT];
-#pragma unroll
-      for (int ct = 0; ct < NT; ++ct) cb[ct] = (wave * NT + ct) * 16;
+    if (wave < CTG / NTG) {
+      f4 acc[RT][NTG];
       zero_acc(acc);
-      mma_tile_k2<RT, NT, HP2>(h1_lds, LD2, w + mw.r1t, HP2, cb, acc);
+      if constexpr (kRegs) mma_regs(h1_lds, LD2, wr1t, acc);
+      else mma_tile_k4<RT, NTG, HP2>(h1_lds, LD2, w + mw.r1t, HP2, cg, acc);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct)
+        for (int ct = 0; ct < NTG; ++ct)
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             const int i = base + rt * 16 + 4 * g + k;
-            if (i < N) gS[(size_t)i * H + cb[ct] + r] = acc[rt][ct][k];
+            if (i < N) gS[(size_t)i * H + cg[ct] + r] = acc[rt][ct][k];
           }
     }
   }
@@ -588,10 +624,10 @@ __global__ __launch_bounds__(kUpdBlock) void update_bwd_kernel(
       const bool in = base + m < N;
       float y1 = 0.f, y2 = 0.f;
       if (gv2 != nullptr) {
-        y1 = q0[k] * x0[k] + q1[k] * x1[k] + q2[k] * x2[k];
-        y2 = q0[k] * (u[0] * x0[k] + u[1] * x1[k] + u[2] * x2[k]) +
-             q1[k] * (u[3] * x0[k] + u[4] * x1[k] + u[5] * x2[k]) +
-             q2[k] * (u[6] * x0[k] + u[7] * x1[k] + u[8] * x2[k]);
+        y1 = dot3(q0[k], q1[k], q2[k], x0[k], x1[k], x2[k]);
+        y2 = dot3(q0[k], q1[k], q2[k], dot3(u[0], u[1], u[2], x0[k], x1[k], x2[k]),
+                  dot3(u[3], u[4], u[5], x0[k], x1[k], x2[k]),
+                  dot3(u[6], u[7], u[8], x0[k], x1[k], x2[k]));
       }
       y_lds[m * LDY + c] = in ? y0[k] : 0.f;
       y_lds[m * LDY + H + c] = in ? y1 : 0.f;
@@ -617,7 +653,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_bwd_kernel(
             av[rt][ct][k] = a_upd[(size_t)i * H + cb[ct] + r];
           }
       zero_acc(acc);
-      mma_tile_k2<RT, NT, 3 * H, 2, true>(y_lds, LDY, w + lw.u2t, 3 * H, cb, acc);
+      mma_tile_k4<RT, NT, 3 * H, 2, true>(y_lds, LDY, w + lw.u2t, 3 * H, cb, acc);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -640,7 +676,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_bwd_kernel(
 #pragma unroll
       for (int ct = 0; ct < NT; ++ct) cb[ct] = (wave * NT + ct) * 16;
       zero_acc(acc);
-      mma_tile_k2<RT, NT, H, 2, true>(a_lds, LDA, w + lw.u1t, H, cb, acc);
+      mma_tile_k4<RT, NT, H, 2, true>(a_lds, LDA, w + lw.u1t, H, cb, acc);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -678,15 +714,253 @@ __global__ __launch_bounds__(kUpdBlock) void update_bwd_kernel(
       const float sc = (n > 0.f) ? gn / n : 0.f;
       float o0 = sc * x0[k], o1 = sc * x1[k], o2 = sc * x2[k];
       if (gv2 != nullptr) {
-        o0 += q0[k] * t1[k] + (u[0] * q0[k] + u[3] * q1[k] + u[6] * q2[k]) * t2[k];
-        o1 += q1[k] * t1[k] + (u[1] * q0[k] + u[4] * q1[k] + u[7] * q2[k]) * t2[k];
-        o2 += q2[k] * t1[k] + (u[2] * q0[k] + u[5] * q1[k] + u[8] * q2[k]) * t2[k];
+        o0 = fma_(dot3(u[0], u[3], u[6], q0[k], q1[k], q2[k]), t2[k], fma_(q0[k], t1[k], o0));
+        o1 = fma_(dot3(u[1], u[4], u[7], q0[k], q1[k], q2[k]), t2[k], fma_(q1[k], t1[k], o1));
+        o2 = fma_(dot3(u[2], u[5], u[8], q0[k], q1[k], q2[k]), t2[k], fma_(q2[k], t1[k], o2));
       }
       float* go = gv1 + (size_t)i * 3 * H;
       go[c] = o0;
       go[H + c] = o1;
       go[2 * H + c] = o2;
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The update block and its adjoint in two kernels each, for few atoms: a block
+// takes 16 atoms and 32 output columns (two waves of one column tile), so the
+// weights (0.3 MB at H = 128, L2-cold in every kernel) come in through many
+// CUs instead of one per atom tile: what one CU can have in flight from memory
+// bounds a whole-tile block at 17 us, however few atoms there are.  All of a
+// wave's weights are requested first.  Same sums as the whole-tile kernels,
+// bit for bit.  Grid (16-atom tiles, H / 32).
+// ---------------------------------------------------------------------------
+constexpr int kSplitBlock = 128;
+
+// a = [s, |v|] W1^T + b1
+template <int H>
+__global__ __launch_bounds__(kSplitBlock, 2) void update_hidden_kernel(
+    int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ s_mid,
+    const float* __restrict__ v_mid, float* __restrict__ a_upd) {
+  constexpr int LDX = 2 * H + 4, PER = 16 * H / kSplitBlock;
+  __shared__ __align__(16) float x_lds[16 * LDX];
+  const int base = blockIdx.x * 16, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int cb[1] = {(int)blockIdx.y * 32 + wave * 16};
+  Weights<1, 2 * H> w1;
+  load_weights(w + lw.u1w, 2 * H, cb, w1);
+  float sv[PER], x0[PER], x1[PER], x2[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, c = idx % H;
+    const int i = min(base + m, N - 1);
+    const float* vv = v_mid + (size_t)i * 3 * H;
+    sv[k] = s_mid[(size_t)i * H + c];
+    x0[k] = vv[c];
+    x1[k] = vv[H + c];
+    x2[k] = vv[2 * H + c];
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, c = idx % H;
+    const bool in = base + m < N;
+    x_lds[m * LDX + c] = in ? sv[k] : 0.f;
+    x_lds[m * LDX + H + c] = in ? norm3_exact(x0[k], x1[k], x2[k]) : 0.f;
+  }
+  __syncthreads();
+  f4 acc[1][1];
+  zero_acc(acc);
+  mma_regs(x_lds, LDX, w1, acc);
+  const int c = cb[0] + r;
+  const float bias = (w + lw.u1b)[c];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = base + 4 * g + k;
+    if (i < N) a_upd[(size_t)i * H + c] = acc[0][0][k] + bias;
+  }
+}
+
+// (ds, g1, g2) = silu(a) W2^T + b2 and the gated outputs
+template <int H>
+__global__ __launch_bounds__(kSplitBlock, 2) void update_gate_kernel(
+    int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ s_mid,
+    const float* __restrict__ v_mid, const float* __restrict__ a_upd, float* __restrict__ s_out,
+    float* __restrict__ v_out, float* __restrict__ g12) {
+  constexpr int LDH = H + 4, PER = 16 * H / kSplitBlock;
+  __shared__ __align__(16) float h_lds[16 * LDH];
+  const int base = blockIdx.x * 16, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int c = blockIdx.y * 32 + wave * 16 + r;
+  const int cb[3] = {c - r, H + c - r, 2 * H + c - r};
+  Weights<3, H> w2;
+  load_weights(w + lw.u2w, H, cb, w2);
+  float av[PER], sm[4], xv[4][3], u[9], bias[3];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, q = idx % H;
+    av[k] = a_upd[(size_t)min(base + m, N - 1) * H + q];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = min(base + 4 * g + k, N - 1);
+    sm[k] = s_mid[(size_t)i * H + c];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) xv[k][x] = v_mid[((size_t)i * 3 + x) * H + c];
+  }
+#pragma unroll
+  for (int k = 0; k < 9; ++k) u[k] = (w + lw.mix)[k];
+#pragma unroll
+  for (int x = 0; x < 3; ++x) bias[x] = (w + lw.u2b)[x * H + c];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, q = idx % H;
+    h_lds[m * LDH + q] = silu(av[k]);
+  }
+  __syncthreads();
+  f4 acc[1][3];
+  zero_acc(acc);
+  mma_regs(h_lds, LDH, w2, acc);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = base + 4 * g + k;
+    if (i >= N) continue;
+    const float ds = acc[0][0][k] + bias[0], gt1 = acc[0][1][k] + bias[1],
+                gt2 = acc[0][2][k] + bias[2];
+    const float x0 = xv[k][0], x1 = xv[k][1], x2 = xv[k][2];
+    s_out[(size_t)i * H + c] = sm[k] + ds;
+    float* vo = v_out + (size_t)i * 3 * H;
+    vo[c] = fma_(dot3(u[0], u[1], u[2], x0, x1, x2), gt2, x0 * gt1);
+    vo[H + c] = fma_(dot3(u[3], u[4], u[5], x0, x1, x2), gt2, x1 * gt1);
+    vo[2 * H + c] = fma_(dot3(u[6], u[7], u[8], x0, x1, x2), gt2, x2 * gt1);
+    g12[(size_t)i * 2 * H + c] = gt1;
+    g12[(size_t)i * 2 * H + H + c] = gt2;
+  }
+}
+
+// ga = silu'(a) (gy W2), gy the gradient of (ds, g1, g2)
+template <int H>
+__global__ __launch_bounds__(kSplitBlock, 2) void update_hidden_bwd_kernel(
+    int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ gs2,
+    const float* __restrict__ gv2, const float* __restrict__ v_mid,
+    const float* __restrict__ a_upd, float* __restrict__ ga) {
+  constexpr int LDY = 3 * H + 4, PER = 16 * H / kSplitBlock, kB = PER < 8 ? PER : 8;
+  __shared__ __align__(16) float y_lds[16 * LDY];
+  const int base = blockIdx.x * 16, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int cb[1] = {(int)blockIdx.y * 32 + wave * 16};
+  const int c1 = cb[0] + r;
+  Weights<1, 3 * H> w1;
+  load_weights(w + lw.u2t, 3 * H, cb, w1);
+  float u[9], av[4];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) u[k] = (w + lw.mix)[k];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) av[k] = a_upd[(size_t)min(base + 4 * g + k, N - 1) * H + c1];
+#pragma unroll
+  for (int kb = 0; kb < PER; kb += kB) {
+    float y0[kB], x0[kB], x1[kB], x2[kB], q0[kB], q1[kB], q2[kB];
+#pragma unroll
+    for (int k = 0; k < kB; ++k) {
+      const int idx = threadIdx.x + (kb + k) * kSplitBlock, m = idx / H, c = idx % H;
+      const int i = min(base + m, N - 1);
+      y0[k] = gs2[(size_t)i * H + c];
+      if (gv2 != nullptr) {
+        const float* vv = v_mid + (size_t)i * 3 * H;
+        const float* gg = gv2 + (size_t)i * 3 * H;
+        x0[k] = vv[c]; x1[k] = vv[H + c]; x2[k] = vv[2 * H + c];
+        q0[k] = gg[c]; q1[k] = gg[H + c]; q2[k] = gg[2 * H + c];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kB; ++k) {
+      const int idx = threadIdx.x + (kb + k) * kSplitBlock, m = idx / H, c = idx % H;
+      const bool in = base + m < N;
+      float y1 = 0.f, y2 = 0.f;
+      if (gv2 != nullptr) {
+        y1 = dot3(q0[k], q1[k], q2[k], x0[k], x1[k], x2[k]);
+        y2 = dot3(q0[k], q1[k], q2[k], dot3(u[0], u[1], u[2], x0[k], x1[k], x2[k]),
+                  dot3(u[3], u[4], u[5], x0[k], x1[k], x2[k]),
+                  dot3(u[6], u[7], u[8], x0[k], x1[k], x2[k]));
+      }
+      y_lds[m * LDY + c] = in ? y0[k] : 0.f;
+      y_lds[m * LDY + H + c] = in ? y1 : 0.f;
+      y_lds[m * LDY + 2 * H + c] = in ? y2 : 0.f;
+    }
+  }
+  __syncthreads();
+  f4 acc[1][1];
+  zero_acc(acc);
+  mma_regs(y_lds, LDY, w1, acc);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = base + 4 * g + k;
+    if (i < N) ga[(size_t)i * H + c1] = acc[0][0][k] * silu_grad(av[k]);
+  }
+}
+
+// gradient of the block's inputs from ga W1 and the gates
+template <int H>
+__global__ __launch_bounds__(kSplitBlock, 2) void update_input_bwd_kernel(
+    int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ gs2,
+    const float* __restrict__ gv2, const float* __restrict__ v_mid, const float* __restrict__ ga,
+    const float* __restrict__ g12, float* __restrict__ gs1, float* __restrict__ gv1) {
+  constexpr int LDA = H + 4, PER = 16 * H / kSplitBlock;
+  __shared__ __align__(16) float a_lds[16 * LDA];
+  const int base = blockIdx.x * 16, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int c = blockIdx.y * 32 + wave * 16 + r;
+  const int cb[2] = {c - r, H + c - r};
+  Weights<2, H> w1;
+  load_weights(w + lw.u1t, H, cb, w1);
+  float av[PER], u[9], s2[4], xv[4][3], t1[4], t2[4], q[4][3];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, cc = idx % H;
+    av[k] = ga[(size_t)min(base + m, N - 1) * H + cc];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = min(base + 4 * g + k, N - 1);
+    s2[k] = gs2[(size_t)i * H + c];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) xv[k][x] = v_mid[((size_t)i * 3 + x) * H + c];
+    if (gv2 != nullptr) {
+      t1[k] = g12[(size_t)i * 2 * H + c];
+      t2[k] = g12[(size_t)i * 2 * H + H + c];
+#pragma unroll
+      for (int x = 0; x < 3; ++x) q[k][x] = gv2[((size_t)i * 3 + x) * H + c];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 9; ++k) u[k] = (w + lw.mix)[k];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, cc = idx % H;
+    a_lds[m * LDA + cc] = base + m < N ? av[k] : 0.f;
+  }
+  __syncthreads();
+  f4 acc[1][2];
+  zero_acc(acc);
+  mma_regs(a_lds, LDA, w1, acc);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = base + 4 * g + k;
+    if (i >= N) continue;
+    gs1[(size_t)i * H + c] = s2[k] + acc[0][0][k];
+    const float gn = acc[0][1][k], x0 = xv[k][0], x1 = xv[k][1], x2 = xv[k][2];
+    const float n = norm3_exact(x0, x1, x2);
+    const float sc = (n > 0.f) ? gn / n : 0.f;
+    float o0 = sc * x0, o1 = sc * x1, o2 = sc * x2;
+    if (gv2 != nullptr) {
+      const float q0 = q[k][0], q1 = q[k][1], q2 = q[k][2];
+      o0 = fma_(dot3(u[0], u[3], u[6], q0, q1, q2), t2[k], fma_(q0, t1[k], o0));
+      o1 = fma_(dot3(u[1], u[4], u[7], q0, q1, q2), t2[k], fma_(q1, t1[k], o1));
+      o2 = fma_(dot3(u[2], u[5], u[8], q0, q1, q2), t2[k], fma_(q2, t1[k], o2));
+    }
+    float* go = gv1 + (size_t)i * 3 * H;
+    go[c] = o0;
+    go[H + c] = o1;
+    go[2 * H + c] = o2;
   }
 }
 
@@ -880,7 +1154,7 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_bwd_kernel(
         zero_acc(pre);
         zero_acc(acc);
         mma_tile<RTW, NT>(e_lds + r0 * 16 * LDE, LDE, w + lw.f1w, RP, RP, cb, pre);
-        mma_tile_k2<RTW, NT, 3 * H, 2, true>(gw_lds + r0 * 16 * LDG, LDG, w + lw.f2t, 3 * H, cb,
+        mma_tile_k4<RTW, NT, 3 * H, 2, true>(gw_lds + r0 * 16 * LDG, LDG, w + lw.f2t, 3 * H, cb,
                                              acc);
         const float* b1 = w + lw.f1b;
 #pragma unroll
@@ -1134,6 +1408,51 @@ void launch_message(const Buffers& b, hipStream_t st, int grid, const float* Wl,
                                                         v_out);
 }
 
+// Atom-side launches: the split or small forms for few atoms (kSplitAtoms,
+// kReadoutSmallAtoms), 32-atom tiles above.  Same bits.
+template <int H>
+void launch_update_fwd(const Buffers& b, hipStream_t s, const LayerW& lw, const float* s_mid,
+                       const float* v_mid, float* s_out, float* v_out, float* a_upd, float* g12) {
+  if (b.N <= kSplitAtoms) {
+    const dim3 grid((b.N + 15) / 16, H / 32);
+    update_hidden_kernel<H><<<grid, kSplitBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, a_upd);
+    update_gate_kernel<H><<<grid, kSplitBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, a_upd, s_out,
+                                                       v_out, g12);
+  } else {
+    update_fwd_kernel<H><<<(b.N + 31) / 32, kUpdBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, s_out,
+                                                               v_out, a_upd, g12);
+  }
+}
+
+template <int H>
+void launch_readout(const Buffers& b, hipStream_t s) {
+  const float* sL = b.S + (size_t)b.L * nh(b);
+  if (b.N <= kReadoutSmallAtoms)
+    readout_kernel<H, 16><<<(b.N + 15) / 16, kBlock, 0, s>>>(b.N, b.w, *b.mw, sL, b.eps, b.gS0);
+  else
+    readout_kernel<H, 32><<<(b.N + 31) / 32, kBlock, 0, s>>>(b.N, b.w, *b.mw, sL, b.eps, b.gS0);
+}
+
+template <int H>
+void launch_update_bwd(const Buffers& b, hipStream_t s, int l, const float* gs2,
+                       const float* gv2) {
+  const LayerW& lw = b.mw->layer[l];
+  const float* vm = b.Vmid + (size_t)l * 3 * nh(b);
+  const float* au = b.Aupd + (size_t)l * nh(b);
+  const float* g12 = b.G12 + (size_t)l * 2 * nh(b);
+  float* gs1 = b.gS1 + (size_t)l * nh(b);
+  float* gv1 = b.gV1 + (size_t)l * 3 * nh(b);
+  if (b.N <= kSplitAtoms) {
+    const dim3 grid((b.N + 15) / 16, H / 32);
+    update_hidden_bwd_kernel<H><<<grid, kSplitBlock, 0, s>>>(b.N, b.w, lw, gs2, gv2, vm, au, b.gA);
+    update_input_bwd_kernel<H><<<grid, kSplitBlock, 0, s>>>(b.N, b.w, lw, gs2, gv2, vm, b.gA, g12,
+                                                            gs1, gv1);
+  } else {
+    update_bwd_kernel<H><<<(b.N + 31) / 32, kUpdBlock, 0, s>>>(b.N, b.w, lw, gs2, gv2, vm, au,
+                                                               g12, gs1, gv1);
+  }
+}
+
 // Fork/join between the caller's stream and the filter stream.  Events order
 // the two streams both eagerly and under graph capture (a wait on an event
 // recorded in a capturing stream pulls the other stream into the capture).
@@ -1172,7 +1491,6 @@ hipError_t forward_impl(const Buffers& b, hipStream_t s) {
   }
   const int rows_per_block = kBlock / H;
   const int msg_grid = ((N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
-  const int atom_grid = (N + 31) / 32;
   for (int l = 0; l < b.L; ++l) {
     const LayerW& lw = mw.layer[l];
     float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
@@ -1182,12 +1500,11 @@ hipError_t forward_impl(const Buffers& b, hipStream_t s) {
     float* Sm = b.Smid + (size_t)l * nh(b);
     float* Vm = b.Vmid + (size_t)l * 3 * nh(b);
     launch_message<H, true>(b, s, msg_grid, Wl, Sl, Vl, Sm, Vm);
-    update_fwd_kernel<H><<<atom_grid, kUpdBlock, 0, s>>>(
-        N, b.w, lw, Sm, Vm, b.S + (size_t)(l + 1) * nh(b), b.V + (size_t)(l + 1) * 3 * nh(b),
-        b.Aupd + (size_t)l * nh(b), b.G12 + (size_t)l * 2 * nh(b));
+    launch_update_fwd<H>(b, s, lw, Sm, Vm, b.S + (size_t)(l + 1) * nh(b),
+                         b.V + (size_t)(l + 1) * 3 * nh(b), b.Aupd + (size_t)l * nh(b),
+                         b.G12 + (size_t)l * 2 * nh(b));
   }
-  readout_kernel<H><<<atom_grid, kBlock, 0, s>>>(N, b.w, mw, b.S + (size_t)b.L * nh(b), b.eps,
-                                                 b.gS0);
+  launch_readout<H>(b, s);
   if (st.err != hipSuccess) return st.err;
   return hipGetLastError();
 }
@@ -1200,7 +1517,6 @@ hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool wa
   const float* widths = b.w + mw.widths;
   const int rows_per_block = kBlock / H;
   const int msg_grid = ((N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
-  const int atom_grid = (N + 31) / 32;
   Streams st(b, s);
   // gradient w.r.t. the update outputs of the last block: (gS0, 0)
   float* gs2 = b.gS0;
@@ -1213,9 +1529,7 @@ hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool wa
     // and update adjoint of block l-1 (caller's stream) run side by side
     float* gS1 = b.gS1 + (size_t)l * nh(b);
     float* gV1 = b.gV1 + (size_t)l * 3 * nh(b);
-    update_bwd_kernel<H><<<atom_grid, kUpdBlock, 0, s>>>(
-        N, b.w, lw, gs2, gv2, b.Vmid + (size_t)l * 3 * nh(b), b.Aupd + (size_t)l * nh(b),
-        b.G12 + (size_t)l * 2 * nh(b), gS1, gV1);
+    launch_update_bwd<H>(b, s, l, gs2, gv2);
     st.order(s, st.filt, b.L + 1 + l);
     launch_filter_bwd<H>(b, st.filt, l, gS1, gV1, l == b.L - 1, l == 0);
     if (l > 0) {
@@ -1240,7 +1554,6 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
   const float* widths = b.w + mw.widths;
   const int rows_per_block = kBlock / H;
   const int msg_grid = ((N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
-  const int atom_grid = (N + 31) / 32;
   const LayerW& lw = mw.layer[l];
   float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
   switch (stage) {
@@ -1253,21 +1566,16 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
                               b.Vmid + (size_t)l * 3 * nh(b));
       break;
     case MLFF_STAGE_UPDATE_FWD:
-      update_fwd_kernel<H><<<atom_grid, kUpdBlock, 0, s>>>(
-          N, b.w, lw, b.Smid + (size_t)l * nh(b), b.Vmid + (size_t)l * 3 * nh(b),
-          b.S + (size_t)(l + 1) * nh(b), b.V + (size_t)(l + 1) * 3 * nh(b),
-          b.Aupd + (size_t)l * nh(b), b.G12 + (size_t)l * 2 * nh(b));
+      launch_update_fwd<H>(b, s, lw, b.Smid + (size_t)l * nh(b), b.Vmid + (size_t)l * 3 * nh(b),
+                           b.S + (size_t)(l + 1) * nh(b), b.V + (size_t)(l + 1) * 3 * nh(b),
+                           b.Aupd + (size_t)l * nh(b), b.G12 + (size_t)l * 2 * nh(b));
       break;
     case MLFF_STAGE_READOUT:
-      readout_kernel<H><<<atom_grid, kBlock, 0, s>>>(N, b.w, mw, b.S + (size_t)b.L * nh(b), b.eps,
-                                                     b.gS0);
+      launch_readout<H>(b, s);
       break;
     case MLFF_STAGE_UPDATE_BWD:
       // reads gS0/gV0, writes block l's slice of gS1/gV1
-      update_bwd_kernel<H><<<atom_grid, kUpdBlock, 0, s>>>(
-          N, b.w, lw, b.gS0, (l == b.L - 1) ? nullptr : b.gV0, b.Vmid + (size_t)l * 3 * nh(b),
-          b.Aupd + (size_t)l * nh(b), b.G12 + (size_t)l * 2 * nh(b), b.gS1 + (size_t)l * nh(b),
-          b.gV1 + (size_t)l * 3 * nh(b));
+      launch_update_bwd<H>(b, s, l, b.gS0, (l == b.L - 1) ? nullptr : b.gV0);
       break;
     case MLFF_STAGE_FILTER_BWD:
       // first=1 overwrites the pair accumulator, so repeated launches agree
