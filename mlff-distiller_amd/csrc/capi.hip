@@ -136,7 +136,7 @@ namespace {
 
 enum Seg {
   S_COUNTS, S_DEG, S_UDEG, S_ROWPTR, S_PAIRPTR, S_COL, S_EPAIR, S_PLO, S_PHI, S_PSHIFT, S_GEOM,
-  S_UNIT,  S_PACC, S_GVEC, S_WF, S_S, S_V, S_SMID, S_VMID, S_AUPD, S_G12, S_GS0, S_GV0, S_GS1, S_GV1,
+  S_UNIT,  S_PACC, S_WF, S_S, S_V, S_SMID, S_VMID, S_AUPD, S_G12, S_GS0, S_GV0, S_GS1, S_GV1,
   S_GA, S_EPS, S_VIR, S_GRID, S_CELLCNT, S_CELLSTART, S_CELLATOMS, S_ATOMCELL, S_TMPSHIFT, S_WBF,
   S_TABBAD, S_TAB,   // the tables last: the static entry keeps them elsewhere
   S_COUNT_
@@ -163,8 +163,7 @@ void carve(mlff_plan* pl) {
   const int64_t P1 = P > 0 ? P : 1;
   sz[S_GEOM] = 16 * P1;
   sz[S_UNIT] = 16 * P1;
-  sz[S_PACC] = 16 * P;
-  sz[S_GVEC] = 16 * P;
+  sz[S_PACC] = 16 * L * P;
   sz[S_WF] = 4 * L * P1 * 3 * H;
   sz[S_S] = 4 * (L + 1) * N * H;
   sz[S_V] = 4 * (L + 1) * N * 3 * H;
@@ -489,7 +488,6 @@ int bind_buffers(mlff_plan* pl, const char* who, void* ws, const float* weights_
   b.geom = segp<float4>(pl, ws, S_GEOM);
   b.unit = segp<float4>(pl, ws, S_UNIT);
   b.pacc = segp<float4>(pl, ws, S_PACC);
-  b.gvec = segp<float4>(pl, ws, S_GVEC);
   b.Wf = segp<float>(pl, ws, S_WF);
   b.S = segp<float>(pl, ws, S_S);
   b.V = segp<float>(pl, ws, S_V);
@@ -601,8 +599,11 @@ static int run_ef(mlff_plan* pl, hipStream_t s, const float* pos, double* energy
   e = launch_forward(pl->buf, s);
   if (e != hipSuccess) return hip_fail(e, "forward");
   if (forces != nullptr || virial != nullptr) {
-    e = launch_backward(pl->buf, s, forces, virial != nullptr);
+    // without a virial the energies are summed beside the forces
+    double* en = virial == nullptr ? energy : nullptr;
+    e = launch_backward(pl->buf, s, forces, virial != nullptr, en);
     if (e != hipSuccess) return hip_fail(e, "adjoint");
+    if (en != nullptr) energy = nullptr;
   }
   e = launch_reduce(pl->buf, s, energy, virial, atom_energy);
   if (e != hipSuccess) return hip_fail(e, "reduce");
@@ -849,10 +850,8 @@ static int run_ef_on(mlff_plan* pl, hipStream_t s, double* energy, float* forces
   b.unit = src.unit;
   e = launch_forward(b, s);
   if (e != hipSuccess) return hip_fail(e, "outer forward");
-  e = launch_backward(b, s, forces, false);
+  e = launch_backward(b, s, forces, false, energy);
   if (e != hipSuccess) return hip_fail(e, "outer adjoint");
-  e = launch_reduce(b, s, energy, nullptr, nullptr);
-  if (e != hipSuccess) return hip_fail(e, "outer reduce");
   return MLFF_OK;
 }
 

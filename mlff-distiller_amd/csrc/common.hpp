@@ -382,11 +382,12 @@ __device__ __forceinline__ void zero_acc(f4 (&acc)[RT][NT]) {
 // gd vec/d + gu/(d+eps) - vec (vec.gu)/(d (d+eps)^2)
 __device__ __forceinline__ float4 pair_gradient(const float4& gm, const float4& acc) {
   const float d = gm.w, den = d + kEdgeEps;
-  const float vdot = gm.x * acc.x + gm.y * acc.y + gm.z * acc.z;
+  const float vdot = fma_(gm.x, acc.x, fma_(gm.y, acc.y, gm.z * acc.z));
   const float a1 = (d > 0.f) ? acc.w / d : 0.f;
   const float a2 = (d > 0.f) ? vdot / (d * den * den) : 0.f;
-  return make_float4(a1 * gm.x + acc.x / den - a2 * gm.x, a1 * gm.y + acc.y / den - a2 * gm.y,
-                     a1 * gm.z + acc.z / den - a2 * gm.z, 0.f);
+  return make_float4(fma_(-a2, gm.x, fma_(a1, gm.x, acc.x / den)),
+                     fma_(-a2, gm.y, fma_(a1, gm.y, acc.y / den)),
+                     fma_(-a2, gm.z, fma_(a1, gm.z, acc.z / den)), 0.f);
 }
 
 // Work tiles of a persistent block: tiles t0, t0 + step, ... below t1.

@@ -235,16 +235,20 @@ __global__ __launch_bounds__(kTabBlock) void table_guard_kernel(
 // ---------------------------------------------------------------------------
 // W_p of every pair, four columns per thread.  Bound by the 3H floats written
 // per pair (HBM) and the 4 x 3H read from the table (L2); kTabUnroll pairs'
-// table rows are in flight per thread.
+// table rows are in flight per thread.  One launch takes all blocks
+// (blockIdx.y): with few pairs a launch is mostly its own latency (60 atoms, three
+// blocks: 7.7 us against 3 x 4.8 us).
 // ---------------------------------------------------------------------------
 constexpr int kTabUnroll = 4;
 
 template <int H>
 __global__ __launch_bounds__(kTabBlock) void filter_table_fwd_kernel(
     const float4* __restrict__ geom, const int32_t* __restrict__ counts, int32_t pcap,
-    TableView tv, const int32_t* __restrict__ gate, float* __restrict__ Wout) {
+    TableView tv, int64_t layer_floats, const int32_t* __restrict__ gate, float* __restrict__ Wf) {
   constexpr int Q = 3 * H / 4;
   if (gate != nullptr && *gate != 0) return;
+  const float* tab = tv.w + blockIdx.y * layer_floats;
+  float* Wout = Wf + blockIdx.y * (size_t)pcap * 3 * H;
   const int P = min(counts[MLFF_COUNT_PAIRS], pcap);
   const int64_t total = (int64_t)P * Q;
   constexpr int kItems = kTabBlock * kTabUnroll;
@@ -258,7 +262,7 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_fwd_kernel(
       const int64_t it = min(base + u * kTabBlock + threadIdx.x, total - 1);
       const int p = (int)(it / Q), c = 4 * (int)(it - (int64_t)p * Q);
       at[u] = table_at(geom[p].w, tv.inv_c, tv.Kc);
-      const float* row = tv.w + (size_t)at[u].k * 2 * 3 * H + c;
+      const float* row = tab + (size_t)at[u].k * 2 * 3 * H + c;
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[u][k] = *reinterpret_cast<const f4*>(row + k * 3 * H);
     }
@@ -278,18 +282,31 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_fwd_kernel(
 // the terms): H/4 lanes per pair, four channels each, gather both endpoints'
 // features and gradients, form dL/dW_p in registers and contract it with
 // W'(d_p) to dL/dd, and (gv_a - gv_b) with Wv2 to dL/du.  Bound by the gathers
-// (16H floats per pair) and the 12H floats of the W' rows, all from L2.
+// (16H floats per pair) and the 12H floats of the W' rows, all from L2.  The
+// blocks' terms meet in force_gather_kernel, so all blocks (blockIdx.y) run in
+// one launch once the last gradients are there (60 atoms, three blocks: 7.6 us
+// against 3 x 4.9 us one by one).  A split into 32-channel slices, one slice's
+// table per XCD's L2, was slower: 282 us a block against 234 us for 256
+// molecules at H = 128, although a block's W' table (7.9 MB) exceeds an L2.
 // ---------------------------------------------------------------------------
 template <int H>
 __global__ __launch_bounds__(kTabBlock) void filter_table_bwd_kernel(
     const int32_t* __restrict__ counts, int32_t pcap, const int32_t* __restrict__ pair_lo,
     const int32_t* __restrict__ pair_hi, const float4* __restrict__ geom, TableView tv,
-    const int32_t* __restrict__ gate, const float* __restrict__ Wf,
+    int64_t layer_floats, const int32_t* __restrict__ gate, const float* __restrict__ Wf, int N,
     const float* __restrict__ s_in, const float* __restrict__ v_in,
-    const float* __restrict__ gs1, const float* __restrict__ gv1, float4* __restrict__ pacc,
-    float4* __restrict__ gvec, int first, int last) {
+    const float* __restrict__ gs1, const float* __restrict__ gv1, float4* __restrict__ pacc) {
   constexpr int G = H / 4, PPB = kTabBlock / G;
   if (gate != nullptr && *gate != 0) return;
+  const int l = blockIdx.y;
+  const size_t nh = (size_t)l * N * H;
+  const float* tab = tv.d + l * layer_floats;
+  Wf += (size_t)l * pcap * 3 * H;
+  s_in += nh;
+  v_in += 3 * nh;
+  gs1 += nh;
+  gv1 += 3 * nh;
+  pacc += (size_t)l * pcap;
   const int P = min(counts[MLFF_COUNT_PAIRS], pcap);
   int t0, t1, tstep;
   persistent_range((P + PPB - 1) / PPB, t0, t1, tstep);
@@ -305,7 +322,7 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_bwd_kernel(
     const float* qa = gv1 + (size_t)a * 3 * H + c;
     const float* qb = gv1 + (size_t)b * 3 * H + c;
     const TableAt at = table_at(gm.w, tv.inv, tv.K);
-    const float* row = tv.d + (size_t)at.k * 2 * 3 * H + c;
+    const float* row = tab + (size_t)at.k * 2 * 3 * H + c;
     const f4 sa = ld(s_in + (size_t)a * H + c), sb = ld(s_in + (size_t)b * H + c);
     const f4 ga = ld(gs1 + (size_t)a * H + c), gb = ld(gs1 + (size_t)b * H + c);
     const f4 wv2 = ld(Wf + (size_t)p * 3 * H + 2 * H + c);
@@ -332,12 +349,7 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_bwd_kernel(
     const float gx = group_sum<G>((w0[0] + w0[1]) + (w0[2] + w0[3]));
     const float gy = group_sum<G>((w1[0] + w1[1]) + (w1[2] + w1[3]));
     const float gz = group_sum<G>((w2[0] + w2[1]) + (w2[2] + w2[3]));
-    if (c == 0 && pr < P) {
-      float4 o = first ? make_float4(0.f, 0.f, 0.f, 0.f) : pacc[p];
-      o.x += gx; o.y += gy; o.z += gz; o.w += gd;
-      if (last) gvec[p] = pair_gradient(gm, o);
-      else pacc[p] = o;
-    }
+    if (c == 0 && pr < P) pacc[p] = make_float4(gx, gy, gz, gd);
   }
 }
 
@@ -394,30 +406,29 @@ hipError_t build_tables(const Buffers& b, hipStream_t s) {
 }
 
 template <int H>
-void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l) {
+void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1) {
   constexpr int Q = 3 * H / 4;
   const int64_t units = ((int64_t)b.pcap * Q + kTabBlock * kTabUnroll - 1) /
                         (kTabBlock * kTabUnroll);
-  filter_table_fwd_kernel<H><<<table_grid(b, units), kTabBlock, 0, s>>>(
-      b.geom, b.counts, b.pcap, table_view(b.ts, b.tab, l, 3 * H), b.gate,
-      b.Wf + (size_t)l * b.pcap * 3 * H);
+  filter_table_fwd_kernel<H><<<dim3(table_grid(b, units), l1 - l0), kTabBlock, 0, s>>>(
+      b.geom, b.counts, b.pcap, table_view(b.ts, b.tab, l0, 3 * H), b.ts.layer_floats, b.gate,
+      b.Wf + (size_t)l0 * b.pcap * 3 * H);
 }
 
 template <int H>
-void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l, const float* gS1,
-                             const float* gV1, int first, int last) {
+void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l0, int l1) {
   constexpr int PPB = kTabBlock / (H / 4);
-  const size_t nh = (size_t)b.N * H;
-  filter_table_bwd_kernel<H><<<table_grid(b, ((int64_t)b.pcap + PPB - 1) / PPB), kTabBlock, 0, s>>>(
-      b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, table_view(b.ts, b.tab, l, 3 * H), b.gate,
-      b.Wf + (size_t)l * b.pcap * 3 * H, b.S + l * nh, b.V + 3 * l * nh, gS1, gV1, b.pacc, b.gvec,
-      first, last);
+  const size_t nh = (size_t)l0 * b.N * H;
+  filter_table_bwd_kernel<H><<<dim3(table_grid(b, ((int64_t)b.pcap + PPB - 1) / PPB), l1 - l0),
+                               kTabBlock, 0, s>>>(
+      b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, table_view(b.ts, b.tab, l0, 3 * H),
+      b.ts.layer_floats, b.gate, b.Wf + (size_t)l0 * b.pcap * 3 * H, b.N, b.S + nh, b.V + 3 * nh,
+      b.gS1 + nh, b.gV1 + 3 * nh, b.pacc + (size_t)l0 * b.pcap);
 }
 
-#define MLFF_TABLE_INST(HH)                                                               \
-  template void launch_filter_table_fwd<HH>(const Buffers&, hipStream_t, int);            \
-  template void launch_filter_table_bwd<HH>(const Buffers&, hipStream_t, int, const float*, \
-                                            const float*, int, int);
+#define MLFF_TABLE_INST(HH)                                                         \
+  template void launch_filter_table_fwd<HH>(const Buffers&, hipStream_t, int, int); \
+  template void launch_filter_table_bwd<HH>(const Buffers&, hipStream_t, int, int);
 MLFF_TABLE_INST(32)
 MLFF_TABLE_INST(64)
 MLFF_TABLE_INST(128)

@@ -125,8 +125,7 @@ struct Buffers {
   const int32_t* pair_lo; const int32_t* pair_hi; const int32_t* pair_shift;
   const float4* geom;               // {p_hi - p_lo, d}
   const float4* unit;               // {(p_hi - p_lo) / (d + eps), d}
-  float4* pacc;                     // per pair (gu.xyz, gd)
-  float4* gvec;                     // per pair dE/dvec
+  float4* pacc;                     // [L][pcap]: per pair and block (dE/du, dE/dd)
   float* Wf;                        // [L][pcap][3H]
   float* S; float* V;               // [L+1][N][H], [L+1][N][3][H]
   float* Smid; float* Vmid;         // [L][N][H], [L][N][3][H]
@@ -156,13 +155,15 @@ int alternative_shape(int H, int which);
 hipError_t prepare_filters(const Buffers& b, hipStream_t s);
 // Fill and check every block's table (tab_bad must be 0 before).
 hipError_t build_tables(const Buffers& b, hipStream_t s);
+// Blocks l0 ... l1 - 1 in one launch.
 template <int H>
-void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l);
+void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1);
 template <int H>
-void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l, const float* gS1,
-                             const float* gV1, int first, int last);
+void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l0, int l1);
 hipError_t launch_forward(const Buffers& b, hipStream_t s);
-hipError_t launch_backward(const Buffers& b, hipStream_t s, float* forces, bool want_virial);
+// energy (may be null): the structures' sums too, in the last launch
+hipError_t launch_backward(const Buffers& b, hipStream_t s, float* forces, bool want_virial,
+                           double* energy);
 // One model stage (mlff_stage 1..8) of block `layer`, on the workspace as the
 // last full evaluation left it.
 hipError_t launch_stage(const Buffers& b, hipStream_t s, int stage, int layer);

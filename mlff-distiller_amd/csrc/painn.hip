@@ -1023,7 +1023,7 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_bwd_kernel(
     const float* __restrict__ widths, int R, int RP, float rc, const float* __restrict__ Wf,
     const float* __restrict__ s_in, const float* __restrict__ v_in,
     const float* __restrict__ gs1, const float* __restrict__ gv1, float4* __restrict__ pacc,
-    float4* __restrict__ gvec, int first, int last, const int32_t* __restrict__ gate) {
+    const int32_t* __restrict__ gate) {
   if (gate != nullptr && *gate == 0) return;
   constexpr int RT = TM / 16;
   constexpr int LDE = kMaxRbf + 4, LDG = 3 * H + 4, LDA = H + 4;
@@ -1190,7 +1190,6 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_bwd_kernel(
     if (threadIdx.x < TM) {
       const int m = threadIdx.x, p = pbase + m;
       if (p < P) {
-        const float4 gm = geom[p];
         const int nparts = (RP > 16) ? 2 * ((H / 16 < 4) ? H / 16 : 4) : ((H / 16 < 8) ? H / 16 : 8);
         float gd = 0.f;
         for (int q = 0; q < nparts; ++q) gd += gd_lds[q * TM + m];
@@ -1201,109 +1200,127 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_bwd_kernel(
           gy += gu_lds[(m * NPART + part) * 3 + 1];
           gz += gu_lds[(m * NPART + part) * 3 + 2];
         }
-        float4 acc = first ? make_float4(0.f, 0.f, 0.f, 0.f) : pacc[p];
-        acc.x += gx; acc.y += gy; acc.z += gz; acc.w += gd;
-        if (last) {
-          gvec[p] = pair_gradient(gm, acc);
-        } else {
-          pacc[p] = acc;
-        }
+        pacc[p] = make_float4(gx, gy, gz, gd);
       }
     }
     __syncthreads();
   }
 }
 
-// forces F_i = sum_{j>i} G_p - sum_{j<i} G_p; per-atom virial sum_{j>i} vec (x) G
-__global__ void force_gather_kernel(int N, const int32_t* __restrict__ row_ptr,
-                                    const int32_t* __restrict__ col,
-                                    const int32_t* __restrict__ edge_pair, int32_t ecap,
-                                    const float4* __restrict__ gvec,
-                                    const float4* __restrict__ geom, float* __restrict__ forces,
-                                    float* __restrict__ vir_atom) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  float fx = 0.f, fy = 0.f, fz = 0.f;
-  float vr[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  const int e0 = min(row_ptr[i], ecap), e1 = min(row_ptr[i + 1], ecap);
-  // one edge's contribution, in edge order
-  auto add = [&](int j, int p, const float4& G, const float4& v) {
-    if (p < 0) return;
-    if (j > i) {
-      fx += G.x; fy += G.y; fz += G.z;
-      if (vir_atom != nullptr) {
-        vr[0] += v.x * G.x; vr[1] += v.x * G.y; vr[2] += v.x * G.z;
-        vr[3] += v.y * G.x; vr[4] += v.y * G.y; vr[5] += v.y * G.z;
-        vr[6] += v.z * G.x; vr[7] += v.z * G.y; vr[8] += v.z * G.z;
-      }
-    } else {
-      fx -= G.x; fy -= G.y; fz -= G.z;
-    }
-  };
-  // four edges' loads in flight before any is added (one thread per atom
-  // leaves about one wave per CU, so the loop is latency bound)
-  constexpr int U = 4;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  int e = e0;
-  for (; e + U - 1 < e1; e += U) {
-    int jj[U], pp[U];
-    float4 GG[U], VV[U];
+// Gradient of pair p: its blocks' terms, from the last block to the first.
+// Four blocks' loads are in flight at a time.
+__device__ __forceinline__ float4 pair_sum(const float4* __restrict__ pacc, int32_t pcap, int L,
+                                           int p, const float4& gm) {
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int lb = L - 1; lb >= 0; lb -= 4) {
+    float4 t[4];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      jj[u] = col[e + u];
-      pp[u] = edge_pair[e + u];
-    }
+    for (int k = 0; k < 4; ++k) t[k] = pacc[(size_t)max(lb - k, 0) * pcap + p];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int pc = pp[u] >= 0 ? pp[u] : 0;
-      GG[u] = gvec[pc];
-      VV[u] = vir_atom != nullptr ? geom[pc] : zero;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) add(jj[u], pp[u], GG[u], VV[u]);
+    for (int k = 0; k < 4; ++k)
+      if (lb - k >= 0) { o.x += t[k].x; o.y += t[k].y; o.z += t[k].z; o.w += t[k].w; }
   }
-  for (; e < e1; ++e) {
-    const int p = edge_pair[e];
-    const int pc = p >= 0 ? p : 0;
-    add(col[e], p, gvec[pc], vir_atom != nullptr ? geom[pc] : zero);
-  }
-  if (forces != nullptr) {
-    forces[3 * i] = fx;
-    forces[3 * i + 1] = fy;
-    forces[3 * i + 2] = fz;
-  }
-  if (vir_atom != nullptr)
-    for (int k = 0; k < 9; ++k) vir_atom[9 * i + k] = vr[k];
+  return pair_gradient(gm, o);
 }
 
-// per-structure FP64 sums in a fixed order (one workgroup per structure)
-__global__ __launch_bounds__(kBlock) void reduce_kernel(int B, const int32_t* __restrict__ mol_ptr,
+// Sums over one structure's atoms in FP64, in a fixed order: thread t of the
+// workgroup takes atoms t, t + 256, ..., then lanes, then waves.  K values per
+// atom: its energy and the nine entries of its virial.
+template <int K>
+__device__ __forceinline__ void structure_sums(int i0, int i1, const float* __restrict__ eps,
+                                               const float* __restrict__ vir_atom,
+                                               double (&acc)[K]) {
+  __shared__ double sh[kBlock / 64][K];
+  for (int k = 0; k < K; ++k) acc[k] = 0.0;
+  for (int i = i0 + threadIdx.x; i < i1; i += kBlock) {
+    acc[0] += (double)eps[i];
+#pragma unroll
+    for (int k = 1; k < K; ++k) acc[k] += (double)vir_atom[9 * (size_t)i + k - 1];
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) acc[k] += __shfl_xor(acc[k], off, 64);
+  if ((threadIdx.x & 63) == 0)
+    for (int k = 0; k < K; ++k) sh[threadIdx.x >> 6][k] = acc[k];
+  __syncthreads();
+  for (int k = 0; k < K; ++k) acc[k] = (sh[0][k] + sh[1][k]) + (sh[2][k] + sh[3][k]);
+}
+
+// Forces F_i = sum_{j>i} G_p - sum_{j<i} G_p; per-atom virial sum_{j>i} vec (x) G.
+// kGatherLanes lanes per atom take its edges in turn and add up at the end: with
+// one thread per atom a row of 60 edges is 15 rounds of loads long (12.4 us in a
+// launch of 60 atoms, 5.3 us so; 25 and 18 us in one of 10,000).  The workgroups past the atoms' add up the
+// structures' energies (energy not null), which saves their launch.
+constexpr int kGatherLanes = 32, kGatherAtoms = kBlock / kGatherLanes;
+
+template <bool VIR>
+__global__ __launch_bounds__(kBlock) void force_gather_kernel(
+    int N, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col,
+    const int32_t* __restrict__ edge_pair, int32_t ecap, const float4* __restrict__ pacc,
+    int32_t pcap, int L, const float4* __restrict__ geom, float* __restrict__ forces,
+    float* __restrict__ vir_atom, int B, const int32_t* __restrict__ mol_ptr,
+    const float* __restrict__ eps, double* __restrict__ energy) {
+  const int atom_blocks = (N + kGatherAtoms - 1) / kGatherAtoms;
+  if ((int)blockIdx.x >= atom_blocks) {
+    const int b = blockIdx.x - atom_blocks;
+    double e[1];
+    structure_sums<1>(mol_ptr[b], mol_ptr[b + 1], eps, nullptr, e);
+    if (threadIdx.x == 0) energy[b] = e[0];
+    return;
+  }
+  const int i = blockIdx.x * kGatherAtoms + threadIdx.x / kGatherLanes;
+  const int lane = threadIdx.x % kGatherLanes;
+  if (i >= N) return;
+  constexpr int K = VIR ? 12 : 3;   // force, virial
+  float o[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) o[k] = 0.f;
+  const int e0 = min(row_ptr[i], ecap), e1 = min(row_ptr[i + 1], ecap);
+  for (int e = e0 + lane; e < e1; e += kGatherLanes) {
+    const int p = edge_pair[e];
+    if (p < 0) continue;
+    const float4 v = geom[p];
+    const float4 G = pair_sum(pacc, pcap, L, p, v);
+    if (col[e] > i) {
+      o[0] += G.x; o[1] += G.y; o[2] += G.z;
+      if constexpr (VIR) {
+        o[3] += v.x * G.x; o[4] += v.x * G.y; o[5] += v.x * G.z;
+        o[6] += v.y * G.x; o[7] += v.y * G.y; o[8] += v.y * G.z;
+        o[9] += v.z * G.x; o[10] += v.z * G.y; o[11] += v.z * G.z;
+      }
+    } else {
+      o[0] -= G.x; o[1] -= G.y; o[2] -= G.z;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) o[k] = group_sum<kGatherLanes>(o[k]);
+  if (lane != 0) return;
+  if (forces != nullptr)
+    for (int k = 0; k < 3; ++k) forces[3 * (size_t)i + k] = o[k];
+  if constexpr (VIR)
+    for (int k = 0; k < 9; ++k) vir_atom[9 * (size_t)i + k] = o[3 + k];
+}
+
+// per-structure FP64 sums (one workgroup per structure)
+__global__ __launch_bounds__(kBlock) void reduce_kernel(const int32_t* __restrict__ mol_ptr,
                                                         const float* __restrict__ eps,
                                                         const float* __restrict__ vir_atom,
                                                         double* __restrict__ energy,
                                                         double* __restrict__ virial) {
-  __shared__ double sh[kBlock][10];
   const int b = blockIdx.x;
-  if (b >= B) return;
   const int i0 = mol_ptr[b], i1 = mol_ptr[b + 1];
-  double acc[10];
-  for (int k = 0; k < 10; ++k) acc[k] = 0.0;
-  for (int i = i0 + threadIdx.x; i < i1; i += kBlock) {
-    acc[0] += (double)eps[i];
-    if (vir_atom != nullptr)
-      for (int k = 0; k < 9; ++k) acc[1 + k] += (double)vir_atom[9 * i + k];
-  }
-  for (int k = 0; k < 10; ++k) sh[threadIdx.x][k] = acc[k];
-  __syncthreads();
-  for (int off = kBlock / 2; off > 0; off >>= 1) {
-    if (threadIdx.x < off)
-      for (int k = 0; k < 10; ++k) sh[threadIdx.x][k] += sh[threadIdx.x + off][k];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    if (energy != nullptr) energy[b] = sh[0][0];
-    if (virial != nullptr)
-      for (int k = 0; k < 9; ++k) virial[9 * b + k] = sh[0][1 + k];
+  if (vir_atom == nullptr) {
+    double e[1];
+    structure_sums<1>(i0, i1, eps, nullptr, e);
+    if (threadIdx.x == 0 && energy != nullptr) energy[b] = e[0];
+  } else {
+    double a[10];
+    structure_sums<10>(i0, i1, eps, vir_atom, a);
+    if (threadIdx.x == 0) {
+      if (energy != nullptr) energy[b] = a[0];
+      for (int k = 0; k < 9; ++k) virial[9 * (size_t)b + k] = a[1 + k];
+    }
   }
 }
 
@@ -1338,12 +1355,12 @@ inline size_t nh(const Buffers& b) { return (size_t)b.N * b.H; }
 
 // Launches in the plan's chosen shapes (Buffers::tile_fwd, tile_bwd,
 // unroll_fwd, unroll_bwd; each is the default or its alternative).
+// the direct filter kernels run: without tables, or beside tables not yet
+// checked on the host (the flag picks one form)
+bool direct_filters(const Buffers& b) { return !b.use_table || b.gate != nullptr; }
+
 template <int H>
 void launch_filter_fwd(const Buffers& b, hipStream_t st, int l) {
-  if (b.use_table) {
-    launch_filter_table_fwd<H>(b, st, l);
-    if (b.gate == nullptr) return;
-  }
   const ModelW& mw = *b.mw;
   const float* centers = b.w + mw.centers;
   const float* widths = b.w + mw.widths;
@@ -1363,33 +1380,31 @@ void launch_filter_fwd(const Buffers& b, hipStream_t st, int l) {
 }
 
 template <int H>
-void launch_filter_bwd(const Buffers& b, hipStream_t st, int l, const float* gS1,
-                       const float* gV1, int first, int last) {
-  if (b.use_table) {
-    launch_filter_table_bwd<H>(b, st, l, gS1, gV1, first, last);
-    if (b.gate == nullptr) return;
-  }
+void launch_filter_bwd(const Buffers& b, hipStream_t st, int l) {
   const ModelW& mw = *b.mw;
   const float* centers = b.w + mw.centers;
   const float* widths = b.w + mw.widths;
   const float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
   const float* Sl = b.S + (size_t)l * nh(b);
   const float* Vl = b.V + (size_t)l * 3 * nh(b);
+  const float* gS1 = b.gS1 + (size_t)l * nh(b);
+  const float* gV1 = b.gV1 + (size_t)l * 3 * nh(b);
+  float4* pacc = b.pacc + (size_t)l * b.pcap;
   if (b.tile_bwd == kBwdPairsAlt<H>) {
     constexpr int TM = kBwdPairsAlt<H>;
     filter_bwd_kernel<H, TM, false><<<pair_grid(b, TM), kPairBlock, 0, st>>>(
         b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, b.w, mw.layer[l], centers, widths, b.R,
-        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, b.pacc, b.gvec, first, last, b.gate);
+        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, pacc, b.gate);
   } else if (b.bwd_variant == 1) {
     constexpr int TM = kBwdPairs<H>;
     filter_bwd_kernel<H, TM, true><<<pair_grid(b, TM), kPairBlock, 0, st>>>(
         b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, b.w, mw.layer[l], centers, widths, b.R,
-        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, b.pacc, b.gvec, first, last, b.gate);
+        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, pacc, b.gate);
   } else {
     constexpr int TM = kBwdPairs<H>;
     filter_bwd_kernel<H, TM, false><<<pair_grid(b, TM), kPairBlock, 0, st>>>(
         b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, b.w, mw.layer[l], centers, widths, b.R,
-        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, b.pacc, b.gvec, first, last, b.gate);
+        mw.RP, b.rc, Wl, Sl, Vl, gS1, gV1, pacc, b.gate);
   }
 }
 
@@ -1453,6 +1468,18 @@ void launch_update_bwd(const Buffers& b, hipStream_t s, int l, const float* gs2,
   }
 }
 
+void launch_force_gather(const Buffers& b, hipStream_t s, float* forces, bool want_virial,
+                         double* energy) {
+  const int grid = (b.N + kGatherAtoms - 1) / kGatherAtoms + (energy != nullptr ? b.B : 0);
+  if (grid == 0) return;
+  auto run = [&](auto kernel, float* vir_atom) {
+    kernel<<<grid, kBlock, 0, s>>>(b.N, b.row_ptr, b.col, b.edge_pair, b.ecap, b.pacc, b.pcap, b.L,
+                                   b.geom, forces, vir_atom, b.B, b.mol_ptr, b.eps, energy);
+  };
+  if (want_virial) run(force_gather_kernel<true>, b.vir_atom);
+  else run(force_gather_kernel<false>, nullptr);
+}
+
 // Fork/join between the caller's stream and the filter stream.  Events order
 // the two streams both eagerly and under graph capture (a wait on an event
 // recorded in a capturing stream pulls the other stream into the capture).
@@ -1480,8 +1507,10 @@ hipError_t forward_impl(const Buffers& b, hipStream_t s) {
   // the filters depend on the pair geometry only: all L of them run on the
   // filter stream while the caller's stream walks the atom-side chain
   st.order(s, st.filt, 0);
+  if (b.use_table && !st.two()) launch_filter_table_fwd<H>(b, s, 0, b.L);
   for (int l = 0; l < b.L; ++l) {
-    launch_filter_fwd<H>(b, st.filt, l);
+    if (b.use_table && st.two()) launch_filter_table_fwd<H>(b, st.filt, l, l + 1);
+    if (direct_filters(b)) launch_filter_fwd<H>(b, st.filt, l);
     if (st.two() && st.err == hipSuccess) st.err = hipEventRecord(b.ev[1 + l], st.filt);
   }
   {
@@ -1510,7 +1539,8 @@ hipError_t forward_impl(const Buffers& b, hipStream_t s) {
 }
 
 template <int H>
-hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool want_virial) {
+hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool want_virial,
+                         double* energy) {
   const ModelW& mw = *b.mw;
   const int N = b.N;
   const float* centers = b.w + mw.centers;
@@ -1531,17 +1561,18 @@ hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool wa
     float* gV1 = b.gV1 + (size_t)l * 3 * nh(b);
     launch_update_bwd<H>(b, s, l, gs2, gv2);
     st.order(s, st.filt, b.L + 1 + l);
-    launch_filter_bwd<H>(b, st.filt, l, gS1, gV1, l == b.L - 1, l == 0);
+    if (b.use_table && st.two()) launch_filter_table_bwd<H>(b, st.filt, l, l + 1);
+    if (direct_filters(b)) launch_filter_bwd<H>(b, st.filt, l);
     if (l > 0) {
       launch_message<H, false>(b, s, msg_grid, Wl, gS1, gV1, b.gS0, b.gV0);
       gs2 = b.gS0;
       gv2 = b.gV0;
     }
   }
+  // on one stream all blocks' adjoints go in one launch
+  if (b.use_table && !st.two()) launch_filter_table_bwd<H>(b, s, 0, b.L);
   st.order(st.filt, s, 2 * b.L + 1);
-  force_gather_kernel<<<(N + 127) / 128, 128, 0, s>>>(N, b.row_ptr, b.col, b.edge_pair, b.ecap,
-                                                      b.gvec, b.geom, forces,
-                                                      want_virial ? b.vir_atom : nullptr);
+  launch_force_gather(b, s, forces, want_virial, energy);
   if (st.err != hipSuccess) return st.err;
   return hipGetLastError();
 }
@@ -1558,7 +1589,8 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
   float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
   switch (stage) {
     case MLFF_STAGE_FILTER_FWD:
-      launch_filter_fwd<H>(b, s, l);
+      if (b.use_table) launch_filter_table_fwd<H>(b, s, l, l + 1);
+      if (direct_filters(b)) launch_filter_fwd<H>(b, s, l);
       break;
     case MLFF_STAGE_MESSAGE_FWD:
       launch_message<H, true>(b, s, msg_grid, Wl, b.S + (size_t)l * nh(b),
@@ -1578,18 +1610,15 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
       launch_update_bwd<H>(b, s, l, b.gS0, (l == b.L - 1) ? nullptr : b.gV0);
       break;
     case MLFF_STAGE_FILTER_BWD:
-      // first=1 overwrites the pair accumulator, so repeated launches agree
-      launch_filter_bwd<H>(b, s, l, b.gS1 + (size_t)l * nh(b), b.gV1 + (size_t)l * 3 * nh(b),
-                           1, 0);
+      if (b.use_table) launch_filter_table_bwd<H>(b, s, l, l + 1);
+      if (direct_filters(b)) launch_filter_bwd<H>(b, s, l);
       break;
     case MLFF_STAGE_MESSAGE_BWD:
       launch_message<H, false>(b, s, msg_grid, Wl, b.gS1 + (size_t)l * nh(b),
                                b.gV1 + (size_t)l * 3 * nh(b), b.gS0, b.gV0);
       break;
     case MLFF_STAGE_FORCES:
-      force_gather_kernel<<<(N + 127) / 128, 128, 0, s>>>(N, b.row_ptr, b.col, b.edge_pair,
-                                                          b.ecap, b.gvec, b.geom, nullptr,
-                                                          b.vir_atom);
+      launch_force_gather(b, s, nullptr, true, nullptr);
       break;
     default:
       return hipErrorInvalidValue;
@@ -1648,19 +1677,20 @@ hipError_t launch_forward(const Buffers& b, hipStream_t s) {
   }
 }
 
-hipError_t launch_backward(const Buffers& b, hipStream_t s, float* forces, bool want_virial) {
+hipError_t launch_backward(const Buffers& b, hipStream_t s, float* forces, bool want_virial,
+                           double* energy) {
   switch (b.H) {
-    case 32: return backward_impl<32>(b, s, forces, want_virial);
-    case 64: return backward_impl<64>(b, s, forces, want_virial);
-    case 128: return backward_impl<128>(b, s, forces, want_virial);
+    case 32: return backward_impl<32>(b, s, forces, want_virial, energy);
+    case 64: return backward_impl<64>(b, s, forces, want_virial, energy);
+    case 128: return backward_impl<128>(b, s, forces, want_virial, energy);
     default: return hipErrorInvalidValue;
   }
 }
 
 hipError_t launch_reduce(const Buffers& b, hipStream_t s, double* energy, double* virial,
                          float* atom_energy) {
-  if (b.B > 0)
-    reduce_kernel<<<b.B, kBlock, 0, s>>>(b.B, b.mol_ptr, b.eps, virial ? b.vir_atom : nullptr,
+  if (b.B > 0 && (energy != nullptr || virial != nullptr))
+    reduce_kernel<<<b.B, kBlock, 0, s>>>(b.mol_ptr, b.eps, virial ? b.vir_atom : nullptr,
                                          energy, virial);
   if (atom_energy != nullptr && b.N > 0)
     copy_f32_kernel<<<(b.N + 255) / 256, 256, 0, s>>>(b.N, b.eps, atom_energy);
