@@ -135,7 +135,7 @@ struct mlff_plan {
 namespace {
 
 enum Seg {
-  S_COUNTS, S_DEG, S_UDEG, S_ROWPTR, S_PAIRPTR, S_COL, S_EPAIR, S_PLO, S_PHI, S_PSHIFT, S_GEOM,
+  S_COUNTS, S_DEG, S_UDEG, S_MASK, S_ROWPTR, S_PAIRPTR, S_COL, S_EPAIR, S_PLO, S_PHI, S_PSHIFT, S_GEOM,
   S_UNIT,  S_PACC, S_WF, S_S, S_V, S_SMID, S_VMID, S_AUPD, S_G12, S_GS0, S_GV0, S_GS1, S_GV1,
   S_GA, S_EPS, S_VIR, S_GRID, S_CELLCNT, S_CELLSTART, S_CELLATOMS, S_ATOMCELL, S_TMPSHIFT, S_WBF,
   S_TABBAD, S_TAB,   // the tables last: the static entry keeps them elsewhere
@@ -151,6 +151,7 @@ void carve(mlff_plan* pl) {
   sz[S_COUNTS] = 4 * MLFF_COUNT_SLOTS;
   sz[S_DEG] = 4 * N;
   sz[S_UDEG] = 4 * N;
+  sz[S_MASK] = N <= kSmallAtoms ? 8 * N * (kSmallAtoms / 64) : 0;
   sz[S_ROWPTR] = 4 * (N + 1);
   sz[S_PAIRPTR] = 4 * (N + 1);
   sz[S_COL] = 4 * E;
@@ -513,6 +514,7 @@ int bind_buffers(mlff_plan* pl, const char* who, void* ws, const float* weights_
   a.cells = c.any_periodic ? cells_dev : nullptr; a.pbc = c.any_periodic ? pbc_dev : nullptr;
   a.rc = c.cutoff;
   a.deg = segp<int32_t>(pl, ws, S_DEG); a.udeg = segp<int32_t>(pl, ws, S_UDEG);
+  a.mask = a.N <= kSmallAtoms ? segp<uint64_t>(pl, ws, S_MASK) : nullptr;
   a.row_ptr = segp<int32_t>(pl, ws, S_ROWPTR); a.pair_ptr = segp<int32_t>(pl, ws, S_PAIRPTR);
   a.col = segp<int32_t>(pl, ws, S_COL); a.edge_shift = nullptr;
   a.edge_pair = segp<int32_t>(pl, ws, S_EPAIR); a.ecap = b.ecap;
@@ -777,7 +779,8 @@ int mlff_md_init_forces(mlff_plan* pl, void* stream) {
 
 static int md_step(mlff_plan* pl, hipStream_t s) {
   const Buffers& b = pl->buf;
-  hipError_t e = launch_vv_first(b.N, pl->x, pl->p, pl->inv_mass, pl->forces, pl->pos32, pl->dt, s);
+  hipError_t e = launch_vv_first(b.N, pl->x, pl->p, pl->inv_mass, pl->forces, pl->pos32, pl->dt,
+                                 b.counts, s);
   if (e != hipSuccess) return hip_fail(e, "vv first half");
   int rc = run_ef(pl, s, pl->pos32, pl->energy, pl->forces, nullptr, nullptr);
   if (rc != MLFF_OK) return rc;
@@ -906,7 +909,7 @@ static int mts_outer_step(mlff_plan* pl, hipStream_t s, bool fallback) {
   hipError_t e = launch_mts_kick(N, pl->p, pl->f_outer, Fin, 0.5 * Dt, s);
   if (e != hipSuccess) return hip_fail(e, "mts outer kick");
   for (int k = 0; k < pl->n_inner; ++k) {
-    e = launch_vv_first(N, pl->x, pl->p, pl->inv_mass, Fin, pl->pos32, dt, s);
+    e = launch_vv_first(N, pl->x, pl->p, pl->inv_mass, Fin, pl->pos32, dt, nullptr, s);
     if (e != hipSuccess) return hip_fail(e, "mts drift");
     int rc = run_ef(in, s, pl->pos32, pl->e_inner, pl->f_inner, nullptr, nullptr);
     if (rc != MLFF_OK) return rc;

@@ -28,6 +28,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -237,15 +239,24 @@ __global__ __launch_bounds__(kTabBlock) void table_guard_kernel(
 // per pair (HBM) and the 4 x 3H read from the table (L2); kTabUnroll pairs'
 // table rows are in flight per thread.  One launch takes all blocks
 // (blockIdx.y): with few pairs a launch is mostly its own latency (60 atoms, three
-// blocks: 7.7 us against 3 x 4.8 us).
+// blocks: 7.7 us against 3 x 4.8 us), and the embedding rides along (blockIdx.y
+// == L; 3.9 us by itself).
 // ---------------------------------------------------------------------------
 constexpr int kTabUnroll = 4;
 
 template <int H>
 __global__ __launch_bounds__(kTabBlock) void filter_table_fwd_kernel(
     const float4* __restrict__ geom, const int32_t* __restrict__ counts, int32_t pcap,
-    TableView tv, int64_t layer_floats, const int32_t* __restrict__ gate, float* __restrict__ Wf) {
+    TableView tv, int64_t layer_floats, const int32_t* __restrict__ gate, float* __restrict__ Wf,
+    int L, int N, const int64_t* __restrict__ Z, const float* __restrict__ emb,
+    float* __restrict__ S0, float* __restrict__ V0) {
   constexpr int Q = 3 * H / 4;
+  if ((int)blockIdx.y == L) {
+    for (int idx = blockIdx.x * kTabBlock + threadIdx.x; idx < N * (H / 4);
+         idx += gridDim.x * kTabBlock)
+      embed_item<H>(idx, Z, emb, S0, V0);
+    return;
+  }
   if (gate != nullptr && *gate != 0) return;
   const float* tab = tv.w + blockIdx.y * layer_floats;
   float* Wout = Wf + blockIdx.y * (size_t)pcap * 3 * H;
@@ -406,13 +417,13 @@ hipError_t build_tables(const Buffers& b, hipStream_t s) {
 }
 
 template <int H>
-void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1) {
+void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1, bool embed) {
   constexpr int Q = 3 * H / 4;
-  const int64_t units = ((int64_t)b.pcap * Q + kTabBlock * kTabUnroll - 1) /
-                        (kTabBlock * kTabUnroll);
-  filter_table_fwd_kernel<H><<<dim3(table_grid(b, units), l1 - l0), kTabBlock, 0, s>>>(
+  int64_t units = ((int64_t)b.pcap * Q + kTabBlock * kTabUnroll - 1) / (kTabBlock * kTabUnroll);
+  if (embed) units = std::max(units, ((int64_t)b.N * (H / 4) + kTabBlock - 1) / kTabBlock);
+  filter_table_fwd_kernel<H><<<dim3(table_grid(b, units), l1 - l0 + embed), kTabBlock, 0, s>>>(
       b.geom, b.counts, b.pcap, table_view(b.ts, b.tab, l0, 3 * H), b.ts.layer_floats, b.gate,
-      b.Wf + (size_t)l0 * b.pcap * 3 * H);
+      b.Wf + (size_t)l0 * b.pcap * 3 * H, l1 - l0, b.N, b.numbers, b.w + b.mw->emb, b.S, b.V);
 }
 
 template <int H>
@@ -427,7 +438,7 @@ void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l0, int l1) {
 }
 
 #define MLFF_TABLE_INST(HH)                                                         \
-  template void launch_filter_table_fwd<HH>(const Buffers&, hipStream_t, int, int); \
+  template void launch_filter_table_fwd<HH>(const Buffers&, hipStream_t, int, int, bool); \
   template void launch_filter_table_bwd<HH>(const Buffers&, hipStream_t, int, int);
 MLFF_TABLE_INST(32)
 MLFF_TABLE_INST(64)

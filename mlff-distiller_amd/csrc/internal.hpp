@@ -32,6 +32,7 @@ int build_layout(int H, int L, int R, int max_z, ModelW* mw, mlff_slot* slots, i
                  int* n_slots);
 
 // Neighbour-list launches (nl.hip).
+constexpr int kSmallAtoms = 1024;   // largest list that is counted and filled in two launches
 struct NLArgs {
   const float* pos; int N; int B;
   const int32_t* mol_ptr; const int32_t* atom_mol;
@@ -43,6 +44,7 @@ struct NLArgs {
   // cell list (periodic structures): grid[b] = {nc0, nc1, nc2, base}, nc0 == 0 -> brute force
   const int4* grid; int32_t n_cells;
   int32_t* cell_count; int32_t* cell_start; int32_t* cell_atoms; int32_t* atom_cell;
+  uint64_t* mask;            // [N][kSmallAtoms / 64] hit masks; null: none
   int32_t* edge_tmp_shift;   // [ecap*3] image shifts of cell-list rows before sorting
 };
 hipError_t launch_neighbor_list(const NLArgs& a, hipStream_t s, bool build_pairs);
@@ -155,9 +157,9 @@ int alternative_shape(int H, int which);
 hipError_t prepare_filters(const Buffers& b, hipStream_t s);
 // Fill and check every block's table (tab_bad must be 0 before).
 hipError_t build_tables(const Buffers& b, hipStream_t s);
-// Blocks l0 ... l1 - 1 in one launch.
+// Blocks l0 ... l1 - 1 in one launch; embed: the atoms' first features too.
 template <int H>
-void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1);
+void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1, bool embed);
 template <int H>
 void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l0, int l1);
 hipError_t launch_forward(const Buffers& b, hipStream_t s);
@@ -171,13 +173,15 @@ hipError_t launch_reduce(const Buffers& b, hipStream_t s, double* energy, double
                          float* atom_energy);
 
 // MD launches (md.hip).
+// counts (may be null): the step counter is advanced here; launch_vv_second
+// then writes the rows of the step before
 hipError_t launch_vv_first(int N, double* x, double* p, const double* inv_mass, const float* F,
-                           float* pos32, double dt, hipStream_t s);
+                           float* pos32, double dt, int32_t* counts, hipStream_t s);
 hipError_t launch_vv_second(int N, int B, const int32_t* mol_ptr, double* p,
                             const double* inv_mass, const float* F, double dt,
                             const double* epot, double* ledger, int ledger_len,
-                            int32_t* counts, const double* x, double* fx, double* fp, float* fF,
-                            int n_frames, hipStream_t s);
+                            const int32_t* counts, const double* x, double* fx, double* fp,
+                            float* fF, int n_frames, hipStream_t s);
 
 hipError_t launch_mts_kick(int N, double* p, const float* Fa, const float* Fb, double coef,
                            hipStream_t s);
@@ -189,6 +193,24 @@ hipError_t launch_mts_disagree(int N, const int32_t* atom_mol, const float* F_fu
 hipError_t launch_mts_ledger(int B, const int32_t* mol_ptr, const double* p,
                              const double* inv_mass, const double* epot, double* ledger,
                              int ledger_len, int32_t* counts, hipStream_t s);
+
+// S0 = emb[Z] and V0 = 0, four channels per item: item t of an atom's H/4
+// writes S0 channels 4t..4t+3 and the same channels of the three V0 components
+// (16-byte stores; rows are 16-byte aligned since H % 4 == 0)
+template <int H>
+__device__ __forceinline__ void embed_item(int idx, const int64_t* __restrict__ Z,
+                                           const float* __restrict__ emb, float* __restrict__ S0,
+                                           float* __restrict__ V0) {
+  constexpr int Q = H / 4;
+  const int i = idx / Q, c = idx % Q;
+  const float4 e = reinterpret_cast<const float4*>(emb + Z[i] * H)[c];
+  reinterpret_cast<float4*>(S0)[idx] = e;
+  float4* v = reinterpret_cast<float4*>(V0) + (size_t)i * 3 * Q + c;
+  const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+  v[0] = z;
+  v[Q] = z;
+  v[2 * Q] = z;
+}
 
 void set_error(const char* fmt, ...);
 

@@ -18,8 +18,11 @@ namespace {
 
 __global__ void vv_first_kernel(int N, double* __restrict__ x, double* __restrict__ p,
                                 const double* __restrict__ inv_mass, const float* __restrict__ F,
-                                float* __restrict__ pos32, double dt) {
+                                float* __restrict__ pos32, double dt,
+                                int32_t* __restrict__ counts) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  // nothing between here and vv_second_kernel reads the step counter
+  if (i == 0 && counts != nullptr) counts[MLFF_COUNT_STEP] += 1;
   if (i >= N) return;
   const double im = inv_mass[i];
 #pragma unroll
@@ -42,9 +45,10 @@ __global__ __launch_bounds__(256) void vv_second_kernel(
   const int b = blockIdx.x;
   if (b >= B) return;
   const int i0 = mol_ptr[b], i1 = mol_ptr[b + 1];
+  // the counter was advanced at the start of the step
+  const int step = counts[MLFF_COUNT_STEP] - 1;
   // frame row of this step (all three frame buffers are bound together)
-  const size_t fbase = n_frames > 0
-      ? (size_t)(counts[MLFF_COUNT_STEP] % n_frames) * (size_t)N * 3 : 0;
+  const size_t fbase = n_frames > 0 ? (size_t)(step % n_frames) * (size_t)N * 3 : 0;
   double ke = 0.0;
   for (int i = i0 + threadIdx.x; i < i1; i += 256) {
     double s = 0.0;
@@ -68,7 +72,7 @@ __global__ __launch_bounds__(256) void vv_second_kernel(
     __syncthreads();
   }
   if (threadIdx.x == 0 && ledger != nullptr && ledger_len > 0) {
-    const int row = counts[MLFF_COUNT_STEP] % ledger_len;
+    const int row = step % ledger_len;
     ledger[((size_t)row * B + b) * 2 + 0] = epot[b];
     ledger[((size_t)row * B + b) * 2 + 1] = sh[0];
   }
@@ -175,20 +179,20 @@ hipError_t launch_mts_ledger(int B, const int32_t* mol_ptr, const double* p,
 }
 
 hipError_t launch_vv_first(int N, double* x, double* p, const double* inv_mass, const float* F,
-                           float* pos32, double dt, hipStream_t s) {
-  if (N > 0) vv_first_kernel<<<(N + 255) / 256, 256, 0, s>>>(N, x, p, inv_mass, F, pos32, dt);
+                           float* pos32, double dt, int32_t* counts, hipStream_t s) {
+  if (N > 0)
+    vv_first_kernel<<<(N + 255) / 256, 256, 0, s>>>(N, x, p, inv_mass, F, pos32, dt, counts);
   return hipGetLastError();
 }
 
 hipError_t launch_vv_second(int N, int B, const int32_t* mol_ptr, double* p,
                             const double* inv_mass, const float* F, double dt,
                             const double* epot, double* ledger, int ledger_len,
-                            int32_t* counts, const double* x, double* fx, double* fp, float* fF,
-                            int n_frames, hipStream_t s) {
+                            const int32_t* counts, const double* x, double* fx, double* fp,
+                            float* fF, int n_frames, hipStream_t s) {
   if (B > 0)
     vv_second_kernel<<<B, 256, 0, s>>>(B, mol_ptr, p, inv_mass, F, dt, epot, ledger, ledger_len,
                                        counts, N, x, fx, fp, fF, n_frames);
-  step_advance_kernel<<<1, 64, 0, s>>>(counts);
   return hipGetLastError();
 }
 

@@ -14,6 +14,7 @@
 //           {p_hi - p_lo (+ shift @ cell), d}
 //   link  : per atom (one wave), edges with j < i find their pair in row j
 //           by binary search among row j's sorted upper neighbours.
+// Small lists: count, then fill with scan and link in it (nl_fill_small_kernel).
 // Every write is guarded by the edge / pair capacity; a run that exceeds a
 // capacity sets counts[MLFF_COUNT_OVERFLOW] and never writes out of bounds.
 //
@@ -206,6 +207,7 @@ __device__ __forceinline__ int cell_candidate(const CellList& cl, const CellWalk
 // longer rows take the one-lane path
 constexpr int kCellRowMax = 256;
 constexpr int kNlBlock = 256;
+constexpr int kMaskWords = kSmallAtoms / 64;   // hit mask of a row, from its structure's first atom
 
 __global__ void cl_zero_kernel(int n, int32_t* __restrict__ a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -314,7 +316,7 @@ __global__ void nl_count_kernel(const float* __restrict__ pos, int N,
                                 const int32_t* __restrict__ atom_mol,
                                 const float* __restrict__ cells, const uint8_t* __restrict__ pbc,
                                 float rc, int32_t* __restrict__ deg, int32_t* __restrict__ udeg,
-                                CellList cl) {
+                                uint64_t* __restrict__ mask, CellList cl) {
   // one wave per atom: the lanes test 64 candidates at a time, the atoms of
   // the structure (brute force) or of the 27 cells around the atom's cell
   const int i = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
@@ -345,14 +347,31 @@ __global__ void nl_count_kernel(const float* __restrict__ pos, int N,
     for (int jb = j0; jb < j1; jb += 64) {
       const int j = jb + lane;
       const bool h = (j < j1) && (j != i) && hit(j);
-      n += __popcll(__ballot(h));
+      const uint64_t mh = __ballot(h);
+      n += __popcll(mh);
       nu += __popcll(__ballot(h && j > i));
+      if (mask != nullptr && lane == 0) mask[(size_t)i * kMaskWords + (jb - j0) / 64] = mh;
     }
   }
   if (lane == 0) {
     deg[i] = n;
     udeg[i] = nu;
   }
+}
+
+// one thread, once per list
+__device__ __forceinline__ void store_totals(int N, int edges, int pairs,
+                                             int32_t* __restrict__ row_ptr,
+                                             int32_t* __restrict__ pair_ptr,
+                                             int32_t* __restrict__ counts, int32_t ecap,
+                                             int32_t pcap) {
+  row_ptr[N] = edges;
+  pair_ptr[N] = pairs;
+  counts[MLFF_COUNT_EDGES] = edges;
+  counts[MLFF_COUNT_PAIRS] = pairs;
+  // the largest count of a run of lists (an MD chunk), for the regrowth
+  if (edges > counts[MLFF_COUNT_EDGES_MAX]) counts[MLFF_COUNT_EDGES_MAX] = edges;
+  if (edges > ecap || pairs > pcap) counts[MLFF_COUNT_OVERFLOW] = 1;
 }
 
 // Exclusive scan of deg and udeg in two passes over 1024-atom slices, one
@@ -456,14 +475,59 @@ __global__ __launch_bounds__(kScanThreads) void nl_scan_offset_kernel(
       pair_ptr[base + i] += o2;
     }
   }
-  if (g == G - 1 && t == 0) {
-    row_ptr[N] = all1;
-    pair_ptr[N] = all2;
-    counts[MLFF_COUNT_EDGES] = all1;
-    counts[MLFF_COUNT_PAIRS] = all2;
-    // the largest count of a run of lists (an MD chunk), for the regrowth
-    if (all1 > counts[MLFF_COUNT_EDGES_MAX]) counts[MLFF_COUNT_EDGES_MAX] = all1;
-    if (all1 > ecap || all2 > pcap) counts[MLFF_COUNT_OVERFLOW] = 1;
+  if (g == G - 1 && t == 0) store_totals(N, all1, all2, row_ptr, pair_ptr, counts, ecap, pcap);
+}
+
+// Row i of the list by a test against every atom of its structure: 64
+// candidates per step; a hit's slot is the number of hits in lower lanes, so the
+// row stays in ascending neighbour order.  lower(j) is the pair of an edge to
+// j < i, or -1 where nl_link_kernel finds it afterwards.
+template <class Lower>
+__device__ __forceinline__ void fill_row(
+    const float* __restrict__ pos, int i, int j0, int j1, const CellInfo& ci, bool periodic,
+    float rc, int e, int p, int32_t* __restrict__ col, int32_t* __restrict__ edge_shift,
+    int32_t* __restrict__ edge_pair, int32_t ecap, int32_t* __restrict__ pair_lo,
+    int32_t* __restrict__ pair_hi, int32_t* __restrict__ pair_shift, float4* __restrict__ geom,
+    float4* __restrict__ unit, int32_t pcap, Lower lower) {
+  const int lane = threadIdx.x & 63;
+  const float xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  for (int jb = j0; jb < j1; jb += 64) {
+    const int j = jb + lane;
+    float vx = 0.f, vy = 0.f, vz = 0.f, d = 0.f;
+    int s0 = 0, s1 = 0, s2 = 0;
+    const bool h = (j < j1) && (j != i) &&
+                   within(pos[3 * j] - xi, pos[3 * j + 1] - yi, pos[3 * j + 2] - zi, rc, periodic,
+                          ci, vx, vy, vz, d, s0, s1, s2);
+    const uint64_t mh = __ballot(h);
+    const uint64_t mu = __ballot(h && j > i);
+    if (h) {
+      const int ek = e + __popcll(mh & below);
+      const bool e_ok = ek < ecap;
+      if (e_ok) {
+        col[ek] = j;
+        if (edge_shift) {
+          edge_shift[3 * ek] = s0; edge_shift[3 * ek + 1] = s1; edge_shift[3 * ek + 2] = s2;
+        }
+      }
+      if (j > i) {
+        const int pk = p + __popcll(mu & below);
+        if (pair_lo != nullptr && pk < pcap) {
+          pair_lo[pk] = i;
+          pair_hi[pk] = j;
+          if (pair_shift) {
+            pair_shift[3 * pk] = s0; pair_shift[3 * pk + 1] = s1; pair_shift[3 * pk + 2] = s2;
+          }
+          store_pair(geom, unit, pk, vx, vy, vz, d);
+        }
+        if (edge_pair != nullptr && e_ok) edge_pair[ek] = (pk < pcap) ? pk : -1;
+      } else if (edge_pair != nullptr && e_ok) {
+        const int pk = lower(j);
+        edge_pair[ek] = (pk < pcap) ? pk : -1;
+      }
+    }
+    e += __popcll(mh);
+    p += __popcll(mu);
   }
 }
 
@@ -611,42 +675,87 @@ __global__ void nl_fill_kernel(const float* __restrict__ pos, int N,
     }
     return;
   }
-  // 64 candidates per step; a hit's slot is the number of hits in lower
-  // lanes, so the row stays in ascending neighbour order
-  for (int jb = j0; jb < j1; jb += 64) {
-    const int j = jb + lane;
-    float vx = 0.f, vy = 0.f, vz = 0.f, d = 0.f;
-    int s0 = 0, s1 = 0, s2 = 0;
-    const bool h = (j < j1) && (j != i) &&
-                   within(pos[3 * j] - xi, pos[3 * j + 1] - yi, pos[3 * j + 2] - zi, rc, periodic,
-                          ci, vx, vy, vz, d, s0, s1, s2);
-    const uint64_t mh = __ballot(h);
-    const uint64_t mu = __ballot(h && j > i);
-    if (h) {
-      const int ek = e + __popcll(mh & below);
-      const bool e_ok = ek < ecap;
-      if (e_ok) {
-        col[ek] = j;
-        if (edge_shift) {
-          edge_shift[3 * ek] = s0; edge_shift[3 * ek + 1] = s1; edge_shift[3 * ek + 2] = s2;
-        }
-      }
-      if (j > i) {
-        const int pk = p + __popcll(mu & below);
-        if (pair_lo != nullptr && pk < pcap) {
-          pair_lo[pk] = i;
-          pair_hi[pk] = j;
-          if (pair_shift) {
-            pair_shift[3 * pk] = s0; pair_shift[3 * pk + 1] = s1; pair_shift[3 * pk + 2] = s2;
-          }
-          store_pair(geom, unit, pk, vx, vy, vz, d);
-        }
-        if (edge_pair != nullptr && e_ok) edge_pair[ek] = (pk < pcap) ? pk : -1;
-      }
-    }
-    e += __popcll(mh);
-    p += __popcll(mu);
+  fill_row(pos, i, j0, j1, ci, periodic, rc, e, p, col, edge_shift, edge_pair, ecap, pair_lo,
+           pair_hi, pair_shift, geom, unit, pcap, [](int) { return -1; });
+}
+
+// Lists of at most kSmallAtoms atoms: the list is a chain of launches with
+// little work in each (60 atoms: 20 us in five), so the rows are filled right
+// after they are counted.  Every workgroup scans all counts by itself, and
+// the pair of an edge to a lower neighbour j is the number of bits of row j's
+// hit mask between j and i.  Without masks (the lists outside a plan)
+// nl_link_kernel follows.
+__global__ __launch_bounds__(kNlBlock) void nl_fill_small_kernel(
+    const float* __restrict__ pos, int N, const int32_t* __restrict__ mol_ptr,
+    const int32_t* __restrict__ atom_mol, const float* __restrict__ cells,
+    const uint8_t* __restrict__ pbc, float rc, const int32_t* __restrict__ deg,
+    const int32_t* __restrict__ udeg, const uint64_t* __restrict__ mask,
+    int32_t* __restrict__ row_ptr, int32_t* __restrict__ pair_ptr, int32_t* __restrict__ counts,
+    int32_t* __restrict__ col, int32_t* __restrict__ edge_shift, int32_t* __restrict__ edge_pair,
+    int32_t ecap, int32_t* __restrict__ pair_lo, int32_t* __restrict__ pair_hi,
+    int32_t* __restrict__ pair_shift, float4* __restrict__ geom, float4* __restrict__ unit,
+    int32_t pcap) {
+  static_assert(kSmallAtoms == 4 * kNlBlock, "four atoms per thread");
+  __shared__ __align__(16) int b1[kSmallAtoms];
+  __shared__ __align__(16) int b2[kSmallAtoms];
+  __shared__ int w1[kNlBlock / 64], w2[kNlBlock / 64];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  int a1[4], a2[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int q = 4 * t + k;
+    a1[k] = q < N ? deg[q] : 0;
+    a2[k] = q < N ? udeg[q] : 0;
   }
+  const int s1 = a1[0] + a1[1] + a1[2] + a1[3], s2 = a2[0] + a2[1] + a2[2] + a2[3];
+  const int i1 = wave_inclusive_scan(s1), i2 = wave_inclusive_scan(s2);
+  if (lane == 63) { w1[wv] = i1; w2[wv] = i2; }
+  __syncthreads();
+  int o1 = i1 - s1, o2 = i2 - s2, all1 = 0, all2 = 0;
+#pragma unroll
+  for (int q = 0; q < kNlBlock / 64; ++q) {
+    if (q < wv) { o1 += w1[q]; o2 += w2[q]; }
+    all1 += w1[q];
+    all2 += w2[q];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    b1[4 * t + k] = o1;
+    b2[4 * t + k] = o2;
+    o1 += a1[k];
+    o2 += a2[k];
+  }
+  __syncthreads();
+  if (blockIdx.x == 0 && t == 0) store_totals(N, all1, all2, row_ptr, pair_ptr, counts, ecap, pcap);
+  const int i = blockIdx.x * (kNlBlock / 64) + wv;
+  if (i >= N) return;
+  if (lane == 0) {
+    row_ptr[i] = b1[i];
+    pair_ptr[i] = b2[i];
+  }
+  const int b = atom_mol[i];
+  const int j0 = mol_ptr[b], j1 = mol_ptr[b + 1];
+  CellInfo ci;
+  bool periodic;
+  load_cell(cells, pbc, b, ci, periodic);
+  fill_row(pos, i, j0, j1, ci, periodic, rc, b1[i], b2[i], col, edge_shift, edge_pair, ecap,
+           pair_lo, pair_hi, pair_shift, geom, unit, pcap, [&](int j) {
+             if (mask == nullptr) return -1;
+             // bits (j, i) of row j's mask, and bit i itself
+             const uint64_t* m = mask + (size_t)j * kMaskWords;
+             const int wi = (i - j0) / 64, bi = (i - j0) % 64, bj = (j - j0) % 64;
+             int pk = b2[j];
+             for (int w = (j - j0) / 64; w <= wi; ++w) {
+               uint64_t v = m[w];
+               if (w == (j - j0) / 64) v &= ~0ull << bj;   // row j has no bit j
+               if (w == wi) {
+                 if (!((v >> bi) & 1)) return -1;
+                 v &= ~(~0ull << bi);
+               }
+               pk += __popcll(v);
+             }
+             return pk;
+           });
 }
 
 // One wave per row i.  Row i's lower neighbours j < i are its first
@@ -690,6 +799,21 @@ hipError_t launch_neighbor_list(const NLArgs& a, hipStream_t s, bool build_pairs
   const int g = (a.N + tb - 1) / tb;
   if (a.N == 0) return hipSuccess;
   CellList cl{nullptr, nullptr, nullptr, nullptr};
+  // count and fill: one wave per atom
+  const int gw = (int)(((int64_t)a.N * 64 + kNlBlock - 1) / kNlBlock);
+  const int32_t pcap = build_pairs ? a.pcap : 0x7fffffff;
+  if (a.N <= kSmallAtoms && !(a.grid != nullptr && a.n_cells > 0)) {
+    nl_count_kernel<<<gw, kNlBlock, 0, s>>>(a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc,
+                                            a.rc, a.deg, a.udeg, a.mask, cl);
+    nl_fill_small_kernel<<<gw, kNlBlock, 0, s>>>(
+        a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc, a.rc, a.deg, a.udeg, a.mask, a.row_ptr,
+        a.pair_ptr, a.counts, a.col, a.edge_shift, build_pairs ? a.edge_pair : nullptr, a.ecap,
+        build_pairs ? a.pair_lo : nullptr, a.pair_hi, a.pair_shift, a.geom, a.unit, pcap);
+    if (build_pairs && a.mask == nullptr)
+      nl_link_kernel<<<gw, kNlBlock, 0, s>>>(a.N, a.row_ptr, a.pair_ptr, a.col, a.edge_pair,
+                                             a.ecap, a.pcap);
+    return hipGetLastError();
+  }
   if (a.grid != nullptr && a.n_cells > 0) {
     const int C = a.n_cells;
     cl_zero_kernel<<<(C + 255) / 256, 256, 0, s>>>(C, a.cell_count);
@@ -701,15 +825,12 @@ hipError_t launch_neighbor_list(const NLArgs& a, hipStream_t s, bool build_pairs
         C, a.cell_start, a.cell_atoms);
     cl = CellList{a.grid, a.cell_start, a.cell_atoms, a.atom_cell};
   }
-  // count and fill: one wave per atom
-  const int gw = (int)(((int64_t)a.N * 64 + kNlBlock - 1) / kNlBlock);
   nl_count_kernel<<<gw, kNlBlock, 0, s>>>(a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc, a.rc,
-                                   a.deg, a.udeg, cl);
+                                   a.deg, a.udeg, nullptr, cl);
   const int slices = (a.N + kScanSlice - 1) / kScanSlice;
   nl_scan_slice_kernel<<<slices, kScanThreads, 0, s>>>(a.deg, a.udeg, a.N, a.row_ptr, a.pair_ptr);
   nl_scan_offset_kernel<<<slices, kScanThreads, 0, s>>>(a.deg, a.udeg, a.N, a.row_ptr, a.pair_ptr,
-                                                        a.counts, a.ecap,
-                                                        build_pairs ? a.pcap : 0x7fffffff);
+                                                        a.counts, a.ecap, pcap);
   nl_fill_kernel<<<gw, kNlBlock, 0, s>>>(a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc, a.rc,
                                   a.row_ptr, a.pair_ptr, a.col, a.edge_shift,
                                   build_pairs ? a.edge_pair : nullptr, a.ecap,

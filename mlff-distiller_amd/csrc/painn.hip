@@ -51,6 +51,9 @@ constexpr int kUpdBlock = 64 * kUpdWaves;
 // Readout: 14 -> 7 us at 60 atoms, 15 -> 9 us at 3000.
 constexpr int kSplitAtoms = 1024;
 constexpr int kReadoutSmallAtoms = 4096;
+// Message rows: sums per row, and the atoms up to which each has threads of its own
+constexpr int kMsgSums = 4;
+constexpr int kMsgSplitAtoms = 1024;
 // edges in flight per row in the message kernels (forward, adjoint)
 constexpr int kMsgUnrollFwd = 8;
 constexpr int kMsgUnrollBwd = 8;
@@ -72,24 +75,12 @@ inline int pair_grid(const Buffers& b, int pairs_per_tile) {
   return std::max(8, std::min(b.blocks, (tiles + 7) / 8 * 8));
 }
 
-// S0 = emb[Z] and V0 = 0, four channels per thread: thread t of an atom's
-// H/4 threads writes S0 channels 4t..4t+3 and the same channels of the
-// three V0 components (16-byte stores; rows are 16-byte aligned since H % 4 == 0)
 template <int H>
 __global__ void embed_kernel(int N, const int64_t* __restrict__ Z,
                              const float* __restrict__ emb, float* __restrict__ S0,
                              float* __restrict__ V0) {
-  constexpr int Q = H / 4;
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= N * Q) return;
-  const int i = idx / Q, c = idx % Q;
-  const float4 e = reinterpret_cast<const float4*>(emb + Z[i] * H)[c];
-  reinterpret_cast<float4*>(S0)[idx] = e;
-  float4* v = reinterpret_cast<float4*>(V0) + (size_t)i * 3 * Q + c;
-  const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-  v[0] = z;
-  v[Q] = z;
-  v[2 * Q] = z;
+  if (idx < N * (H / 4)) embed_item<H>(idx, Z, emb, S0, V0);
 }
 
 // ---------------------------------------------------------------------------
@@ -219,8 +210,9 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_fwd_kernel(
 // FWD:  s'_i = s_i + sum_j s_j * Ws_p ;  v'_i = v_i + sum_j v_j * Wv1_p + u_ji (x) Wv2_p
 // BWD:  gs_i = gs'_i + sum_j gs'_j * Ws_p ; gv_i = gv'_i + sum_j gv'_j * Wv1_p
 // One channel per lane, H lanes per row, neighbours in ascending j; the operands
-// of UNROLL edges are requested before any is added.  Even and odd
-// edges have sums of their own (shorter rounding chains).
+// of UNROLL edges are requested before any is added.  Edges
+// e, e + 4, ... of a row have a sum of their own: shorter rounding chains, and with
+// few rows (SPLIT) four times the threads, one sum each, same bits.
 // A wave works on one row (H >= 64), so a row's neighbour and pair indices and
 // unit vectors are scalar loads and the loop spends its vector registers on
 // operands in flight only.  Bound by reading every W_p once per direction
@@ -229,19 +221,26 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_fwd_kernel(
 // adjoint) for 256 molecules of 10-100 atoms at H = 128, 55 / 36 us for 1000
 // waters and 32 / 21 us for one molecule of 60 atoms; this form 180 / 144,
 // 47 / 32 and 10 / 7 us.  Twelve edges in flight: 180 / 143, 48 / 33, 12 / 7.
+// SPLIT: 6.3 / 4.8 us for the molecule of 60 atoms.
 // ---------------------------------------------------------------------------
-template <int H, bool FWD, int UNROLL>
-__global__ __launch_bounds__(kBlock) void message_kernel(
+template <int H, bool FWD, int UNROLL, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? kMsgSums * H : kBlock) void message_kernel(
     int N, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col,
     const int32_t* __restrict__ edge_pair, int32_t ecap, const float4* __restrict__ unit,
     const float* __restrict__ Wf, const float* __restrict__ s_in, const float* __restrict__ v_in,
     float* __restrict__ s_out, float* __restrict__ v_out) {
-  constexpr int RPB = kBlock / H;
+  constexpr int RPB = SPLIT ? 1 : kBlock / H;
+  constexpr int NA = SPLIT ? 1 : kMsgSums;       // sums of a thread
+  constexpr int STEP = SPLIT ? kMsgSums : 1;     // edges from one of its edges to the next
   const int c = threadIdx.x % H;
-  int i = xcd_block() * RPB + threadIdx.x / H;
+  int i = xcd_block() * RPB + (SPLIT ? 0 : threadIdx.x / H);
+  int part = SPLIT ? threadIdx.x / H : 0;
+  if (H >= 64) part = __builtin_amdgcn_readfirstlane(part);
   if (H >= 64) i = __builtin_amdgcn_readfirstlane(i);   // uniform: indices in scalar registers
   if (i >= N) return;
-  float as[2] = {0.f, 0.f}, a0[2] = {0.f, 0.f}, a1[2] = {0.f, 0.f}, a2[2] = {0.f, 0.f};
+  float as[NA], a0[NA], a1[NA], a2[NA];
+#pragma unroll
+  for (int o = 0; o < NA; ++o) as[o] = a0[o] = a1[o] = a2[o] = 0.f;
   const int e0 = min(row_ptr[i], ecap), e1 = min(row_ptr[i + 1], ecap);
   // neighbour and pair indices of the next step, requested a step ahead (past
   // the row's end: the last edge's)
@@ -249,7 +248,7 @@ __global__ __launch_bounds__(kBlock) void message_kernel(
   auto indices = [&](int e) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      const int ec = min(e + u, e1 - 1);
+      const int ec = min(e + STEP * u, e1 - 1);
       jn[u] = col[ec];
       pn[u] = edge_pair[ec];
     }
@@ -267,7 +266,7 @@ __global__ __launch_bounds__(kBlock) void message_kernel(
     for (int u = 0; u < UNROLL; ++u) {
       const int p = max(pn[u], 0);
       jc[u] = jn[u];
-      on[u] = (!TAIL || e + u < e1) && pn[u] >= 0;
+      on[u] = (!TAIL || e + STEP * u < e1) && pn[u] >= 0;
       const float* wp = Wf + (size_t)p * 3 * H;
       const float* vj = v_in + (size_t)jc[u] * 3 * H;
       ws[u] = wp[c];
@@ -281,12 +280,12 @@ __global__ __launch_bounds__(kBlock) void message_kernel(
         uu[u] = unit[p];
       }
     }
-    if (!TAIL) indices(e + UNROLL);
+    if (!TAIL) indices(e + STEP * UNROLL);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       const float w0 = on[u] ? ws[u] : 0.f, w1 = on[u] ? wv1[u] : 0.f;
-      const int o = u & 1;   // UNROLL is even: the edge's parity in its row
+      const int o = u % NA;   // UNROLL is a multiple of NA
       as[o] = fma_(sj[u], w0, as[o]);
       a0[o] = fma_(v0[u], w1, a0[o]);
       a1[o] = fma_(v1[u], w1, a1[o]);
@@ -300,16 +299,39 @@ __global__ __launch_bounds__(kBlock) void message_kernel(
       }
     }
   };
-  if (e0 < e1) indices(e0);
-  int e = e0;
-  for (; e + UNROLL <= e1; e += UNROLL) step(e, std::false_type{});
+  int e = e0 + part;
+  if (e < e1) indices(e);
+  for (; e + STEP * (UNROLL - 1) < e1; e += STEP * UNROLL) step(e, std::false_type{});
   if (e < e1) step(e, std::true_type{});
+  float t[kMsgSums][4];
+  if constexpr (SPLIT) {
+    __shared__ float sh[kMsgSums][4][H];
+    sh[part][0][c] = as[0];
+    sh[part][1][c] = a0[0];
+    sh[part][2][c] = a1[0];
+    sh[part][3][c] = a2[0];
+    __syncthreads();
+    if (part != 0) return;
+#pragma unroll
+    for (int o = 0; o < kMsgSums; ++o)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) t[o][k] = sh[o][k][c];
+  } else {
+#pragma unroll
+    for (int o = 0; o < kMsgSums; ++o) {
+      t[o][0] = as[o];
+      t[o][1] = a0[o];
+      t[o][2] = a1[o];
+      t[o][3] = a2[o];
+    }
+  }
+  auto sum = [&](int k) { return (t[0][k] + t[1][k]) + (t[2][k] + t[3][k]); };
   const float* vi = v_in + (size_t)i * 3 * H + c;
   float* vo = v_out + (size_t)i * 3 * H + c;
-  s_out[(size_t)i * H + c] = s_in[(size_t)i * H + c] + (as[0] + as[1]);
-  vo[0] = vi[0] + (a0[0] + a0[1]);
-  vo[H] = vi[H] + (a1[0] + a1[1]);
-  vo[2 * H] = vi[2 * H] + (a2[0] + a2[1]);
+  s_out[(size_t)i * H + c] = s_in[(size_t)i * H + c] + sum(0);
+  vo[0] = vi[0] + sum(1);
+  vo[H] = vi[H] + sum(2);
+  vo[2 * H] = vi[2 * H] + sum(3);
 }
 
 // a . b in x order, with the fused operations spelled out: every tile shape of a
@@ -1409,18 +1431,21 @@ void launch_filter_bwd(const Buffers& b, hipStream_t st, int l) {
 }
 
 template <int H, bool FWD>
-void launch_message(const Buffers& b, hipStream_t st, int grid, const float* Wl,
-                    const float* s_in, const float* v_in, float* s_out, float* v_out) {
+void launch_message(const Buffers& b, hipStream_t st, const float* Wl, const float* s_in,
+                    const float* v_in, float* s_out, float* v_out) {
   constexpr int U0 = FWD ? kMsgUnrollFwd : kMsgUnrollBwd;
   constexpr int U1 = FWD ? kMsgUnrollFwdAlt : kMsgUnrollBwdAlt;
-  if ((FWD ? b.unroll_fwd : b.unroll_bwd) == U1)
-    message_kernel<H, FWD, U1><<<grid, kBlock, 0, st>>>(b.N, b.row_ptr, b.col, b.edge_pair,
-                                                        b.ecap, b.unit, Wl, s_in, v_in, s_out,
-                                                        v_out);
+  auto run = [&](auto kernel, int rows_per_block, int block) {
+    const int grid = ((b.N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
+    kernel<<<grid, block, 0, st>>>(b.N, b.row_ptr, b.col, b.edge_pair, b.ecap, b.unit, Wl, s_in,
+                                   v_in, s_out, v_out);
+  };
+  if (b.N <= kMsgSplitAtoms)
+    run(message_kernel<H, FWD, U0, true>, 1, kMsgSums * H);
+  else if ((FWD ? b.unroll_fwd : b.unroll_bwd) == U1)
+    run(message_kernel<H, FWD, U1, false>, kBlock / H, kBlock);
   else
-    message_kernel<H, FWD, U0><<<grid, kBlock, 0, st>>>(b.N, b.row_ptr, b.col, b.edge_pair,
-                                                        b.ecap, b.unit, Wl, s_in, v_in, s_out,
-                                                        v_out);
+    run(message_kernel<H, FWD, U0, false>, kBlock / H, kBlock);
 }
 
 // Atom-side launches: the split or small forms for few atoms (kSplitAtoms,
@@ -1507,19 +1532,18 @@ hipError_t forward_impl(const Buffers& b, hipStream_t s) {
   // the filters depend on the pair geometry only: all L of them run on the
   // filter stream while the caller's stream walks the atom-side chain
   st.order(s, st.filt, 0);
-  if (b.use_table && !st.two()) launch_filter_table_fwd<H>(b, s, 0, b.L);
+  const bool one = b.use_table && !st.two();
+  if (one) launch_filter_table_fwd<H>(b, s, 0, b.L, true);
   for (int l = 0; l < b.L; ++l) {
-    if (b.use_table && st.two()) launch_filter_table_fwd<H>(b, st.filt, l, l + 1);
+    if (b.use_table && st.two()) launch_filter_table_fwd<H>(b, st.filt, l, l + 1, false);
     if (direct_filters(b)) launch_filter_fwd<H>(b, st.filt, l);
     if (st.two() && st.err == hipSuccess) st.err = hipEventRecord(b.ev[1 + l], st.filt);
   }
-  {
+  if (!one) {
     const int total = N * (H / 4);
     embed_kernel<H><<<(unsigned)((total + kBlock - 1) / kBlock), kBlock, 0, s>>>(
         N, b.numbers, b.w + mw.emb, b.S, b.V);
   }
-  const int rows_per_block = kBlock / H;
-  const int msg_grid = ((N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
   for (int l = 0; l < b.L; ++l) {
     const LayerW& lw = mw.layer[l];
     float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
@@ -1528,7 +1552,7 @@ hipError_t forward_impl(const Buffers& b, hipStream_t s) {
     float* Vl = b.V + (size_t)l * 3 * nh(b);
     float* Sm = b.Smid + (size_t)l * nh(b);
     float* Vm = b.Vmid + (size_t)l * 3 * nh(b);
-    launch_message<H, true>(b, s, msg_grid, Wl, Sl, Vl, Sm, Vm);
+    launch_message<H, true>(b, s, Wl, Sl, Vl, Sm, Vm);
     launch_update_fwd<H>(b, s, lw, Sm, Vm, b.S + (size_t)(l + 1) * nh(b),
                          b.V + (size_t)(l + 1) * 3 * nh(b), b.Aupd + (size_t)l * nh(b),
                          b.G12 + (size_t)l * 2 * nh(b));
@@ -1545,8 +1569,6 @@ hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool wa
   const int N = b.N;
   const float* centers = b.w + mw.centers;
   const float* widths = b.w + mw.widths;
-  const int rows_per_block = kBlock / H;
-  const int msg_grid = ((N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
   Streams st(b, s);
   // gradient w.r.t. the update outputs of the last block: (gS0, 0)
   float* gs2 = b.gS0;
@@ -1564,7 +1586,7 @@ hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool wa
     if (b.use_table && st.two()) launch_filter_table_bwd<H>(b, st.filt, l, l + 1);
     if (direct_filters(b)) launch_filter_bwd<H>(b, st.filt, l);
     if (l > 0) {
-      launch_message<H, false>(b, s, msg_grid, Wl, gS1, gV1, b.gS0, b.gV0);
+      launch_message<H, false>(b, s, Wl, gS1, gV1, b.gS0, b.gV0);
       gs2 = b.gS0;
       gv2 = b.gV0;
     }
@@ -1583,17 +1605,15 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
   const int N = b.N;
   const float* centers = b.w + mw.centers;
   const float* widths = b.w + mw.widths;
-  const int rows_per_block = kBlock / H;
-  const int msg_grid = ((N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
   const LayerW& lw = mw.layer[l];
   float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
   switch (stage) {
     case MLFF_STAGE_FILTER_FWD:
-      if (b.use_table) launch_filter_table_fwd<H>(b, s, l, l + 1);
+      if (b.use_table) launch_filter_table_fwd<H>(b, s, l, l + 1, false);
       if (direct_filters(b)) launch_filter_fwd<H>(b, s, l);
       break;
     case MLFF_STAGE_MESSAGE_FWD:
-      launch_message<H, true>(b, s, msg_grid, Wl, b.S + (size_t)l * nh(b),
+      launch_message<H, true>(b, s, Wl, b.S + (size_t)l * nh(b),
                               b.V + (size_t)l * 3 * nh(b), b.Smid + (size_t)l * nh(b),
                               b.Vmid + (size_t)l * 3 * nh(b));
       break;
@@ -1614,7 +1634,7 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
       if (direct_filters(b)) launch_filter_bwd<H>(b, s, l);
       break;
     case MLFF_STAGE_MESSAGE_BWD:
-      launch_message<H, false>(b, s, msg_grid, Wl, b.gS1 + (size_t)l * nh(b),
+      launch_message<H, false>(b, s, Wl, b.gS1 + (size_t)l * nh(b),
                                b.gV1 + (size_t)l * 3 * nh(b), b.gS0, b.gV0);
       break;
     case MLFF_STAGE_FORCES:
