@@ -397,6 +397,17 @@ int mlff_train_pair_grad(void* stream, int hidden_dim, int n_pairs, const int32_
                          const float* dgs_dev, const float* dgv_dev, float* gw_dev,
                          float* dgw_dev);
 
+/* Groups E directed edges src[e] -> dst[e] (int64, endpoints in [0, N)) by
+ * receiver (list 0) and, with lists = 2, by source (list 1), each group in
+ * ascending edge order: row_ptr [lists][N+1], the other endpoint col
+ * [lists][E] and the edge's index edge_id [lists][E].  ends [2][E] receives
+ * dst and src as int32.  An endpoint out of range sets *bad to 1 and the
+ * edge is in no list.  scratch: lists * (N + E) int32. */
+int mlff_edge_csr(void* stream, int n_edges, int n_atoms, int lists, const int64_t* src_dev,
+                  const int64_t* dst_dev, int32_t* row_ptr_dev, int32_t* col_dev,
+                  int32_t* edge_id_dev, int32_t* ends_dev, int32_t* scratch_dev,
+                  int32_t* bad_dev);
+
 /* PaiNNMessage.forward on a caller-given directed edge list
  * (student_model.py:346-387, the interaction submodules' own forward):
  * each edge e (src -> dst) has its own filter row w[e] [3H] and edge vector

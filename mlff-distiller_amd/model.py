@@ -75,13 +75,22 @@ class CosineCutoff(nn.Module):
         return f * (distances < self.cutoff).to(distances.dtype)
 
 
-def _edge_csr(key: torch.Tensor, other: torch.Tensor, n: int):
-    """Edges grouped by ``key`` (stable, so each group keeps the caller's
-    edge order): row_ptr [n+1], the other endpoint of each edge, its index."""
-    order = torch.sort(key, stable=True).indices
-    row_ptr = torch.zeros(n + 1, dtype=torch.int32, device=key.device)
-    row_ptr[1:] = torch.cumsum(torch.bincount(key, minlength=n), 0).to(torch.int32)
-    return row_ptr, other[order].to(torch.int32).contiguous(), order.to(torch.int32).contiguous()
+def _edge_csr(src: torch.Tensor, dst: torch.Tensor, n: int, lists: int):
+    """Edges grouped by receiver and, with ``lists`` = 2, by source, each group
+    in the caller's edge order (mlff_edge_csr): row_ptr [lists, n+1], the other
+    endpoint and the index of each edge [lists, E], and the endpoints as int32
+    [2, E] (receivers, sources)."""
+    from . import _capi as C
+    E = src.numel()
+    i32 = lambda *shape: torch.empty(*shape, dtype=torch.int32, device=src.device)
+    row_ptr, col, eid, ends = i32(lists, n + 1), i32(lists, E), i32(lists, E), i32(2, E)
+    scratch, bad = i32(lists * (n + E) + 1), i32(1)
+    C.check("mlff_edge_csr", C.lib().mlff_edge_csr(
+        C.stream_handle(), E, n, lists, C.ptr(src.contiguous()), C.ptr(dst.contiguous()),
+        C.ptr(row_ptr), C.ptr(col), C.ptr(eid), C.ptr(ends), C.ptr(scratch), C.ptr(bad)))
+    if E and bad.item():
+        raise ValueError("edge_index refers to atoms outside [0, num_atoms)")
+    return row_ptr, col, eid, ends
 
 
 def _device_f32(*ts):
@@ -94,9 +103,9 @@ def _device_f32(*ts):
 class _EdgeMessage(torch.autograd.Function):
     """The gathers of PaiNNMessage.forward (student_model.py:357-387) on a
     caller-given directed edge list: the receiver-row HIP kernel forward; the
-    backward groups the edges by source for the feature gradients and takes
+    backward takes the edges grouped by source for the feature gradients and
     the filter and edge-vector gradients per edge (all on HIP kernels, fixed
-    order, no atomics)."""
+    order, no float atomics)."""
 
     @staticmethod
     def forward(ctx, s, v, W, ev, src, dst):
@@ -104,38 +113,174 @@ class _EdgeMessage(torch.autograd.Function):
         _device_f32(s, v, W, ev)
         N, H = s.shape
         s, v, W, ev = s.contiguous(), v.contiguous(), W.contiguous(), ev.contiguous()
-        src, dst = src.long(), dst.long()
-        if src.numel() and (int(src.min()) < 0 or int(src.max()) >= N or int(dst.min()) < 0
-                            or int(dst.max()) >= N):
-            raise ValueError("edge_index refers to atoms outside [0, num_atoms)")
-        row_ptr, col, eid = _edge_csr(dst, src, N)
+        row_ptr, col, eid, ends = _edge_csr(src.long(), dst.long(), N,
+                                            2 if any(ctx.needs_input_grad) else 1)
         so, vo = torch.empty_like(s), torch.empty_like(v)
         C.check("mlff_edge_message", C.lib().mlff_edge_message(
             C.stream_handle(), H, N, C.ptr(row_ptr), C.ptr(col), C.ptr(eid), C.ptr(s), C.ptr(v),
             C.ptr(W), C.ptr(ev), C.ptr(so), C.ptr(vo)))
-        ctx.save_for_backward(s, v, W, ev, src, dst)
+        ctx.save_for_backward(s, v, W, ev, ends, row_ptr[-1], col[-1], eid[-1])
         return so, vo
 
     @staticmethod
     def backward(ctx, gso, gvo):
         from . import _capi as C
-        s, v, W, ev, src, dst = ctx.saved_tensors
+        s, v, W, ev, ends, row_ptr, col, eid = ctx.saved_tensors
         N, H = s.shape
-        E = src.numel()
+        E = ends.shape[1]
         gso = torch.zeros_like(s) if gso is None else gso.contiguous().float()
         gvo = torch.zeros_like(v) if gvo is None else gvo.contiguous().float()
-        row_ptr, col, eid = _edge_csr(src, dst, N)
         gs, gv = torch.empty_like(s), torch.empty_like(v)
         C.check("mlff_train_message_adjoint", C.lib().mlff_train_message_adjoint(
             C.stream_handle(), H, N, C.ptr(row_ptr), C.ptr(col), C.ptr(eid), C.ptr(gso),
             C.ptr(gvo), C.ptr(W), None, None, None, C.ptr(gs), C.ptr(gv), None, None))
         gW = torch.empty(E, 3 * H, dtype=torch.float32, device=s.device)
         gev = torch.empty(E, 3, dtype=torch.float32, device=s.device)
-        s32, d32 = src.to(torch.int32).contiguous(), dst.to(torch.int32).contiguous()
         C.check("mlff_edge_grad", C.lib().mlff_edge_grad(
-            C.stream_handle(), H, E, C.ptr(s32), C.ptr(d32), C.ptr(s), C.ptr(v), C.ptr(W),
+            C.stream_handle(), H, E, C.ptr(ends[1]), C.ptr(ends[0]), C.ptr(s), C.ptr(v), C.ptr(W),
             C.ptr(ev), C.ptr(gso), C.ptr(gvo), C.ptr(gW), C.ptr(gev)))
         return gs, gv, gW, gev, None, None
+
+
+_MLP_TYPES = (nn.Linear, nn.SiLU, nn.Linear)
+
+
+def _fused_mlp(seq, *tensors) -> bool:
+    """Whether an MLP block on ``tensors`` may run as one autograd function with
+    its own weight-gradient kernels.  Everything else takes the module path:
+    replaced, hooked or parametrized layers, other types, devices and empty
+    inputs, autocast, tracing, function transforms and forward-mode AD."""
+    if type(seq) is not nn.Sequential or tuple(type(m) for m in seq) != _MLP_TYPES:
+        return False
+    m = nn.modules.module
+    if (m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
+            or m._global_backward_pre_hooks):
+        return False
+    for mod in (seq, *seq):
+        if (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks
+                or mod._backward_pre_hooks or "forward" in mod.__dict__):
+            return False
+    if seq[0].bias is None or seq[2].bias is None:
+        return False
+    for t in (*tensors, seq[0].weight, seq[0].bias, seq[2].weight, seq[2].bias):
+        if (type(t) not in (torch.Tensor, nn.Parameter) or not t.is_cuda or t.numel() == 0
+                or t.dtype != torch.float32):
+            return False
+    return not (torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
+                or torch.compiler.is_compiling()
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
+def _plain_grads(ctx, outputs, inputs, grads):
+    """Gradients of a block that can be differentiated again, from its plain
+    formula (create_graph)."""
+    need = [k for k, on in enumerate(ctx.needs_input_grad) if on]
+    got = torch.autograd.grad(outputs, [inputs[k] for k in need], grads, create_graph=True,
+                              allow_unused=True)
+    out = [None] * len(inputs)
+    for k, g in zip(need, got):
+        out[k] = g
+    return tuple(out)
+
+
+class _EdgeFilter(torch.autograd.Function):
+    """rbf_to_scalar on edge rows: W2 silu(W1 x + b1) + b2.  The weight and bias
+    gradients are sums over all edges; the library product for them runs on a
+    few workgroups (135 us each for 40,000 edges at H = 64), so the backward
+    takes the split-row kernel of the training pass."""
+
+    @staticmethod
+    def forward(ctx, x, w1, b1, w2, b2):
+        a = torch.addmm(b1, x, w1.t())
+        h = nn.functional.silu(a)
+        ctx.save_for_backward(x, w1, b1, w2, b2, a, h)
+        return torch.addmm(b2, h, w2.t())
+
+    @staticmethod
+    def backward(ctx, g):
+        from . import train
+        x, w1, b1, w2, b2, a, h = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            F = nn.functional
+            return _plain_grads(ctx, F.linear(F.silu(F.linear(x, w1, b1)), w2, b2),
+                                (x, w1, b1, w2, b2), g)
+        need = ctx.needs_input_grad
+        g = g.contiguous()
+        grp = train._WgGroup()
+        gx = gw1 = gb1 = gw2 = gb2 = None
+        if need[3] or need[4]:
+            gw2, gb2 = train._wgrad(g, h, bias=True, group=grp)
+        if any(need[:3]):
+            ga = torch.ops.aten.silu_backward(g @ w2, a)
+            if need[1] or need[2]:
+                gw1, gb1 = train._wgrad(ga, x, bias=True, group=grp)
+            if need[0]:
+                gx = ga @ w1
+        grp.flush()
+        return tuple(t if on else None for t, on in zip((gx, gw1, gb1, gw2, gb2), need))
+
+
+def _update_plain(s, v, w1, b1, w2, b2, mix):
+    F = nn.functional
+    H = s.shape[1]
+    norms = torch.linalg.vector_norm(v, dim=1)
+    upd = F.linear(F.silu(F.linear(torch.cat([s, norms], dim=-1), w1, b1)), w2, b2)
+    ds, g1, g2 = upd[:, :H], upd[:, H:2 * H], upd[:, 2 * H:]
+    return s + ds, v * g1.unsqueeze(1) + torch.matmul(mix, v) * g2.unsqueeze(1)
+
+
+class _UpdateBlock(torch.autograd.Function):
+    """PaiNNUpdate.forward on the elementwise and weight-gradient kernels of the
+    training pass (the library's product for the 3x3 mixing gradient alone took
+    220 us for 1,700 atoms at H = 64)."""
+
+    @staticmethod
+    def forward(ctx, s, v, w1, b1, w2, b2, mix):
+        from . import train
+        n, H = s.shape
+        xin = torch.empty(n, 2 * H, dtype=torch.float32, device=s.device)
+        train._glue("mlff_update_norm", n, H, s, v, xin)
+        a = torch.addmm(b1, xin, w1.t())
+        h = nn.functional.silu(a)
+        y = torch.addmm(b2, h, w2.t())
+        so = torch.empty(n, H, dtype=torch.float32, device=s.device)
+        vo = torch.empty(n, 3, H, dtype=torch.float32, device=s.device)
+        mv = torch.empty_like(vo)
+        train._glue("mlff_update_apply", n, H, mix, y, s, v, so, vo, mv)
+        ctx.save_for_backward(s, v, w1, b1, w2, b2, mix, xin, a, h, y, mv)
+        return so, vo
+
+    @staticmethod
+    def backward(ctx, gs, gv):
+        from . import train
+        s, v, w1, b1, w2, b2, mix, xin, a, h, y, mv = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            ins = (s, v, w1, b1, w2, b2, mix)
+            return _plain_grads(ctx, _update_plain(*ins), ins, (gs, gv))
+        need = ctx.needs_input_grad
+        n, H = s.shape
+        gs, gv = train._dense(gs), train._dense(gv)
+        new = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=s.device)
+        gy = new(n, 3 * H)
+        train._glue("mlff_update_gate_adjoint", n, H, gs, gv, v, mv, None, None, None, None, gy,
+                    None)
+        ga = torch.ops.aten.silu_backward(gy @ w2, a)
+        gx = ga @ w1
+        gso, gvo, gvg2 = new(n, H), new(n, 3, H), new(n, 3, H)
+        train._glue("mlff_update_input_adjoint", n, H, mix, gx, gs, gv, y, v, xin, None, None,
+                    None, None, None, None, gso, gvo, gvg2, None, None, None)
+        grp = train._WgGroup()
+        gw1 = gb1 = gw2 = gb2 = gm = None
+        if need[4] or need[5]:
+            gw2, gb2 = train._wgrad(gy, h, bias=True, group=grp)
+        if need[2] or need[3]:
+            gw1, gb1 = train._wgrad(ga, xin, bias=True, group=grp)
+        if need[6]:
+            gm = train._xyz_outer(gvg2, v, group=grp)
+        grp.flush()
+        return tuple(t if on else None
+                     for t, on in zip((gso, gvo, gw1, gb1, gw2, gb2, gm), need))
 
 
 class PaiNNMessage(nn.Module):
@@ -154,7 +299,12 @@ class PaiNNMessage(nn.Module):
                 edge_vector: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         """s_i + sum_{j->i} s_j Ws, v_i + sum_{j->i} (v_j Wv1 + e_ji (x) Wv2)
         with (Ws, Wv1, Wv2) = rbf_to_scalar(edge_rbf) per edge."""
-        filt = self.rbf_to_scalar(edge_rbf)
+        mlp = self.rbf_to_scalar
+        if edge_rbf.dim() == 2 and _fused_mlp(mlp, edge_rbf):
+            filt = _EdgeFilter.apply(edge_rbf, mlp[0].weight, mlp[0].bias, mlp[2].weight,
+                                     mlp[2].bias)
+        else:
+            filt = mlp(edge_rbf)
         return _EdgeMessage.apply(scalar_features, vector_features, filt, edge_vector,
                                   edge_index[0], edge_index[1])
 
@@ -175,6 +325,11 @@ class PaiNNUpdate(nn.Module):
                 vector_features: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         _device_f32(scalar_features, vector_features)
         H = self.hidden_dim
+        n, mlp, mix = scalar_features.shape[0], self.update_mlp, self.mixing_matrix
+        if (H % 4 == 0 and scalar_features.shape == (n, H) and vector_features.shape == (n, 3, H)
+                and mix.shape == (3, 3) and _fused_mlp(mlp, scalar_features, vector_features, mix)):
+            return _UpdateBlock.apply(scalar_features, vector_features, mlp[0].weight,
+                                      mlp[0].bias, mlp[2].weight, mlp[2].bias, mix)
         norms = torch.linalg.vector_norm(vector_features, dim=1)
         upd = self.update_mlp(torch.cat([scalar_features, norms], dim=-1))
         ds, g1, g2 = upd[:, :H], upd[:, H:2 * H], upd[:, 2 * H:]

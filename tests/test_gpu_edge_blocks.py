@@ -1,0 +1,72 @@
+"""Interaction blocks on a caller-given edge list: the grouping kernels and the
+blocks' own autograd functions against torch's sort and the module path."""
+import pytest
+import torch
+
+from conftest import pkg_mod
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sizes", [[0, 1, 0], [64, 65, 63, 0], [2048, 2049, 5], [300] * 40, [1]])
+def test_edge_groups_equal_a_stable_sort(gpu, sizes):
+    """Every row form (registers, ranking, scan), empty rows, duplicate edges."""
+    print(f"[case] edge groups {sizes[:4]}", flush=True)
+    model = pkg_mod("model")
+    n = len(sizes)
+    gen = torch.Generator().manual_seed(1)
+    dst = torch.repeat_interleave(torch.arange(n), torch.tensor(sizes))
+    dst = dst[torch.randperm(len(dst), generator=gen)].to(gpu)
+    src = torch.randint(0, n, (len(dst),), generator=gen).to(gpu)
+    row_ptr, col, eid, ends = model._edge_csr(src, dst, n, 2)
+    assert torch.equal(ends[0].long(), dst) and torch.equal(ends[1].long(), src)
+    for l, (key, other) in enumerate(((dst, src), (src, dst))):
+        order = torch.sort(key, stable=True).indices
+        assert torch.equal(eid[l].long(), order) and torch.equal(col[l].long(), other[order])
+        assert torch.equal(row_ptr[l, 1:].long(), torch.cumsum(torch.bincount(key, minlength=n), 0))
+
+
+@pytest.mark.parametrize("bad", [-1, 5])
+def test_edges_out_of_range_are_refused(gpu, bad):
+    print(f"[case] edge out of range {bad}", flush=True)
+    model = pkg_mod("model")
+    ok = torch.tensor([0, 1, 2], device=gpu)
+    for src, dst in ((torch.tensor([0, bad, 1], device=gpu), ok),
+                     (ok, torch.tensor([0, 1, bad], device=gpu))):
+        with pytest.raises(ValueError, match="outside"):
+            model._edge_csr(src, dst, 5, 2)
+
+
+@pytest.mark.parametrize("H,R,n,E", [(64, 20, 50, 3000), (32, 9, 3, 1), (128, 32, 70, 2049)])
+def test_blocks_equal_the_module_path(gpu, H, R, n, E):
+    """A forward hook takes the module path.  Outputs, gradients and gradients of
+    a gradient norm agree to 2e-5 of their norm: sums of up to 3,000 float32
+    products have an error of about sqrt(3000) 2^-24 = 3.3e-6."""
+    print(f"[case] blocks H{H} R{R} n{n} E{E}", flush=True)
+    model = pkg_mod("model")
+    torch.manual_seed(5)
+    blk = model.PaiNNInteraction(H, R).to(gpu)
+    ins = [torch.randn(*sh, device=gpu).requires_grad_(True)
+           for sh in ((n, H), (n, 3, H), (E, R), (E, 3))]
+    edges = torch.randint(0, n, (2, E), device=gpu)
+    leaves = ins + list(blk.parameters())
+    gs, gv = torch.randn(n, H, device=gpu), torch.randn(n, 3, H, device=gpu)
+
+    def run():
+        out = blk(ins[0], ins[1], edges, ins[2], ins[3])
+        first = torch.autograd.grad(out, leaves, (gs, gv), retain_graph=True)
+        s, v = blk.update(ins[0], ins[1])
+        g = torch.autograd.grad((s * gs).sum() + (v * gv).sum(), ins[:2], create_graph=True)
+        second = torch.autograd.grad(sum((t ** 2).sum() for t in g),
+                                     ins[:2] + list(blk.update.parameters()))
+        return list(out) + list(first) + list(second)
+
+    fused = run()
+    names = [type(t.grad_fn).__name__ for t in blk.update(ins[0], ins[1])]
+    assert names[0].startswith("_UpdateBlock")
+    for seq in (blk.message.rbf_to_scalar, blk.update.update_mlp):
+        seq.register_forward_hook(lambda *a: None)
+    plain = run()
+    assert not type(blk.update(ins[0], ins[1])[0].grad_fn).__name__.startswith("_UpdateBlock")
+    for k, (a, b) in enumerate(zip(fused, plain)):
+        assert (a - b).norm() <= 2e-5 * b.norm() + 1e-30, k
