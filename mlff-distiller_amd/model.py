@@ -425,8 +425,23 @@ class _Session:
         from . import train
         p, g, c = self._prepared()
         _, tg = train.reverse(p, c, g, gE.reshape(-1), lam=self._to_sorted(lam),
-                              rbf_grads=self._rbf_grads())
+                              rbf_grads=self._rbf_grads(), primal=False)
         return tg
+
+
+def _any_runs(nodes) -> bool:
+    """Whether the backward pass that is running goes on to any of ``nodes``.
+    A gradient with respect to the positions alone does not visit the
+    parameters', though they require grad."""
+    for node, _ in nodes:
+        if node is None:
+            continue
+        try:
+            if torch._C._will_engine_execute_node(node):
+                return True
+        except RuntimeError:   # a leaf whose gradient the call asked for
+            return True
+    return False
 
 
 def _grads_tuple(names, grads, params):
@@ -462,7 +477,7 @@ class _TrainableEnergy(torch.autograd.Function):
                 g = g[s.batch_index] if s.batch_index is not None else g.expand(s.forces.shape[0])
                 g_pos = -s.forces * g.unsqueeze(1)
         pg = (None,) * len(ctx.names)
-        if any(ctx.needs_input_grad[3:]):
+        if any(ctx.needs_input_grad[3:]) and _any_runs(ctx.next_functions[1:]):
             params = [p for _, p in s.model.named_parameters()]
             pg = _grads_tuple(ctx.names, s.param_grads(gE_vec.detach()), params)
         return (g_pos, None, None) + pg

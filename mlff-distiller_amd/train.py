@@ -661,11 +661,12 @@ def _z_segments(Z: Tensor, n_rows: int):
 
 def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
             lam: Optional[Tensor] = None, gw: Optional[Tensor] = None,
-            rbf_grads: bool = False):
+            rbf_grads: bool = False, primal: bool = True):
     """Parameter gradients of sum_b gw_b E_b (gw defaults to gE) and -- with
     the tangent along ``lam`` [N,3] (reused from the cache when forward()
     already computed it for the same lam) -- the parameter gradients of
-    < lam, grad_x (sum_b gE_b E_b) >.  Returns (grads, tgrads or None).
+    < lam, grad_x (sum_b gE_b E_b) >.  Returns (grads, tgrads or None); without
+    ``primal`` the tangent's only ({}, tgrads).
 
     gw is applied as a per-row weight on the gE adjoint (structures do not
     interact), so gE must then be all ones.  ``rbf_grads`` adds the basis
@@ -703,9 +704,10 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
     geps = gE[g.batch]
     r1, h3, r2, h4, sL = c["r1"], c["h3"], c["r2"], c["h4"], c["sL"]
     Q3 = p["energy_head.4.weight"]
-    wgeps = wa(geps)
-    acc(grads, "energy_head.4.weight", (wgeps @ h4).reshape(1, -1))
-    acc(grads, "energy_head.4.bias", wgeps.sum().reshape(1))
+    if primal:
+        wgeps = wa(geps)
+        acc(grads, "energy_head.4.weight", (wgeps @ h4).reshape(1, -1))
+        acc(grads, "energy_head.4.bias", wgeps.sum().reshape(1))
     gh4 = geps.unsqueeze(1) * Q3
     R2w, R1w = p["energy_head.2.weight"], p["energy_head.0.weight"]
     if T:
@@ -723,12 +725,13 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         gr2 = _silu_d(r2, gh4)
         gr1 = _silu_d(r1, gr2 @ R2w)
         gs = (gr1 @ R1w).contiguous()
-    gw_, gb_ = _wgrad(gr2, h3, w=w_atom, bias=True, group=grp)
-    acc(grads, "energy_head.2.weight", gw_)
-    acc(grads, "energy_head.2.bias", gb_)
-    gw_, gb_ = _wgrad(gr1, sL, w=w_atom, bias=True, group=grp)
-    acc(grads, "energy_head.0.weight", gw_)
-    acc(grads, "energy_head.0.bias", gb_)
+    if primal:
+        gw_, gb_ = _wgrad(gr2, h3, w=w_atom, bias=True, group=grp)
+        acc(grads, "energy_head.2.weight", gw_)
+        acc(grads, "energy_head.2.bias", gb_)
+        gw_, gb_ = _wgrad(gr1, sL, w=w_atom, bias=True, group=grp)
+        acc(grads, "energy_head.0.weight", gw_)
+        acc(grads, "energy_head.0.bias", gb_)
     gv = torch.zeros(n, 3, H, dtype=torch.float32, device=dev)
     if T:
         acc(tg, "energy_head.4.weight", (geps @ dh4).reshape(1, -1))
@@ -768,12 +771,13 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         else:
             ga2 = _silu_d(lay["a2"], gy @ U2)
             gx, dgx = ga2 @ U1, None
-        gw_, gb_ = _wgrad(gy, lay["h2"], w=w_atom, bias=True, group=grp)
-        acc(grads, upre + ".update_mlp.2.weight", gw_)
-        acc(grads, upre + ".update_mlp.2.bias", gb_)
-        gw_, gb_ = _wgrad(ga2, xin, w=w_atom, bias=True, group=grp)
-        acc(grads, upre + ".update_mlp.0.weight", gw_)
-        acc(grads, upre + ".update_mlp.0.bias", gb_)
+        if primal:
+            gw_, gb_ = _wgrad(gy, lay["h2"], w=w_atom, bias=True, group=grp)
+            acc(grads, upre + ".update_mlp.2.weight", gw_)
+            acc(grads, upre + ".update_mlp.2.bias", gb_)
+            gw_, gb_ = _wgrad(ga2, xin, w=w_atom, bias=True, group=grp)
+            acc(grads, upre + ".update_mlp.0.weight", gw_)
+            acc(grads, upre + ".update_mlp.0.bias", gb_)
         if T:
             gw_, gb_ = _wgrad(dgy, lay["h2"], gy, lay["dh2"], bias=True, group=grp)
             acc(tg, upre + ".update_mlp.2.weight", gw_)
@@ -790,7 +794,8 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         _glue("mlff_update_input_adjoint", n, H, M, gx, gs, gv, y, v_m, xin, dgx,
               dgs if T else None, dgv if T else None, lay["dy"] if T else None, dvm, dxin,
               gs_m, gv_m, gvg2, dgs_m, dgv_m, dgvg2)
-        acc(grads, upre + ".mixing_matrix", _xyz_outer(gvg2, v_m, w=w_atom, group=grp))
+        if primal:
+            acc(grads, upre + ".mixing_matrix", _xyz_outer(gvg2, v_m, w=w_atom, group=grp))
         if T:
             acc(tg, upre + ".mixing_matrix", _xyz_outer(dgvg2, v_m, gvg2, dvm, group=grp))
         # message reverse (student_model.py:346-387): filter-output gradients per pair
@@ -801,19 +806,21 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         else:
             gW, _ = _pair_grad(g, H, u, s, v, gs_m, gv_m)
         W1 = p[mpre + ".0.weight"]
-        gw_, gb_ = _wgrad(gW, lay["h"], w=w_pair, bias=True, group=grp)
-        acc(grads, mpre + ".2.weight", gw_)
-        acc(grads, mpre + ".2.bias", gb_)
+        if primal:
+            gw_, gb_ = _wgrad(gW, lay["h"], w=w_pair, bias=True, group=grp)
+            acc(grads, mpre + ".2.weight", gw_)
+            acc(grads, mpre + ".2.bias", gb_)
         # gW W2 through the SiLU (and its tangent) on the fused pair kernel
         ga1, dga1 = _filter_adjoint(p, mpre, gW, lay["a1"], dgW if T else None,
                                     lay["da1"] if T else None)
-        gw_, gb_ = _wgrad(ga1, c["e"], w=w_pair, bias=True, group=grp)
-        acc(grads, mpre + ".0.weight", gw_)
-        acc(grads, mpre + ".0.bias", gb_)
-        if rbf_grads:
-            ge = ga1 @ W1
-            acc(grads, "rbf.centers", (wp(ge) * e_mu).sum(0))
-            acc(grads, "rbf.widths", (wp(ge) * e_w).sum(0))
+        ge = ga1 @ W1 if rbf_grads else None
+        if primal:
+            gw_, gb_ = _wgrad(ga1, c["e"], w=w_pair, bias=True, group=grp)
+            acc(grads, mpre + ".0.weight", gw_)
+            acc(grads, mpre + ".0.bias", gb_)
+            if rbf_grads:
+                acc(grads, "rbf.centers", (wp(ge) * e_mu).sum(0))
+                acc(grads, "rbf.widths", (wp(ge) * e_w).sum(0))
         if T:
             dh = lay["dh"]
             gw_, gb_ = _wgrad(dgW, lay["h"], gW, dh, bias=True, group=grp)
@@ -832,7 +839,8 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
             gs, gv, _, _ = _message_adjoint(g, H, gs_m, gv_m, W)
     emb_rows = p["embedding.weight"].shape[0]
     zptr, zorder = _z_segments(c["Z"], emb_rows)
-    acc(grads, "embedding.weight", _segment_sum(zptr, wa(gs), zorder))
+    if primal:
+        acc(grads, "embedding.weight", _segment_sum(zptr, wa(gs), zorder))
     if T:
         acc(tg, "embedding.weight", _segment_sum(zptr, dgs, zorder))
     grp.flush()
