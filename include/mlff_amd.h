@@ -461,6 +461,17 @@ int mlff_weight_grad(void* stream, int K, int M, int N, const float* a0_dev, int
                      const float* b1_dev, int ldb1, const float* row_w_dev, void* ws_dev,
                      size_t ws_bytes, float* out_dev, float* bias_out_dev);
 
+/* The two weight gradients of a force-matching step in one (the weighted sum
+ * of a1 (x) b0, less a0 (x) b0 + a1 (x) b1), as partials like
+ * mlff_weight_grad_partials: with c = row_w a1 - a0,
+ *   out[m][n] = sum_k (c[k][m] b0[k][n] - a1[k][m] b1[k][n]),  bias[m] = sum_k c[k][m].
+ * All operands are needed. */
+int mlff_weight_grad_diff_partials(void* stream, int K, int M, int N, const float* a0_dev,
+                                   int lda0, const float* b0_dev, int ldb0, const float* a1_dev,
+                                   int lda1, const float* b1_dev, int ldb1,
+                                   const float* row_w_dev, int with_bias, void* ws_dev,
+                                   size_t ws_bytes);
+
 /* The same weight gradients in two steps, so that the partial sums of many
  * gradients (one training pass's) are added by one launch.  The products the
  * reference's backward computes are the same as for mlff_weight_grad.
@@ -524,6 +535,11 @@ int mlff_xyz_outer_partial_count(int n_atoms);
 int mlff_xyz_outer_partials(void* stream, int n_atoms, int hidden, const float* a0_dev,
                             const float* b0_dev, const float* a1_dev, const float* b1_dev,
                             const float* row_w_dev, float* part_dev);
+
+/* mlff_xyz_outer_partials of (row_w a1 - a0) with b0, less a1 with b1. */
+int mlff_xyz_outer_diff_partials(void* stream, int n_atoms, int hidden, const float* a0_dev,
+                                 const float* b0_dev, const float* a1_dev, const float* b1_dev,
+                                 const float* row_w_dev, float* part_dev);
 
 /* The filter MLP of PaiNNMessage (student_model.py:313-322, 350-355) over
  * n_pairs pairs in the training pass, fused in one pair-tile kernel:

@@ -437,7 +437,12 @@ __global__ __launch_bounds__(kTrainBlock) void segment_sum_kernel(
 // ---------------------------------------------------------------------------
 // Weight gradients over K rows (pairs or atoms):
 //   out[m][n] = sum_k w_k (a0[k][m] b0[k][n] + a1[k][m] b1[k][n]),
-//   bias[m]   = sum_k w_k a0[k][m].
+//   bias[m]   = sum_k w_k a0[k][m],
+// or, DIFF (a force-matching step's two gradients in one: the weighted sum of
+// a1 (x) b0 less the tangent's a0 (x) b0 + a1 (x) b1), with c = w a1 - a0,
+//   out[m][n] = sum_k (c[k][m] b0[k][n] - a1[k][m] b1[k][n]),
+//   bias[m]   = sum_k c[k][m]:
+// two products per row instead of three, each operand read once.
 //
 // One wave owns a 64 x 64 output tile over RW consecutive rows; the four waves
 // of a block take four consecutive row ranges of the same tile, and waves 1-3
@@ -504,7 +509,7 @@ struct WgBatch {
   }
 };
 
-template <bool TWO, bool ROWW, bool BIAS>
+template <bool TWO, bool ROWW, bool BIAS, bool DIFF>
 __global__ __launch_bounds__(64 * kWgWaves, 3) void weight_grad_kernel(
     int K, int M, int N, int RW, int tiles_m, int tiles_n, int S,
     const float* __restrict__ a0, int lda0, const float* __restrict__ b0, int ldb0,
@@ -555,8 +560,13 @@ __global__ __launch_bounds__(64 * kWgWaves, 3) void weight_grad_kernel(
         }
         if (ROWW) {
           const float w = kok ? cur.w[u] : 0.f;
-          a = a * w;
-          if (TWO) a2 = a2 * w;
+          if (DIFF) {
+            a = fma_(w, a2, -a);
+            a2 = -a2;
+          } else {
+            a = a * w;
+            if (TWO) a2 = a2 * w;
+          }
         }
         if (BIAS) cs += a;
         wg_mfma(acc, a, b);
@@ -709,17 +719,17 @@ void weight_grad_split(int K, int M, int N, int& RW, int& S) {
   S = K > 0 ? (int)(((long)K + 4 * rw - 1) / (4 * rw)) : 1;
 }
 
-template <bool TWO, bool ROWW>
+template <bool TWO, bool ROWW, bool DIFF = false>
 void launch_weight_grad(hipStream_t st, bool bias, int blocks, int K, int M, int N, int RW,
                         int tiles_m, int tiles_n, int S, const float* a0, int lda0,
                         const float* b0, int ldb0, const float* a1, int lda1, const float* b1,
                         int ldb1, const float* roww, float* part, float* part_bias) {
   if (bias)
-    weight_grad_kernel<TWO, ROWW, true><<<blocks, 64 * kWgWaves, 0, st>>>(
+    weight_grad_kernel<TWO, ROWW, true, DIFF><<<blocks, 64 * kWgWaves, 0, st>>>(
         K, M, N, RW, tiles_m, tiles_n, S, a0, lda0, b0, ldb0, a1, lda1, b1, ldb1, roww, part,
         part_bias);
   else
-    weight_grad_kernel<TWO, ROWW, false><<<blocks, 64 * kWgWaves, 0, st>>>(
+    weight_grad_kernel<TWO, ROWW, false, DIFF><<<blocks, 64 * kWgWaves, 0, st>>>(
         K, M, N, RW, tiles_m, tiles_n, S, a0, lda0, b0, ldb0, a1, lda1, b1, ldb1, roww, part,
         part_bias);
 }
@@ -1140,7 +1150,7 @@ static int weight_grad_partials(const char* who, void* stream, int K, int M, int
                                 const float* a0_dev, int lda0, const float* b0_dev, int ldb0,
                                 const float* a1_dev, int lda1, const float* b1_dev, int ldb1,
                                 const float* row_w_dev, bool bias, void* ws_dev,
-                                size_t ws_bytes, int* s_out) {
+                                size_t ws_bytes, int* s_out, bool diff = false) {
   if (K < 0 || M < 4 || N < 4 || M % 4 || N % 4) {
     set_error("%s: need K >= 0 and M, N positive multiples of 4 (K=%d M=%d N=%d)", who, K, M,
               N);
@@ -1174,7 +1184,11 @@ static int weight_grad_partials(const char* who, void* stream, int K, int M, int
   const int blocks = (tiles_m * tiles_n * S + 7) / 8 * 8;
   float* part = static_cast<float*>(ws_dev);
   float* part_bias = part + (size_t)S * M * N;
-  if (two && row_w_dev)
+  if (diff)
+    launch_weight_grad<true, true, true>(st, bias, blocks, K, M, N, RW, tiles_m, tiles_n, S, a0_dev,
+                                         lda0, b0_dev, ldb0, a1_dev, lda1, b1_dev, ldb1, row_w_dev,
+                                         part, part_bias);
+  else if (two && row_w_dev)
     launch_weight_grad<true, true>(st, bias, blocks, K, M, N, RW, tiles_m, tiles_n, S, a0_dev,
                                    lda0, b0_dev, ldb0, a1_dev, lda1, b1_dev, ldb1, row_w_dev,
                                    part, part_bias);
@@ -1242,6 +1256,29 @@ int mlff_weight_grad_partials(void* stream, int K, int M, int N, const float* a0
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error("mlff_weight_grad_partials: %s", hipGetErrorString(e));
+    return MLFF_ERR_HIP;
+  }
+  return MLFF_OK;
+}
+
+int mlff_weight_grad_diff_partials(void* stream, int K, int M, int N, const float* a0_dev,
+                                   int lda0, const float* b0_dev, int ldb0, const float* a1_dev,
+                                   int lda1, const float* b1_dev, int ldb1,
+                                   const float* row_w_dev, int with_bias, void* ws_dev,
+                                   size_t ws_bytes) {
+  const char* nm = "mlff_weight_grad_diff_partials";
+  if (!a1_dev || !row_w_dev) {
+    set_error("%s: need a1, b1 and row weights", nm);
+    return MLFF_ERR_INVALID;
+  }
+  int S = 0;
+  const int rc = weight_grad_partials(nm, stream, K, M, N, a0_dev, lda0, b0_dev, ldb0, a1_dev,
+                                      lda1, b1_dev, ldb1, row_w_dev, with_bias != 0, ws_dev,
+                                      ws_bytes, &S, true);
+  if (rc != MLFF_OK) return rc;
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error("%s: %s", nm, hipGetErrorString(e));
     return MLFF_ERR_HIP;
   }
   return MLFF_OK;

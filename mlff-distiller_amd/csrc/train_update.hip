@@ -266,7 +266,8 @@ int xyz_atoms(int n) {
 }
 int xyz_parts(int n) { return n > 0 ? (n + xyz_atoms(n) - 1) / xyz_atoms(n) : 1; }
 
-template <bool TWO, bool ROWW>
+// DIFF, with c = w a1 - a0: sum_n sum_h (c[n][x][h] b0[n][z][h] - a1[n][x][h] b1[n][z][h]).
+template <bool TWO, bool ROWW, bool DIFF = false>
 __global__ __launch_bounds__(kGlueBlock) void xyz_outer_kernel(
     int n, int H, int A, const float* __restrict__ a0, const float* __restrict__ b0,
     const float* __restrict__ a1, const float* __restrict__ b1, const float* __restrict__ w,
@@ -289,6 +290,13 @@ __global__ __launch_bounds__(kGlueBlock) void xyz_outer_kernel(
       load3(b1, i, H, c, bv1);
     }
     const float wi = ROWW ? w[i] : 1.f;
+    if (DIFF) {
+#pragma unroll
+      for (int x = 0; x < 3; ++x) {
+        av[x] = fma_(wi, av1[x], -av[x]);
+        av1[x] = -av1[x];
+      }
+    }
 #pragma unroll
     for (int x = 0; x < 3; ++x)
 #pragma unroll
@@ -299,7 +307,7 @@ __global__ __launch_bounds__(kGlueBlock) void xyz_outer_kernel(
           const f4 q1 = av1[x] * bv1[z];
           d += (q1[0] + q1[1]) + (q1[2] + q1[3]);
         }
-        acc[3 * x + z] += ROWW ? wi * d : d;
+        acc[3 * x + z] += ROWW && !DIFF ? wi * d : d;
       }
   }
 #pragma unroll
@@ -481,6 +489,23 @@ int mlff_update_input_adjoint(void* stream, int n_atoms, int hidden, const float
 }
 
 int mlff_xyz_outer_partial_count(int n_atoms) { return n_atoms < 0 ? 0 : xyz_parts(n_atoms); }
+
+int mlff_xyz_outer_diff_partials(void* stream, int n_atoms, int hidden, const float* a0_dev,
+                                 const float* b0_dev, const float* a1_dev, const float* b1_dev,
+                                 const float* row_w_dev, float* part_dev) {
+  const char* nm = "mlff_xyz_outer_diff_partials";
+  if (int rc = check_glue(nm, n_atoms, hidden, {part_dev},
+                          {a0_dev, b0_dev, a1_dev, b1_dev, part_dev}))
+    return rc;
+  if (n_atoms > 0 && (!a0_dev || !b0_dev || !a1_dev || !b1_dev || !row_w_dev)) {
+    set_error("%s: null buffer", nm);
+    return MLFF_ERR_INVALID;
+  }
+  xyz_outer_kernel<true, true, true><<<xyz_parts(n_atoms), kGlueBlock, 0,
+                                       static_cast<hipStream_t>(stream)>>>(
+      n_atoms, hidden, xyz_atoms(n_atoms), a0_dev, b0_dev, a1_dev, b1_dev, row_w_dev, part_dev);
+  return finish(nm);
+}
 
 int mlff_xyz_outer_partials(void* stream, int n_atoms, int hidden, const float* a0_dev,
                             const float* b0_dev, const float* a1_dev, const float* b1_dev,

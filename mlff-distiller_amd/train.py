@@ -477,13 +477,16 @@ class _WgGroup:
 
 
 def _wgrad(a0: Tensor, b0: Tensor, a1: Optional[Tensor] = None, b1: Optional[Tensor] = None,
-           w: Optional[Tensor] = None, bias: bool = False, group: Optional[_WgGroup] = None):
+           w: Optional[Tensor] = None, bias: bool = False, group: Optional[_WgGroup] = None,
+           diff: bool = False):
     """sum_k w_k (a0[k] (x) b0[k] + a1[k] (x) b1[k]) [M, N] and, with
     ``bias``, sum_k w_k a0[k] [M] over the K rows (pairs or atoms): a Linear
     layer's weight and bias gradients, on the MFMA kernel with a fixed split
     and order of the row sum (mlff_weight_grad).  Returns (weight, bias or
     None).  With ``group`` only the partial sums are launched here; the
-    outputs are filled, with the same bits, by group.flush()."""
+    outputs are filled, with the same bits, by group.flush().  ``diff`` (with a
+    group): (w a1 - a0) (x) b0 - a1 (x) b1 and the sum of w a1 - a0
+    (mlff_weight_grad_diff_partials)."""
     M, N = a0.shape[1], b0.shape[1]
     K = a0.shape[0]
     A0, B0 = _wg_operand(a0), _wg_operand(b0)
@@ -511,8 +514,8 @@ def _wgrad(a0: Tensor, b0: Tensor, a1: Optional[Tensor] = None, b1: Optional[Ten
         C.check("mlff_weight_grad", lib.mlff_weight_grad(
             *operands, buf.data_ptr(), ws_floats * 4, out.data_ptr(), C.ptr(bout)))
     else:
-        C.check("mlff_weight_grad_partials", lib.mlff_weight_grad_partials(
-            *operands, int(bias), buf.data_ptr(), ws_floats * 4))
+        fn = "mlff_weight_grad_diff_partials" if diff else "mlff_weight_grad_partials"
+        C.check(fn, getattr(lib, fn)(*operands, int(bias), buf.data_ptr(), ws_floats * 4))
         S = _WG_S.get(key)
         if S is None:
             S = _WG_S[key] = int(lib.mlff_weight_grad_partial_count(K, M4, N4))
@@ -530,18 +533,21 @@ def _lin(x, p, name):
     return torch.addmm(p[name + ".bias"], x, p[name + ".weight"].T)
 
 
-def _xyz_outer(a, b, a1=None, b1=None, w=None, group: Optional[_WgGroup] = None):
+def _xyz_outer(a, b, a1=None, b1=None, w=None, group: Optional[_WgGroup] = None,
+               diff: bool = False):
     """sum_n w_n sum_h (a[n,x,h] b[n,z,h] + a1[n,x,h] b1[n,z,h]) -> [3,3]
     (gradient of a 3x3 mixing matrix), on one partial-sum kernel
     (mlff_xyz_outer_partials) whose partials the weight-gradient reduce adds:
-    at ``group``'s flush when one is given, else at once."""
+    at ``group``'s flush when one is given, else at once.  ``diff`` as in
+    _wgrad."""
     n, _, H = a.shape
     lib = C.lib()
     S = int(lib.mlff_xyz_outer_partial_count(n))
     buf = torch.empty(12 * S + 12, dtype=torch.float32, device=a.device)
     opt = lambda t: None if t is None else _dense(t)
     wv = None if w is None else _dense(w.to(torch.float32))
-    C.check("mlff_xyz_outer_partials", lib.mlff_xyz_outer_partials(
+    fn = "mlff_xyz_outer_diff_partials" if diff else "mlff_xyz_outer_partials"
+    C.check(fn, getattr(lib, fn)(
         C.stream_handle(), n, H, C.ptr(_dense(a)), C.ptr(_dense(b)), C.ptr(opt(a1)),
         C.ptr(opt(b1)), C.ptr(wv), buf.data_ptr()))
     out = buf[12 * S:]
@@ -559,7 +565,9 @@ def _xyz_outer(a, b, a1=None, b1=None, w=None, group: Optional[_WgGroup] = None)
 def forward(p: Dict[str, Tensor], Z: Tensor, x: Tensor, g: PairGraph, rc: float,
             lam: Optional[Tensor] = None):
     """Primal pass (student_model.py:634-757); returns (E [B] float64, cache).
-    With ``lam`` [N,3] the tangent along lam is computed too."""
+    With ``lam`` [N,3] the tangent along lam is computed too, block by block
+    beside the primal pass: the message kernel's tangent form gives both, so
+    a block's filters are read once."""
     H = p["embedding.weight"].shape[1]
     L = len({int(k.split(".")[1]) for k in p if k.startswith("interactions.")})
     n = Z.shape[0]
@@ -568,10 +576,18 @@ def forward(p: Dict[str, Tensor], Z: Tensor, x: Tensor, g: PairGraph, rc: float,
     s = p["embedding.weight"][Z].contiguous()
     v = torch.zeros(n, 3, H, dtype=torch.float32, device=x.device)
     layers = []
+    cache = dict(H=H, L=L, n=n, x=x, vec=vec, d=d, den=den, u=u, e=e, de=de, layers=layers,
+                 Z=Z, rc=rc, lam=None)
+    t = None if lam is None else _Tangent(p, cache, lam)
     for k in range(L):
         pre = f"interactions.{k}.message.rbf_to_scalar"
         a1, h, W = _filter(p, pre, e)
-        s_m, v_m, _, _ = _message(g, H, s, v, W, u)
+        lay = dict(s=s, v=v, a1=a1, h=h, W=W)
+        layers.append(lay)
+        if t is None:
+            s_m, v_m, _, _ = _message(g, H, s, v, W, u)
+        else:
+            s_m, v_m = t.message(k, g)
         upre = f"interactions.{k}.update"
         # PaiNNUpdate.forward (student_model.py:430-470)
         xin = torch.empty(n, 2 * H, dtype=torch.float32, device=x.device)
@@ -584,8 +600,9 @@ def forward(p: Dict[str, Tensor], Z: Tensor, x: Tensor, g: PairGraph, rc: float,
         v_new = torch.empty_like(v_m)
         Mv = torch.empty_like(v_m)
         _glue("mlff_update_apply", n, H, M, y, s_m, v_m, s_new, v_new, Mv)
-        layers.append(dict(s=s, v=v, a1=a1, h=h, W=W, s_m=s_m, v_m=v_m, xin=xin, a2=a2, h2=h2,
-                           y=y, Mv=Mv, M=M))
+        lay.update(s_m=s_m, v_m=v_m, xin=xin, a2=a2, h2=h2, y=y, Mv=Mv, M=M)
+        if t is not None:
+            t.update(k)
         s, v = s_new, v_new
     r1 = _lin(s, p, "energy_head.0")
     h3 = _silu(r1)
@@ -593,46 +610,72 @@ def forward(p: Dict[str, Tensor], Z: Tensor, x: Tensor, g: PairGraph, rc: float,
     h4 = _silu(r2)
     eps = _lin(h4, p, "energy_head.4")[:, 0]
     E = _segment_sum(g.mol_ptr, eps, f64=True)
-    cache = dict(H=H, L=L, n=n, x=x, vec=vec, d=d, den=den, u=u, e=e, de=de, layers=layers,
-                 sL=s, r1=r1, h3=h3, r2=r2, h4=h4, Z=Z, rc=rc, lam=None)
-    if lam is not None:
-        tangent(p, cache, g, lam)
+    cache.update(sL=s, r1=r1, h3=h3, r2=r2, h4=h4)
+    if t is not None:
+        t.finish()
     return E, cache
 
 
-def tangent(p: Dict[str, Tensor], c: dict, g: PairGraph, lam: Tensor):
-    """Tangent of the forward pass along the position direction lam [N,3],
-    stored in the cache (the message tangents on the HIP row kernel)."""
-    H, n = c["H"], c["n"]
-    lam32 = lam.to(torch.float32)
-    dd, du, de_t = _geometry(g, c["x"], p["rbf.centers"], p["rbf.widths"], c["rc"], lam32)
-    vec = c["vec"]
-    ds_ = torch.zeros(n, H, dtype=torch.float32, device=vec.device)
-    dv_ = torch.zeros(n, 3, H, dtype=torch.float32, device=vec.device)
-    for k, lay in enumerate(c["layers"]):
-        pre = f"interactions.{k}.message.rbf_to_scalar"
-        lay["ds"], lay["dv"] = ds_, dv_
-        da1, dh, dW = _filter(p, pre, de_t, lay["a1"])
+class _Tangent:
+    """Tangent of the forward pass along the position direction lam [N,3], block
+    by block behind the primal pass of each; stored in the cache."""
+
+    def __init__(self, p: Dict[str, Tensor], c: dict, lam: Tensor):
+        self.p, self.c, self.lam = p, c, lam
+        self.geometry = None
+
+    def message(self, k: int, g: PairGraph):
+        """Block k's filters and message outputs; returns the primal outputs."""
+        p, c, H = self.p, self.c, self.c["H"]
+        if self.geometry is None:
+            self.geometry = _geometry(g, c["x"], p["rbf.centers"], p["rbf.widths"], c["rc"],
+                                      self.lam.to(torch.float32))
+            f = lambda *shape: torch.zeros(*shape, dtype=torch.float32, device=c["x"].device)
+            self.ds, self.dv = f(c["n"], H), f(c["n"], 3, H)
+        _, du, de_t = self.geometry
+        lay = c["layers"][k]
+        lay["ds"], lay["dv"] = self.ds, self.dv
+        da1, dh, dW = _filter(p, f"interactions.{k}.message.rbf_to_scalar", de_t, lay["a1"])
         lay["da1"], lay["dh"], lay["dW"] = da1, dh, dW
-        _, _, dsm, dvm = _message(g, H, lay["s"], lay["v"], lay["W"], c["u"], ds_, dv_, dW, du)
+        s_m, v_m, self.dsm, self.dvm = _message(g, H, lay["s"], lay["v"], lay["W"], c["u"],
+                                                self.ds, self.dv, dW, du)
+        return s_m, v_m
+
+    def update(self, k: int):
+        p, c, H, n = self.p, self.c, self.c["H"], self.c["n"]
+        lay, dsm, dvm = c["layers"][k], self.dsm, self.dvm
         v_m = lay["v_m"]
-        dxin = torch.empty(n, 2 * H, dtype=torch.float32, device=vec.device)
+        dxin = torch.empty(n, 2 * H, dtype=torch.float32, device=v_m.device)
         _glue("mlff_update_norm_tangent", n, H, v_m, lay["xin"], dsm, dvm, dxin)
         upre = f"interactions.{k}.update"
         da2 = dxin @ p[upre + ".update_mlp.0.weight"].T
         dh2 = _silu_d(lay["a2"], da2)
         dy = dh2 @ p[upre + ".update_mlp.2.weight"].T
-        ds_ = torch.empty_like(dsm)
-        dv_ = torch.empty_like(dvm)
+        self.ds = torch.empty_like(dsm)
+        self.dv = torch.empty_like(dvm)
         dMv = torch.empty_like(dvm)
         _glue("mlff_update_apply_tangent", n, H, lay["M"], lay["y"], dy, dsm, v_m, dvm,
-              lay["Mv"], ds_, dv_, dMv)
+              lay["Mv"], self.ds, self.dv, dMv)
         lay.update(dsm=dsm, dvm=dvm, dxin=dxin, da2=da2, dh2=dh2, dy=dy, dMv=dMv)
-    dr1 = ds_ @ p["energy_head.0.weight"].T
-    dh3 = _silu_d(c["r1"], dr1)
-    dr2 = dh3 @ p["energy_head.2.weight"].T
-    dh4 = _silu_d(c["r2"], dr2)
-    c.update(lam=lam, dd=dd, du=du, de_t=de_t, dsL=ds_, dr1=dr1, dh3=dh3, dr2=dr2, dh4=dh4)
+
+    def finish(self):
+        p, c = self.p, self.c
+        dd, du, de_t = self.geometry
+        dr1 = self.ds @ p["energy_head.0.weight"].T
+        dh3 = _silu_d(c["r1"], dr1)
+        dr2 = dh3 @ p["energy_head.2.weight"].T
+        dh4 = _silu_d(c["r2"], dr2)
+        c.update(lam=self.lam, dd=dd, du=du, de_t=de_t, dsL=self.ds, dr1=dr1, dh3=dh3, dr2=dr2,
+                 dh4=dh4)
+
+
+def tangent(p: Dict[str, Tensor], c: dict, g: PairGraph, lam: Tensor):
+    """Tangent of a finished forward pass along lam [N,3], stored in the cache."""
+    t = _Tangent(p, c, lam)
+    for k in range(c["L"]):
+        t.message(k, g)
+        t.update(k)
+    t.finish()
 
 
 # ---------------------------------------------------------------------------
@@ -661,12 +704,14 @@ def _z_segments(Z: Tensor, n_rows: int):
 
 def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
             lam: Optional[Tensor] = None, gw: Optional[Tensor] = None,
-            rbf_grads: bool = False, primal: bool = True):
+            rbf_grads: bool = False, primal: bool = True, diff: bool = False):
     """Parameter gradients of sum_b gw_b E_b (gw defaults to gE) and -- with
     the tangent along ``lam`` [N,3] (reused from the cache when forward()
     already computed it for the same lam) -- the parameter gradients of
     < lam, grad_x (sum_b gE_b E_b) >.  Returns (grads, tgrads or None); without
-    ``primal`` the tangent's only ({}, tgrads).
+    ``primal`` the tangent's only ({}, tgrads), with ``diff`` (lam and gw
+    given) their difference (grads - tgrads, None) from two products per
+    weight instead of three.
 
     gw is applied as a per-row weight on the gE adjoint (structures do not
     interact), so gE must then be all ones.  ``rbf_grads`` adds the basis
@@ -689,6 +734,32 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         else:
             store[name] = val
 
+    def linear(name, ga, b, dga, db, w):
+        """Weight and bias gradients of a Linear with adjoint ga and input b."""
+        if diff:
+            gw_, gb_ = _wgrad(dga, b, ga, db, w=w, bias=True, group=grp, diff=True)
+            acc(grads, name + ".weight", gw_)
+            acc(grads, name + ".bias", gb_)
+            return
+        if primal:
+            gw_, gb_ = _wgrad(ga, b, w=w, bias=True, group=grp)
+            acc(grads, name + ".weight", gw_)
+            acc(grads, name + ".bias", gb_)
+        if T:
+            gw_, gb_ = _wgrad(dga, b, ga, db, bias=True, group=grp)
+            acc(tg, name + ".weight", gw_)
+            acc(tg, name + ".bias", gb_)
+
+    def direct(name, val, dval):
+        """A gradient and its tangent's, each given as a function."""
+        if diff:
+            acc(grads, name, val() - dval())
+            return
+        if primal:
+            acc(grads, name, val())
+        if T:
+            acc(tg, name, dval())
+
     gE = gE.to(torch.float32)
     w_atom = w_pair = None
     if gw is not None:
@@ -704,10 +775,10 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
     geps = gE[g.batch]
     r1, h3, r2, h4, sL = c["r1"], c["h3"], c["r2"], c["h4"], c["sL"]
     Q3 = p["energy_head.4.weight"]
-    if primal:
-        wgeps = wa(geps)
-        acc(grads, "energy_head.4.weight", (wgeps @ h4).reshape(1, -1))
-        acc(grads, "energy_head.4.bias", wgeps.sum().reshape(1))
+    direct("energy_head.4.weight", lambda: (wa(geps) @ h4).reshape(1, -1),
+           lambda: (geps @ c["dh4"]).reshape(1, -1))
+    direct("energy_head.4.bias", lambda: wa(geps).sum().reshape(1),
+           lambda: torch.zeros(1, dtype=torch.float32, device=dev))
     gh4 = geps.unsqueeze(1) * Q3
     R2w, R1w = p["energy_head.2.weight"], p["energy_head.0.weight"]
     if T:
@@ -725,23 +796,11 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         gr2 = _silu_d(r2, gh4)
         gr1 = _silu_d(r1, gr2 @ R2w)
         gs = (gr1 @ R1w).contiguous()
-    if primal:
-        gw_, gb_ = _wgrad(gr2, h3, w=w_atom, bias=True, group=grp)
-        acc(grads, "energy_head.2.weight", gw_)
-        acc(grads, "energy_head.2.bias", gb_)
-        gw_, gb_ = _wgrad(gr1, sL, w=w_atom, bias=True, group=grp)
-        acc(grads, "energy_head.0.weight", gw_)
-        acc(grads, "energy_head.0.bias", gb_)
+        dgr2 = dgr1 = dh3 = None
+    linear("energy_head.2", gr2, h3, dgr2, dh3, w_atom)
+    linear("energy_head.0", gr1, sL, dgr1, c["dsL"] if T else None, w_atom)
     gv = torch.zeros(n, 3, H, dtype=torch.float32, device=dev)
     if T:
-        acc(tg, "energy_head.4.weight", (geps @ dh4).reshape(1, -1))
-        acc(tg, "energy_head.4.bias", torch.zeros(1, dtype=torch.float32, device=dev))
-        gw_, gb_ = _wgrad(dgr2, h3, gr2, dh3, bias=True, group=grp)
-        acc(tg, "energy_head.2.weight", gw_)
-        acc(tg, "energy_head.2.bias", gb_)
-        gw_, gb_ = _wgrad(dgr1, sL, gr1, c["dsL"], bias=True, group=grp)
-        acc(tg, "energy_head.0.weight", gw_)
-        acc(tg, "energy_head.0.bias", gb_)
         dgv = torch.zeros_like(gv)
 
     u = c["u"]
@@ -771,20 +830,9 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         else:
             ga2 = _silu_d(lay["a2"], gy @ U2)
             gx, dgx = ga2 @ U1, None
-        if primal:
-            gw_, gb_ = _wgrad(gy, lay["h2"], w=w_atom, bias=True, group=grp)
-            acc(grads, upre + ".update_mlp.2.weight", gw_)
-            acc(grads, upre + ".update_mlp.2.bias", gb_)
-            gw_, gb_ = _wgrad(ga2, xin, w=w_atom, bias=True, group=grp)
-            acc(grads, upre + ".update_mlp.0.weight", gw_)
-            acc(grads, upre + ".update_mlp.0.bias", gb_)
-        if T:
-            gw_, gb_ = _wgrad(dgy, lay["h2"], gy, lay["dh2"], bias=True, group=grp)
-            acc(tg, upre + ".update_mlp.2.weight", gw_)
-            acc(tg, upre + ".update_mlp.2.bias", gb_)
-            gw_, gb_ = _wgrad(dga2, xin, ga2, dxin, bias=True, group=grp)
-            acc(tg, upre + ".update_mlp.0.weight", gw_)
-            acc(tg, upre + ".update_mlp.0.bias", gb_)
+            dga2 = None
+        linear(upre + ".update_mlp.2", gy, lay["h2"], dgy, lay["dh2"] if T else None, w_atom)
+        linear(upre + ".update_mlp.0", ga2, xin, dga2, dxin, w_atom)
         gs_m = torch.empty(n, H, dtype=torch.float32, device=dev)
         gv_m = torch.empty(n, 3, H, dtype=torch.float32, device=dev)
         gvg2 = torch.empty_like(gv_m)
@@ -794,57 +842,45 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         _glue("mlff_update_input_adjoint", n, H, M, gx, gs, gv, y, v_m, xin, dgx,
               dgs if T else None, dgv if T else None, lay["dy"] if T else None, dvm, dxin,
               gs_m, gv_m, gvg2, dgs_m, dgv_m, dgvg2)
-        if primal:
-            acc(grads, upre + ".mixing_matrix", _xyz_outer(gvg2, v_m, w=w_atom, group=grp))
-        if T:
-            acc(tg, upre + ".mixing_matrix", _xyz_outer(dgvg2, v_m, gvg2, dvm, group=grp))
+        if diff:
+            acc(grads, upre + ".mixing_matrix",
+                _xyz_outer(dgvg2, v_m, gvg2, dvm, w=w_atom, group=grp, diff=True))
+        else:
+            direct(upre + ".mixing_matrix", lambda: _xyz_outer(gvg2, v_m, w=w_atom, group=grp),
+                   lambda: _xyz_outer(dgvg2, v_m, gvg2, dvm, group=grp))
         # message reverse (student_model.py:346-387): filter-output gradients per pair
         s, v, W = lay["s"], lay["v"], lay["W"]
         if T:
             gW, dgW = _pair_grad(g, H, u, s, v, gs_m, gv_m, c["du"], lay["ds"], lay["dv"],
                                  dgs_m, dgv_m)
         else:
-            gW, _ = _pair_grad(g, H, u, s, v, gs_m, gv_m)
+            gW, dgW = _pair_grad(g, H, u, s, v, gs_m, gv_m)
         W1 = p[mpre + ".0.weight"]
-        if primal:
-            gw_, gb_ = _wgrad(gW, lay["h"], w=w_pair, bias=True, group=grp)
-            acc(grads, mpre + ".2.weight", gw_)
-            acc(grads, mpre + ".2.bias", gb_)
+        linear(mpre + ".2", gW, lay["h"], dgW, lay["dh"] if T else None, w_pair)
         # gW W2 through the SiLU (and its tangent) on the fused pair kernel
         ga1, dga1 = _filter_adjoint(p, mpre, gW, lay["a1"], dgW if T else None,
                                     lay["da1"] if T else None)
-        ge = ga1 @ W1 if rbf_grads else None
-        if primal:
-            gw_, gb_ = _wgrad(ga1, c["e"], w=w_pair, bias=True, group=grp)
-            acc(grads, mpre + ".0.weight", gw_)
-            acc(grads, mpre + ".0.bias", gb_)
-            if rbf_grads:
-                acc(grads, "rbf.centers", (wp(ge) * e_mu).sum(0))
-                acc(grads, "rbf.widths", (wp(ge) * e_w).sum(0))
+        linear(mpre + ".0", ga1, c["e"], dga1, c["de_t"] if T else None, w_pair)
+        if rbf_grads:
+            ge = ga1 @ W1
+            if T:
+                dge, dd = dga1 @ W1, c["dd"].unsqueeze(-1)
+            for name, ek, dek in (("rbf.centers", e_mu, de_mu), ("rbf.widths", e_w, de_w)):
+                direct(name, lambda: (wp(ge) * ek).sum(0),
+                       lambda: (dge * ek + ge * dek * dd).sum(0))
         if T:
-            dh = lay["dh"]
-            gw_, gb_ = _wgrad(dgW, lay["h"], gW, dh, bias=True, group=grp)
-            acc(tg, mpre + ".2.weight", gw_)
-            acc(tg, mpre + ".2.bias", gb_)
-            gw_, gb_ = _wgrad(dga1, c["e"], ga1, c["de_t"], bias=True, group=grp)
-            acc(tg, mpre + ".0.weight", gw_)
-            acc(tg, mpre + ".0.bias", gb_)
-            if rbf_grads:
-                dge = dga1 @ W1
-                dd = c["dd"].unsqueeze(-1)
-                acc(tg, "rbf.centers", (dge * e_mu + ge * de_mu * dd).sum(0))
-                acc(tg, "rbf.widths", (dge * e_w + ge * de_w * dd).sum(0))
             gs, gv, dgs, dgv = _message_adjoint(g, H, gs_m, gv_m, W, dgs_m, dgv_m, lay["dW"])
         else:
             gs, gv, _, _ = _message_adjoint(g, H, gs_m, gv_m, W)
     emb_rows = p["embedding.weight"].shape[0]
     zptr, zorder = _z_segments(c["Z"], emb_rows)
-    if primal:
-        acc(grads, "embedding.weight", _segment_sum(zptr, wa(gs), zorder))
-    if T:
-        acc(tg, "embedding.weight", _segment_sum(zptr, dgs, zorder))
+    if diff:
+        acc(grads, "embedding.weight", _segment_sum(zptr, wa(gs) - dgs, zorder))
+    else:
+        direct("embedding.weight", lambda: _segment_sum(zptr, wa(gs), zorder),
+               lambda: _segment_sum(zptr, dgs, zorder))
     grp.flush()
-    return grads, (tg if T else None)
+    return grads, (tg if T and not diff else None)
 
 
 # ---------------------------------------------------------------------------
@@ -869,25 +905,8 @@ def force_matching_grads(p: Dict[str, Tensor], Z: Tensor, x: Tensor, g: PairGrap
     # one reverse pass gives both parts:
     #   d/dtheta of wE MSE(E): the unit adjoint's terms weighted by dL/dE (gw)
     #   d/dtheta of wF MSE(F) = - d/dtheta < dL/dF, grad_x sum E >
-    gE, tg = reverse(p, cache, g, torch.ones(B, dtype=torch.float32, device=x.device),
-                     lam=dLdF, gw=dLdE, rbf_grads=rbf_grads)
-    grads = {}
-    both, A, B = [], [], []
-    for name in p:
-        a = gE.get(name)
-        b = tg.get(name)
-        if a is None and b is None:
-            continue
-        if a is not None and b is not None:
-            both.append(name)
-            A.append(a)
-            B.append(b)
-        else:
-            grads[name] = a if b is None else torch.neg(b)
-    # one multi-tensor launch for every parameter with both parts
-    if both:
-        for name, d in zip(both, torch._foreach_sub(A, B)):
-            grads[name] = d
+    grads, _ = reverse(p, cache, g, torch.ones(B, dtype=torch.float32, device=x.device),
+                       lam=dLdF, gw=dLdE, rbf_grads=rbf_grads, diff=True)
     return loss, E, F, grads
 
 
