@@ -397,6 +397,11 @@ int mlff_train_pair_grad(void* stream, int hidden_dim, int n_pairs, const int32_
                          const float* dgs_dev, const float* dgv_dev, float* gw_dev,
                          float* dgw_dev);
 
+/* (row, column) of every entry of a receiver CSR list (row_ptr [N+1], col [E])
+ * as int64, edge_index [2][E], in list order. */
+int mlff_edge_index(void* stream, int n_atoms, int n_edges, const int32_t* row_ptr_dev,
+                    const int32_t* col_dev, int64_t* edge_index_dev);
+
 /* Groups E directed edges src[e] -> dst[e] (int64, endpoints in [0, N)) by
  * receiver (list 0) and, with lists = 2, by source (list 1), each group in
  * ascending edge order: row_ptr [lists][N+1], the other endpoint col

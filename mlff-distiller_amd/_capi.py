@@ -44,7 +44,7 @@ EXPORTS = (
     "mlff_mts_run", "mlff_mts_graph_run", "mlff_plan_set_streams", "mlff_energy_forces_static",
     "mlff_train_message", "mlff_train_message_adjoint", "mlff_train_pair_grad",
     "mlff_segment_sum", "mlff_plan_set_tiles", "mlff_edge_message", "mlff_edge_grad",
-    "mlff_edge_csr",
+    "mlff_edge_csr", "mlff_edge_index",
     "mlff_weight_grad_workspace_bytes", "mlff_weight_grad", "mlff_weight_grad_partial_count",
     "mlff_weight_grad_partials", "mlff_weight_grad_diff_partials", "mlff_weight_grad_reduce_group", "mlff_xyz_outer_partial_count",
     "mlff_xyz_outer_partials", "mlff_xyz_outer_diff_partials", "mlff_train_geometry", "mlff_silu_chain",
@@ -159,6 +159,8 @@ def _declare(lib):
     lib.mlff_edge_message.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 9
     lib.mlff_edge_csr.restype = ctypes.c_int
     lib.mlff_edge_csr.argtypes = [vp] + [ctypes.c_int] * 3 + [vp] * 8
+    lib.mlff_edge_index.restype = ctypes.c_int
+    lib.mlff_edge_index.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 3
     lib.mlff_edge_grad.restype = ctypes.c_int
     lib.mlff_edge_grad.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 10
     lib.mlff_segment_sum.restype = ctypes.c_int

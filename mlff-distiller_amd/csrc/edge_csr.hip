@@ -141,10 +141,46 @@ __global__ __launch_bounds__(kCsrBlock) void csr_rows_kernel(
   }
 }
 
+// (row, column) of every entry of a CSR list as int64, one wave per row
+__global__ __launch_bounds__(kCsrBlock) void edge_index_kernel(int N, int E,
+                                                               const int32_t* __restrict__ row_ptr,
+                                                               const int32_t* __restrict__ col,
+                                                               int64_t* __restrict__ out) {
+  const int i = (int)(((int64_t)blockIdx.x * kCsrBlock + threadIdx.x) >> 6);
+  if (i >= N) return;
+  const int e1 = min(row_ptr[i + 1], E);
+  for (int e = row_ptr[i] + (int)(threadIdx.x & 63); e < e1; e += 64) {
+    out[e] = i;
+    out[(size_t)E + e] = col[e];
+  }
+}
+
 }  // namespace
 }  // namespace mlff
 
 using namespace mlff;
+
+extern "C" int mlff_edge_index(void* stream, int n_atoms, int n_edges, const int32_t* row_ptr_dev,
+                               const int32_t* col_dev, int64_t* edge_index_dev) {
+  if (n_atoms < 0 || n_edges < 0) {
+    set_error("mlff_edge_index: invalid sizes");
+    return MLFF_ERR_INVALID;
+  }
+  if (n_atoms == 0 || n_edges == 0) return MLFF_OK;
+  if (!row_ptr_dev || !col_dev || !edge_index_dev) {
+    set_error("mlff_edge_index: null pointer");
+    return MLFF_ERR_INVALID;
+  }
+  const int blocks = (int)(((int64_t)n_atoms * 64 + kCsrBlock - 1) / kCsrBlock);
+  edge_index_kernel<<<blocks, kCsrBlock, 0, static_cast<hipStream_t>(stream)>>>(
+      n_atoms, n_edges, row_ptr_dev, col_dev, edge_index_dev);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error("mlff_edge_index: %s", hipGetErrorString(e));
+    return MLFF_ERR_HIP;
+  }
+  return MLFF_OK;
+}
 
 extern "C" int mlff_edge_csr(void* stream, int n_edges, int n_atoms, int lists,
                              const int64_t* src_dev, const int64_t* dst_dev, int32_t* row_ptr_dev,

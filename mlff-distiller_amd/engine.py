@@ -160,8 +160,9 @@ def make_layout(sizes: Sequence[int], device, cells=None, pbc=None) -> BatchLayo
             cells_np = np.asarray(cells, dtype=np.float32).reshape(len(sizes), 3, 3)
             ct = torch.from_numpy(np.ascontiguousarray(cells_np)).to(device)
             pt = torch.from_numpy(pbc_np.astype(np.uint8)).to(device)
-    return BatchLayout(int(mol_ptr[-1]), sizes, torch.from_numpy(mol_ptr).to(device),
-                       torch.from_numpy(atom_mol).to(device), ct, pt, periodic,
+    both = torch.from_numpy(np.concatenate([atom_mol, mol_ptr])).to(device)   # one copy
+    return BatchLayout(int(mol_ptr[-1]), sizes, both[len(atom_mol):], both[:len(atom_mol)], ct, pt,
+                       periodic,
                        cells_np if periodic else None, pbc_np if periodic else None)
 
 
@@ -399,6 +400,15 @@ def neighbor_pairs(positions: torch.Tensor, layout: BatchLayout, cutoff: float):
             return row_ptr, col[:E], edge_pair[:E], pair_lo[:P], pair_hi[:P]
         cap = max(E, 2 * P)
     raise RuntimeError("neighbour list capacity did not converge")
+
+
+def edge_index(row_ptr: torch.Tensor, col: torch.Tensor) -> torch.Tensor:
+    """The entries of a receiver CSR list as an int64 [2, E] (row, column) tensor."""
+    out = torch.empty(2, col.numel(), dtype=torch.int64, device=col.device)
+    C.check("mlff_edge_index", C.lib().mlff_edge_index(
+        C.stream_handle(), row_ptr.numel() - 1, col.numel(), C.ptr(row_ptr), C.ptr(col),
+        C.ptr(out)))
+    return out
 
 
 def neighbor_list(positions: torch.Tensor, layout: BatchLayout, cutoff: float,

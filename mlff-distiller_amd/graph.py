@@ -60,9 +60,10 @@ def radius_graph(positions: torch.Tensor, r: float, batch: Optional[torch.Tensor
     layout = engine.make_layout(sizes, positions.device)
     row_ptr, col, _ = engine.neighbor_list(pos.detach().to(torch.float32).contiguous(), layout,
                                            float(np.float32(r)))
-    deg = row_ptr[1:] - row_ptr[:-1]
-    src = torch.repeat_interleave(torch.arange(n, device=positions.device), deg.long())
-    dst = col.long()
+    edges = engine.edge_index(row_ptr, col)
+    if order is None and not loop:
+        return edges
+    src, dst = edges
     if order is not None:
         src, dst = perm[src], perm[dst]
     if loop:
