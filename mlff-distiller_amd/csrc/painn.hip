@@ -45,12 +45,15 @@ template <int H>
 constexpr int kBwdPairs = H <= 32 ? 64 : 32;
 constexpr int kUpdWaves = 8;          // update kernels: waves per 32-atom tile
 constexpr int kUpdBlock = 64 * kUpdWaves;
-// Atoms up to which the update blocks run split over columns, and the readout on
-// 16-atom tiles.  H = 128, forward + adjoint of a block: 60 atoms 24 us split,
-// 34 us whole (33 with 16-atom tiles); 3000 atoms 42 us split, 41 us whole.
+// Atoms up to which the update blocks run split over columns, and the update
+// blocks and the readout on 16-atom tiles.  H = 128, forward + adjoint of a
+// block: 60 atoms 24 us split, 34 us whole (33 with 16-atom tiles); 3000 atoms
+// 42 us split, 41 us in 32-atom and 34 us in 16-atom tiles (one round of the
+// CUs in either, half the products per CU); 14,000 atoms 89 us in 32-atom and
+// 109 us in 16-atom tiles, which read the weights twice as often.
 // Readout: 14 -> 7 us at 60 atoms, 15 -> 9 us at 3000.
 constexpr int kSplitAtoms = 1024;
-constexpr int kReadoutSmallAtoms = 4096;
+constexpr int kSmallTileAtoms = 4096;
 // Message rows: sums per row, and the atoms up to which each has threads of its own
 constexpr int kMsgSums = 4;
 constexpr int kMsgSplitAtoms = 1024;
@@ -341,17 +344,17 @@ __device__ __forceinline__ float dot3(float a0, float a1, float a2, float b0, fl
 }
 
 // ---------------------------------------------------------------------------
-// update forward, 32 atoms per tile.  The products run on four accumulator sets
+// update forward, TM atoms per tile.  The products run on four accumulator sets
 // (mma_tile_k4): on one set they are the largest part of an energy's error
 // (molecules with large biases: 4.7e-5 eV/atom rms with one set, 3.1e-5 with
 // two, 2.3e-5 with four, in the same time).
 // ---------------------------------------------------------------------------
-template <int H>
+template <int H, int TM>
 __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
     int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ s_mid,
     const float* __restrict__ v_mid, float* __restrict__ s_out, float* __restrict__ v_out,
     float* __restrict__ a_upd, float* __restrict__ g12) {
-  constexpr int TM = 32, RT = 2;
+  constexpr int RT = TM / 16;
   constexpr int LDX = 2 * H + 4, LDH = H + 4;
   constexpr int CT1 = H / 16, NT1 = (CT1 + kUpdWaves - 1) / kUpdWaves;
   constexpr int NTC = NT1, NT2 = 3 * NTC;
@@ -466,7 +469,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// readout: eps_i = head(s_i) and gs_i = d eps_i / d s_i, 32 atoms per tile
+// readout: eps_i = head(s_i) and gs_i = d eps_i / d s_i, TM atoms per tile
 // ---------------------------------------------------------------------------
 template <int H, int TM>
 __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __restrict__ w,
@@ -602,15 +605,15 @@ __global__ __launch_bounds__(kBlock) void readout_kernel(int N, const float* __r
 }
 
 // ---------------------------------------------------------------------------
-// update backward, 32 atoms per tile.  gv2 == nullptr means a zero gradient.
+// update backward, TM atoms per tile.  gv2 == nullptr means a zero gradient.
 // ---------------------------------------------------------------------------
-template <int H>
+template <int H, int TM>
 __global__ __launch_bounds__(kUpdBlock) void update_bwd_kernel(
     int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ gs2,
     const float* __restrict__ gv2, const float* __restrict__ v_mid,
     const float* __restrict__ a_upd, const float* __restrict__ g12, float* __restrict__ gs1,
     float* __restrict__ gv1) {
-  constexpr int TM = 32, RT = 2;
+  constexpr int RT = TM / 16;
   constexpr int LDY = 3 * H + 4, LDA = H + 4, LDX = 2 * H + 4;
   __shared__ __align__(16) float y_lds[TM * LDY];
   __shared__ __align__(16) float a_lds[TM * LDA];
@@ -1449,7 +1452,7 @@ void launch_message(const Buffers& b, hipStream_t st, const float* Wl, const flo
 }
 
 // Atom-side launches: the split or small forms for few atoms (kSplitAtoms,
-// kReadoutSmallAtoms), 32-atom tiles above.  Same bits.
+// kSmallTileAtoms), 32-atom tiles above.  Same bits.
 template <int H>
 void launch_update_fwd(const Buffers& b, hipStream_t s, const LayerW& lw, const float* s_mid,
                        const float* v_mid, float* s_out, float* v_out, float* a_upd, float* g12) {
@@ -1459,15 +1462,19 @@ void launch_update_fwd(const Buffers& b, hipStream_t s, const LayerW& lw, const 
     update_gate_kernel<H><<<grid, kSplitBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, a_upd, s_out,
                                                        v_out, g12);
   } else {
-    update_fwd_kernel<H><<<(b.N + 31) / 32, kUpdBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, s_out,
-                                                               v_out, a_upd, g12);
+    auto run = [&](auto kernel, int tm) {
+      kernel<<<(b.N + tm - 1) / tm, kUpdBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, s_out, v_out,
+                                                       a_upd, g12);
+    };
+    if (b.N <= kSmallTileAtoms) run(update_fwd_kernel<H, 16>, 16);
+    else run(update_fwd_kernel<H, 32>, 32);
   }
 }
 
 template <int H>
 void launch_readout(const Buffers& b, hipStream_t s) {
   const float* sL = b.S + (size_t)b.L * nh(b);
-  if (b.N <= kReadoutSmallAtoms)
+  if (b.N <= kSmallTileAtoms)
     readout_kernel<H, 16><<<(b.N + 15) / 16, kBlock, 0, s>>>(b.N, b.w, *b.mw, sL, b.eps, b.gS0);
   else
     readout_kernel<H, 32><<<(b.N + 31) / 32, kBlock, 0, s>>>(b.N, b.w, *b.mw, sL, b.eps, b.gS0);
@@ -1488,8 +1495,12 @@ void launch_update_bwd(const Buffers& b, hipStream_t s, int l, const float* gs2,
     update_input_bwd_kernel<H><<<grid, kSplitBlock, 0, s>>>(b.N, b.w, lw, gs2, gv2, vm, b.gA, g12,
                                                             gs1, gv1);
   } else {
-    update_bwd_kernel<H><<<(b.N + 31) / 32, kUpdBlock, 0, s>>>(b.N, b.w, lw, gs2, gv2, vm, au,
-                                                               g12, gs1, gv1);
+    auto run = [&](auto kernel, int tm) {
+      kernel<<<(b.N + tm - 1) / tm, kUpdBlock, 0, s>>>(b.N, b.w, lw, gs2, gv2, vm, au, g12, gs1,
+                                                       gv1);
+    };
+    if (b.N <= kSmallTileAtoms) run(update_bwd_kernel<H, 16>, 16);
+    else run(update_bwd_kernel<H, 32>, 32);
   }
 }
 
