@@ -623,6 +623,38 @@ int mlff_update_input_adjoint(void* stream, int n_atoms, int hidden, const float
                               float* gs_out_dev, float* gv_out_dev, float* gvg2_out_dev,
                               float* dgs_out_dev, float* dgv_out_dev, float* dgvg2_out_dev);
 
+/* The update block (student_model.py:430-470) of the training pass in one
+ * launch, hidden_dim 32, 64 or 128.  parts: 1 the primal pass, 2 its tangent
+ * along (ds, dv) from the primal pass's stored xin, a, y, 3 both.
+ *   n = |v|_xyz, xin = (s, n) [N][2H], a = xin w1^T + b1, h = silu(a) [N][H],
+ *   y = h w2^T + b2 [N][3H] = (ds, g1, g2), mv = mix v [N][3][H],
+ *   s_out = s + ds, v_out = v g1 + mv g2.
+ * w1 [H][2H], w2 [3H][H].  Feature and input buffers and the weights are 16-byte
+ * aligned. */
+int mlff_train_update(void* stream, int parts, int n_atoms, int hidden_dim, const float* s_dev,
+                      const float* v_dev, const float* ds_dev, const float* dv_dev,
+                      const float* w1_dev, const float* b1_dev, const float* w2_dev,
+                      const float* b2_dev, const float* mix_dev, float* xin_dev, float* a_dev,
+                      float* h_dev, float* y_dev, float* mv_dev, float* s_out_dev,
+                      float* v_out_dev, float* dxin_dev, float* da_dev, float* dh_dev,
+                      float* dy_dev, float* dmv_dev, float* ds_out_dev, float* dv_out_dev);
+
+/* Its adjoint from the output gradients (gs, gv), and with (dgs, dgv) the
+ * adjoint's tangent:
+ *   gy = (gs, sum_x gv v, sum_x gv mv), ga = silu'(a) (gy w2),
+ *   (gsx, gn) = ga w1, gvg2 = gv g2,
+ *   gs_out = gs + gsx, gv_out = gv g1 + mix^T gvg2 + gn v / n (0 where n = 0). */
+int mlff_train_update_adjoint(void* stream, int n_atoms, int hidden_dim, const float* gs_dev,
+                              const float* gv_dev, const float* dgs_dev, const float* dgv_dev,
+                              const float* v_dev, const float* mv_dev, const float* y_dev,
+                              const float* a_dev, const float* xin_dev, const float* dv_dev,
+                              const float* dmv_dev, const float* dy_dev, const float* da_dev,
+                              const float* dxin_dev, const float* w1_dev, const float* w2_dev,
+                              const float* mix_dev, float* gy_dev, float* ga_dev,
+                              float* gs_out_dev, float* gv_out_dev, float* gvg2_dev,
+                              float* dgy_dev, float* dga_dev, float* dgs_out_dev,
+                              float* dgv_out_dev, float* dgvg2_dev);
+
 /* ---------------------------------------------------------------------------
  * Matrix-core throughput probe, for the measured peak next to the published
  * one in roofline figures (no counterpart in the reference, which has no GPU

@@ -23,6 +23,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "_lib")
 LIBNAME = "libmlff_amd.so"
 SOURCES = ("capi.hip", "nl.hip", "painn.hip", "filter_table.hip", "md.hip", "train.hip", "train_update.hip", "train_filter.hip",
+           "train_block.hip",
            "edge_csr.hip", "pack.hip", "probe.hip")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

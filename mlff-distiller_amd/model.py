@@ -231,25 +231,19 @@ def _update_plain(s, v, w1, b1, w2, b2, mix):
 
 
 class _UpdateBlock(torch.autograd.Function):
-    """PaiNNUpdate.forward on the elementwise and weight-gradient kernels of the
-    training pass (the library's product for the 3x3 mixing gradient alone took
-    220 us for 1,700 atoms at H = 64)."""
+    """PaiNNUpdate.forward on the training pass's kernels: one launch each way and
+    the weight gradients (the library's product for the 3x3 mixing gradient
+    alone took 220 us for 1,700 atoms at H = 64)."""
 
     @staticmethod
     def forward(ctx, s, v, w1, b1, w2, b2, mix):
         from . import train
-        n, H = s.shape
-        xin = torch.empty(n, 2 * H, dtype=torch.float32, device=s.device)
-        train._glue("mlff_update_norm", n, H, s, v, xin)
-        a = torch.addmm(b1, xin, w1.t())
-        h = nn.functional.silu(a)
-        y = torch.addmm(b2, h, w2.t())
-        so = torch.empty(n, H, dtype=torch.float32, device=s.device)
-        vo = torch.empty(n, 3, H, dtype=torch.float32, device=s.device)
-        mv = torch.empty_like(vo)
-        train._glue("mlff_update_apply", n, H, mix, y, s, v, so, vo, mv)
-        ctx.save_for_backward(s, v, w1, b1, w2, b2, mix, xin, a, h, y, mv)
-        return so, vo
+        w = tuple(train._dense(t) for t in (w1, b1, w2, b2, mix))
+        sd, vd = train._dense(s), train._dense(v)
+        o = train._update(w, sd, vd)
+        ctx.save_for_backward(s, v, w1, b1, w2, b2, mix, *[o[k] for k in
+                                                           ("xin", "a2", "h2", "y", "Mv")])
+        return o["s_out"], o["v_out"]
 
     @staticmethod
     def backward(ctx, gs, gv):
@@ -259,17 +253,10 @@ class _UpdateBlock(torch.autograd.Function):
             ins = (s, v, w1, b1, w2, b2, mix)
             return _plain_grads(ctx, _update_plain(*ins), ins, (gs, gv))
         need = ctx.needs_input_grad
-        n, H = s.shape
-        gs, gv = train._dense(gs), train._dense(gv)
-        new = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=s.device)
-        gy = new(n, 3 * H)
-        train._glue("mlff_update_gate_adjoint", n, H, gs, gv, v, mv, None, None, None, None, gy,
-                    None)
-        ga = torch.ops.aten.silu_backward(gy @ w2, a)
-        gx = ga @ w1
-        gso, gvo, gvg2 = new(n, H), new(n, 3, H), new(n, 3, H)
-        train._glue("mlff_update_input_adjoint", n, H, mix, gx, gs, gv, y, v, xin, None, None,
-                    None, None, None, None, gso, gvo, gvg2, None, None, None)
+        w = tuple(train._dense(t) for t in (w1, b1, w2, b2, mix))
+        lay = dict(v_m=train._dense(v), Mv=mv, y=y, a2=a, xin=xin)
+        (gy, ga, gso, gvo, gvg2), _ = train._update_adjoint(w, lay, train._dense(gs),
+                                                            train._dense(gv))
         grp = train._WgGroup()
         gw1 = gb1 = gw2 = gb2 = gm = None
         if need[4] or need[5]:
@@ -326,7 +313,7 @@ class PaiNNUpdate(nn.Module):
         _device_f32(scalar_features, vector_features)
         H = self.hidden_dim
         n, mlp, mix = scalar_features.shape[0], self.update_mlp, self.mixing_matrix
-        if (H % 4 == 0 and scalar_features.shape == (n, H) and vector_features.shape == (n, 3, H)
+        if (H in (32, 64, 128) and scalar_features.shape == (n, H) and vector_features.shape == (n, 3, H)
                 and mix.shape == (3, 3) and _fused_mlp(mlp, scalar_features, vector_features, mix)):
             return _UpdateBlock.apply(scalar_features, vector_features, mlp[0].weight,
                                       mlp[0].bias, mlp[2].weight, mlp[2].bias, mix)

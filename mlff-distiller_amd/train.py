@@ -24,9 +24,11 @@ Where the work runs:
   per unordered pair from both endpoints -- no scatter-adds, no atomics;
 * per-structure energies and the embedding gradient by fixed-order segment
   sums (mlff_segment_sum);
-* the dense products (filter and update MLPs, weight gradients) as plain
-  library GEMMs; weight gradients over many rows are split into 2048-row
-  chunks and summed, so no library split-K reduction is involved.
+* the update block with its products, and its reverse, on one kernel each
+  (mlff_train_update, mlff_train_update_adjoint), primal and tangent together;
+  the readout's small products as library GEMMs;
+* weight gradients on a split-row kernel with a fixed order
+  (mlff_weight_grad_partials).
 Every reduction runs in a fixed order: two runs give bit-identical gradients.
 
 The forces the loss needs come from the fused HIP evaluation of the current
@@ -249,6 +251,56 @@ def _glue(name: str, *args):
             a = None
         conv.append(a)
     C.check(name, getattr(C.lib(), name)(C.stream_handle(), *conv))
+
+
+def _update(w, s, v, lay: Optional[dict] = None, ds=None, dv=None, primal: bool = True):
+    """The update block on inputs (s, v) and, with (ds, dv), its tangent, in one
+    launch (mlff_train_update); ``primal`` False: the tangent of the pass stored
+    in ``lay``.  w = (W1, b1, W2, b2, M), dense.  Returns what the reverse pass
+    needs, outputs included (s_out, v_out, ds_out, dv_out)."""
+    n, _, H = v.shape
+    new = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=v.device)
+    out = {}
+    if primal:
+        out.update(xin=new(n, 2 * H), a2=new(n, H), h2=new(n, H), y=new(n, 3 * H),
+                   Mv=new(n, 3, H), s_out=new(n, H), v_out=new(n, 3, H))
+    if ds is not None:
+        out.update(dxin=new(n, 2 * H), da2=new(n, H), dh2=new(n, H), dy=new(n, 3 * H),
+                   dMv=new(n, 3, H), ds_out=new(n, H), dv_out=new(n, 3, H))
+    src = out if primal else lay
+    P = C.ptr
+    W1, b1, W2, b2, M = w
+    C.check("mlff_train_update", C.lib().mlff_train_update(
+        C.stream_handle(), int(primal) + 2 * (ds is not None), n, H, P(s), P(v), P(ds), P(dv),
+        P(W1), P(b1), P(W2), P(b2), P(M), P(src["xin"]), P(src["a2"]), P(src["h2"]), P(src["y"]),
+        P(src["Mv"]), P(out.get("s_out")), P(out.get("v_out")), P(out.get("dxin")),
+        P(out.get("da2")), P(out.get("dh2")), P(out.get("dy")), P(out.get("dMv")),
+        P(out.get("ds_out")), P(out.get("dv_out"))))
+    return out
+
+
+def _update_adjoint(w, lay: dict, gs, gv, dgs=None, dgv=None):
+    """Adjoint of _update from the output gradients and, with (dgs, dgv), its
+    tangent (mlff_train_update_adjoint): ([gy, ga, gs_m, gv_m, gvg2], the same of
+    the tangent or Nones)."""
+    n, _, H = gv.shape
+    new = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=gv.device)
+    outs = lambda: [new(n, 3 * H), new(n, H), new(n, H), new(n, 3, H), new(n, 3, H)]
+    T = dgs is not None
+    out, dout = outs(), outs() if T else [None] * 5
+    t = (lambda k: lay[k]) if T else (lambda k: None)
+    W1, _, W2, _, M = w
+    C.check("mlff_train_update_adjoint", C.lib().mlff_train_update_adjoint(
+        C.stream_handle(), n, H, *[C.ptr(q) for q in (
+            gs, gv, dgs, dgv, lay["v_m"], lay["Mv"], lay["y"], lay["a2"], lay["xin"], t("dvm"),
+            t("dMv"), t("dy"), t("da2"), t("dxin"), W1, W2, M, *out, *dout)]))
+    return out, dout
+
+
+def _update_weights(p: Dict[str, Tensor], upre: str):
+    return tuple(_dense(p[upre + k]) for k in (".update_mlp.0.weight", ".update_mlp.0.bias",
+                                               ".update_mlp.2.weight", ".update_mlp.2.bias",
+                                               ".mixing_matrix"))
 
 
 def _silu_call(a, da=None, g=None, dg=None, h=False, dh=False, dga=False):
@@ -588,22 +640,14 @@ def forward(p: Dict[str, Tensor], Z: Tensor, x: Tensor, g: PairGraph, rc: float,
             s_m, v_m, _, _ = _message(g, H, s, v, W, u)
         else:
             s_m, v_m = t.message(k, g)
-        upre = f"interactions.{k}.update"
         # PaiNNUpdate.forward (student_model.py:430-470)
-        xin = torch.empty(n, 2 * H, dtype=torch.float32, device=x.device)
-        _glue("mlff_update_norm", n, H, s_m, v_m, xin)
-        a2 = _lin(xin, p, upre + ".update_mlp.0")
-        h2 = _silu(a2)
-        y = _lin(h2, p, upre + ".update_mlp.2")
-        M = _dense(p[upre + ".mixing_matrix"])
-        s_new = torch.empty_like(s_m)
-        v_new = torch.empty_like(v_m)
-        Mv = torch.empty_like(v_m)
-        _glue("mlff_update_apply", n, H, M, y, s_m, v_m, s_new, v_new, Mv)
-        lay.update(s_m=s_m, v_m=v_m, xin=xin, a2=a2, h2=h2, y=y, Mv=Mv, M=M)
-        if t is not None:
-            t.update(k)
-        s, v = s_new, v_new
+        lay.update(s_m=s_m, v_m=v_m, w=_update_weights(p, f"interactions.{k}.update"))
+        if t is None:
+            lay.update(_update(lay["w"], s_m, v_m))
+        else:
+            lay.update(_update(lay["w"], s_m, v_m, None, *t.moved(k)))
+            t.updated(k)
+        s, v = lay["s_out"], lay["v_out"]
     r1 = _lin(s, p, "energy_head.0")
     h3 = _silu(r1)
     r2 = _lin(h3, p, "energy_head.2")
@@ -641,22 +685,14 @@ class _Tangent:
                                                 self.ds, self.dv, dW, du)
         return s_m, v_m
 
-    def update(self, k: int):
-        p, c, H, n = self.p, self.c, self.c["H"], self.c["n"]
-        lay, dsm, dvm = c["layers"][k], self.dsm, self.dvm
-        v_m = lay["v_m"]
-        dxin = torch.empty(n, 2 * H, dtype=torch.float32, device=v_m.device)
-        _glue("mlff_update_norm_tangent", n, H, v_m, lay["xin"], dsm, dvm, dxin)
-        upre = f"interactions.{k}.update"
-        da2 = dxin @ p[upre + ".update_mlp.0.weight"].T
-        dh2 = _silu_d(lay["a2"], da2)
-        dy = dh2 @ p[upre + ".update_mlp.2.weight"].T
-        self.ds = torch.empty_like(dsm)
-        self.dv = torch.empty_like(dvm)
-        dMv = torch.empty_like(dvm)
-        _glue("mlff_update_apply_tangent", n, H, lay["M"], lay["y"], dy, dsm, v_m, dvm,
-              lay["Mv"], self.ds, self.dv, dMv)
-        lay.update(dsm=dsm, dvm=dvm, dxin=dxin, da2=da2, dh2=dh2, dy=dy, dMv=dMv)
+    def moved(self, k: int):
+        """Tangents of block k's message outputs."""
+        return self.dsm, self.dvm
+
+    def updated(self, k: int):
+        lay = self.c["layers"][k]
+        lay.update(dsm=self.dsm, dvm=self.dvm)
+        self.ds, self.dv = lay["ds_out"], lay["dv_out"]
 
     def finish(self):
         p, c = self.p, self.c
@@ -674,7 +710,9 @@ def tangent(p: Dict[str, Tensor], c: dict, g: PairGraph, lam: Tensor):
     t = _Tangent(p, c, lam)
     for k in range(c["L"]):
         t.message(k, g)
-        t.update(k)
+        lay = c["layers"][k]
+        lay.update(_update(lay["w"], None, lay["v_m"], lay, *t.moved(k), primal=False))
+        t.updated(k)
     t.finish()
 
 
@@ -791,7 +829,7 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         GR1 = _silu_pair(r1, gh3, dr1, dgh3)
         gr1, dgr1 = GR1[0], GR1[1]
         GS = GR1.view(2 * n, -1) @ R1w
-        gs, dgs = GS[:n], GS[n:]
+        gs, dgs = GS[:n], _dense(GS[n:])
     else:
         gr2 = _silu_d(r2, gh4)
         gr1 = _silu_d(r1, gr2 @ R2w)
@@ -811,37 +849,13 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         lay = c["layers"][k]
         upre = f"interactions.{k}.update"
         mpre = f"interactions.{k}.message.rbf_to_scalar"
-        U1 = p[upre + ".update_mlp.0.weight"]
-        U2 = p[upre + ".update_mlp.2.weight"]
-        M, v_m, Mv, y, xin = lay["M"], lay["v_m"], lay["Mv"], lay["y"], lay["xin"]
-        # update reverse (student_model.py:434-470), gates and their tangent
-        # the adjoint and its tangent stacked ([2, n, ...]): one product for both
-        YY = torch.empty(2 if T else 1, n, 3 * H, dtype=torch.float32, device=dev)
-        gy, dgy = YY[0], (YY[1] if T else None)
-        dvm, dMv, dxin = (lay["dvm"], lay["dMv"], lay["dxin"]) if T else (None, None, None)
-        _glue("mlff_update_gate_adjoint", n, H, gs, gv, v_m, Mv, dgs if T else None,
-              dgv if T else None, dvm, dMv, gy, dgy)
-        if T:
-            GH2 = YY.view(2 * n, 3 * H) @ U2
-            GA2 = _silu_pair(lay["a2"], GH2[:n], lay["da2"], GH2[n:])
-            ga2, dga2 = GA2[0], GA2[1]
-            GX = GA2.view(2 * n, -1) @ U1
-            gx, dgx = GX[:n], GX[n:]
-        else:
-            ga2 = _silu_d(lay["a2"], gy @ U2)
-            gx, dgx = ga2 @ U1, None
-            dga2 = None
+        v_m, xin = lay["v_m"], lay["xin"]
+        # update reverse (student_model.py:434-470) and its tangent
+        dvm, dxin = (lay["dvm"], lay["dxin"]) if T else (None, None)
+        (gy, ga2, gs_m, gv_m, gvg2), (dgy, dga2, dgs_m, dgv_m, dgvg2) = _update_adjoint(
+            lay["w"], lay, gs, gv, dgs if T else None, dgv if T else None)
         linear(upre + ".update_mlp.2", gy, lay["h2"], dgy, lay["dh2"] if T else None, w_atom)
         linear(upre + ".update_mlp.0", ga2, xin, dga2, dxin, w_atom)
-        gs_m = torch.empty(n, H, dtype=torch.float32, device=dev)
-        gv_m = torch.empty(n, 3, H, dtype=torch.float32, device=dev)
-        gvg2 = torch.empty_like(gv_m)
-        dgs_m = torch.empty_like(gs_m) if T else None
-        dgv_m = torch.empty_like(gv_m) if T else None
-        dgvg2 = torch.empty_like(gv_m) if T else None
-        _glue("mlff_update_input_adjoint", n, H, M, gx, gs, gv, y, v_m, xin, dgx,
-              dgs if T else None, dgv if T else None, lay["dy"] if T else None, dvm, dxin,
-              gs_m, gv_m, gvg2, dgs_m, dgv_m, dgvg2)
         if diff:
             acc(grads, upre + ".mixing_matrix",
                 _xyz_outer(dgvg2, v_m, gvg2, dvm, w=w_atom, group=grp, diff=True))
