@@ -477,6 +477,17 @@ int mlff_weight_grad_diff_partials(void* stream, int K, int M, int N, const floa
                                    const float* row_w_dev, int with_bias, void* ws_dev,
                                    size_t ws_bytes);
 
+/* Partials of several weight gradients in one launch.  kind: 0 plain, 1 row
+ * weights, 2 two terms, 3 the difference of mlff_weight_grad_diff_partials; all
+ * with bias.  A table row is 14 int64 words: the problem's first block (each has
+ * ceil(M / 64) ceil(N / 64) S), then as int32 pairs K, M; N, rows_per_wave;
+ * ceil(M / 64), ceil(N / 64); S, lda0; ldb0, lda1; ldb1, 0, with rows_per_wave and
+ * S of mlff_weight_grad_split, then the addresses a0, b0, a1, b1, row_w, weight
+ * partials [S][M][N], bias partials [S][M].  n_blocks: the sum of their blocks. */
+int mlff_weight_grad_split(int K, int M, int N, int* rows_per_wave, int* n_partials);
+int mlff_weight_grad_group(void* stream, int kind, int n_problems, const int64_t* table_dev,
+                           int n_blocks);
+
 /* The same weight gradients in two steps, so that the partial sums of many
  * gradients (one training pass's) are added by one launch.  The products the
  * reference's backward computes are the same as for mlff_weight_grad.

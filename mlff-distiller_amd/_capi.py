@@ -46,7 +46,8 @@ EXPORTS = (
     "mlff_segment_sum", "mlff_plan_set_tiles", "mlff_edge_message", "mlff_edge_grad",
     "mlff_edge_csr", "mlff_edge_index",
     "mlff_weight_grad_workspace_bytes", "mlff_weight_grad", "mlff_weight_grad_partial_count",
-    "mlff_weight_grad_partials", "mlff_weight_grad_diff_partials", "mlff_weight_grad_reduce_group", "mlff_xyz_outer_partial_count",
+    "mlff_weight_grad_partials", "mlff_weight_grad_diff_partials",
+    "mlff_weight_grad_split", "mlff_weight_grad_group", "mlff_weight_grad_reduce_group", "mlff_xyz_outer_partial_count",
     "mlff_xyz_outer_partials", "mlff_xyz_outer_diff_partials", "mlff_train_geometry", "mlff_silu_chain",
     "mlff_update_norm", "mlff_update_apply", "mlff_update_norm_tangent",
     "mlff_update_apply_tangent", "mlff_update_gate_adjoint", "mlff_update_input_adjoint",
@@ -180,6 +181,10 @@ def _declare(lib):
     lib.mlff_weight_grad_partials.restype = ctypes.c_int
     lib.mlff_weight_grad_partials.argtypes = ([vp] + [ctypes.c_int] * 3 + [vp, ctypes.c_int] * 4
                                               + [vp, ctypes.c_int, vp, ctypes.c_size_t])
+    lib.mlff_weight_grad_split.restype = ctypes.c_int
+    lib.mlff_weight_grad_split.argtypes = [ctypes.c_int] * 3 + [vp, vp]
+    lib.mlff_weight_grad_group.restype = ctypes.c_int
+    lib.mlff_weight_grad_group.argtypes = [vp, ctypes.c_int, ctypes.c_int, vp, ctypes.c_int]
     lib.mlff_weight_grad_diff_partials.restype = ctypes.c_int
     lib.mlff_weight_grad_diff_partials.argtypes = lib.mlff_weight_grad_partials.argtypes
     lib.mlff_train_geometry.restype = ctypes.c_int

@@ -509,16 +509,30 @@ struct WgBatch {
   }
 };
 
+// One problem of the kernel; the grouped form reads them from a device table.
+struct WgProblem {
+  int64_t first;                    // grouped: the problem's first block
+  int K, M, N, RW, tiles_m, tiles_n, S, lda0, ldb0, lda1, ldb1, pad;
+  const float *a0, *b0, *a1, *b1, *roww;
+  float *part, *part_bias;
+};
+static_assert(sizeof(WgProblem) == 8 * 14, "14 int64 words per table row");
+
+// logical: consecutive blocks of a problem hold the tiles of one row range
 template <bool TWO, bool ROWW, bool BIAS, bool DIFF>
-__global__ __launch_bounds__(64 * kWgWaves, 3) void weight_grad_kernel(
-    int K, int M, int N, int RW, int tiles_m, int tiles_n, int S,
-    const float* __restrict__ a0, int lda0, const float* __restrict__ b0, int ldb0,
-    const float* __restrict__ a1, int lda1, const float* __restrict__ b1, int ldb1,
-    const float* __restrict__ roww, float* __restrict__ part, float* __restrict__ part_bias) {
+__device__ __forceinline__ void weight_grad_block(const WgProblem& p, int logical) {
+  const int K = p.K, M = p.M, N = p.N, RW = p.RW, tiles_m = p.tiles_m, tiles_n = p.tiles_n,
+            S = p.S, lda0 = p.lda0, ldb0 = p.ldb0, lda1 = p.lda1, ldb1 = p.ldb1;
+  const float* __restrict__ a0 = p.a0;
+  const float* __restrict__ b0 = p.b0;
+  const float* __restrict__ a1 = p.a1;
+  const float* __restrict__ b1 = p.b1;
+  const float* __restrict__ roww = p.roww;
+  float* __restrict__ part = p.part;
+  float* __restrict__ part_bias = p.part_bias;
   __shared__ __align__(16) f4 red[kWgWaves - 1][16 * 64];
   __shared__ f4 bred[kWgWaves][64];
   const int tiles = tiles_m * tiles_n;
-  const int logical = xcd_block();          // consecutive: the tiles of one row range
   if (logical >= tiles * S) return;         // grid padding (whole block)
   const int s = logical / tiles, tile = logical - s * tiles;
   const int tm = tile / tiles_n, tn = tile - tm * tiles_n;
@@ -614,6 +628,23 @@ __global__ __launch_bounds__(64 * kWgWaves, 3) void weight_grad_kernel(
     }
     if (m0 + lane < M) part_bias[(size_t)s * M + m0 + lane] = sum;
   }
+}
+
+template <bool TWO, bool ROWW, bool BIAS, bool DIFF>
+__global__ __launch_bounds__(64 * kWgWaves, 3) void weight_grad_kernel(WgProblem p) {
+  weight_grad_block<TWO, ROWW, BIAS, DIFF>(p, xcd_block());
+}
+
+// Several problems in one launch, each with the blocks, the split and the bits
+// it has by itself: the gradients of a few thousand rows are short launches.
+template <bool TWO, bool ROWW, bool DIFF>
+__global__ __launch_bounds__(64 * kWgWaves, 3) void weight_grad_group_kernel(
+    int n, const WgProblem* __restrict__ table) {
+  const int logical = xcd_block();
+  int q = 0;
+  while (q + 1 < n && table[q + 1].first <= logical) ++q;
+  const WgProblem p = table[q];
+  weight_grad_block<TWO, ROWW, true, DIFF>(p, logical - (int)p.first);
 }
 
 // One float4 of a weight gradient from its S partials: the partials added in
@@ -720,18 +751,9 @@ void weight_grad_split(int K, int M, int N, int& RW, int& S) {
 }
 
 template <bool TWO, bool ROWW, bool DIFF = false>
-void launch_weight_grad(hipStream_t st, bool bias, int blocks, int K, int M, int N, int RW,
-                        int tiles_m, int tiles_n, int S, const float* a0, int lda0,
-                        const float* b0, int ldb0, const float* a1, int lda1, const float* b1,
-                        int ldb1, const float* roww, float* part, float* part_bias) {
-  if (bias)
-    weight_grad_kernel<TWO, ROWW, true, DIFF><<<blocks, 64 * kWgWaves, 0, st>>>(
-        K, M, N, RW, tiles_m, tiles_n, S, a0, lda0, b0, ldb0, a1, lda1, b1, ldb1, roww, part,
-        part_bias);
-  else
-    weight_grad_kernel<TWO, ROWW, false, DIFF><<<blocks, 64 * kWgWaves, 0, st>>>(
-        K, M, N, RW, tiles_m, tiles_n, S, a0, lda0, b0, ldb0, a1, lda1, b1, ldb1, roww, part,
-        part_bias);
+void launch_weight_grad(hipStream_t st, bool bias, int blocks, const WgProblem& p) {
+  if (bias) weight_grad_kernel<TWO, ROWW, true, DIFF><<<blocks, 64 * kWgWaves, 0, st>>>(p);
+  else weight_grad_kernel<TWO, ROWW, false, DIFF><<<blocks, 64 * kWgWaves, 0, st>>>(p);
 }
 
 // Pair geometry and radial basis of the training pass, one thread per pair
@@ -1183,27 +1205,13 @@ static int weight_grad_partials(const char* who, void* stream, int K, int M, int
   // a multiple of 8 blocks, so that xcd_block() groups them by XCD
   const int blocks = (tiles_m * tiles_n * S + 7) / 8 * 8;
   float* part = static_cast<float*>(ws_dev);
-  float* part_bias = part + (size_t)S * M * N;
-  if (diff)
-    launch_weight_grad<true, true, true>(st, bias, blocks, K, M, N, RW, tiles_m, tiles_n, S, a0_dev,
-                                         lda0, b0_dev, ldb0, a1_dev, lda1, b1_dev, ldb1, row_w_dev,
-                                         part, part_bias);
-  else if (two && row_w_dev)
-    launch_weight_grad<true, true>(st, bias, blocks, K, M, N, RW, tiles_m, tiles_n, S, a0_dev,
-                                   lda0, b0_dev, ldb0, a1_dev, lda1, b1_dev, ldb1, row_w_dev,
-                                   part, part_bias);
-  else if (two)
-    launch_weight_grad<true, false>(st, bias, blocks, K, M, N, RW, tiles_m, tiles_n, S, a0_dev,
-                                    lda0, b0_dev, ldb0, a1_dev, lda1, b1_dev, ldb1, row_w_dev,
-                                    part, part_bias);
-  else if (row_w_dev)
-    launch_weight_grad<false, true>(st, bias, blocks, K, M, N, RW, tiles_m, tiles_n, S, a0_dev,
-                                    lda0, b0_dev, ldb0, a1_dev, lda1, b1_dev, ldb1, row_w_dev,
-                                    part, part_bias);
-  else
-    launch_weight_grad<false, false>(st, bias, blocks, K, M, N, RW, tiles_m, tiles_n, S,
-                                     a0_dev, lda0, b0_dev, ldb0, a1_dev, lda1, b1_dev, ldb1,
-                                     row_w_dev, part, part_bias);
+  const WgProblem p = {0, K, M, N, RW, tiles_m, tiles_n, S, lda0, ldb0, lda1, ldb1, 0, a0_dev,
+                       b0_dev, a1_dev, b1_dev, row_w_dev, part, part + (size_t)S * M * N};
+  if (diff) launch_weight_grad<true, true, true>(st, bias, blocks, p);
+  else if (two && row_w_dev) launch_weight_grad<true, true>(st, bias, blocks, p);
+  else if (two) launch_weight_grad<true, false>(st, bias, blocks, p);
+  else if (row_w_dev) launch_weight_grad<false, true>(st, bias, blocks, p);
+  else launch_weight_grad<false, false>(st, bias, blocks, p);
   *s_out = S;
   return MLFF_OK;
 }
@@ -1279,6 +1287,39 @@ int mlff_weight_grad_diff_partials(void* stream, int K, int M, int N, const floa
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error("%s: %s", nm, hipGetErrorString(e));
+    return MLFF_ERR_HIP;
+  }
+  return MLFF_OK;
+}
+
+int mlff_weight_grad_split(int K, int M, int N, int* rows_per_wave, int* n_partials) {
+  if (K < 0 || M < 4 || N < 4 || M % 4 || N % 4 || !rows_per_wave || !n_partials) {
+    set_error("mlff_weight_grad_split: need K >= 0 and M, N positive multiples of 4");
+    return MLFF_ERR_INVALID;
+  }
+  weight_grad_split(K, M, N, *rows_per_wave, *n_partials);
+  return MLFF_OK;
+}
+
+int mlff_weight_grad_group(void* stream, int kind, int n_problems, const int64_t* table_dev,
+                           int n_blocks) {
+  if (kind < 0 || kind > 3 || n_problems < 1 || n_blocks < 1 || !table_dev ||
+      !aligned16(table_dev)) {
+    set_error("mlff_weight_grad_group: need kind 0 to 3, problems, a 16-byte aligned table and "
+              "blocks");
+    return MLFF_ERR_INVALID;
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const WgProblem* t = reinterpret_cast<const WgProblem*>(table_dev);
+  const int blocks = (n_blocks + 7) / 8 * 8;
+  auto run = [&](auto kernel) { kernel<<<blocks, 64 * kWgWaves, 0, st>>>(n_problems, t); };
+  if (kind == 0) run(weight_grad_group_kernel<false, false, false>);
+  else if (kind == 1) run(weight_grad_group_kernel<false, true, false>);
+  else if (kind == 2) run(weight_grad_group_kernel<true, false, false>);
+  else run(weight_grad_group_kernel<true, true, true>);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error("mlff_weight_grad_group: %s", hipGetErrorString(e));
     return MLFF_ERR_HIP;
   }
   return MLFF_OK;

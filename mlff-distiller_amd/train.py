@@ -500,37 +500,84 @@ _WG_S: Dict[tuple, int] = {}    # partial sums of mlff_weight_grad by (K, M, N)
 
 
 class _WgGroup:
-    """Weight gradients whose split-K partial sums are added later, all in one
-    launch (mlff_weight_grad_reduce_group), instead of one launch each.  The
-    outputs _wgrad returns with a group hold their values only after
-    flush(); the partial buffers are kept alive until then."""
+    """Weight gradients that are finished later: the partial sums of all are
+    added in one launch (mlff_weight_grad_reduce_group), and those of the short
+    ones (the atoms' rows) are formed in one launch per kind
+    (mlff_weight_grad_group).  The outputs _wgrad returns with a group hold
+    their values only after flush(); operands and partials are kept until then."""
 
     def __init__(self):
         self.rows = []
         self.keep = []
+        self.short = {}     # kind: [(K, M, N, operands, out, bias)]
 
     def add(self, S: int, n4: int, part: int, out: int, buf: Tensor):
         self.rows.append((S, n4, part, out))
         self.keep.append(buf)
 
     def flush(self):
+        words, launches = [], []
+        for kind, probs in self.short.items():
+            splits = [_wg_split(*q[:3]) for q in probs]
+            part = torch.empty(sum(S * (M * N + M) for (_, S), (_, M, N, *_) in
+                                   zip(splits, probs)), dtype=torch.float32,
+                               device=probs[0][3][0].device)
+            self.keep.append((part, probs))
+            at, first, start = part.data_ptr(), 0, len(words) // 14
+            for (RW, S), (K, M, N, ops, out) in zip(splits, probs):
+                a0, b0, a1, b1, w = ops
+                tm, tn = (M + 63) // 64, (N + 63) // 64
+                ld = lambda t: 0 if t is None else t.stride(0)
+                pair = lambda x, y: x | y << 32
+                words += [first, pair(K, M), pair(N, RW), pair(tm, tn), pair(S, ld(a0)),
+                          pair(ld(b0), ld(a1)), ld(b1), _p(a0), _p(b0), _p(a1), _p(b1), _p(w), at,
+                          at + 4 * S * M * N]
+                self.rows += [(S, M * N // 4, at, out.data_ptr()),
+                              (S, M // 4, at + 4 * S * M * N, out.data_ptr() + 4 * M * N)]
+                at += 4 * S * (M * N + M)
+                first += tm * tn * S
+            launches.append((kind, len(probs), start, first))
+        self.short = {}
         if not self.rows:
             return
         lib = C.lib()
-        dev = self.keep[0].device
+        keep = self.keep[0]
+        dev = (keep[0] if isinstance(keep, tuple) else keep).device
+        n = len(words)
+        for row in self.rows:
+            words += row
+        table = torch.tensor(words, dtype=torch.int64, pin_memory=True).to(dev, non_blocking=True)
+        at = table.data_ptr()
+        for kind, n_probs, start, blocks in launches:
+            C.check("mlff_weight_grad_group", lib.mlff_weight_grad_group(
+                C.stream_handle(), kind, n_probs, at + 112 * start, blocks))
         for i in range(0, len(self.rows), 256):   # at most 256 rows per launch
             rows = self.rows[i:i + 256]
-            table = torch.tensor(rows, dtype=torch.int64, pin_memory=True).to(
-                dev, non_blocking=True)
             n_blocks = sum((n4 + 255) // 256 for _, n4, _, _ in rows)
             C.check("mlff_weight_grad_reduce_group", lib.mlff_weight_grad_reduce_group(
-                C.stream_handle(), len(rows), table.data_ptr(), min(n_blocks, 1 << 16)))
+                C.stream_handle(), len(rows), at + 8 * n + 32 * i, min(n_blocks, 1 << 16)))
         self.rows, self.keep = [], []
+
+
+_WG_SPLIT: Dict[tuple, tuple] = {}   # (rows per wave, partials) by (K, M, N)
+
+
+def _wg_split(K: int, M: int, N: int):
+    got = _WG_SPLIT.get((K, M, N))
+    if got is None:
+        import ctypes
+        rw, S = ctypes.c_int(), ctypes.c_int()
+        C.check("mlff_weight_grad_split", C.lib().mlff_weight_grad_split(
+            K, M, N, ctypes.byref(rw), ctypes.byref(S)))
+        if len(_WG_SPLIT) > 4096:
+            _WG_SPLIT.clear()
+        got = _WG_SPLIT[(K, M, N)] = (rw.value, S.value)
+    return got
 
 
 def _wgrad(a0: Tensor, b0: Tensor, a1: Optional[Tensor] = None, b1: Optional[Tensor] = None,
            w: Optional[Tensor] = None, bias: bool = False, group: Optional[_WgGroup] = None,
-           diff: bool = False):
+           diff: bool = False, short: bool = False):
     """sum_k w_k (a0[k] (x) b0[k] + a1[k] (x) b1[k]) [M, N] and, with
     ``bias``, sum_k w_k a0[k] [M] over the K rows (pairs or atoms): a Linear
     layer's weight and bias gradients, on the MFMA kernel with a fixed split
@@ -538,7 +585,8 @@ def _wgrad(a0: Tensor, b0: Tensor, a1: Optional[Tensor] = None, b1: Optional[Ten
     None).  With ``group`` only the partial sums are launched here; the
     outputs are filled, with the same bits, by group.flush().  ``diff`` (with a
     group): (w a1 - a0) (x) b0 - a1 (x) b1 and the sum of w a1 - a0
-    (mlff_weight_grad_diff_partials)."""
+    (mlff_weight_grad_diff_partials).  ``short`` (with a group and bias): one of
+    the launch of short ones at the flush."""
     M, N = a0.shape[1], b0.shape[1]
     K = a0.shape[0]
     A0, B0 = _wg_operand(a0), _wg_operand(b0)
@@ -546,6 +594,14 @@ def _wgrad(a0: Tensor, b0: Tensor, a1: Optional[Tensor] = None, b1: Optional[Ten
     if a1 is not None:
         A1, B1 = _wg_operand(a1), _wg_operand(b1)
     M4, N4 = A0.shape[1], B0.shape[1]
+    if short:
+        wv = None if w is None else _dense(w.to(torch.float32))
+        buf = torch.empty(M4 * N4 + M4, dtype=torch.float32, device=a0.device)
+        if not diff and A1 is not None and wv is not None:
+            raise ValueError("short weight gradients: two terms take no row weights")
+        kind = 3 if diff else 2 if A1 is not None else int(wv is not None)
+        group.short.setdefault(kind, []).append((K, M4, N4, (A0, B0, A1, B1, wv), buf))
+        return buf[:M4 * N4].view(M4, N4)[:M, :N], buf[M4 * N4:][:M]
     lib = C.lib()
     key = (K, M4, N4)
     ws_floats = _WG_WS.get(key)
@@ -772,21 +828,20 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         else:
             store[name] = val
 
-    def linear(name, ga, b, dga, db, w):
+    def linear(name, ga, b, dga, db, w, short=True):
         """Weight and bias gradients of a Linear with adjoint ga and input b."""
+        def put(store, *a, **kw):
+            gw_, gb_ = _wgrad(*a, bias=True, group=grp, short=short, **kw)
+            acc(store, name + ".weight", gw_)
+            acc(store, name + ".bias", gb_)
+
         if diff:
-            gw_, gb_ = _wgrad(dga, b, ga, db, w=w, bias=True, group=grp, diff=True)
-            acc(grads, name + ".weight", gw_)
-            acc(grads, name + ".bias", gb_)
+            put(grads, dga, b, ga, db, w=w, diff=True)
             return
         if primal:
-            gw_, gb_ = _wgrad(ga, b, w=w, bias=True, group=grp)
-            acc(grads, name + ".weight", gw_)
-            acc(grads, name + ".bias", gb_)
+            put(grads, ga, b, w=w)
         if T:
-            gw_, gb_ = _wgrad(dga, b, ga, db, bias=True, group=grp)
-            acc(tg, name + ".weight", gw_)
-            acc(tg, name + ".bias", gb_)
+            put(tg, dga, b, ga, db)
 
     def direct(name, val, dval):
         """A gradient and its tangent's, each given as a function."""
@@ -870,11 +925,13 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         else:
             gW, dgW = _pair_grad(g, H, u, s, v, gs_m, gv_m)
         W1 = p[mpre + ".0.weight"]
-        linear(mpre + ".2", gW, lay["h"], dgW, lay["dh"] if T else None, w_pair)
+        linear(mpre + ".2", gW, lay["h"], dgW, lay["dh"] if T else None, w_pair,
+               short=False)
         # gW W2 through the SiLU (and its tangent) on the fused pair kernel
         ga1, dga1 = _filter_adjoint(p, mpre, gW, lay["a1"], dgW if T else None,
                                     lay["da1"] if T else None)
-        linear(mpre + ".0", ga1, c["e"], dga1, c["de_t"] if T else None, w_pair)
+        linear(mpre + ".0", ga1, c["e"], dga1, c["de_t"] if T else None, w_pair,
+               short=False)
         if rbf_grads:
             ge = ga1 @ W1
             if T:
