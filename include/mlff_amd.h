@@ -666,6 +666,27 @@ int mlff_train_update_adjoint(void* stream, int n_atoms, int hidden_dim, const f
                               float* dgy_dev, float* dga_dev, float* dgs_out_dev,
                               float* dgv_out_dev, float* dgvg2_dev);
 
+/* The readout (student_model.py:606-618) of the training pass in one launch:
+ * r1 = s w1^T + b1, h3 = silu(r1) [N][H/2], r2 = h3 w2^T + b2, h4 = silu(r2)
+ * [N][H/4], eps = h4 . w3 + b3 [N]; parts as in mlff_train_update (2 reads r1 and
+ * r2).  s, ds and the weights are 16-byte aligned. */
+int mlff_train_readout(void* stream, int parts, int n_atoms, int hidden_dim, const float* s_dev,
+                       const float* ds_dev, const float* w1_dev, const float* b1_dev,
+                       const float* w2_dev, const float* b2_dev, const float* w3_dev,
+                       const float* b3_dev, float* r1_dev, float* h3_dev, float* r2_dev,
+                       float* h4_dev, float* eps_dev, float* dr1_dev, float* dh3_dev,
+                       float* dr2_dev, float* dh4_dev);
+
+/* Its adjoint from the seed g = seed[batch[i]] of each atom's energy and, with
+ * dr1 and dr2, the adjoint's tangent: gr2 = g w3 silu'(r2), gr1 = (gr2 w2) silu'(r1),
+ * gs = gr1 w1, g4 [N][4] = (g, 0, 0, 0). */
+int mlff_train_readout_adjoint(void* stream, int n_atoms, int hidden_dim, const float* seed_dev,
+                               const int64_t* batch_dev, const float* r1_dev, const float* r2_dev,
+                               const float* dr1_dev, const float* dr2_dev, const float* w1_dev,
+                               const float* w2_dev, const float* w3_dev, float* g4_dev,
+                               float* gr2_dev, float* gr1_dev, float* gs_dev, float* dgr2_dev,
+                               float* dgr1_dev, float* dgs_dev);
+
 /* ---------------------------------------------------------------------------
  * Matrix-core throughput probe, for the measured peak next to the published
  * one in roofline figures (no counterpart in the reference, which has no GPU

@@ -51,7 +51,8 @@ EXPORTS = (
     "mlff_xyz_outer_partials", "mlff_xyz_outer_diff_partials", "mlff_train_geometry", "mlff_silu_chain",
     "mlff_update_norm", "mlff_update_apply", "mlff_update_norm_tangent",
     "mlff_update_apply_tangent", "mlff_update_gate_adjoint", "mlff_update_input_adjoint",
-    "mlff_train_update", "mlff_train_update_adjoint",
+    "mlff_train_update", "mlff_train_update_adjoint", "mlff_train_readout",
+    "mlff_train_readout_adjoint",
     "mlff_probe_mfma_flops", "mlff_probe_mfma", "mlff_plan_set_weights",
     "mlff_train_filter", "mlff_train_filter_adjoint", "mlff_split_bf16x3", "mlff_pack_weights",
 )
@@ -165,6 +166,10 @@ def _declare(lib):
     lib.mlff_train_update.argtypes = [vp] + [ctypes.c_int] * 3 + [vp] * 23
     lib.mlff_train_update_adjoint.restype = ctypes.c_int
     lib.mlff_train_update_adjoint.argtypes = [vp] + [ctypes.c_int] * 2 + [vp] * 27
+    lib.mlff_train_readout.restype = ctypes.c_int
+    lib.mlff_train_readout.argtypes = [vp] + [ctypes.c_int] * 3 + [vp] * 17
+    lib.mlff_train_readout_adjoint.restype = ctypes.c_int
+    lib.mlff_train_readout_adjoint.argtypes = [vp] + [ctypes.c_int] * 2 + [vp] * 16
     lib.mlff_edge_index.restype = ctypes.c_int
     lib.mlff_edge_index.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 3
     lib.mlff_edge_grad.restype = ctypes.c_int

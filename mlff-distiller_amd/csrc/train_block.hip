@@ -1,6 +1,6 @@
 // The update block of the training pass (PaiNNUpdate, student_model.py:430-470)
 // with its tangent along a position direction, one launch per block and
-// direction:
+// direction (the readout's kernels follow):
 //   forward:  n = |v|_xyz, xin = (s, n), a = xin W1^T + b1, h = silu(a),
 //             y = (ds, g1, g2) = h W2^T + b2, Mv = M v,
 //             s' = s + ds, v' = v g1 + Mv g2, and/or the tangent of all of it;
@@ -315,6 +315,31 @@ __global__ __launch_bounds__(4 * H) void train_update_bwd_kernel(BwdArgs p) {
 #pragma unroll
   for (int k = 0; k < 9; ++k) mx[k] = p.mix[k];
   const int cb[2] = {16 * wave, H + 16 * wave};
+  // the epilogue's operands are requested before the product
+  float y1[4], y2[4], nm[4], qv[4][3], vr[4][3], e1[4], e2[4], en[4], dqv[4][3], dvr[4][3];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const size_t i = min(base + 4 * g + k, p.n - 1);
+    y1[k] = p.y[i * 3 * H + H + c];
+    y2[k] = p.y[i * 3 * H + 2 * H + c];
+    nm[k] = p.xin[i * 2 * H + H + c];
+    if (TAN) {
+      e1[k] = p.dy[i * 3 * H + H + c];
+      e2[k] = p.dy[i * 3 * H + 2 * H + c];
+      en[k] = p.dxin[i * 2 * H + H + c];
+    }
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      const size_t o = (i * 3 + x) * H + c;
+      qv[k][x] = p.gv[o];
+      vr[k][x] = p.v[o];
+      if (TAN) {
+        dqv[k][x] = p.dgv[o];
+        dvr[k][x] = p.dv[o];
+      }
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
   f4 acc[RT][2];
   zero_acc(acc);
   mma_tile_t<RT, 2, H>(a_lds, LDA, p.w1, 2 * H, cb, acc);
@@ -323,18 +348,17 @@ __global__ __launch_bounds__(4 * H) void train_update_bwd_kernel(BwdArgs p) {
     const int m = 4 * g + k;
     if (base + m >= p.n) continue;
     const size_t i = base + m;
-    const float g1 = p.y[i * 3 * H + H + c], g2 = p.y[i * 3 * H + 2 * H + c];
-    const float nrm = p.xin[i * 2 * H + H + c], inv = nrm > 0.f ? 1.0f / nrm : 0.f;
+    const float g1 = y1[k], g2 = y2[k];
+    const float nrm = nm[k], inv = nrm > 0.f ? 1.0f / nrm : 0.f;
     const float gn = acc[0][1][k];
-    float q[3], vv[3], qg[3], unit[3];
+    const float(&q)[3] = qv[k];
+    const float(&vv)[3] = vr[k];
+    float qg[3], unit[3];
 #pragma unroll
     for (int x = 0; x < 3; ++x) {
-      const size_t o = (i * 3 + x) * H + c;
-      q[x] = p.gv[o];
-      vv[x] = p.v[o];
       qg[x] = q[x] * g2;
       unit[x] = vv[x] * inv;
-      p.gvg2[o] = qg[x];
+      p.gvg2[(i * 3 + x) * H + c] = qg[x];
     }
     p.gs_out[i * H + c] = y_lds[m * LDY + c] + acc[0][0][k];
 #pragma unroll
@@ -342,17 +366,15 @@ __global__ __launch_bounds__(4 * H) void train_update_bwd_kernel(BwdArgs p) {
       p.gv_out[(i * 3 + x) * H + c] =
           q[x] * g1 + (mx[x] * qg[0] + mx[3 + x] * qg[1] + mx[6 + x] * qg[2]) + gn * unit[x];
     if (TAN) {
-      const float dg1 = p.dy[i * 3 * H + H + c], dg2 = p.dy[i * 3 * H + 2 * H + c];
-      const float dn = p.dxin[i * 2 * H + H + c], dninv2 = dn * inv * inv;
+      const float dg1 = e1[k], dg2 = e2[k], dninv2 = en[k] * inv * inv;
       const float dgn = acc[RT - 1][1][k];
-      float dq[3], dqg[3], dunit[3];
+      const float(&dq)[3] = dqv[k];
+      float dqg[3], dunit[3];
 #pragma unroll
       for (int x = 0; x < 3; ++x) {
-        const size_t o = (i * 3 + x) * H + c;
-        dq[x] = p.dgv[o];
         dqg[x] = dq[x] * g2 + q[x] * dg2;
-        dunit[x] = p.dv[o] * inv - vv[x] * dninv2;
-        p.dgvg2[o] = dqg[x];
+        dunit[x] = dvr[k][x] * inv - vv[x] * dninv2;
+        p.dgvg2[(i * 3 + x) * H + c] = dqg[x];
       }
       p.dgs_out[i * H + c] = y_lds[(kTM + m) * LDY + c] + acc[RT - 1][0][k];
 #pragma unroll
@@ -361,6 +383,225 @@ __global__ __launch_bounds__(4 * H) void train_update_bwd_kernel(BwdArgs p) {
             dq[x] * g1 + q[x] * dg1 + (mx[x] * dqg[0] + mx[3 + x] * dqg[1] + mx[6 + x] * dqg[2]) +
             dgn * unit[x] + gn * dunit[x];
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The readout (student_model.py:606-618: H -> H/2 -> H/4 -> 1, SiLU between) of
+// the training pass, 16 atoms per workgroup:
+//   forward: r1 = s W1^T + b1, h3 = silu(r1), r2 = h3 W2^T + b2, h4 = silu(r2),
+//            eps = h4 W3^T + b3, and/or the tangent;
+//   adjoint: gr2 = g W3 silu'(r2), gr1 = (gr2 W2) silu'(r1), gs = gr1 W1 with the
+//            atom's seed g, and with it the tangent.
+// The products are a few thousand multiplications per atom, on the vector units:
+// a thread takes one output column for four (two) of the tile's atoms and reads
+// its weights once for them, its inputs from LDS.  Bound by its launches; as
+// library products and elementwise kernels it was ten launches forward with the
+// tangent, and eight adjoint.
+// ---------------------------------------------------------------------------
+constexpr int kReadBlock = 256;
+
+struct ReadArgs {
+  int n;
+  const float *s, *ds, *w1, *b1, *w2, *b2, *w3, *b3;
+  float *r1, *h3, *r2, *h4, *eps;
+  float *dr1, *dh3, *dr2, *dh4;
+};
+
+// out[j][q] = sum_k x_j[q][k] w(k) for four atoms q of NX tiles x_j, four partial
+// sums each; w(k) gives the weights k ... k + 3
+template <int K, int LD, int NX, class W>
+__device__ __forceinline__ void dot_rows(const float* const (&x)[NX], W w, float (&out)[NX][4]) {
+  f4 acc[NX][4];
+#pragma unroll
+  for (int j = 0; j < NX; ++j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[j][q] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int k = 0; k < K; k += 4) {
+    const f4 wk = w(k);
+#pragma unroll
+    for (int j = 0; j < NX; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[j][q] = fma_(ld4(x[j] + q * LD + k), wk, acc[j][q]);
+  }
+#pragma unroll
+  for (int j = 0; j < NX; ++j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      out[j][q] = (acc[j][q][0] + acc[j][q][1]) + (acc[j][q][2] + acc[j][q][3]);
+}
+__device__ __forceinline__ auto row_of(const float* w) {
+  return [=](int k) { return ld4(w + k); };
+}
+// the same with a column of a matrix of ldw columns; a pass per tile: with two
+// tiles on one pass fewer loads are in flight (19 against 14 us)
+template <int K, int LD>
+__device__ __forceinline__ void dot_column(const float* x, const float* w, int ldw,
+                                           float (&out)[4]) {
+  const float* const rows[1] = {x};
+  float v[1][4];
+  dot_rows<K, LD, 1>(rows, [=](int k) {
+    return f4{w[(size_t)k * ldw], w[(size_t)(k + 1) * ldw], w[(size_t)(k + 2) * ldw],
+              w[(size_t)(k + 3) * ldw]};
+  }, v);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) out[q] = v[0][q];
+}
+
+template <int H, bool PRIM, bool TAN>
+__global__ __launch_bounds__(kReadBlock) void train_readout_fwd_kernel(ReadArgs p) {
+  constexpr int H2 = H / 2, H4 = H / 4, LX = H + 4, L2 = H2 + 4, L4 = H4 + 4;
+  __shared__ __align__(16) float x[2][kTM * LX];
+  __shared__ __align__(16) float h3[2][kTM * L2];
+  __shared__ __align__(16) float h4[kTM * L4];
+  __shared__ __align__(16) float w1[H2 * LX];    // rows a lane apart are far apart in memory
+  constexpr int NX = PRIM && TAN ? 2 : 1, X0 = PRIM ? 0 : 1;
+  const int base = blockIdx.x * kTM;
+  for (int it = threadIdx.x; it < H2 * H / 4; it += kReadBlock) {
+    const int c = it / (H / 4), k = 4 * (it % (H / 4));
+    st4(w1 + c * LX + k, ld4(p.w1 + (size_t)c * H + k));
+  }
+  for (int it = threadIdx.x; it < kTM * H / 4; it += kReadBlock) {
+    const int m = it / (H / 4), c = 4 * (it % (H / 4));
+    const size_t o = (size_t)min(base + m, p.n - 1) * H + c;
+    if (PRIM) st4(x[0] + m * LX + c, ld4(p.s + o));
+    if (TAN) st4(x[1] + m * LX + c, ld4(p.ds + o));
+  }
+  __syncthreads();
+  // items of four consecutive atoms and one column
+  for (int it = threadIdx.x; it < H2 * kTM / 4; it += kReadBlock) {
+    const int c = it % H2, m0 = 4 * (it / H2);
+    const float* in_rows[NX];
+    float v[NX][4];
+#pragma unroll
+    for (int j = 0; j < NX; ++j) in_rows[j] = x[X0 + j] + m0 * LX;
+    dot_rows<H, LX, NX>(in_rows, row_of(w1 + c * LX), v);
+    const float(&r)[4] = v[0];
+    const float(&d)[4] = v[NX - 1];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int m = m0 + q;
+      const bool in = base + m < p.n;
+      const size_t o = (size_t)min(base + m, p.n - 1) * H2 + c;
+      const float a = PRIM ? r[q] + p.b1[c] : p.r1[o], s = sigmoid(a);
+      if (PRIM) {
+        h3[0][m * L2 + c] = a * s;
+        if (in) { p.r1[o] = a; p.h3[o] = a * s; }
+      }
+      if (TAN) {
+        const float dh = silu_d1(a, s, sigmoid(-a)) * d[q];
+        h3[1][m * L2 + c] = dh;
+        if (in) { p.dr1[o] = d[q]; p.dh3[o] = dh; }
+      }
+    }
+  }
+  __syncthreads();
+  for (int it = threadIdx.x; it < H4 * kTM / 4; it += kReadBlock) {
+    const int c = it % H4, m0 = 4 * (it / H4);
+    const float* in_rows[NX];
+    float v[NX][4];
+#pragma unroll
+    for (int j = 0; j < NX; ++j) in_rows[j] = h3[X0 + j] + m0 * L2;
+    dot_rows<H2, L2, NX>(in_rows, row_of(p.w2 + (size_t)c * H2), v);
+    const float(&r)[4] = v[0];
+    const float(&d)[4] = v[NX - 1];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int m = m0 + q;
+      const bool in = base + m < p.n;
+      const size_t o = (size_t)min(base + m, p.n - 1) * H4 + c;
+      const float a = PRIM ? r[q] + p.b2[c] : p.r2[o], s = sigmoid(a);
+      if (PRIM) {
+        h4[m * L4 + c] = a * s;
+        if (in) { p.r2[o] = a; p.h4[o] = a * s; }
+      }
+      if (TAN && in) {
+        p.dr2[o] = d[q];
+        p.dh4[o] = silu_d1(a, s, sigmoid(-a)) * d[q];
+      }
+    }
+  }
+  if constexpr (PRIM) {
+    __syncthreads();
+    if (threadIdx.x < kTM / 4) {
+      const int m0 = 4 * threadIdx.x;
+      const float* in_rows[1] = {h4 + m0 * L4};
+      float e[1][4];
+      dot_rows<H4, L4, 1>(in_rows, row_of(p.w3), e);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (base + m0 + q < p.n) p.eps[base + m0 + q] = e[0][q] + p.b3[0];
+    }
+  }
+}
+
+struct ReadAdjArgs {
+  int n;
+  const float *seed;                 // g of each structure
+  const int64_t* batch;              // structure of each atom
+  const float *r1, *r2, *dr1, *dr2, *w1, *w2, *w3;
+  float *g4, *gr2, *gr1, *gs;        // g4 [n][4]: (g, 0, 0, 0)
+  float *dgr2, *dgr1, *dgs;
+};
+
+template <int H, bool TAN>
+__global__ __launch_bounds__(kReadBlock) void train_readout_bwd_kernel(ReadAdjArgs p) {
+  constexpr int H2 = H / 2, H4 = H / 4, L2 = H2 + 4, L4 = H4 + 4;
+  __shared__ __align__(16) float g2[2][kTM * L4];
+  __shared__ __align__(16) float g1[2][kTM * L2];
+  const int base = blockIdx.x * kTM;
+  for (int it = threadIdx.x; it < kTM * H4; it += kReadBlock) {
+    const int m = it / H4, c = it % H4;
+    const bool in = base + m < p.n;
+    const size_t i = min(base + m, p.n - 1), o = i * H4 + c;
+    const float g = p.seed[p.batch[i]], gh = g * p.w3[c];
+    const float a = p.r2[o], s = sigmoid(a), q = sigmoid(-a);
+    const float v = gh * silu_d1(a, s, q);
+    g2[0][m * L4 + c] = v;
+    if (in) p.gr2[o] = v;
+    if (TAN) {
+      const float d = gh * silu_d2(a, s, q) * p.dr2[o];
+      g2[1][m * L4 + c] = d;
+      if (in) p.dgr2[o] = d;
+    }
+    if (in && c < 4) p.g4[4 * i + c] = c == 0 ? g : 0.f;
+  }
+  __syncthreads();
+  for (int it = threadIdx.x; it < H2 * kTM / 4; it += kReadBlock) {
+    const int c = it % H2, m0 = 4 * (it / H2);
+    float v[4], d[4];
+    dot_column<H4, L4>(g2[0] + m0 * L4, p.w2 + c, H2, v);
+    if (TAN) dot_column<H4, L4>(g2[1] + m0 * L4, p.w2 + c, H2, d);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int m = m0 + k;
+      const bool in = base + m < p.n;
+      const size_t o = (size_t)min(base + m, p.n - 1) * H2 + c;
+      const float a = p.r1[o], s = sigmoid(a), q = sigmoid(-a), d1 = silu_d1(a, s, q);
+      const float t = v[k] * d1;
+      g1[0][m * L2 + c] = t;
+      if (in) p.gr1[o] = t;
+      if (TAN) {
+        const float u = fma_(d[k], d1, v[k] * silu_d2(a, s, q) * p.dr1[o]);
+        g1[1][m * L2 + c] = u;
+        if (in) p.dgr1[o] = u;
+      }
+    }
+  }
+  __syncthreads();
+  for (int it = threadIdx.x; it < H * kTM / 4; it += kReadBlock) {
+    const int c = it % H, m0 = 4 * (it / H);
+    float v[4], d[4];
+    dot_column<H2, L2>(g1[0] + m0 * L2, p.w1 + c, H, v);
+    if (TAN) dot_column<H2, L2>(g1[1] + m0 * L2, p.w1 + c, H, d);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (base + m0 + k < p.n) {
+        const size_t o = (size_t)(base + m0 + k) * H + c;
+        p.gs[o] = v[k];
+        if (TAN) p.dgs[o] = d[k];
+      }
   }
 }
 
@@ -477,6 +718,85 @@ int mlff_train_update_adjoint(void* stream, int n_atoms, int hidden_dim, const f
     case 32: return tan ? run(train_update_bwd_kernel<32, true>) : run(train_update_bwd_kernel<32, false>);
     case 64: return tan ? run(train_update_bwd_kernel<64, true>) : run(train_update_bwd_kernel<64, false>);
     case 128: return tan ? run(train_update_bwd_kernel<128, true>) : run(train_update_bwd_kernel<128, false>);
+  }
+  set_error("%s: hidden_dim %d not supported (32, 64, 128)", nm, hidden_dim);
+  return MLFF_ERR_UNSUPPORTED;
+}
+
+int mlff_train_readout(void* stream, int parts, int n_atoms, int hidden_dim, const float* s_dev,
+                       const float* ds_dev, const float* w1_dev, const float* b1_dev,
+                       const float* w2_dev, const float* b2_dev, const float* w3_dev,
+                       const float* b3_dev, float* r1_dev, float* h3_dev, float* r2_dev,
+                       float* h4_dev, float* eps_dev, float* dr1_dev, float* dh3_dev,
+                       float* dr2_dev, float* dh4_dev) {
+  const char* nm = "mlff_train_readout";
+  const bool prim = parts & 1, tan = parts & 2;
+  if (n_atoms < 0 || parts < 1 || parts > 3) {
+    set_error("%s: invalid size or parts", nm);
+    return MLFF_ERR_INVALID;
+  }
+  if (n_atoms == 0) return MLFF_OK;
+  if (!present({w1_dev, w2_dev, r1_dev, r2_dev}) ||
+      (prim && !present({s_dev, b1_dev, b2_dev, w3_dev, b3_dev, h3_dev, h4_dev, eps_dev})) ||
+      (tan && !present({ds_dev, dr1_dev, dh3_dev, dr2_dev, dh4_dev}))) {
+    set_error("%s: null buffer", nm);
+    return MLFF_ERR_INVALID;
+  }
+  if (!aligned({s_dev, ds_dev, w1_dev, w2_dev, w3_dev})) {
+    set_error("%s: buffers must be 16-byte aligned", nm);
+    return MLFF_ERR_INVALID;
+  }
+  const ReadArgs p = {n_atoms, s_dev, ds_dev, w1_dev, b1_dev, w2_dev, b2_dev, w3_dev, b3_dev,
+                      r1_dev, h3_dev, r2_dev, h4_dev, eps_dev, dr1_dev, dh3_dev, dr2_dev, dh4_dev};
+  auto run = [&](auto kernel) {
+    kernel<<<(n_atoms + kTM - 1) / kTM, kReadBlock, 0, static_cast<hipStream_t>(stream)>>>(p);
+    return finish(nm);
+  };
+#define MLFF_READ(H)                                                   \
+  case H:                                                              \
+    return prim && tan ? run(train_readout_fwd_kernel<H, true, true>)  \
+           : prim      ? run(train_readout_fwd_kernel<H, true, false>) \
+                       : run(train_readout_fwd_kernel<H, false, true>);
+  switch (hidden_dim) {
+    MLFF_READ(32)
+    MLFF_READ(64)
+    MLFF_READ(128)
+  }
+#undef MLFF_READ
+  set_error("%s: hidden_dim %d not supported (32, 64, 128)", nm, hidden_dim);
+  return MLFF_ERR_UNSUPPORTED;
+}
+
+int mlff_train_readout_adjoint(void* stream, int n_atoms, int hidden_dim, const float* seed_dev,
+                               const int64_t* batch_dev, const float* r1_dev, const float* r2_dev,
+                               const float* dr1_dev, const float* dr2_dev, const float* w1_dev,
+                               const float* w2_dev, const float* w3_dev, float* g4_dev,
+                               float* gr2_dev, float* gr1_dev, float* gs_dev, float* dgr2_dev,
+                               float* dgr1_dev, float* dgs_dev) {
+  const char* nm = "mlff_train_readout_adjoint";
+  const bool tan = dr1_dev != nullptr;
+  if (n_atoms < 0) {
+    set_error("%s: invalid size", nm);
+    return MLFF_ERR_INVALID;
+  }
+  if (n_atoms == 0) return MLFF_OK;
+  if (!present({seed_dev, batch_dev, r1_dev, r2_dev, w1_dev, w2_dev, w3_dev, g4_dev, gr2_dev,
+                gr1_dev, gs_dev}) ||
+      (tan && !present({dr2_dev, dgr2_dev, dgr1_dev, dgs_dev}))) {
+    set_error("%s: null buffer", nm);
+    return MLFF_ERR_INVALID;
+  }
+  const ReadAdjArgs p = {n_atoms, seed_dev, batch_dev, r1_dev, r2_dev, dr1_dev, dr2_dev, w1_dev,
+                         w2_dev, w3_dev, g4_dev, gr2_dev, gr1_dev, gs_dev, dgr2_dev, dgr1_dev,
+                         dgs_dev};
+  auto run = [&](auto kernel) {
+    kernel<<<(n_atoms + kTM - 1) / kTM, kReadBlock, 0, static_cast<hipStream_t>(stream)>>>(p);
+    return finish(nm);
+  };
+  switch (hidden_dim) {
+    case 32: return tan ? run(train_readout_bwd_kernel<32, true>) : run(train_readout_bwd_kernel<32, false>);
+    case 64: return tan ? run(train_readout_bwd_kernel<64, true>) : run(train_readout_bwd_kernel<64, false>);
+    case 128: return tan ? run(train_readout_bwd_kernel<128, true>) : run(train_readout_bwd_kernel<128, false>);
   }
   set_error("%s: hidden_dim %d not supported (32, 64, 128)", nm, hidden_dim);
   return MLFF_ERR_UNSUPPORTED;

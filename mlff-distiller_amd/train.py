@@ -24,9 +24,9 @@ Where the work runs:
   per unordered pair from both endpoints -- no scatter-adds, no atomics;
 * per-structure energies and the embedding gradient by fixed-order segment
   sums (mlff_segment_sum);
-* the update block with its products, and its reverse, on one kernel each
-  (mlff_train_update, mlff_train_update_adjoint), primal and tangent together;
-  the readout's small products as library GEMMs;
+* the update block and the readout with their products, and their reverses,
+  on one kernel each (mlff_train_update, mlff_train_readout and their
+  adjoints), primal and tangent together;
 * weight gradients on a split-row kernel with a fixed order
   (mlff_weight_grad_partials).
 Every reduction runs in a fixed order: two runs give bit-identical gradients.
@@ -303,6 +303,49 @@ def _update_weights(p: Dict[str, Tensor], upre: str):
                                                ".mixing_matrix"))
 
 
+def _readout(w, s, c: Optional[dict] = None, ds=None, primal: bool = True):
+    """The readout of s and, with ds, its tangent, in one launch
+    (mlff_train_readout); w = (W1, b1, W2, b2, W3, b3), dense.  ``primal`` False:
+    the tangent of the pass stored in ``c``."""
+    n, H = (s if primal else ds).shape
+    dev = w[0].device
+    new = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=dev)
+    out = {}
+    if primal:
+        out.update(r1=new(n, H // 2), h3=new(n, H // 2), r2=new(n, H // 4), h4=new(n, H // 4),
+                   eps=new(n))
+    if ds is not None:
+        out.update(dr1=new(n, H // 2), dh3=new(n, H // 2), dr2=new(n, H // 4),
+                   dh4=new(n, H // 4))
+    src = out if primal else c
+    keys = ("dr1", "dh3", "dr2", "dh4")
+    C.check("mlff_train_readout", C.lib().mlff_train_readout(
+        C.stream_handle(), int(primal) + 2 * (ds is not None), n, H, C.ptr(s), C.ptr(ds),
+        *[C.ptr(t) for t in w], C.ptr(src["r1"]), C.ptr(src["h3"]), C.ptr(src["r2"]),
+        C.ptr(src["h4"]), C.ptr(src.get("eps")), *[C.ptr(out.get(k)) for k in keys]))
+    return out
+
+
+def _readout_adjoint(w, c: dict, seed, batch, T: bool):
+    """(g4, gr2, gr1, gs) from the structures' seeds and, with T, the tangents
+    (dgr2, dgr1, dgs) or Nones (mlff_train_readout_adjoint)."""
+    r1, r2 = c["r1"], c["r2"]
+    n, H = r1.shape[0], 2 * r1.shape[1]
+    new = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=r1.device)
+    outs = lambda: [new(n, H // 4), new(n, H // 2), new(n, H)]
+    g4, out, dout = new(n, 4), outs(), outs() if T else [None] * 3
+    C.check("mlff_train_readout_adjoint", C.lib().mlff_train_readout_adjoint(
+        C.stream_handle(), n, H, C.ptr(seed), C.ptr(batch), C.ptr(r1), C.ptr(r2),
+        C.ptr(c["dr1"] if T else None), C.ptr(c["dr2"] if T else None), C.ptr(w[0]), C.ptr(w[2]),
+        C.ptr(w[4]), C.ptr(g4), *[C.ptr(t) for t in out + dout]))
+    return (g4, *out), dout
+
+
+def _readout_weights(p: Dict[str, Tensor]):
+    return tuple(_dense(p["energy_head." + k]) for k in ("0.weight", "0.bias", "2.weight",
+                                                         "2.bias", "4.weight", "4.bias"))
+
+
 def _silu_call(a, da=None, g=None, dg=None, h=False, dh=False, dga=False):
     a = _dense(a)
     opt = lambda t: None if t is None else _dense(t)
@@ -312,19 +355,6 @@ def _silu_call(a, da=None, g=None, dg=None, h=False, dh=False, dga=False):
         C.stream_handle(), a.numel(), C.ptr(a), C.ptr(da), C.ptr(g), C.ptr(dg),
         C.ptr(outs[0]), C.ptr(outs[1]), None, C.ptr(outs[2])))
     return [o for o in outs if o is not None][0]
-
-
-def _silu_pair(x, g, dx, dg=None):
-    """The adjoint g silu'(x) and its tangent dg silu'(x) + g silu''(x) dx
-    (dg None is zero) from one pass, stacked in one [2, *x.shape] buffer, so
-    the products that follow take both as one operand."""
-    x, g, dx = _dense(x), _dense(g), _dense(dx)
-    dg = None if dg is None else _dense(dg)
-    out = torch.empty((2,) + tuple(x.shape), dtype=torch.float32, device=x.device)
-    C.check("mlff_silu_chain", C.lib().mlff_silu_chain(
-        C.stream_handle(), x.numel(), C.ptr(x), C.ptr(dx), C.ptr(g), C.ptr(dg), None, None,
-        C.ptr(out[0]), C.ptr(out[1])))
-    return out
 
 
 def _silu(x):
@@ -637,10 +667,6 @@ def _wgrad(a0: Tensor, b0: Tensor, a1: Optional[Tensor] = None, b1: Optional[Ten
     return out, bout
 
 
-def _lin(x, p, name):
-    return torch.addmm(p[name + ".bias"], x, p[name + ".weight"].T)
-
-
 def _xyz_outer(a, b, a1=None, b1=None, w=None, group: Optional[_WgGroup] = None,
                diff: bool = False):
     """sum_n w_n sum_h (a[n,x,h] b[n,z,h] + a1[n,x,h] b1[n,z,h]) -> [3,3]
@@ -704,15 +730,13 @@ def forward(p: Dict[str, Tensor], Z: Tensor, x: Tensor, g: PairGraph, rc: float,
             lay.update(_update(lay["w"], s_m, v_m, None, *t.moved(k)))
             t.updated(k)
         s, v = lay["s_out"], lay["v_out"]
-    r1 = _lin(s, p, "energy_head.0")
-    h3 = _silu(r1)
-    r2 = _lin(h3, p, "energy_head.2")
-    h4 = _silu(r2)
-    eps = _lin(h4, p, "energy_head.4")[:, 0]
-    E = _segment_sum(g.mol_ptr, eps, f64=True)
-    cache.update(sL=s, r1=r1, h3=h3, r2=r2, h4=h4)
-    if t is not None:
+    cache.update(sL=s, wr=_readout_weights(p))
+    if t is None:
+        cache.update(_readout(cache["wr"], s))
+    else:
+        cache.update(_readout(cache["wr"], s, None, t.ds))
         t.finish()
+    E = _segment_sum(g.mol_ptr, cache["eps"], f64=True)
     return E, cache
 
 
@@ -751,14 +775,9 @@ class _Tangent:
         self.ds, self.dv = lay["ds_out"], lay["dv_out"]
 
     def finish(self):
-        p, c = self.p, self.c
+        c = self.c
         dd, du, de_t = self.geometry
-        dr1 = self.ds @ p["energy_head.0.weight"].T
-        dh3 = _silu_d(c["r1"], dr1)
-        dr2 = dh3 @ p["energy_head.2.weight"].T
-        dh4 = _silu_d(c["r2"], dr2)
-        c.update(lam=self.lam, dd=dd, du=du, de_t=de_t, dsL=self.ds, dr1=dr1, dh3=dh3, dr2=dr2,
-                 dh4=dh4)
+        c.update(lam=self.lam, dd=dd, du=du, de_t=de_t, dsL=self.ds)
 
 
 def tangent(p: Dict[str, Tensor], c: dict, g: PairGraph, lam: Tensor):
@@ -769,6 +788,7 @@ def tangent(p: Dict[str, Tensor], c: dict, g: PairGraph, lam: Tensor):
         lay = c["layers"][k]
         lay.update(_update(lay["w"], None, lay["v_m"], lay, *t.moved(k), primal=False))
         t.updated(k)
+    c.update(_readout(c["wr"], None, c, t.ds, primal=False))
     t.finish()
 
 
@@ -865,33 +885,16 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         wa = wp = lambda t: t
 
     # ---- readout reverse ------------------------------------------------------
-    geps = gE[g.batch]
-    r1, h3, r2, h4, sL = c["r1"], c["h3"], c["r2"], c["h4"], c["sL"]
-    Q3 = p["energy_head.4.weight"]
-    direct("energy_head.4.weight", lambda: (wa(geps) @ h4).reshape(1, -1),
-           lambda: (geps @ c["dh4"]).reshape(1, -1))
-    direct("energy_head.4.bias", lambda: wa(geps).sum().reshape(1),
-           lambda: torch.zeros(1, dtype=torch.float32, device=dev))
-    gh4 = geps.unsqueeze(1) * Q3
-    R2w, R1w = p["energy_head.2.weight"], p["energy_head.0.weight"]
-    if T:
-        # each adjoint is stacked with its tangent: one product for both
-        dr1, dh3, dr2, dh4 = c["dr1"], c["dh3"], c["dr2"], c["dh4"]
-        GR2 = _silu_pair(r2, gh4, dr2)
-        gr2, dgr2 = GR2[0], GR2[1]
-        GH3 = GR2.view(2 * n, -1) @ R2w
-        gh3, dgh3 = GH3[:n], GH3[n:]
-        GR1 = _silu_pair(r1, gh3, dr1, dgh3)
-        gr1, dgr1 = GR1[0], GR1[1]
-        GS = GR1.view(2 * n, -1) @ R1w
-        gs, dgs = GS[:n], _dense(GS[n:])
-    else:
-        gr2 = _silu_d(r2, gh4)
-        gr1 = _silu_d(r1, gr2 @ R2w)
-        gs = (gr1 @ R1w).contiguous()
-        dgr2 = dgr1 = dh3 = None
-    linear("energy_head.2", gr2, h3, dgr2, dh3, w_atom)
-    linear("energy_head.0", gr1, sL, dgr1, c["dsL"] if T else None, w_atom)
+    (g4, gr2, gr1, gs), (dgr2, dgr1, dgs) = _readout_adjoint(c["wr"], c, gE.contiguous(), g.batch, T)
+    d = (lambda key: c[key]) if T else (lambda key: None)
+    # the seeds as a one-column Linear of four columns, whose tangent is zero
+    linear("energy_head.4", g4, c["h4"], torch.zeros_like(g4) if T else None, d("dh4"), w_atom)
+    linear("energy_head.2", gr2, c["h3"], dgr2, d("dh3"), w_atom)
+    linear("energy_head.0", gr1, c["sL"], dgr1, d("dsL"), w_atom)
+    for store in (grads, tg):
+        for k, rows in (("energy_head.4.weight", slice(0, 1)), ("energy_head.4.bias", slice(0, 1))):
+            if k in store:
+                store[k] = store[k][rows]
     gv = torch.zeros(n, 3, H, dtype=torch.float32, device=dev)
     if T:
         dgv = torch.zeros_like(gv)

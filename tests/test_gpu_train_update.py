@@ -76,3 +76,53 @@ def test_zero_vectors_have_no_direction(gpu):
     lay = dict(o, v_m=z, dvm=r(n, 3, H))
     for t in sum(train._update_adjoint(w, lay, r(n, H), r(n, 3, H), r(n, H), r(n, 3, H)), []):
         assert torch.isfinite(t).all()
+
+
+@pytest.mark.parametrize("H", [32, 64, 128])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 50])
+def test_readout_and_its_derivatives(gpu, n, H):
+    """As above: sums of up to 128 products through three layers."""
+    print(f"[case] train readout n{n} H{H}", flush=True)
+    train = pkg_mod("train")
+    g = torch.Generator().manual_seed(7 * n + H)
+    r = lambda *sh: torch.randn(*sh, generator=g)
+    w = (r(H // 2, H) / H ** 0.5, 0.1 * r(H // 2), r(H // 4, H // 2) / (H / 2) ** 0.5,
+         0.1 * r(H // 4), r(1, H // 4), r(1))
+    s, ds, seed = r(n, H), r(n, H), r(3)
+    batch = torch.randint(0, 3, (n,), generator=g)
+    W1, b1, W2, b2, W3, b3 = (t.double() for t in w)
+    silu = torch.nn.functional.silu
+
+    def plain(x):
+        return (silu(silu(x @ W1.T + b1) @ W2.T + b2) @ W3.T + b3)[:, 0]
+
+    def vjp(x):
+        with torch.enable_grad():
+            if not x.requires_grad:
+                x = x.requires_grad_(True)
+            return torch.autograd.grad(plain(x), x, seed.double()[batch], create_graph=True)[0]
+
+    eps = plain(s.double())
+    gs, dgs = torch.autograd.functional.jvp(vjp, s.double(), ds.double())
+    h4 = lambda x: silu(silu(x @ W1.T + b1) @ W2.T + b2)
+    _, dh4 = torch.autograd.functional.jvp(h4, s.double(), ds.double())
+    wg = tuple(t.to(gpu) for t in w)
+
+    def close(a, b, what):
+        assert (a.cpu().double() - b.detach()).norm() <= 1e-5 * b.detach().norm(), what
+
+    both = train._readout(wg, s.to(gpu), None, ds.to(gpu))
+    first = train._readout(wg, s.to(gpu))
+    then = train._readout(wg, None, first, ds.to(gpu), primal=False)
+    for o in (both, {**first, **then}):
+        close(o["eps"], eps, "eps")
+        close(o["h4"], h4(s.double()), "h4")
+        close(o["dh4"], dh4, "dh4")
+    sg, bg = seed.to(gpu), batch.to(gpu)
+    one, none = train._readout_adjoint(wg, both, sg, bg, False)
+    two, tan = train._readout_adjoint(wg, both, sg, bg, True)
+    assert none == [None] * 3
+    for o in (one, two):
+        assert torch.equal(o[0][:, 0].cpu(), seed[batch]) and not o[0][:, 1:].any()
+        close(o[3], gs, "gs")
+    close(tan[2], dgs, "dgs")
