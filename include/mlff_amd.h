@@ -589,6 +589,20 @@ int mlff_train_filter_adjoint(void* stream, int tangent, int hidden, int n_pairs
                               const float* a_dev, const float* da_dev, float* ga_out_dev,
                               float* dga_out_dev);
 
+/* What the pair kernels of the training pass read of a filter MLP, in one launch:
+ * W1 [H][R] padded to [H][16 or 32], the three bf16 planes of W2 [3H][H] and of
+ * its transpose [H][3H], and the transpose. */
+int mlff_filter_planes(void* stream, int hidden_dim, int R, const float* w1_dev,
+                       const float* w2_dev, float* w1p_dev, uint16_t* planes_dev,
+                       uint16_t* planes_t_dev, float* w2t_dev);
+
+/* mlff_train_filter_adjoint on the bf16 matrix cores (hidden_dim 64 or 128), with
+ * the planes of W2^T that mlff_filter_planes makes. */
+int mlff_train_filter_adjoint_x6(void* stream, int hidden_dim, int n_pairs, const float* gw_dev,
+                                 const float* dgw_dev, const uint16_t* planes_t_dev,
+                                 const float* a_dev, const float* da_dev, float* ga_dev,
+                                 float* dga_dev);
+
 /* Split n float32 values into three bfloat16 planes (planes_dev [3][n]):
  * x = hi + mid + lo, each part the round-to-nearest-even bfloat16 of what the
  * previous parts leave (24 significant bits together). */

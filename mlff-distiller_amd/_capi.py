@@ -54,7 +54,8 @@ EXPORTS = (
     "mlff_train_update", "mlff_train_update_adjoint", "mlff_train_readout",
     "mlff_train_readout_adjoint",
     "mlff_probe_mfma_flops", "mlff_probe_mfma", "mlff_plan_set_weights",
-    "mlff_train_filter", "mlff_train_filter_adjoint", "mlff_split_bf16x3", "mlff_pack_weights",
+    "mlff_train_filter", "mlff_train_filter_adjoint",
+    "mlff_filter_planes", "mlff_train_filter_adjoint_x6", "mlff_split_bf16x3", "mlff_pack_weights",
 )
 
 # bytes of the static device scratch behind mlff_energy_forces_static
@@ -170,6 +171,10 @@ def _declare(lib):
     lib.mlff_train_readout.argtypes = [vp] + [ctypes.c_int] * 3 + [vp] * 17
     lib.mlff_train_readout_adjoint.restype = ctypes.c_int
     lib.mlff_train_readout_adjoint.argtypes = [vp] + [ctypes.c_int] * 2 + [vp] * 16
+    lib.mlff_filter_planes.restype = ctypes.c_int
+    lib.mlff_filter_planes.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 6
+    lib.mlff_train_filter_adjoint_x6.restype = ctypes.c_int
+    lib.mlff_train_filter_adjoint_x6.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 7
     lib.mlff_edge_index.restype = ctypes.c_int
     lib.mlff_edge_index.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 3
     lib.mlff_edge_grad.restype = ctypes.c_int

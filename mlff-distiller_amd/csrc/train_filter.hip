@@ -15,12 +15,13 @@
 //   gh = gW W2,   ga = silu'(a) gh,
 //   dgh = dgW W2, dga = silu'(a) dgh + silu''(a) da gh
 //
-// with the products on the FP32 matrix cores (W2 comes transposed, [H][3H]).  The first product runs on the FP32 matrix
-// cores; the second, the large one, on the bf16 matrix cores with both
+// on the FP32 matrix cores (W2 comes transposed, [H][3H]) or, for H >= 64, the
+// bf16 ones.  In the forward and the tangent the first product runs on the FP32
+// matrix cores; the second, the large one, on the bf16 matrix cores with both
 // operands split into three bf16 parts (six part products, float32
 // accuracy), as in the evaluation's filter kernel.  W1 comes padded to RP
-// columns (16 or 32, zeros beyond R) and W2 as three bf16 planes
-// (mlff_split_bf16x3), so a caller re-splits W2 once per weight update.
+// columns (16 or 32, zeros beyond R) and W2 and its transpose as three bf16
+// planes, which mlff_filter_planes makes once per weight update.
 
 #include <stdint.h>
 
@@ -310,6 +311,130 @@ __global__ __launch_bounds__(kTaBlock, 4) void train_filter_adjoint_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// The filter adjoint on the bf16 matrix cores (H >= 64): each K chunk of gW and
+// dgW is split into three bf16 parts on its way to LDS and multiplied with the
+// split W2^T (six part products, float32 accuracy).  Bound by the 10H floats per
+// pair read and written and the splitting.  64 molecules, H = 128: 90 us per
+// block against 117 us of the FP32 form above, which its products bound (121
+// TFLOP/s).  At H = 32 that form's products are short enough (29 us).
+// ---------------------------------------------------------------------------
+template <int H, int TM, bool TAN>
+__global__ __launch_bounds__(kTfBlock, 4) void train_filter_adjoint_x6_kernel(
+    int P, const float* __restrict__ gw, const float* __restrict__ dgw,
+    const uint16_t* __restrict__ w2t, const float* __restrict__ a, const float* __restrict__ da,
+    float* __restrict__ ga, float* __restrict__ dga) {
+  constexpr int LDA = H + 8, PA = TM * LDA, NS = TAN ? 2 : 1;
+  constexpr int CT = H / 16, RG = kTfWaves / CT, RTW = TM / 16 / RG;
+  constexpr int PB = 3 * H * H;                // plane stride of W2^T
+  static_assert(RG * CT == kTfWaves && RTW * RG * 16 == TM, "wave split");
+  constexpr int NV = TM * (H / 4) / kTfBlock;
+  static_assert(NV * kTfBlock == TM * (H / 4), "chunk split");
+  __shared__ __align__(16) uint16_t a_bf[NS][3 * PA];
+  const int ntiles = (P + TM - 1) / TM;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int cw = 16 * (wave % CT), rg = wave / CT;
+  // a thread's share of the next chunk is in flight during the products
+  f4 st[NS][NV];
+  auto fetch = [&](int t, int ch) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int idx = threadIdx.x + v * kTfBlock;
+      const int m = idx / (H / 4), c = 4 * (idx % (H / 4));
+      const size_t o = (size_t)min(t * TM + m, P - 1) * 3 * H + ch * H + c;
+      st[0][v] = *reinterpret_cast<const f4*>(gw + o);
+      if (TAN) st[NS - 1][v] = *reinterpret_cast<const f4*>(dgw + o);
+    }
+  };
+  if ((int)blockIdx.x < ntiles) fetch(blockIdx.x, 0);
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int pbase = tile * TM;
+    f4 acc[RTW][1], dacc[RTW][1];
+    zero_acc(acc);
+    zero_acc(dacc);
+#pragma unroll 1
+    for (int ch = 0; ch < 3; ++ch) {
+      __syncthreads();   // the products before are done with the LDS
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int j = 0; j < NS; ++j) {
+          const int idx = threadIdx.x + v * kTfBlock;
+          uint16_t* o = a_bf[j] + (idx / (H / 4)) * LDA + 4 * (idx % (H / 4));
+          ushort4 h, md, l;
+          split3_bf16(st[j][v][0], h.x, md.x, l.x);
+          split3_bf16(st[j][v][1], h.y, md.y, l.y);
+          split3_bf16(st[j][v][2], h.z, md.z, l.z);
+          split3_bf16(st[j][v][3], h.w, md.w, l.w);
+          *reinterpret_cast<ushort4*>(o) = h;
+          *reinterpret_cast<ushort4*>(o + PA) = md;
+          *reinterpret_cast<ushort4*>(o + 2 * PA) = l;
+        }
+      __syncthreads();
+      const int nt = ch < 2 ? tile : tile + gridDim.x;
+      if (nt < ntiles) fetch(nt, ch < 2 ? ch + 1 : 0);
+      const uint16_t* B = w2t + (size_t)(cw + r) * 3 * H + ch * H + 8 * g;
+      const int ao = (rg * RTW * 16 + r) * LDA + 8 * g;
+#pragma unroll
+      for (int k0 = 0; k0 < H; k0 += 32) {
+        auto b8 = [&](const uint16_t* q) { return *reinterpret_cast<const bf8*>(q); };
+        const bf8 bh = b8(B + k0), bm = b8(B + PB + k0), bl = b8(B + 2 * PB + k0);
+        auto six = [&](const uint16_t* A, f4& c) {
+          const bf8 ah = b8(A), am = b8(A + PA), al = b8(A + 2 * PA);
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bm, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bh, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bm, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, c, 0, 0, 0);
+        };
+#pragma unroll
+        for (int rt = 0; rt < RTW; ++rt) {
+          six(a_bf[0] + ao + rt * 16 * LDA + k0, acc[rt][0]);
+          if (TAN) six(a_bf[NS - 1] + ao + rt * 16 * LDA + k0, dacc[rt][0]);
+        }
+      }
+    }
+#pragma unroll
+    for (int rt = 0; rt < RTW; ++rt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int p = pbase + (rg * RTW + rt) * 16 + 4 * g + i;
+        if (p >= P) continue;
+        const size_t o = (size_t)p * H + cw + r;
+        const float x = a[o];
+        // s = sigmoid(x); 1 - s as 1 / (1 + exp(x)) (exact for large x)
+        const float sg = 1.0f / (1.0f + expf(-x)), sm = 1.0f / (1.0f + expf(x));
+        const float d1 = sg * (1.0f + x * sm), gh = acc[rt][0][i];
+        ga[o] = gh * d1;
+        if (TAN) dga[o] = dacc[rt][0][i] * d1 + gh * (sg * sm * (2.0f + x * (sm - sg))) * da[o];
+      }
+  }
+}
+
+// What the pair kernels read of a filter MLP, remade for new weights in one
+// launch: W1 [H][R] padded with zeros to RP columns, the bf16 planes of W2 [3H][H]
+// and of its transpose, and the transpose.
+__global__ void filter_planes_kernel(int H, int R, int RP, const float* __restrict__ w1,
+                                     const float* __restrict__ w2, float* __restrict__ w1p,
+                                     uint16_t* __restrict__ planes,
+                                     uint16_t* __restrict__ planes_t, float* __restrict__ w2t) {
+  const int n = 3 * H * H;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    uint16_t h, m, l;
+    split3_bf16(w2[i], h, m, l);
+    planes[i] = h;
+    planes[n + i] = m;
+    planes[2 * n + i] = l;
+    const int t = (i % H) * 3 * H + i / H;
+    planes_t[t] = h;
+    planes_t[n + t] = m;
+    planes_t[2 * n + t] = l;
+    w2t[t] = w2[i];
+    if (i < H * RP) w1p[i] = i % RP < R ? w1[(i / RP) * R + i % RP] : 0.f;
+  }
+}
+
 __global__ void split_bf16x3_kernel(int64_t n, const float* __restrict__ src,
                                     uint16_t* __restrict__ dst) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -349,6 +474,17 @@ hipError_t launch_train_filter_adjoint(hipStream_t s, int P, const float* gw, co
   return hipGetLastError();
 }
 
+template <int H>
+hipError_t launch_adjoint_x6(hipStream_t st, int P, const float* gw, const float* dgw,
+                             const uint16_t* w2t, const float* a, const float* da, float* ga,
+                             float* dga) {
+  constexpr int TM = H >= 128 ? 32 : 64;
+  const int tiles = (P + TM - 1) / TM, grid = tiles < 8192 ? tiles : 8192;
+  if (dgw) train_filter_adjoint_x6_kernel<H, TM, true><<<grid, kTfBlock, 0, st>>>(P, gw, dgw, w2t, a, da, ga, dga);
+  else train_filter_adjoint_x6_kernel<H, TM, false><<<grid, kTfBlock, 0, st>>>(P, gw, dgw, w2t, a, da, ga, dga);
+  return hipGetLastError();
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
@@ -357,6 +493,58 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 using namespace mlff;
 
 extern "C" {
+
+int mlff_filter_planes(void* stream, int hidden_dim, int R, const float* w1_dev,
+                       const float* w2_dev, float* w1p_dev, uint16_t* planes_dev,
+                       uint16_t* planes_t_dev, float* w2t_dev) {
+  if (hidden_dim < 32 || hidden_dim > 4096 || R < 1 || R > kTfMaxRbf || !w1_dev || !w2_dev ||
+      !w1p_dev || !planes_dev || !planes_t_dev || !w2t_dev) {
+    set_error("mlff_filter_planes: need 32 <= hidden_dim <= 4096, 1 <= R <= %d and non-null "
+              "buffers", kTfMaxRbf);
+    return MLFF_ERR_INVALID;
+  }
+  const int n = 3 * hidden_dim * hidden_dim;
+  filter_planes_kernel<<<(n + 255) / 256, 256, 0, static_cast<hipStream_t>(stream)>>>(
+      hidden_dim, R, R <= 16 ? 16 : 32, w1_dev, w2_dev, w1p_dev, planes_dev, planes_t_dev,
+      w2t_dev);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error("mlff_filter_planes: %s", hipGetErrorString(e));
+    return MLFF_ERR_HIP;
+  }
+  return MLFF_OK;
+}
+
+int mlff_train_filter_adjoint_x6(void* stream, int hidden_dim, int n_pairs, const float* gw_dev,
+                                 const float* dgw_dev, const uint16_t* planes_t_dev,
+                                 const float* a_dev, const float* da_dev, float* ga_dev,
+                                 float* dga_dev) {
+  const char* nm = "mlff_train_filter_adjoint_x6";
+  if (n_pairs < 0) { set_error("%s: negative size", nm); return MLFF_ERR_INVALID; }
+  if (n_pairs == 0) return MLFF_OK;
+  if (!gw_dev || !planes_t_dev || !a_dev || !ga_dev || (dgw_dev && (!da_dev || !dga_dev))) {
+    set_error("%s: null pointer", nm);
+    return MLFF_ERR_INVALID;
+  }
+  if (!aligned16(gw_dev) || !aligned16(dgw_dev) || !aligned16(planes_t_dev)) {
+    set_error("%s: buffers must be 16-byte aligned", nm);
+    return MLFF_ERR_INVALID;
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  hipError_t e;
+  switch (hidden_dim) {
+    case 64: e = launch_adjoint_x6<64>(st, n_pairs, gw_dev, dgw_dev, planes_t_dev, a_dev, da_dev, ga_dev, dga_dev); break;
+    case 128: e = launch_adjoint_x6<128>(st, n_pairs, gw_dev, dgw_dev, planes_t_dev, a_dev, da_dev, ga_dev, dga_dev); break;
+    default:
+      set_error("%s: hidden_dim %d not supported (64, 128)", nm, hidden_dim);
+      return MLFF_ERR_UNSUPPORTED;
+  }
+  if (e != hipSuccess) {
+    set_error("%s: %s", nm, hipGetErrorString(e));
+    return MLFF_ERR_HIP;
+  }
+  return MLFF_OK;
+}
 
 int mlff_split_bf16x3(void* stream, int64_t n, const float* src_dev, uint16_t* planes_dev) {
   if (n < 0 || (n > 0 && (!src_dev || !planes_dev))) {

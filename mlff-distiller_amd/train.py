@@ -374,9 +374,10 @@ def _silu_dd(x, g, dx, dg=None):
 
 
 # prepared filter weights per (W1, W2) tensor pair: W1 padded to 16 or 32
-# columns, W2 as three bf16 planes and W2 transposed.  An entry belongs to the two tensor
-# objects themselves (weak references: a tensor allocated later at a freed
-# one's address, or under its id, never matches) and is remade when the
+# columns, W2 and its transpose as three bf16 planes each, and the transpose
+# itself.  An entry belongs to
+# the two tensor objects themselves (weak references: a tensor allocated later at
+# a freed one's address, or under its id, never matches) and is remade when the
 # optimizer has written either tensor (its version counter moved).
 _FILTER_W: Dict[tuple, tuple] = {}
 
@@ -388,28 +389,28 @@ def _filter_weights(p: Dict[str, Tensor], pre: str):
     ent = _FILTER_W.get(key)
     same = ent is not None and ent[0]() is W1o and ent[1]() is W2o
     if same and ent[2] == state:
-        return ent[3], ent[4], ent[5]
+        return ent[3:]
     W1, W2 = _dense(W1o), _dense(W2o)
     H, R = W1.shape
+    if W2.shape != (3 * H, H):
+        raise RuntimeError("filter layers do not match: W2 must be [3H, H]")
     RP = 16 if R <= 16 else 32
     if len(_FILTER_W) > 64:
         for k in [k for k, e in _FILTER_W.items() if e[0]() is None or e[1]() is None]:
             del _FILTER_W[k]
-    if (same and ent[3].shape == (H, RP) and ent[4].numel() == 3 * W2.numel()
-            and ent[5].shape == W2.T.shape):
+    if same and ent[3].shape == (H, RP):
         # the same tensors, written by the optimizer: refill the buffers in place
-        # (W1's padding columns stay zero)
-        w1p, planes, w2t = ent[3], ent[4], ent[5]
+        w1p, planes, planes_t, w2t = ent[3:]
     else:
-        w1p = torch.zeros(H, RP, dtype=torch.float32, device=W1.device)
+        w1p = torch.empty(H, RP, dtype=torch.float32, device=W1.device)
         planes = torch.empty(3 * W2.numel(), dtype=torch.int16, device=W2.device)
-        w2t = torch.empty(W2.shape[1], W2.shape[0], dtype=torch.float32, device=W2.device)
-    w1p[:, :R].copy_(W1)
-    w2t.copy_(W2.T)
-    C.check("mlff_split_bf16x3", C.lib().mlff_split_bf16x3(
-        C.stream_handle(), W2.numel(), C.ptr(W2), C.ptr(planes)))
-    _FILTER_W[key] = (weakref.ref(W1o), weakref.ref(W2o), state, w1p, planes, w2t)
-    return w1p, planes, w2t
+        planes_t = torch.empty_like(planes)
+        w2t = torch.empty(H, 3 * H, dtype=torch.float32, device=W2.device)
+    C.check("mlff_filter_planes", C.lib().mlff_filter_planes(
+        C.stream_handle(), H, R, C.ptr(W1), C.ptr(W2), C.ptr(w1p), C.ptr(planes),
+        C.ptr(planes_t), C.ptr(w2t)))
+    _FILTER_W[key] = (weakref.ref(W1o), weakref.ref(W2o), state, w1p, planes, planes_t, w2t)
+    return w1p, planes, planes_t, w2t
 
 
 def _filter(p: Dict[str, Tensor], pre: str, x: Tensor, a: Optional[Tensor] = None):
@@ -417,7 +418,7 @@ def _filter(p: Dict[str, Tensor], pre: str, x: Tensor, a: Optional[Tensor] = Non
     (a None): x = e gives (a1, h, W) with a1 = e W1^T + b1, h = silu(a1),
     W = h W2^T + b2.  Tangent: x = de and a = a1 give (da1, dh, dW) with
     da1 = de W1^T, dh = silu'(a1) da1, dW = dh W2^T."""
-    w1p, planes, _ = _filter_weights(p, pre)
+    w1p, planes, _, _ = _filter_weights(p, pre)
     x = _dense(x)
     P, R = x.shape
     H = p[pre + ".0.weight"].shape[0]
@@ -442,7 +443,7 @@ def _filter_adjoint(p: Dict[str, Tensor], pre: str, gW: Tensor, a1: Tensor,
     (mlff_train_filter_adjoint): ga1 = silu'(a1) (gW W2) and, with the
     tangent (dgW, da1), dga1 = silu'(a1) (dgW W2) + silu''(a1) da1 (gW W2).
     Returns (ga1, dga1 or None)."""
-    _, _, w2t = _filter_weights(p, pre)
+    _, _, planes_t, w2t = _filter_weights(p, pre)
     gW, a1 = _dense(gW), _dense(a1)
     P, H = a1.shape
     if w2t.shape != (H, 3 * H) or gW.shape != (P, 3 * H):
@@ -450,6 +451,12 @@ def _filter_adjoint(p: Dict[str, Tensor], pre: str, gW: Tensor, a1: Tensor,
     tan = dgW is not None
     ga = torch.empty(P, H, dtype=torch.float32, device=a1.device)
     dga = torch.empty_like(ga) if tan else None
+    if H > 32:
+        C.check("mlff_train_filter_adjoint_x6", C.lib().mlff_train_filter_adjoint_x6(
+            C.stream_handle(), H, P, C.ptr(gW), C.ptr(_dense(dgW) if tan else None),
+            C.ptr(planes_t), C.ptr(a1), C.ptr(_dense(da1) if tan else None), C.ptr(ga),
+            C.ptr(dga)))
+        return ga, dga
     C.check("mlff_train_filter_adjoint", C.lib().mlff_train_filter_adjoint(
         C.stream_handle(), int(tan), H, P, C.ptr(gW), C.ptr(_dense(dgW) if tan else None),
         C.ptr(w2t), C.ptr(a1), C.ptr(_dense(da1) if tan else None), C.ptr(ga), C.ptr(dga)))
@@ -922,11 +929,8 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
                    lambda: _xyz_outer(dgvg2, v_m, gvg2, dvm, group=grp))
         # message reverse (student_model.py:346-387): filter-output gradients per pair
         s, v, W = lay["s"], lay["v"], lay["W"]
-        if T:
-            gW, dgW = _pair_grad(g, H, u, s, v, gs_m, gv_m, c["du"], lay["ds"], lay["dv"],
-                                 dgs_m, dgv_m)
-        else:
-            gW, dgW = _pair_grad(g, H, u, s, v, gs_m, gv_m)
+        moved = (c["du"], lay["ds"], lay["dv"], dgs_m, dgv_m) if T else ()
+        gW, dgW = _pair_grad(g, H, u, s, v, gs_m, gv_m, *moved)
         W1 = p[mpre + ".0.weight"]
         linear(mpre + ".2", gW, lay["h"], dgW, lay["dh"] if T else None, w_pair,
                short=False)
