@@ -137,7 +137,8 @@ namespace {
 enum Seg {
   S_COUNTS, S_DEG, S_UDEG, S_MASK, S_ROWPTR, S_PAIRPTR, S_COL, S_EPAIR, S_PLO, S_PHI, S_PSHIFT, S_GEOM,
   S_UNIT,  S_PACC, S_WF, S_S, S_V, S_SMID, S_VMID, S_AUPD, S_G12, S_GS0, S_GV0, S_GS1, S_GV1,
-  S_GA, S_EPS, S_VIR, S_GRID, S_CELLCNT, S_CELLSTART, S_CELLATOMS, S_ATOMCELL, S_TMPSHIFT, S_WBF,
+  S_GA, S_EPS, S_VIR, S_GRID, S_CELLCNT, S_CELLSTART, S_CELLATOMS, S_ATOMCELL, S_TMPSHIFT,
+  S_HITS, S_WBF,
   S_TABBAD, S_TAB,   // the tables last: the static entry keeps them elsewhere
   S_COUNT_
 };
@@ -151,7 +152,7 @@ void carve(mlff_plan* pl) {
   sz[S_COUNTS] = 4 * MLFF_COUNT_SLOTS;
   sz[S_DEG] = 4 * N;
   sz[S_UDEG] = 4 * N;
-  sz[S_MASK] = N <= kSmallAtoms ? 8 * N * (kSmallAtoms / 64) : 0;
+  sz[S_MASK] = N <= kSmallAtoms ? 8 * N * ((N + 63) / 64) : 0;
   sz[S_ROWPTR] = 4 * (N + 1);
   sz[S_PAIRPTR] = 4 * (N + 1);
   sz[S_COL] = 4 * E;
@@ -186,6 +187,7 @@ void carve(mlff_plan* pl) {
   sz[S_CELLATOMS] = CC ? 4 * N : 0;
   sz[S_ATOMCELL] = CC ? 4 * N : 0;
   sz[S_TMPSHIFT] = CC ? 12 * E : 0;
+  sz[S_HITS] = CC ? 4 * N * kCellRowMax : 0;
   sz[S_WBF] = 2 * wbf_elems((int)H, (int)L);
   pl->buf.ts = table_shape((int)H, c.num_rbf, (int)L, c.cutoff);
   sz[S_TABBAD] = pl->buf.ts.bytes ? 4 : 0;
@@ -529,6 +531,7 @@ int bind_buffers(mlff_plan* pl, const char* who, void* ws, const float* weights_
   a.cell_atoms = segp<int32_t>(pl, ws, S_CELLATOMS);
   a.atom_cell = segp<int32_t>(pl, ws, S_ATOMCELL);
   a.edge_tmp_shift = segp<int32_t>(pl, ws, S_TMPSHIFT);
+  a.hits = segp<int32_t>(pl, ws, S_HITS);
   pl->grid_dev = segp<int4>(pl, ws, S_GRID);
   return MLFF_OK;
 }

@@ -32,7 +32,8 @@ int build_layout(int H, int L, int R, int max_z, ModelW* mw, mlff_slot* slots, i
                  int* n_slots);
 
 // Neighbour-list launches (nl.hip).
-constexpr int kSmallAtoms = 1024;   // largest list that is counted and filled in two launches
+constexpr int kSmallAtoms = 4096;   // largest list that is counted and filled in two launches
+constexpr int kCellRowMax = 256;    // cell-list rows up to here are kept from the count pass
 struct NLArgs {
   const float* pos; int N; int B;
   const int32_t* mol_ptr; const int32_t* atom_mol;
@@ -44,7 +45,8 @@ struct NLArgs {
   // cell list (periodic structures): grid[b] = {nc0, nc1, nc2, base}, nc0 == 0 -> brute force
   const int4* grid; int32_t n_cells;
   int32_t* cell_count; int32_t* cell_start; int32_t* cell_atoms; int32_t* atom_cell;
-  uint64_t* mask;            // [N][kSmallAtoms / 64] hit masks; null: none
+  uint64_t* mask;            // [N][ceil(N / 64)] hit masks; null: none
+  int32_t* hits;             // [N][kCellRowMax] neighbours of the cell-list rows, unsorted
   int32_t* edge_tmp_shift;   // [ecap*3] image shifts of cell-list rows before sorting
 };
 hipError_t launch_neighbor_list(const NLArgs& a, hipStream_t s, bool build_pairs);

@@ -23,6 +23,8 @@
 // cells need nothing more when rc is below half the box); for skewed cells
 // the 27 neighbouring images of that vector are searched for the shortest.
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -203,28 +205,24 @@ __device__ __forceinline__ int cell_candidate(const CellList& cl, const CellWalk
   return f < w.total ? cl.cell_atoms[slot] : -1;
 }
 
-// cell-list rows of up to this many neighbours are sorted in LDS by a wave;
+// cell-list rows of up to kCellRowMax neighbours are sorted in LDS by a wave;
 // longer rows take the one-lane path
-constexpr int kCellRowMax = 256;
 constexpr int kNlBlock = 256;
-constexpr int kMaskWords = kSmallAtoms / 64;   // hit mask of a row, from its structure's first atom
 
 __global__ void cl_zero_kernel(int n, int32_t* __restrict__ a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) a[i] = 0;
 }
 
-// cell of every cell-list atom from its wrapped fractional coordinates
-__global__ void cl_bin_kernel(const float* __restrict__ pos, int N,
-                              const int32_t* __restrict__ atom_mol,
-                              const float* __restrict__ cells, const uint8_t* __restrict__ pbc,
-                              const int4* __restrict__ grid, int32_t* __restrict__ atom_cell,
-                              int32_t* __restrict__ cell_count) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
+// cell of atom i from its wrapped fractional coordinates, -1 without a grid
+__device__ __forceinline__ int cell_of(const float* __restrict__ pos, int i,
+                                       const int32_t* __restrict__ atom_mol,
+                                       const float* __restrict__ cells,
+                                       const uint8_t* __restrict__ pbc,
+                                       const int4* __restrict__ grid) {
   const int b = atom_mol[i];
   const int4 g = grid[b];
-  if (g.x == 0) { atom_cell[i] = -1; return; }
+  if (g.x == 0) return -1;
   CellInfo ci;
   bool periodic;
   load_cell(cells, pbc, b, ci, periodic);
@@ -241,9 +239,85 @@ __global__ void cl_bin_kernel(const float* __restrict__ pos, int N,
     int k = (int)(w * (float)nc[a]);
     c[a] = k < 0 ? 0 : (k >= nc[a] ? nc[a] - 1 : k);
   }
-  const int cell = g.w + (c[0] * g.y + c[1]) * g.z + c[2];
+  return g.w + (c[0] * g.y + c[1]) * g.z + c[2];
+}
+
+__global__ void cl_bin_kernel(const float* __restrict__ pos, int N,
+                              const int32_t* __restrict__ atom_mol,
+                              const float* __restrict__ cells, const uint8_t* __restrict__ pbc,
+                              const int4* __restrict__ grid, int32_t* __restrict__ atom_cell,
+                              int32_t* __restrict__ cell_count) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= N) return;
+  const int cell = cell_of(pos, i, atom_mol, cells, pbc, grid);
   atom_cell[i] = cell;
-  atomicAdd(&cell_count[cell], 1);
+  if (cell >= 0) atomicAdd(&cell_count[cell], 1);
+}
+
+// The whole cell list of at most kSmallAtoms atoms and cells in one workgroup:
+// bin, scan, place and sort in LDS.  For 3000 atoms 14 us, as five launches 19
+// us and the gaps between them.
+__global__ __launch_bounds__(1024) void cl_build_kernel(
+    const float* __restrict__ pos, int N, int C, const int32_t* __restrict__ atom_mol,
+    const float* __restrict__ cells, const uint8_t* __restrict__ pbc,
+    const int4* __restrict__ grid, int32_t* __restrict__ atom_cell,
+    int32_t* __restrict__ cell_start, int32_t* __restrict__ cell_atoms) {
+  constexpr int kPer = kSmallAtoms / 1024;
+  __shared__ int cursor[kSmallAtoms], atoms[kSmallAtoms], wsum[16];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+#pragma unroll
+  for (int a = 0; a < kPer; ++a) cursor[t + 1024 * a] = 0;
+  __syncthreads();
+  int cell[kPer];
+#pragma unroll
+  for (int a = 0; a < kPer; ++a) {
+    const int i = t + 1024 * a;
+    cell[a] = -1;
+    if (i < N) {
+      cell[a] = cell_of(pos, i, atom_mol, cells, pbc, grid);
+      atom_cell[i] = cell[a];
+      if (cell[a] >= 0) atomicAdd(&cursor[cell[a]], 1);
+    }
+  }
+  __syncthreads();
+  int n[kPer], sum = 0;
+#pragma unroll
+  for (int a = 0; a < kPer; ++a) {
+    n[a] = cursor[kPer * t + a];
+    sum += n[a];
+  }
+  const int incl = wave_inclusive_scan(sum);
+  if (lane == 63) wsum[wv] = incl;
+  __syncthreads();
+  int start = incl - sum, total = 0;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    if (q < wv) start += wsum[q];
+    total += wsum[q];
+  }
+#pragma unroll
+  for (int a = 0; a < kPer; ++a) {
+    const int c = kPer * t + a;
+    cursor[c] = start;
+    if (c < C) cell_start[c] = start;
+    start += n[a];
+  }
+  if (t == 0) cell_start[C] = total;
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < kPer; ++a)
+    if (cell[a] >= 0) atoms[atomicAdd(&cursor[cell[a]], 1)] = t + 1024 * a;
+  __syncthreads();
+  // ascending atoms in every cell: an atom's place is the number of smaller ones
+  // (cursor[c] now ends cell c)
+#pragma unroll
+  for (int a = 0; a < kPer; ++a) {
+    if (cell[a] < 0) continue;
+    const int i = t + 1024 * a, lo = cell[a] > 0 ? cursor[cell[a] - 1] : 0, hi = cursor[cell[a]];
+    int rank = 0;
+    for (int k = lo; k < hi; ++k) rank += atoms[k] < i ? 1 : 0;
+    cell_atoms[lo + rank] = i;
+  }
 }
 
 // exclusive scan of the cell counts (one workgroup), then reset the counts
@@ -316,7 +390,8 @@ __global__ void nl_count_kernel(const float* __restrict__ pos, int N,
                                 const int32_t* __restrict__ atom_mol,
                                 const float* __restrict__ cells, const uint8_t* __restrict__ pbc,
                                 float rc, int32_t* __restrict__ deg, int32_t* __restrict__ udeg,
-                                uint64_t* __restrict__ mask, CellList cl) {
+                                uint64_t* __restrict__ mask, int mask_words, CellList cl,
+                                int32_t* __restrict__ hits) {
   // one wave per atom: the lanes test 64 candidates at a time, the atoms of
   // the structure (brute force) or of the 27 cells around the atom's cell
   const int i = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
@@ -327,6 +402,7 @@ __global__ void nl_count_kernel(const float* __restrict__ pos, int N,
   bool periodic;
   load_cell(cells, pbc, b, ci, periodic);
   const float xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   int n = 0, nu = 0;
   auto hit = [&](int j) {
     float vx, vy, vz, d;
@@ -339,7 +415,11 @@ __global__ void nl_count_kernel(const float* __restrict__ pos, int N,
     for (int fb = 0; fb < w.total; fb += 64) {
       const int j = cell_candidate(cl, w, fb + lane);
       const bool h = (j >= 0) && (j != i) && hit(j);
-      n += __popcll(__ballot(h));
+      const uint64_t mh = __ballot(h);
+      // the fill pass starts from the row's hits
+      const int slot = n + __popcll(mh & below);
+      if (h && slot < kCellRowMax) hits[(size_t)i * kCellRowMax + slot] = j;
+      n += __popcll(mh);
       nu += __popcll(__ballot(h && j > i));
     }
   } else {
@@ -350,7 +430,7 @@ __global__ void nl_count_kernel(const float* __restrict__ pos, int N,
       const uint64_t mh = __ballot(h);
       n += __popcll(mh);
       nu += __popcll(__ballot(h && j > i));
-      if (mask != nullptr && lane == 0) mask[(size_t)i * kMaskWords + (jb - j0) / 64] = mh;
+      if (mask != nullptr && lane == 0) mask[(size_t)i * mask_words + (jb - j0) / 64] = mh;
     }
   }
   if (lane == 0) {
@@ -478,6 +558,55 @@ __global__ __launch_bounds__(kScanThreads) void nl_scan_offset_kernel(
   if (g == G - 1 && t == 0) store_totals(N, all1, all2, row_ptr, pair_ptr, counts, ecap, pcap);
 }
 
+// Exclusive scans of deg and udeg over all N <= kSmallAtoms atoms into LDS
+// (entry N: the totals), by every workgroup for itself; its rows' entries go to
+// memory, and the totals from the first workgroup.
+struct SmallScan {
+  int b1[kSmallAtoms + 1], b2[kSmallAtoms + 1];
+  int w1[kNlBlock / 64], w2[kNlBlock / 64];
+};
+__device__ __forceinline__ void small_scan(SmallScan& sc, int N, const int32_t* __restrict__ deg,
+                                           const int32_t* __restrict__ udeg,
+                                           int32_t* __restrict__ row_ptr,
+                                           int32_t* __restrict__ pair_ptr,
+                                           int32_t* __restrict__ counts, int32_t ecap,
+                                           int32_t pcap) {
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int per = (N + kNlBlock - 1) / kNlBlock, q0 = min(N, per * t), q1 = min(N, q0 + per);
+  int s1 = 0, s2 = 0;
+  for (int q = q0; q < q1; ++q) {
+    s1 += deg[q];
+    s2 += udeg[q];
+  }
+  const int i1 = wave_inclusive_scan(s1), i2 = wave_inclusive_scan(s2);
+  if (lane == 63) { sc.w1[wv] = i1; sc.w2[wv] = i2; }
+  __syncthreads();
+  int o1 = i1 - s1, o2 = i2 - s2, all1 = 0, all2 = 0;
+#pragma unroll
+  for (int q = 0; q < kNlBlock / 64; ++q) {
+    if (q < wv) { o1 += sc.w1[q]; o2 += sc.w2[q]; }
+    all1 += sc.w1[q];
+    all2 += sc.w2[q];
+  }
+  for (int q = q0; q < q1; ++q) {
+    sc.b1[q] = o1;
+    sc.b2[q] = o2;
+    o1 += deg[q];
+    o2 += udeg[q];
+  }
+  if (t == 0) {
+    sc.b1[N] = all1;
+    sc.b2[N] = all2;
+    if (blockIdx.x == 0) store_totals(N, all1, all2, row_ptr, pair_ptr, counts, ecap, pcap);
+  }
+  __syncthreads();
+  const int i = blockIdx.x * (kNlBlock / 64) + wv;
+  if (i < N && lane == 0) {
+    row_ptr[i] = sc.b1[i];
+    pair_ptr[i] = sc.b2[i];
+  }
+}
+
 // Row i of the list by a test against every atom of its structure: 64
 // candidates per step; a hit's slot is the number of hits in lower lanes, so the
 // row stays in ascending neighbour order.  lower(j) is the pair of an edge to
@@ -531,20 +660,28 @@ __device__ __forceinline__ void fill_row(
   }
 }
 
+// SCAN (at most kSmallAtoms atoms): row_ptr and pair_ptr are made here as well.
+template <bool SCAN>
 __global__ void nl_fill_kernel(const float* __restrict__ pos, int N,
                                const int32_t* __restrict__ mol_ptr,
                                const int32_t* __restrict__ atom_mol,
                                const float* __restrict__ cells, const uint8_t* __restrict__ pbc,
-                               float rc, const int32_t* __restrict__ row_ptr,
-                               const int32_t* __restrict__ pair_ptr, int32_t* __restrict__ col,
+                               float rc, const int32_t* __restrict__ deg_in,
+                               const int32_t* __restrict__ udeg_in,
+                               int32_t* __restrict__ row_ptr, int32_t* __restrict__ pair_ptr,
+                               int32_t* __restrict__ counts, int32_t* __restrict__ col,
                                int32_t* __restrict__ edge_shift, int32_t* __restrict__ edge_pair,
                                int32_t ecap, int32_t* __restrict__ pair_lo,
                                int32_t* __restrict__ pair_hi, int32_t* __restrict__ pair_shift,
                                float4* __restrict__ geom, float4* __restrict__ unit,
-                               int32_t pcap, CellList cl,
-                               int32_t* __restrict__ tmp_shift) {
+                               int32_t pcap, int32_t pairs_max, CellList cl,
+                               int32_t* __restrict__ tmp_shift,
+                               const int32_t* __restrict__ hits) {
   // one wave per atom, as the count pass
   __shared__ int4 hits_lds[(kNlBlock / 64) * kCellRowMax];
+  __shared__ std::conditional_t<SCAN, SmallScan, int> sc;
+  if constexpr (SCAN)
+    small_scan(sc, N, deg_in, udeg_in, row_ptr, pair_ptr, counts, ecap, pairs_max);
   const int i = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int lane = threadIdx.x & 63;
   if (i >= N) return;
@@ -554,35 +691,37 @@ __global__ void nl_fill_kernel(const float* __restrict__ pos, int N,
   bool periodic;
   load_cell(cells, pbc, b, ci, periodic);
   const float xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-  int e = row_ptr[i];
-  int p = pair_ptr[i];
-  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int deg = row_ptr[i + 1] - e;
+  int e, p, deg, udeg;
+  if constexpr (SCAN) {
+    e = sc.b1[i];
+    p = sc.b2[i];
+    deg = sc.b1[i + 1] - e;
+    udeg = sc.b2[i + 1] - p;
+  } else {
+    e = row_ptr[i];
+    p = pair_ptr[i];
+    deg = row_ptr[i + 1] - e;
+    udeg = pair_ptr[i + 1] - p;
+  }
   if (cl.grid != nullptr && cl.atom_cell[i] >= 0 && deg <= kCellRowMax) {
-    // cell-list row: the wave collects the hits {j, shift} in candidate order
-    // into LDS, then every hit's place in the row is the number of hits with
-    // a smaller neighbour index (the neighbours of a row are distinct)
+    // cell-list row: the count pass's hits with their shifts into LDS, then
+    // every hit's place in the row is the number of hits with a smaller
+    // neighbour index (the neighbours of a row are distinct)
     int4* hl = hits_lds + (threadIdx.x >> 6) * kCellRowMax;
-    const CellWalk w = cell_walk(cl, i, b);
-    int k = 0;
-    for (int fb = 0; fb < w.total; fb += 64) {
-      const int j = cell_candidate(cl, w, fb + lane);
+    const int k = deg;
+    for (int q = lane; q < k; q += 64) {
+      const int j = hits[(size_t)i * kCellRowMax + q];
       float vx, vy, vz, d;
       int s0 = 0, s1 = 0, s2 = 0;
-      const bool h = (j >= 0) && (j != i) &&
-                     within(pos[3 * j] - xi, pos[3 * j + 1] - yi, pos[3 * j + 2] - zi, rc,
-                            periodic, ci, vx, vy, vz, d, s0, s1, s2);
-      const uint64_t mh = __ballot(h);
-      const int slot = k + __popcll(mh & below);
-      if (h && slot < kCellRowMax) hl[slot] = make_int4(j, s0, s1, s2);
-      k += __popcll(mh);
+      within(pos[3 * j] - xi, pos[3 * j + 1] - yi, pos[3 * j + 2] - zi, rc, periodic, ci, vx, vy,
+             vz, d, s0, s1, s2);
+      hl[q] = make_int4(j, s0, s1, s2);
     }
-    k = min(k, kCellRowMax);
     // the LDS writes above are visible to every lane of the wave below
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int n_lower = deg - (pair_ptr[i + 1] - p);   // neighbours j < i
+    const int n_lower = deg - udeg;   // neighbours j < i
     for (int q = lane; q < k; q += 64) {
       const int4 hq = hl[q];
       int rank = 0;
@@ -689,62 +828,28 @@ __global__ __launch_bounds__(kNlBlock) void nl_fill_small_kernel(
     const float* __restrict__ pos, int N, const int32_t* __restrict__ mol_ptr,
     const int32_t* __restrict__ atom_mol, const float* __restrict__ cells,
     const uint8_t* __restrict__ pbc, float rc, const int32_t* __restrict__ deg,
-    const int32_t* __restrict__ udeg, const uint64_t* __restrict__ mask,
+    const int32_t* __restrict__ udeg, const uint64_t* __restrict__ mask, int mask_words,
     int32_t* __restrict__ row_ptr, int32_t* __restrict__ pair_ptr, int32_t* __restrict__ counts,
     int32_t* __restrict__ col, int32_t* __restrict__ edge_shift, int32_t* __restrict__ edge_pair,
     int32_t ecap, int32_t* __restrict__ pair_lo, int32_t* __restrict__ pair_hi,
     int32_t* __restrict__ pair_shift, float4* __restrict__ geom, float4* __restrict__ unit,
     int32_t pcap) {
-  static_assert(kSmallAtoms == 4 * kNlBlock, "four atoms per thread");
-  __shared__ __align__(16) int b1[kSmallAtoms];
-  __shared__ __align__(16) int b2[kSmallAtoms];
-  __shared__ int w1[kNlBlock / 64], w2[kNlBlock / 64];
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  int a1[4], a2[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int q = 4 * t + k;
-    a1[k] = q < N ? deg[q] : 0;
-    a2[k] = q < N ? udeg[q] : 0;
-  }
-  const int s1 = a1[0] + a1[1] + a1[2] + a1[3], s2 = a2[0] + a2[1] + a2[2] + a2[3];
-  const int i1 = wave_inclusive_scan(s1), i2 = wave_inclusive_scan(s2);
-  if (lane == 63) { w1[wv] = i1; w2[wv] = i2; }
-  __syncthreads();
-  int o1 = i1 - s1, o2 = i2 - s2, all1 = 0, all2 = 0;
-#pragma unroll
-  for (int q = 0; q < kNlBlock / 64; ++q) {
-    if (q < wv) { o1 += w1[q]; o2 += w2[q]; }
-    all1 += w1[q];
-    all2 += w2[q];
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    b1[4 * t + k] = o1;
-    b2[4 * t + k] = o2;
-    o1 += a1[k];
-    o2 += a2[k];
-  }
-  __syncthreads();
-  if (blockIdx.x == 0 && t == 0) store_totals(N, all1, all2, row_ptr, pair_ptr, counts, ecap, pcap);
-  const int i = blockIdx.x * (kNlBlock / 64) + wv;
+  __shared__ SmallScan sc;
+  small_scan(sc, N, deg, udeg, row_ptr, pair_ptr, counts, ecap, pcap);
+  const int i = blockIdx.x * (kNlBlock / 64) + (threadIdx.x >> 6);
   if (i >= N) return;
-  if (lane == 0) {
-    row_ptr[i] = b1[i];
-    pair_ptr[i] = b2[i];
-  }
   const int b = atom_mol[i];
   const int j0 = mol_ptr[b], j1 = mol_ptr[b + 1];
   CellInfo ci;
   bool periodic;
   load_cell(cells, pbc, b, ci, periodic);
-  fill_row(pos, i, j0, j1, ci, periodic, rc, b1[i], b2[i], col, edge_shift, edge_pair, ecap,
+  fill_row(pos, i, j0, j1, ci, periodic, rc, sc.b1[i], sc.b2[i], col, edge_shift, edge_pair, ecap,
            pair_lo, pair_hi, pair_shift, geom, unit, pcap, [&](int j) {
              if (mask == nullptr) return -1;
              // bits (j, i) of row j's mask, and bit i itself
-             const uint64_t* m = mask + (size_t)j * kMaskWords;
+             const uint64_t* m = mask + (size_t)j * mask_words;
              const int wi = (i - j0) / 64, bi = (i - j0) % 64, bj = (j - j0) % 64;
-             int pk = b2[j];
+             int pk = sc.b2[j];
              for (int w = (j - j0) / 64; w <= wi; ++w) {
                uint64_t v = m[w];
                if (w == (j - j0) / 64) v &= ~0ull << bj;   // row j has no bit j
@@ -802,12 +907,13 @@ hipError_t launch_neighbor_list(const NLArgs& a, hipStream_t s, bool build_pairs
   // count and fill: one wave per atom
   const int gw = (int)(((int64_t)a.N * 64 + kNlBlock - 1) / kNlBlock);
   const int32_t pcap = build_pairs ? a.pcap : 0x7fffffff;
+  const int mask_words = (a.N + 63) / 64;
   if (a.N <= kSmallAtoms && !(a.grid != nullptr && a.n_cells > 0)) {
     nl_count_kernel<<<gw, kNlBlock, 0, s>>>(a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc,
-                                            a.rc, a.deg, a.udeg, a.mask, cl);
+                                            a.rc, a.deg, a.udeg, a.mask, mask_words, cl, nullptr);
     nl_fill_small_kernel<<<gw, kNlBlock, 0, s>>>(
-        a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc, a.rc, a.deg, a.udeg, a.mask, a.row_ptr,
-        a.pair_ptr, a.counts, a.col, a.edge_shift, build_pairs ? a.edge_pair : nullptr, a.ecap,
+        a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc, a.rc, a.deg, a.udeg, a.mask, mask_words,
+        a.row_ptr, a.pair_ptr, a.counts, a.col, a.edge_shift, build_pairs ? a.edge_pair : nullptr, a.ecap,
         build_pairs ? a.pair_lo : nullptr, a.pair_hi, a.pair_shift, a.geom, a.unit, pcap);
     if (build_pairs && a.mask == nullptr)
       nl_link_kernel<<<gw, kNlBlock, 0, s>>>(a.N, a.row_ptr, a.pair_ptr, a.col, a.edge_pair,
@@ -816,26 +922,39 @@ hipError_t launch_neighbor_list(const NLArgs& a, hipStream_t s, bool build_pairs
   }
   if (a.grid != nullptr && a.n_cells > 0) {
     const int C = a.n_cells;
-    cl_zero_kernel<<<(C + 255) / 256, 256, 0, s>>>(C, a.cell_count);
-    cl_bin_kernel<<<g, tb, 0, s>>>(a.pos, a.N, a.atom_mol, a.cells, a.pbc, a.grid, a.atom_cell,
-                                   a.cell_count);
-    cl_scan_kernel<<<1, 1024, 0, s>>>(a.cell_count, C, a.cell_start);
-    cl_place_kernel<<<g, tb, 0, s>>>(a.N, a.atom_cell, a.cell_start, a.cell_count, a.cell_atoms);
-    cl_sort_cells_kernel<<<(unsigned)(((int64_t)C * 64 + 255) / 256), 256, 0, s>>>(
-        C, a.cell_start, a.cell_atoms);
+    if (a.N <= kSmallAtoms && C <= kSmallAtoms) {
+      cl_build_kernel<<<1, 1024, 0, s>>>(a.pos, a.N, C, a.atom_mol, a.cells, a.pbc, a.grid,
+                                         a.atom_cell, a.cell_start, a.cell_atoms);
+    } else {
+      cl_zero_kernel<<<(C + 255) / 256, 256, 0, s>>>(C, a.cell_count);
+      cl_bin_kernel<<<g, tb, 0, s>>>(a.pos, a.N, a.atom_mol, a.cells, a.pbc, a.grid, a.atom_cell,
+                                     a.cell_count);
+      cl_scan_kernel<<<1, 1024, 0, s>>>(a.cell_count, C, a.cell_start);
+      cl_place_kernel<<<g, tb, 0, s>>>(a.N, a.atom_cell, a.cell_start, a.cell_count, a.cell_atoms);
+      cl_sort_cells_kernel<<<(unsigned)(((int64_t)C * 64 + 255) / 256), 256, 0, s>>>(
+          C, a.cell_start, a.cell_atoms);
+    }
     cl = CellList{a.grid, a.cell_start, a.cell_atoms, a.atom_cell};
   }
   nl_count_kernel<<<gw, kNlBlock, 0, s>>>(a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc, a.rc,
-                                   a.deg, a.udeg, nullptr, cl);
-  const int slices = (a.N + kScanSlice - 1) / kScanSlice;
-  nl_scan_slice_kernel<<<slices, kScanThreads, 0, s>>>(a.deg, a.udeg, a.N, a.row_ptr, a.pair_ptr);
-  nl_scan_offset_kernel<<<slices, kScanThreads, 0, s>>>(a.deg, a.udeg, a.N, a.row_ptr, a.pair_ptr,
-                                                        a.counts, a.ecap, pcap);
-  nl_fill_kernel<<<gw, kNlBlock, 0, s>>>(a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc, a.rc,
-                                  a.row_ptr, a.pair_ptr, a.col, a.edge_shift,
-                                  build_pairs ? a.edge_pair : nullptr, a.ecap,
-                                  build_pairs ? a.pair_lo : nullptr, a.pair_hi, a.pair_shift,
-                                  a.geom, a.unit, a.pcap, cl, a.edge_tmp_shift);
+                                          a.deg, a.udeg, nullptr, 0, cl, a.hits);
+  const bool scan = a.N > kSmallAtoms;
+  if (scan) {
+    const int slices = (a.N + kScanSlice - 1) / kScanSlice;
+    nl_scan_slice_kernel<<<slices, kScanThreads, 0, s>>>(a.deg, a.udeg, a.N, a.row_ptr,
+                                                         a.pair_ptr);
+    nl_scan_offset_kernel<<<slices, kScanThreads, 0, s>>>(a.deg, a.udeg, a.N, a.row_ptr,
+                                                          a.pair_ptr, a.counts, a.ecap, pcap);
+  }
+  auto fill = [&](auto kernel) {
+    kernel<<<gw, kNlBlock, 0, s>>>(a.pos, a.N, a.mol_ptr, a.atom_mol, a.cells, a.pbc, a.rc, a.deg,
+                                   a.udeg, a.row_ptr, a.pair_ptr, a.counts, a.col, a.edge_shift,
+                                   build_pairs ? a.edge_pair : nullptr, a.ecap,
+                                   build_pairs ? a.pair_lo : nullptr, a.pair_hi, a.pair_shift,
+                                   a.geom, a.unit, a.pcap, pcap, cl, a.edge_tmp_shift, a.hits);
+  };
+  if (scan) fill(nl_fill_kernel<false>);
+  else fill(nl_fill_kernel<true>);
   if (build_pairs) {
     nl_link_kernel<<<gw, kNlBlock, 0, s>>>(a.N, a.row_ptr, a.pair_ptr, a.col, a.edge_pair,
                                             a.ecap, a.pcap);

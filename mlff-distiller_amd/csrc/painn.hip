@@ -1257,6 +1257,7 @@ __device__ __forceinline__ void structure_sums(int i0, int i1, const float* __re
                                                double (&acc)[K]) {
   __shared__ double sh[kBlock / 64][K];
   for (int k = 0; k < K; ++k) acc[k] = 0.0;
+#pragma unroll 4
   for (int i = i0 + threadIdx.x; i < i1; i += kBlock) {
     acc[0] += (double)eps[i];
 #pragma unroll
