@@ -752,105 +752,105 @@ __global__ __launch_bounds__(kUpdBlock) void update_bwd_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// The update block and its adjoint in two kernels each, for few atoms: a block
-// takes 16 atoms and 32 output columns (two waves of one column tile), so the
-// weights (0.3 MB at H = 128, L2-cold in every kernel) come in through many
-// CUs instead of one per atom tile: what one CU can have in flight from memory
-// bounds a whole-tile block at 17 us, however few atoms there are.  All of a
-// wave's weights are requested first.  Same sums as the whole-tile kernels,
-// bit for bit.  Grid (16-atom tiles, H / 32).
+// Update kernels for few atoms.  What one compute unit can have in flight from
+// memory bounds a workgroup that takes a whole tile through the block at 17 us
+// (it reads every weight, 0.3 MB at H = 128), however few atoms there are.  So a
+// workgroup takes a 16-atom tile and 32 of the output channels.  Forward, its
+// waves share the whole hidden layer between them (computed H / 32 times over,
+// 0.9 us of products) and then the slice's columns of the second product: 10.1 us
+// for 60 atoms, against 6.3 + 6.1 us as two launches.  The adjoint's first product
+// has three times the weights, and there two launches are faster (7.3 + 4.4 us
+// against 13.6).  All of a wave's weights are requested first.  Same sums as the
+// whole-tile kernels, bit for bit.  Grid (16-atom tiles, H / 32).
 // ---------------------------------------------------------------------------
-constexpr int kSplitBlock = 128;
-
-// a = [s, |v|] W1^T + b1
 template <int H>
-__global__ __launch_bounds__(kSplitBlock, 2) void update_hidden_kernel(
+__global__ __launch_bounds__(4 * H) void update_fwd_split_kernel(
     int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ s_mid,
-    const float* __restrict__ v_mid, float* __restrict__ a_upd) {
-  constexpr int LDX = 2 * H + 4, PER = 16 * H / kSplitBlock;
+    const float* __restrict__ v_mid, float* __restrict__ s_out, float* __restrict__ v_out,
+    float* __restrict__ a_upd, float* __restrict__ g12) {
+  constexpr int BLK = 4 * H, WAVES = H / 16;
+  constexpr int LDX = 2 * H + 4, LDH = H + 4, LDY = 96 + 4;
+  constexpr int NT = (6 + WAVES - 1) / WAVES;    // second product: 6 column tiles, ds, g1, g2
+  constexpr int PE = 16 * 32 / BLK;              // outputs per thread
   __shared__ __align__(16) float x_lds[16 * LDX];
-  const int base = blockIdx.x * 16, wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int cb[1] = {(int)blockIdx.y * 32 + wave * 16};
+  __shared__ __align__(16) float h_lds[16 * LDH];
+  __shared__ float y_lds[16 * LDY];
+  const int base = blockIdx.x * 16, slice = blockIdx.y * 32;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int cb[1] = {16 * wave};
   Weights<1, 2 * H> w1;
   load_weights(w + lw.u1w, 2 * H, cb, w1);
-  float sv[PER], x0[PER], x1[PER], x2[PER];
+  Weights<1, H> w2[NT];
+  int col[NT];
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, c = idx % H;
-    const int i = min(base + m, N - 1);
-    const float* vv = v_mid + (size_t)i * 3 * H;
-    sv[k] = s_mid[(size_t)i * H + c];
-    x0[k] = vv[c];
-    x1[k] = vv[H + c];
-    x2[k] = vv[2 * H + c];
+  for (int q = 0; q < NT; ++q) {
+    const int t = min(wave + q * WAVES, 5);
+    col[q] = t / 2 * H + slice + 16 * (t % 2);
+    const int c2[1] = {col[q]};
+    load_weights(w + lw.u2w, H, c2, w2[q]);
   }
+  {
+    const int m = threadIdx.x / (H / 4), c = 4 * (threadIdx.x % (H / 4));
+    const size_t i = min(base + m, N - 1);
+    const float* vr = v_mid + i * 3 * H + c;
+    auto ld = [](const float* q) { return *reinterpret_cast<const f4*>(q); };
+    f4 sv = ld(s_mid + i * H + c);
+    const f4 x0 = ld(vr), x1 = ld(vr + H), x2 = ld(vr + 2 * H);
+    f4 n;
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, c = idx % H;
-    const bool in = base + m < N;
-    x_lds[m * LDX + c] = in ? sv[k] : 0.f;
-    x_lds[m * LDX + H + c] = in ? norm3_exact(x0[k], x1[k], x2[k]) : 0.f;
+    for (int k = 0; k < 4; ++k) n[k] = norm3_exact(x0[k], x1[k], x2[k]);
+    if (base + m >= N) sv = n = f4{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<f4*>(x_lds + m * LDX + c) = sv;
+    *reinterpret_cast<f4*>(x_lds + m * LDX + H + c) = n;
   }
-  __syncthreads();
-  f4 acc[1][1];
-  zero_acc(acc);
-  mma_regs(x_lds, LDX, w1, acc);
-  const int c = cb[0] + r;
-  const float bias = (w + lw.u1b)[c];
+  float sm[PE], xv[PE][3], u[9];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int i = base + 4 * g + k;
-    if (i < N) a_upd[(size_t)i * H + c] = acc[0][0][k] + bias;
-  }
-}
-
-// (ds, g1, g2) = silu(a) W2^T + b2 and the gated outputs
-template <int H>
-__global__ __launch_bounds__(kSplitBlock, 2) void update_gate_kernel(
-    int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ s_mid,
-    const float* __restrict__ v_mid, const float* __restrict__ a_upd, float* __restrict__ s_out,
-    float* __restrict__ v_out, float* __restrict__ g12) {
-  constexpr int LDH = H + 4, PER = 16 * H / kSplitBlock;
-  __shared__ __align__(16) float h_lds[16 * LDH];
-  const int base = blockIdx.x * 16, wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int c = blockIdx.y * 32 + wave * 16 + r;
-  const int cb[3] = {c - r, H + c - r, 2 * H + c - r};
-  Weights<3, H> w2;
-  load_weights(w + lw.u2w, H, cb, w2);
-  float av[PER], sm[4], xv[4][3], u[9], bias[3];
+  for (int k = 0; k < PE; ++k) {
+    const int e = threadIdx.x + k * BLK, c = slice + e % 32;
+    const size_t i = min(base + e / 32, N - 1);
+    sm[k] = s_mid[i * H + c];
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, q = idx % H;
-    av[k] = a_upd[(size_t)min(base + m, N - 1) * H + q];
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int i = min(base + 4 * g + k, N - 1);
-    sm[k] = s_mid[(size_t)i * H + c];
-#pragma unroll
-    for (int x = 0; x < 3; ++x) xv[k][x] = v_mid[((size_t)i * 3 + x) * H + c];
+    for (int x = 0; x < 3; ++x) xv[k][x] = v_mid[(i * 3 + x) * H + c];
   }
 #pragma unroll
   for (int k = 0; k < 9; ++k) u[k] = (w + lw.mix)[k];
+  const float b1 = (w + lw.u1b)[cb[0] + r];
+  float b2[NT];
 #pragma unroll
-  for (int x = 0; x < 3; ++x) bias[x] = (w + lw.u2b)[x * H + c];
+  for (int q = 0; q < NT; ++q) b2[q] = (w + lw.u2b)[col[q] + r];
+  __syncthreads();
+  {
+    f4 acc[1][1];
+    zero_acc(acc);
+    mma_regs(x_lds, LDX, w1, acc);
+    const int c = cb[0] + r;
+    const bool own = cb[0] >= slice && cb[0] < slice + 32;
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int idx = threadIdx.x + k * kSplitBlock, m = idx / H, q = idx % H;
-    h_lds[m * LDH + q] = silu(av[k]);
+    for (int k = 0; k < 4; ++k) {
+      const int i = base + 4 * g + k;
+      const float a = acc[0][0][k] + b1;
+      if (own && i < N) a_upd[(size_t)i * H + c] = a;
+      h_lds[(4 * g + k) * LDH + c] = silu(a);
+    }
   }
   __syncthreads();
-  f4 acc[1][3];
-  zero_acc(acc);
-  mma_regs(h_lds, LDH, w2, acc);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int i = base + 4 * g + k;
+  for (int q = 0; q < NT; ++q) {
+    const int t = wave + q * WAVES;
+    if (t >= 6) break;
+    f4 acc[1][1];
+    zero_acc(acc);
+    mma_regs(h_lds, LDH, w2[q], acc);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) y_lds[(4 * g + k) * LDY + 16 * t + r] = acc[0][0][k] + b2[q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PE; ++k) {
+    const int e = threadIdx.x + k * BLK, m = e / 32, c = slice + e % 32, i = base + m;
     if (i >= N) continue;
-    const float ds = acc[0][0][k] + bias[0], gt1 = acc[0][1][k] + bias[1],
-                gt2 = acc[0][2][k] + bias[2];
+    const float* y = y_lds + m * LDY + e % 32;
+    const float ds = y[0], gt1 = y[32], gt2 = y[64];
     const float x0 = xv[k][0], x1 = xv[k][1], x2 = xv[k][2];
     s_out[(size_t)i * H + c] = sm[k] + ds;
     float* vo = v_out + (size_t)i * 3 * H;
@@ -861,6 +861,8 @@ __global__ __launch_bounds__(kSplitBlock, 2) void update_gate_kernel(
     g12[(size_t)i * 2 * H + H + c] = gt2;
   }
 }
+
+constexpr int kSplitBlock = 128;
 
 // ga = silu'(a) (gy W2), gy the gradient of (ds, g1, g2)
 template <int H>
@@ -1459,9 +1461,8 @@ void launch_update_fwd(const Buffers& b, hipStream_t s, const LayerW& lw, const 
                        const float* v_mid, float* s_out, float* v_out, float* a_upd, float* g12) {
   if (b.N <= kSplitAtoms) {
     const dim3 grid((b.N + 15) / 16, H / 32);
-    update_hidden_kernel<H><<<grid, kSplitBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, a_upd);
-    update_gate_kernel<H><<<grid, kSplitBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, a_upd, s_out,
-                                                       v_out, g12);
+    update_fwd_split_kernel<H><<<grid, 4 * H, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, s_out, v_out,
+                                                      a_upd, g12);
   } else {
     auto run = [&](auto kernel, int tm) {
       kernel<<<(b.N + tm - 1) / tm, kUpdBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, s_out, v_out,
