@@ -29,6 +29,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "internal.hpp"
@@ -249,8 +250,7 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_fwd_kernel(
     const float4* __restrict__ geom, const int32_t* __restrict__ counts, int32_t pcap,
     TableView tv, int64_t layer_floats, const int32_t* __restrict__ gate, float* __restrict__ Wf,
     int L, int N, const int64_t* __restrict__ Z, const float* __restrict__ emb,
-    float* __restrict__ S0, float* __restrict__ V0) {
-  constexpr int Q = 3 * H / 4;
+    float* __restrict__ S0, float* __restrict__ V0, bool skip) {
   if ((int)blockIdx.y == L) {
     for (int idx = blockIdx.x * kTabBlock + threadIdx.x; idx < N * (H / 4);
          idx += gridDim.x * kTabBlock)
@@ -261,31 +261,40 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_fwd_kernel(
   const float* tab = tv.w + blockIdx.y * layer_floats;
   float* Wout = Wf + blockIdx.y * (size_t)pcap * 3 * H;
   const int P = min(counts[MLFF_COUNT_PAIRS], pcap);
-  const int64_t total = (int64_t)P * Q;
-  constexpr int kItems = kTabBlock * kTabUnroll;
-  for (int64_t base = (int64_t)blockIdx.x * kItems; base < total;
-       base += (int64_t)gridDim.x * kItems) {
-    TableAt at[kTabUnroll];
-    f4 v[kTabUnroll][4];
-    // items past the end read the last pair and are not stored
+  // Q items of four columns per pair: all of W, or (zero_vectors) without Wv1
+  auto fill = [&](auto items) {
+    constexpr int Q = decltype(items)::value;
+    const int64_t total = (int64_t)P * Q;
+    constexpr int kItems = kTabBlock * kTabUnroll;
+    auto column = [](int q) { return 4 * q + (Q < 3 * H / 4 && q >= H / 4 ? H : 0); };
+    for (int64_t base = (int64_t)blockIdx.x * kItems; base < total;
+         base += (int64_t)gridDim.x * kItems) {
+      TableAt at[kTabUnroll];
+      f4 v[kTabUnroll][4];
+      // items past the end read the last pair and are not stored
 #pragma unroll
-    for (int u = 0; u < kTabUnroll; ++u) {
-      const int64_t it = min(base + u * kTabBlock + threadIdx.x, total - 1);
-      const int p = (int)(it / Q), c = 4 * (int)(it - (int64_t)p * Q);
-      at[u] = table_at(geom[p].w, tv.inv_c, tv.Kc);
-      const float* row = tab + (size_t)at[u].k * 2 * 3 * H + c;
+      for (int u = 0; u < kTabUnroll; ++u) {
+        const int64_t it = min(base + u * kTabBlock + threadIdx.x, total - 1);
+        const int p = (int)(it / Q), c = column((int)(it - (int64_t)p * Q));
+        at[u] = table_at(geom[p].w, tv.inv_c, tv.Kc);
+        const float* row = tab + (size_t)at[u].k * 2 * 3 * H + c;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[u][k] = *reinterpret_cast<const f4*>(row + k * 3 * H);
-    }
+        for (int k = 0; k < 4; ++k) v[u][k] = *reinterpret_cast<const f4*>(row + k * 3 * H);
+      }
 #pragma unroll
-    for (int u = 0; u < kTabUnroll; ++u) {
-      const int64_t it = base + u * kTabBlock + threadIdx.x;
-      if (it < total) {
-        const f4 o = hermite(at[u], v[u][0], v[u][1], v[u][2], v[u][3]);
-        __builtin_nontemporal_store(o, reinterpret_cast<f4*>(Wout) + it);
+      for (int u = 0; u < kTabUnroll; ++u) {
+        const int64_t it = base + u * kTabBlock + threadIdx.x;
+        if (it < total) {
+          const f4 o = hermite(at[u], v[u][0], v[u][1], v[u][2], v[u][3]);
+          const int64_t p = it / Q;
+          __builtin_nontemporal_store(
+              o, reinterpret_cast<f4*>(Wout + p * 3 * H + column((int)(it - p * Q))));
+        }
       }
     }
-  }
+  };
+  if (skip && blockIdx.y == 0) fill(std::integral_constant<int, 2 * H / 4>{});
+  else fill(std::integral_constant<int, 3 * H / 4>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -306,10 +315,12 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_bwd_kernel(
     const int32_t* __restrict__ pair_hi, const float4* __restrict__ geom, TableView tv,
     int64_t layer_floats, const int32_t* __restrict__ gate, const float* __restrict__ Wf, int N,
     const float* __restrict__ s_in, const float* __restrict__ v_in,
-    const float* __restrict__ gs1, const float* __restrict__ gv1, float4* __restrict__ pacc) {
+    const float* __restrict__ gs1, const float* __restrict__ gv1, float4* __restrict__ pacc,
+    bool skip) {
   constexpr int G = H / 4, PPB = kTabBlock / G;
   if (gate != nullptr && *gate != 0) return;
   const int l = blockIdx.y;
+  const bool vectors = !(skip && l == 0);
   const size_t nh = (size_t)l * N * H;
   const float* tab = tv.d + l * layer_floats;
   Wf += (size_t)l * pcap * 3 * H;
@@ -341,7 +352,7 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_bwd_kernel(
              hermite(at, ld(row), ld(row + 3 * H), ld(row + 6 * H), ld(row + 9 * H));
     const f4 qa0 = ld(qa), qa1 = ld(qa + H), qa2 = ld(qa + 2 * H);
     const f4 qb0 = ld(qb), qb1 = ld(qb + H), qb2 = ld(qb + 2 * H);
-    {
+    if (vectors) {
       const f4 g1 = qa0 * ld(vb) + qa1 * ld(vb + H) + qa2 * ld(vb + 2 * H) + qb0 * ld(va) +
                     qb1 * ld(va + H) + qb2 * ld(va + 2 * H);
       const float* r1 = row + H;
@@ -423,7 +434,8 @@ void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1, bo
   if (embed) units = std::max(units, ((int64_t)b.N * (H / 4) + kTabBlock - 1) / kTabBlock);
   filter_table_fwd_kernel<H><<<dim3(table_grid(b, units), l1 - l0 + embed), kTabBlock, 0, s>>>(
       b.geom, b.counts, b.pcap, table_view(b.ts, b.tab, l0, 3 * H), b.ts.layer_floats, b.gate,
-      b.Wf + (size_t)l0 * b.pcap * 3 * H, l1 - l0, b.N, b.numbers, b.w + b.mw->emb, b.S, b.V);
+      b.Wf + (size_t)l0 * b.pcap * 3 * H, l1 - l0, b.N, b.numbers, b.w + b.mw->emb, b.S, b.V,
+      l0 == 0 && zero_vectors(b));
 }
 
 template <int H>
@@ -434,7 +446,7 @@ void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l0, int l1) {
                                kTabBlock, 0, s>>>(
       b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, table_view(b.ts, b.tab, l0, 3 * H),
       b.ts.layer_floats, b.gate, b.Wf + (size_t)l0 * b.pcap * 3 * H, b.N, b.S + nh, b.V + 3 * nh,
-      b.gS1 + nh, b.gV1 + 3 * nh, b.pacc + (size_t)l0 * b.pcap);
+      b.gS1 + nh, b.gV1 + 3 * nh, b.pacc + (size_t)l0 * b.pcap, l0 == 0 && zero_vectors(b));
 }
 
 #define MLFF_TABLE_INST(HH)                                                         \

@@ -144,6 +144,10 @@ struct Buffers {
   hipStream_t aux;
   hipEvent_t* ev;
 };
+// The first block reads neither its vectors, which are zero, nor what multiplies
+// them (Wv1 and its derivative).  Only with checked tables: the check fails for
+// infinities and NaN in a filter, whose products with zero are no zeros.
+inline bool zero_vectors(const Buffers& b) { return b.use_table && b.gate == nullptr; }
 __host__ __device__ inline int64_t wbf_plane(int H) { return 3 * (int64_t)H * H; }
 __host__ __device__ inline int64_t wbf_f2w(int H, int l) { return (int64_t)l * 3 * wbf_plane(H); }
 __host__ __device__ inline int64_t wbf_elems(int H, int L) { return (int64_t)L * 3 * wbf_plane(H); }

@@ -225,8 +225,10 @@ __global__ __launch_bounds__(kPairBlock, 4) void filter_fwd_kernel(
 // waters and 32 / 21 us for one molecule of 60 atoms; this form 180 / 144,
 // 47 / 32 and 10 / 7 us.  Twelve edges in flight: 180 / 143, 48 / 33, 12 / 7.
 // SPLIT: 6.3 / 4.8 us for the molecule of 60 atoms.
+// ZEROV: the first block, whose vectors are zero: their products with Wv1 add
+// exact zeros (zero_vectors()), so neither is read.
 // ---------------------------------------------------------------------------
-template <int H, bool FWD, int UNROLL, bool SPLIT>
+template <int H, bool FWD, int UNROLL, bool SPLIT, bool ZEROV>
 __global__ __launch_bounds__(SPLIT ? kMsgSums * H : kBlock) void message_kernel(
     int N, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col,
     const int32_t* __restrict__ edge_pair, int32_t ecap, const float4* __restrict__ unit,
@@ -273,11 +275,13 @@ __global__ __launch_bounds__(SPLIT ? kMsgSums * H : kBlock) void message_kernel(
       const float* wp = Wf + (size_t)p * 3 * H;
       const float* vj = v_in + (size_t)jc[u] * 3 * H;
       ws[u] = wp[c];
-      wv1[u] = wp[H + c];
       sj[u] = (s_in + (size_t)jc[u] * H)[c];
-      v0[u] = vj[c];
-      v1[u] = vj[H + c];
-      v2[u] = vj[2 * H + c];
+      if (!ZEROV) {
+        wv1[u] = wp[H + c];
+        v0[u] = vj[c];
+        v1[u] = vj[H + c];
+        v2[u] = vj[2 * H + c];
+      }
       if (FWD) {
         wv2[u] = wp[2 * H + c];
         uu[u] = unit[p];
@@ -287,12 +291,15 @@ __global__ __launch_bounds__(SPLIT ? kMsgSums * H : kBlock) void message_kernel(
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      const float w0 = on[u] ? ws[u] : 0.f, w1 = on[u] ? wv1[u] : 0.f;
+      const float w0 = on[u] ? ws[u] : 0.f;
       const int o = u % NA;   // UNROLL is a multiple of NA
       as[o] = fma_(sj[u], w0, as[o]);
-      a0[o] = fma_(v0[u], w1, a0[o]);
-      a1[o] = fma_(v1[u], w1, a1[o]);
-      a2[o] = fma_(v2[u], w1, a2[o]);
+      if (!ZEROV) {
+        const float w1 = on[u] ? wv1[u] : 0.f;
+        a0[o] = fma_(v0[u], w1, a0[o]);
+        a1[o] = fma_(v1[u], w1, a1[o]);
+        a2[o] = fma_(v2[u], w1, a2[o]);
+      }
       if (FWD) {
         // u_ji = (p_j - p_i)/(d + eps): +pair vector when j is the pair's hi atom
         const float w2 = on[u] ? (jc[u] < i ? -wv2[u] : wv2[u]) : 0.f;
@@ -1437,21 +1444,29 @@ void launch_filter_bwd(const Buffers& b, hipStream_t st, int l) {
 }
 
 template <int H, bool FWD>
-void launch_message(const Buffers& b, hipStream_t st, const float* Wl, const float* s_in,
-                    const float* v_in, float* s_out, float* v_out) {
+void launch_message(const Buffers& b, hipStream_t st, int l, const float* s_in, const float* v_in,
+                    float* s_out, float* v_out) {
   constexpr int U0 = FWD ? kMsgUnrollFwd : kMsgUnrollBwd;
   constexpr int U1 = FWD ? kMsgUnrollFwdAlt : kMsgUnrollBwdAlt;
+  const float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
   auto run = [&](auto kernel, int rows_per_block, int block) {
     const int grid = ((b.N + rows_per_block - 1) / rows_per_block + 7) / 8 * 8;
     kernel<<<grid, block, 0, st>>>(b.N, b.row_ptr, b.col, b.edge_pair, b.ecap, b.unit, Wl, s_in,
                                    v_in, s_out, v_out);
   };
-  if (b.N <= kMsgSplitAtoms)
-    run(message_kernel<H, FWD, U0, true>, 1, kMsgSums * H);
-  else if ((FWD ? b.unroll_fwd : b.unroll_bwd) == U1)
-    run(message_kernel<H, FWD, U1, false>, kBlock / H, kBlock);
-  else
-    run(message_kernel<H, FWD, U0, false>, kBlock / H, kBlock);
+  auto shapes = [&](auto zero) {
+    constexpr bool Z = decltype(zero)::value;
+    if (b.N <= kMsgSplitAtoms)
+      run(message_kernel<H, FWD, U0, true, Z>, 1, kMsgSums * H);
+    else if ((FWD ? b.unroll_fwd : b.unroll_bwd) == U1)
+      run(message_kernel<H, FWD, U1, false, Z>, kBlock / H, kBlock);
+    else
+      run(message_kernel<H, FWD, U0, false, Z>, kBlock / H, kBlock);
+  };
+  if constexpr (FWD) {
+    if (l == 0 && zero_vectors(b)) return shapes(std::true_type{});
+  }
+  shapes(std::false_type{});
 }
 
 // Atom-side launches: the split or small forms for few atoms (kSplitAtoms,
@@ -1559,13 +1574,12 @@ hipError_t forward_impl(const Buffers& b, hipStream_t s) {
   }
   for (int l = 0; l < b.L; ++l) {
     const LayerW& lw = mw.layer[l];
-    float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
     if (st.two() && st.err == hipSuccess) st.err = hipStreamWaitEvent(s, b.ev[1 + l], 0);
     float* Sl = b.S + (size_t)l * nh(b);
     float* Vl = b.V + (size_t)l * 3 * nh(b);
     float* Sm = b.Smid + (size_t)l * nh(b);
     float* Vm = b.Vmid + (size_t)l * 3 * nh(b);
-    launch_message<H, true>(b, s, Wl, Sl, Vl, Sm, Vm);
+    launch_message<H, true>(b, s, l, Sl, Vl, Sm, Vm);
     launch_update_fwd<H>(b, s, lw, Sm, Vm, b.S + (size_t)(l + 1) * nh(b),
                          b.V + (size_t)(l + 1) * 3 * nh(b), b.Aupd + (size_t)l * nh(b),
                          b.G12 + (size_t)l * 2 * nh(b));
@@ -1588,7 +1602,6 @@ hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool wa
   float* gv2 = nullptr;
   for (int l = b.L - 1; l >= 0; --l) {
     const LayerW& lw = mw.layer[l];
-    const float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
     // block l's message gradient has a slice of its own, so the filter
     // adjoint of block l (filter stream) and the message adjoint of block l
     // and update adjoint of block l-1 (caller's stream) run side by side
@@ -1599,7 +1612,7 @@ hipError_t backward_impl(const Buffers& b, hipStream_t s, float* forces, bool wa
     if (b.use_table && st.two()) launch_filter_table_bwd<H>(b, st.filt, l, l + 1);
     if (direct_filters(b)) launch_filter_bwd<H>(b, st.filt, l);
     if (l > 0) {
-      launch_message<H, false>(b, s, Wl, gS1, gV1, b.gS0, b.gV0);
+      launch_message<H, false>(b, s, l, gS1, gV1, b.gS0, b.gV0);
       gs2 = b.gS0;
       gv2 = b.gV0;
     }
@@ -1619,14 +1632,13 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
   const float* centers = b.w + mw.centers;
   const float* widths = b.w + mw.widths;
   const LayerW& lw = mw.layer[l];
-  float* Wl = b.Wf + (size_t)l * b.pcap * 3 * H;
   switch (stage) {
     case MLFF_STAGE_FILTER_FWD:
       if (b.use_table) launch_filter_table_fwd<H>(b, s, l, l + 1, false);
       if (direct_filters(b)) launch_filter_fwd<H>(b, s, l);
       break;
     case MLFF_STAGE_MESSAGE_FWD:
-      launch_message<H, true>(b, s, Wl, b.S + (size_t)l * nh(b),
+      launch_message<H, true>(b, s, l, b.S + (size_t)l * nh(b),
                               b.V + (size_t)l * 3 * nh(b), b.Smid + (size_t)l * nh(b),
                               b.Vmid + (size_t)l * 3 * nh(b));
       break;
@@ -1647,7 +1659,7 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
       if (direct_filters(b)) launch_filter_bwd<H>(b, s, l);
       break;
     case MLFF_STAGE_MESSAGE_BWD:
-      launch_message<H, false>(b, s, Wl, b.gS1 + (size_t)l * nh(b),
+      launch_message<H, false>(b, s, l, b.gS1 + (size_t)l * nh(b),
                                b.gV1 + (size_t)l * 3 * nh(b), b.gS0, b.gV0);
       break;
     case MLFF_STAGE_FORCES:

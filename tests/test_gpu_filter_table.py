@@ -104,3 +104,31 @@ def test_evaluations_after_a_weight_change(gpu, narrow):
     assert not torch.equal(before[1], runs[0][1])
     for e, f in runs[1:]:
         assert torch.equal(e, runs[0][0]) and torch.equal(f, runs[0][1])
+
+
+@pytest.mark.parametrize("H,n", [(32, 40), (64, 40), (128, 40), (128, 400)])
+def test_first_block_without_its_zero_vectors(gpu, H, n):
+    """The first evaluation with new weights runs before its tables are checked
+    and multiplies the first block's zero vectors out; the ones after leave them
+    out (row forms of up to and beyond 1,024 atoms).  The same bits; a NaN in the
+    filter rows that only they meet still reaches the energy."""
+    print(f"[case] first block H{H} n{n}", flush=True)
+    synth = pkg_mod("synth")
+    rng = np.random.Generator(np.random.PCG64(n))
+    Z, P, ptr = synth.flatten([synth.random_molecule(40, rng) for _ in range(n // 10)])
+    torch.manual_seed(1)
+    m = pkg().StudentForceField(hidden_dim=H, num_interactions=2, num_rbf=20).to(gpu)
+    Zt, Pt = torch.tensor(Z, device=gpu), torch.tensor(P.astype(np.float32), device=gpu)
+    sizes = np.diff(ptr)
+    ev = lambda: m.evaluate(Zt, Pt, sizes, need_virial=True)
+    for a in (ev(), ev()):     # resolve the tables
+        assert torch.isfinite(a[0]).all()
+    with torch.no_grad():
+        m.interactions[0].message.rbf_to_scalar[2].weight.mul_(1.0)
+    runs = [ev() for _ in range(4)]
+    for r in runs[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(runs[0], r))
+    with torch.no_grad():
+        m.interactions[0].message.rbf_to_scalar[2].weight[H + 3, 5] = float("nan")
+    for _ in range(4):
+        assert torch.isnan(ev()[0]).all()
