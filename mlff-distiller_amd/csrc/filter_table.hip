@@ -300,7 +300,8 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_fwd_kernel(
 // ---------------------------------------------------------------------------
 // Filter adjoint of pair p = (a < b) from the table (see filter_bwd_kernel for
 // the terms): H/4 lanes per pair, four channels each, gather both endpoints'
-// features and gradients, form dL/dW_p in registers and contract it with
+// features and gradients (the lower atom's once for a run of consecutive pairs,
+// see pair_run), form dL/dW_p in registers and contract it with
 // W'(d_p) to dL/dd, and (gv_a - gv_b) with Wv2 to dL/du.  Bound by the gathers
 // (16H floats per pair) and the 12H floats of the W' rows, all from L2.  The
 // blocks' terms meet in force_gather_kernel, so all blocks (blockIdx.y) run in
@@ -316,7 +317,7 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_bwd_kernel(
     int64_t layer_floats, const int32_t* __restrict__ gate, const float* __restrict__ Wf, int N,
     const float* __restrict__ s_in, const float* __restrict__ v_in,
     const float* __restrict__ gs1, const float* __restrict__ gv1, float4* __restrict__ pacc,
-    bool skip) {
+    bool skip, int run) {
   constexpr int G = H / 4, PPB = kTabBlock / G;
   if (gate != nullptr && *gate != 0) return;
   const int l = blockIdx.y;
@@ -331,47 +332,57 @@ __global__ __launch_bounds__(kTabBlock) void filter_table_bwd_kernel(
   pacc += (size_t)l * pcap;
   const int P = min(counts[MLFF_COUNT_PAIRS], pcap);
   int t0, t1, tstep;
-  persistent_range((P + PPB - 1) / PPB, t0, t1, tstep);
+  persistent_range((P + PPB * run - 1) / (PPB * run), t0, t1, tstep);
   const int c = 4 * (threadIdx.x % G);
   auto ld = [&](const float* q) { return *reinterpret_cast<const f4*>(q); };
   for (int tile = t0; tile < t1; tile += tstep) {
-    const int pr = tile * PPB + threadIdx.x / G;
-    const int p = min(pr, P - 1);   // past the end: the last pair, not stored
-    const int a = pair_lo[p], b = pair_hi[p];
-    const float4 gm = geom[p];
-    const float* va = v_in + (size_t)a * 3 * H + c;
-    const float* vb = v_in + (size_t)b * 3 * H + c;
-    const float* qa = gv1 + (size_t)a * 3 * H + c;
-    const float* qb = gv1 + (size_t)b * 3 * H + c;
-    const TableAt at = table_at(gm.w, tv.inv, tv.K);
-    const float* row = tab + (size_t)at.k * 2 * 3 * H + c;
-    const f4 sa = ld(s_in + (size_t)a * H + c), sb = ld(s_in + (size_t)b * H + c);
-    const f4 ga = ld(gs1 + (size_t)a * H + c), gb = ld(gs1 + (size_t)b * H + c);
-    const f4 wv2 = ld(Wf + (size_t)p * 3 * H + 2 * H + c);
-    f4 acc = (ga * sb + gb * sa) *
-             hermite(at, ld(row), ld(row + 3 * H), ld(row + 6 * H), ld(row + 9 * H));
-    const f4 qa0 = ld(qa), qa1 = ld(qa + H), qa2 = ld(qa + 2 * H);
-    const f4 qb0 = ld(qb), qb1 = ld(qb + H), qb2 = ld(qb + 2 * H);
-    if (vectors) {
-      const f4 g1 = qa0 * ld(vb) + qa1 * ld(vb + H) + qa2 * ld(vb + 2 * H) + qb0 * ld(va) +
-                    qb1 * ld(va + H) + qb2 * ld(va + 2 * H);
-      const float* r1 = row + H;
-      acc += g1 * hermite(at, ld(r1), ld(r1 + 3 * H), ld(r1 + 6 * H), ld(r1 + 9 * H));
+    const int first = (tile * PPB + threadIdx.x / G) * run;
+    int a = -1;
+    f4 sa = {}, ga = {}, va0 = {}, va1 = {}, va2 = {}, qa0 = {}, qa1 = {}, qa2 = {};
+    for (int r = 0; r < run; ++r) {
+      const int p = min(first + r, P - 1);   // past the end: the last pair, not stored
+      const int lo = pair_lo[p], b = pair_hi[p];
+      const float4 gm = geom[p];
+      const float* vb = v_in + (size_t)b * 3 * H + c;
+      const float* qb = gv1 + (size_t)b * 3 * H + c;
+      const TableAt at = table_at(gm.w, tv.inv, tv.K);
+      const float* row = tab + (size_t)at.k * 2 * 3 * H + c;
+      if (lo != a) {
+        a = lo;
+        const float* va = v_in + (size_t)a * 3 * H + c;
+        const float* qa = gv1 + (size_t)a * 3 * H + c;
+        sa = ld(s_in + (size_t)a * H + c);
+        ga = ld(gs1 + (size_t)a * H + c);
+        qa0 = ld(qa), qa1 = ld(qa + H), qa2 = ld(qa + 2 * H);
+        if (vectors) va0 = ld(va), va1 = ld(va + H), va2 = ld(va + 2 * H);
+      }
+      const f4 sb = ld(s_in + (size_t)b * H + c);
+      const f4 gb = ld(gs1 + (size_t)b * H + c);
+      const f4 wv2 = ld(Wf + (size_t)p * 3 * H + 2 * H + c);
+      f4 acc = (ga * sb + gb * sa) *
+               hermite(at, ld(row), ld(row + 3 * H), ld(row + 6 * H), ld(row + 9 * H));
+      const f4 qb0 = ld(qb), qb1 = ld(qb + H), qb2 = ld(qb + 2 * H);
+      if (vectors) {
+        const f4 g1 = qa0 * ld(vb) + qa1 * ld(vb + H) + qa2 * ld(vb + 2 * H) + qb0 * va0 +
+                      qb1 * va1 + qb2 * va2;
+        const float* r1 = row + H;
+        acc += g1 * hermite(at, ld(r1), ld(r1 + 3 * H), ld(r1 + 6 * H), ld(r1 + 9 * H));
+      }
+      const float den = gm.w + kEdgeEps;
+      const float ux = gm.x / den, uy = gm.y / den, uz = gm.z / den;
+      const f4 d0 = qa0 - qb0, d1 = qa1 - qb1, d2 = qa2 - qb2;
+      {
+        const float* r2 = row + 2 * H;
+        acc += (ux * d0 + uy * d1 + uz * d2) *
+               hermite(at, ld(r2), ld(r2 + 3 * H), ld(r2 + 6 * H), ld(r2 + 9 * H));
+      }
+      const f4 w0 = wv2 * d0, w1 = wv2 * d1, w2 = wv2 * d2;
+      const float gd = group_sum<G>((acc[0] + acc[1]) + (acc[2] + acc[3]));
+      const float gx = group_sum<G>((w0[0] + w0[1]) + (w0[2] + w0[3]));
+      const float gy = group_sum<G>((w1[0] + w1[1]) + (w1[2] + w1[3]));
+      const float gz = group_sum<G>((w2[0] + w2[1]) + (w2[2] + w2[3]));
+      if (c == 0 && first + r < P) pacc[p] = make_float4(gx, gy, gz, gd);
     }
-    const float den = gm.w + kEdgeEps;
-    const float ux = gm.x / den, uy = gm.y / den, uz = gm.z / den;
-    const f4 d0 = qa0 - qb0, d1 = qa1 - qb1, d2 = qa2 - qb2;
-    {
-      const float* r2 = row + 2 * H;
-      acc += (ux * d0 + uy * d1 + uz * d2) *
-             hermite(at, ld(r2), ld(r2 + 3 * H), ld(r2 + 6 * H), ld(r2 + 9 * H));
-    }
-    const f4 w0 = wv2 * d0, w1 = wv2 * d1, w2 = wv2 * d2;
-    const float gd = group_sum<G>((acc[0] + acc[1]) + (acc[2] + acc[3]));
-    const float gx = group_sum<G>((w0[0] + w0[1]) + (w0[2] + w0[3]));
-    const float gy = group_sum<G>((w1[0] + w1[1]) + (w1[2] + w1[3]));
-    const float gz = group_sum<G>((w2[0] + w2[1]) + (w2[2] + w2[3]));
-    if (c == 0 && pr < P) pacc[p] = make_float4(gx, gy, gz, gd);
   }
 }
 
@@ -393,6 +404,17 @@ hipError_t build_impl(const Buffers& b, hipStream_t s) {
 int table_grid(const Buffers& b, int64_t units) {
   const int64_t n = (units + 7) / 8 * 8;
   return (int)(n < 8 ? 8 : (n < b.blocks ? n : b.blocks));
+}
+
+// Consecutive pairs that one group of lanes of the filter adjoint takes, so that
+// the features of their common lower atom are read once: four from 64 rounds of
+// resident wavefronts (256 CUs x 16) on, two from 16 on, one below.  Runs of
+// 1 / 2 / 4 / 8 took 621 / 583 / 575 / 607 us for 256 molecules at H = 128 (100
+// rounds), 150 / 143 / 146 / 168 us for 1000 periodic waters (24 rounds), 7.5 / 8.0
+// / 10.4 / 17.3 us for 60 atoms.  Indices read one pair ahead: 1-2 % slower.
+int pair_run(int H, int64_t pcap, int blocks) {
+  const int64_t rounds = pcap * (H / 4) * blocks / (256 * 16 * 64);
+  return rounds >= 64 ? 4 : rounds >= 16 ? 2 : 1;
 }
 
 }  // namespace
@@ -442,11 +464,12 @@ template <int H>
 void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l0, int l1) {
   constexpr int PPB = kTabBlock / (H / 4);
   const size_t nh = (size_t)l0 * b.N * H;
-  filter_table_bwd_kernel<H><<<dim3(table_grid(b, ((int64_t)b.pcap + PPB - 1) / PPB), l1 - l0),
+  const int run = pair_run(H, b.pcap, l1 - l0), per = PPB * run;
+  filter_table_bwd_kernel<H><<<dim3(table_grid(b, ((int64_t)b.pcap + per - 1) / per), l1 - l0),
                                kTabBlock, 0, s>>>(
       b.counts, b.pcap, b.pair_lo, b.pair_hi, b.geom, table_view(b.ts, b.tab, l0, 3 * H),
       b.ts.layer_floats, b.gate, b.Wf + (size_t)l0 * b.pcap * 3 * H, b.N, b.S + nh, b.V + 3 * nh,
-      b.gS1 + nh, b.gV1 + 3 * nh, b.pacc + (size_t)l0 * b.pcap, l0 == 0 && zero_vectors(b));
+      b.gS1 + nh, b.gV1 + 3 * nh, b.pacc + (size_t)l0 * b.pcap, l0 == 0 && zero_vectors(b), run);
 }
 
 #define MLFF_TABLE_INST(HH)                                                         \

@@ -132,3 +132,25 @@ def test_first_block_without_its_zero_vectors(gpu, H, n):
         m.interactions[0].message.rbf_to_scalar[2].weight[H + 3, 5] = float("nan")
     for _ in range(4):
         assert torch.isnan(ev()[0]).all()
+
+
+@pytest.mark.parametrize("H,n", [(32, 8), (64, 70), (128, 30), (128, 141)])
+def test_runs_of_pairs_keep_a_structures_bits(gpu, H, n):
+    """The filter adjoint takes one, two or four pairs per group of lanes with the
+    batch's size; an atom's run of pairs ends anywhere in them.  A structure gives
+    the bits it gives alone (one pair per group)."""
+    print(f"[case] pair runs H{H} n{n}", flush=True)
+    synth = pkg_mod("synth")
+    rng = np.random.Generator(np.random.PCG64(n))
+    Z, P, ptr = synth.flatten([synth.random_molecule(41 + k % 20, rng) for k in range(n)])
+    torch.manual_seed(1)
+    m = pkg().StudentForceField(hidden_dim=H, num_interactions=3, num_rbf=20, cutoff=8.0).to(gpu)
+    Zt, Pt = torch.tensor(Z, device=gpu), torch.tensor(P.astype(np.float32), device=gpu)
+    for _ in range(3):         # resolve the tables
+        e, f, v = m.evaluate(Zt, Pt, np.diff(ptr), need_virial=True)
+    for k in (0, n // 2, n - 1):
+        at = slice(int(ptr[k]), int(ptr[k + 1]))
+        for _ in range(3):
+            one = m.evaluate(Zt[at], Pt[at], np.diff(ptr)[k:k + 1], need_virial=True)
+        assert torch.equal(one[0][0], e[k]) and torch.equal(one[1], f[at])
+        assert torch.equal(one[2][0], v[k])
