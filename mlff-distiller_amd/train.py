@@ -590,7 +590,7 @@ class _WgGroup:
                 C.stream_handle(), kind, n_probs, at + 112 * start, blocks))
         for i in range(0, len(self.rows), 256):   # at most 256 rows per launch
             rows = self.rows[i:i + 256]
-            n_blocks = sum((n4 + 255) // 256 for _, n4, _, _ in rows)
+            n_blocks = sum((n4 + 31) // 32 for _, n4, _, _ in rows)
             C.check("mlff_weight_grad_reduce_group", lib.mlff_weight_grad_reduce_group(
                 C.stream_handle(), len(rows), at + 8 * n + 32 * i, min(n_blocks, 1 << 16)))
         self.rows, self.keep = [], []

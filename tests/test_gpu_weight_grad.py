@@ -304,3 +304,28 @@ def test_train_filter_weights_follow_the_tensor_objects(gpu):
         assert W.shape == (300, 3 * H)
         err = (W.double().cpu() - rW).abs().max().item()
         assert err <= 2e-6 * max(rW.abs().max().item(), 1.0), (H, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [1, 7, 8, 9, 65, 256, 257, 1000])
+def test_partial_sums_are_added_in_chunks_of_eight(gpu, S):
+    """The order of the partial sums (eight to a chunk, then the chunks) for every
+    number of partials: the float32 sums of that order on the CPU, bit for bit."""
+    print(f"[case] partial sums S={S}", flush=True)
+    g = torch.Generator().manual_seed(S)
+    n4s = [1, 31, 32, 33, 500]
+    parts = [torch.randn(S, 4 * n, generator=g) for n in n4s]
+    dev = [p.to(gpu) for p in parts]
+    outs = [torch.empty(4 * n, device=gpu) for n in n4s]
+    table = torch.tensor([(S, n, p.data_ptr(), o.data_ptr()) for n, p, o in
+                          zip(n4s, dev, outs)], dtype=torch.int64).to(gpu)
+    train.C.check("reduce_group", train.C.lib().mlff_weight_grad_reduce_group(
+        train.C.stream_handle(), len(n4s), table.data_ptr(), 9))
+    for p, o in zip(parts, outs):
+        total = None
+        for c in range(0, S, 8):
+            chunk = p[c]
+            for row in p[c + 1:c + 8]:
+                chunk = chunk + row
+            total = chunk if total is None else total + chunk
+        assert torch.equal(o.cpu(), total)
