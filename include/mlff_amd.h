@@ -574,6 +574,13 @@ int mlff_train_filter(void* stream, int tangent, int hidden, int n_pairs, int nu
                       const uint16_t* w2_planes_dev, const float* b2_dev, const float* a_dev,
                       float* a_out_dev, float* h_out_dev, float* w_out_dev);
 
+/* The same for n_blocks (up to 8) interaction blocks over one basis e in one
+ * launch, with de_dev (may be null) their tangents too.  rows: ten pointers per
+ * block on the host, {W1 padded, b1, W2 planes, b2, a, h, W, da, dh, dW}; the last
+ * three only with de_dev. */
+int mlff_train_filters(void* stream, int hidden, int n_blocks, int n_pairs, int num_rbf,
+                       const float* e_dev, const float* de_dev, const void* const* rows);
+
 /* The reverse of the same MLP's first layer in the training pass (the
  * autograd backward of rbf_to_scalar, student_model.py:318-322, in the
  * reference's double backward, distillation_wrapper.py:86-91), over n_pairs

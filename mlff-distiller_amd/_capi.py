@@ -54,7 +54,7 @@ EXPORTS = (
     "mlff_train_update", "mlff_train_update_adjoint", "mlff_train_readout",
     "mlff_train_readout_adjoint",
     "mlff_probe_mfma_flops", "mlff_probe_mfma", "mlff_plan_set_weights",
-    "mlff_train_filter", "mlff_train_filter_adjoint",
+    "mlff_train_filter", "mlff_train_filters", "mlff_train_filter_adjoint",
     "mlff_filter_planes", "mlff_train_filter_adjoint_x6", "mlff_split_bf16x3", "mlff_pack_weights",
 )
 
@@ -221,6 +221,9 @@ def _declare(lib):
     lib.mlff_train_filter.restype = ctypes.c_int
     lib.mlff_train_filter.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                       ctypes.c_int] + [vp] * 9
+    lib.mlff_train_filters.restype = ctypes.c_int
+    lib.mlff_train_filters.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                       ctypes.c_int, vp, vp, vp]
     lib.mlff_train_filter_adjoint.restype = ctypes.c_int
     lib.mlff_train_filter_adjoint.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int] + [vp] * 7
     lib.mlff_split_bf16x3.restype = ctypes.c_int

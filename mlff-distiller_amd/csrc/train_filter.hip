@@ -39,12 +39,24 @@ constexpr int kTfMaxRbf = 32;
 template <int H>
 constexpr int kTfPairs = H <= 32 ? 128 : 64;
 
+// One block's filters: weights and outputs of the forward (a, h, w) and of its
+// tangent (da, dh, dw).
+struct FilterRow {
+  const float *w1p, *b1;
+  const uint16_t* w2;
+  const float *b2;
+  float *a, *h, *w, *da, *dh, *dw;
+};
+constexpr int kTfMaxLayers = 8;
+struct FilterRows {
+  FilterRow row[kTfMaxLayers];
+};
+
+// One pair tile's forward (or tangent, TAN) of the filter MLP.
 template <int H, int TM, bool TAN>
-__global__ __launch_bounds__(kTfBlock, 4) void train_filter_kernel(
-    int P, int R, int RP, const float* __restrict__ x, const float* __restrict__ w1p,
-    const float* __restrict__ b1, const uint16_t* __restrict__ w2bf,
-    const float* __restrict__ b2, const float* __restrict__ a_in, float* __restrict__ a_out,
-    float* __restrict__ h_out, float* __restrict__ w_out) {
+__device__ __forceinline__ void train_filter_tile(int pbase, int P, int R, int RP, const float* x,
+                                                  const FilterRow& q, float* e_lds,
+                                                  uint16_t* h_bf) {
   constexpr int RT = TM / 16;
   constexpr int LDE = kTfMaxRbf + 4;
   constexpr int LDHB = H + 8;          // bf16 row stride of the split hidden activations
@@ -52,83 +64,104 @@ __global__ __launch_bounds__(kTfBlock, 4) void train_filter_kernel(
   constexpr int CT1 = H / 16, NT1 = (CT1 + kTfWaves - 1) / kTfWaves;
   constexpr int CT2 = 3 * H / 16, NT2 = (CT2 + kTfWaves - 1) / kTfWaves;
   static_assert(CT1 % NT1 == 0 && CT2 % NT2 == 0, "tile split");
-  __shared__ __align__(16) float e_lds[TM * LDE];
-  __shared__ __align__(16) uint16_t h_bf[3 * PHB];
-  const int ntiles = (P + TM - 1) / TM;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int pbase = tile * TM;
-    // the tile's basis rows, zero past R and past the last pair
-    for (int idx = threadIdx.x; idx < TM * RP; idx += kTfBlock) {
-      const int m = idx / RP, k = idx - m * RP, p = pbase + m;
-      e_lds[m * LDE + k] = (p < P && k < R) ? x[(size_t)p * R + k] : 0.f;
-    }
-    __syncthreads();
-    if (wave < CT1 / NT1) {
-      int cb[NT1];
-      f4 acc[RT][NT1];
+  const float* a_in = q.a;
+  float* a_out = TAN ? q.da : q.a;
+  float* h_out = TAN ? q.dh : q.h;
+  float* w_out = TAN ? q.dw : q.w;
+  // the tile's basis rows, zero past R and past the last pair
+  for (int idx = threadIdx.x; idx < TM * RP; idx += kTfBlock) {
+    const int m = idx / RP, k = idx - m * RP, p = pbase + m;
+    e_lds[m * LDE + k] = (p < P && k < R) ? x[(size_t)p * R + k] : 0.f;
+  }
+  __syncthreads();
+  if (wave < CT1 / NT1) {
+    int cb[NT1];
+    f4 acc[RT][NT1];
 #pragma unroll
-      for (int ct = 0; ct < NT1; ++ct) cb[ct] = (wave * NT1 + ct) * 16;
-      zero_acc(acc);
-      mma_tile<RT, NT1>(e_lds, LDE, w1p, RP, RP, cb, acc);
+    for (int ct = 0; ct < NT1; ++ct) cb[ct] = (wave * NT1 + ct) * 16;
+    zero_acc(acc);
+    mma_tile<RT, NT1>(e_lds, LDE, q.w1p, RP, RP, cb, acc);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int ct = 0; ct < NT1; ++ct) {
+        const int c = cb[ct] + r;
+        const float bias = TAN ? 0.f : q.b1[c];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = rt * 16 + 4 * g + i, p = pbase + m;
+          const size_t o = (size_t)p * H + c;
+          float a = acc[rt][ct][i] + bias, hv = 0.f;
+          if (p < P) {
+            hv = TAN ? silu_grad(a_in[o]) * a : silu(a);
+            a_out[o] = a;
+            h_out[o] = hv;
+          }
+          uint16_t hh, hm, hl;
+          split3_bf16(hv, hh, hm, hl);
+          h_bf[m * LDHB + c] = hh;
+          h_bf[PHB + m * LDHB + c] = hm;
+          h_bf[2 * PHB + m * LDHB + c] = hl;
+        }
+      }
+  }
+  __syncthreads();
+  if (wave < CT2 / NT2) {
+    int cb[NT2];
+    f4 acc[RT][NT2];
+#pragma unroll
+    for (int ct = 0; ct < NT2; ++ct) cb[ct] = (wave * NT2 + ct) * 16;
+    zero_acc(acc);
+    mma_tile_x6<RT, NT2, H>(h_bf, LDHB, PHB, q.w2, H, 3 * H * H, cb, acc);
+    float bias[NT2];
+#pragma unroll
+    for (int ct = 0; ct < NT2; ++ct) bias[ct] = TAN ? 0.f : q.b2[cb[ct] + r];
+    // lane (r, g) holds rows rt*16 + 4g + i, columns cb[ct] + r
+    float* out = w_out + (size_t)(pbase + 4 * g) * 3 * H + r;
+    if (pbase + TM <= P) {   // full tile: no per-element bounds checks
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int ct = 0; ct < NT1; ++ct) {
-          const int c = cb[ct] + r;
-          const float bias = TAN ? 0.f : b1[c];
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int m = rt * 16 + 4 * g + i, p = pbase + m;
-            const size_t o = (size_t)p * H + c;
-            float a = acc[rt][ct][i] + bias, hv = 0.f;
-            if (p < P) {
-              hv = TAN ? silu_grad(a_in[o]) * a : silu(a);
-              a_out[o] = a;
-              h_out[o] = hv;
-            }
-            uint16_t hh, hm, hl;
-            split3_bf16(hv, hh, hm, hl);
-            h_bf[m * LDHB + c] = hh;
-            h_bf[PHB + m * LDHB + c] = hm;
-            h_bf[2 * PHB + m * LDHB + c] = hl;
-          }
+          for (int ct = 0; ct < NT2; ++ct)
+            out[(size_t)(rt * 16 + i) * 3 * H + cb[ct]] = acc[rt][ct][i] + bias[ct];
+    } else {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (pbase + rt * 16 + 4 * g + i >= P) continue;
+#pragma unroll
+          for (int ct = 0; ct < NT2; ++ct)
+            out[(size_t)(rt * 16 + i) * 3 * H + cb[ct]] = acc[rt][ct][i] + bias[ct];
         }
     }
-    __syncthreads();
-    if (wave < CT2 / NT2) {
-      int cb[NT2];
-      f4 acc[RT][NT2];
-#pragma unroll
-      for (int ct = 0; ct < NT2; ++ct) cb[ct] = (wave * NT2 + ct) * 16;
-      zero_acc(acc);
-      mma_tile_x6<RT, NT2, H>(h_bf, LDHB, PHB, w2bf, H, 3 * H * H, cb, acc);
-      float bias[NT2];
-#pragma unroll
-      for (int ct = 0; ct < NT2; ++ct) bias[ct] = TAN ? 0.f : b2[cb[ct] + r];
-      // lane (r, g) holds rows rt*16 + 4g + i, columns cb[ct] + r
-      float* out = w_out + (size_t)(pbase + 4 * g) * 3 * H + r;
-      if (pbase + TM <= P) {   // full tile: no per-element bounds checks
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int ct = 0; ct < NT2; ++ct)
-              out[(size_t)(rt * 16 + i) * 3 * H + cb[ct]] = acc[rt][ct][i] + bias[ct];
-      } else {
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if (pbase + rt * 16 + 4 * g + i >= P) continue;
-#pragma unroll
-            for (int ct = 0; ct < NT2; ++ct)
-              out[(size_t)(rt * 16 + i) * 3 * H + cb[ct]] = acc[rt][ct][i] + bias[ct];
-          }
-      }
-    }
-    __syncthreads();
+  }
+  __syncthreads();
+}
+
+// The filters of several blocks (blockIdx.y) in one launch, the forward from e, its
+// tangent from de, or (WHAT = 2) both, the tangent of a tile behind its forward: the
+// activations it needs are still in the L2, and a launch of all blocks leaves one
+// last round of part-filled CUs instead of two per block (50000 pairs: 1.5 rounds of
+// two blocks per CU).  64 molecules, three blocks at H = 128: 368 us in six launches,
+// 287 us in one; two blocks at H = 32: 147 and 111 us.  The messages then read the
+// filters from further away (70 -> 77 us a block).  Bound by the matrix cores and
+// the stores by turns: 2 blocks per CU do not fully overlap a tile's phases.
+template <int H, int TM, int WHAT>
+__global__ __launch_bounds__(kTfBlock, 4) void train_filter_kernel(int P, int R, int RP,
+                                                                   const float* e,
+                                                                   const float* de,
+                                                                   FilterRows rows) {
+  __shared__ __align__(16) float e_lds[TM * (kTfMaxRbf + 4)];
+  __shared__ __align__(16) uint16_t h_bf[3 * TM * (H + 8)];
+  const FilterRow& q = rows.row[blockIdx.y];
+  const int ntiles = (P + TM - 1) / TM;
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    if (WHAT != 1) train_filter_tile<H, TM, false>(tile * TM, P, R, RP, e, q, e_lds, h_bf);
+    if (WHAT != 0) train_filter_tile<H, TM, true>(tile * TM, P, R, RP, de, q, e_lds, h_bf);
   }
 }
 
@@ -447,18 +480,33 @@ __global__ void split_bf16x3_kernel(int64_t n, const float* __restrict__ src,
   }
 }
 
-template <int H, bool TAN>
-hipError_t launch_train_filter(hipStream_t s, int P, int R, int RP, const float* x,
-                               const float* w1p, const float* b1, const uint16_t* w2bf,
-                               const float* b2, const float* a_in, float* a_out, float* h_out,
-                               float* w_out) {
+template <int H, int WHAT>
+hipError_t launch_train_filter(hipStream_t s, int P, int R, int RP, const float* e,
+                               const float* de, int layers, const FilterRows& rows) {
   constexpr int TM = kTfPairs<H>;
   const int tiles = (P + TM - 1) / TM;
   // two blocks per CU fit the LDS; a few rounds of them
   const int grid = tiles < 2048 ? tiles : 2048;
-  train_filter_kernel<H, TM, TAN><<<grid, kTfBlock, 0, s>>>(P, R, RP, x, w1p, b1, w2bf, b2,
-                                                            a_in, a_out, h_out, w_out);
+  train_filter_kernel<H, TM, WHAT><<<dim3(grid, layers), kTfBlock, 0, s>>>(P, R, RP, e, de,
+                                                                           rows);
   return hipGetLastError();
+}
+
+hipError_t dispatch_train_filter(hipStream_t s, int hidden, int what, int P, int R,
+                                 const float* e, const float* de, int layers,
+                                 const FilterRows& rows) {
+  const int RP = R <= 16 ? 16 : 32;
+  switch (hidden * 4 + what) {
+#define MLFF_TF(HH, WW) \
+  case HH * 4 + WW: return launch_train_filter<HH, WW>(s, P, R, RP, e, de, layers, rows);
+#define MLFF_TF3(HH) MLFF_TF(HH, 0) MLFF_TF(HH, 1) MLFF_TF(HH, 2)
+    MLFF_TF3(32)
+    MLFF_TF3(64)
+    MLFF_TF3(128)
+#undef MLFF_TF3
+#undef MLFF_TF
+    default: return hipErrorInvalidValue;
+  }
 }
 
 template <int H, bool TAN>
@@ -587,26 +635,60 @@ int mlff_train_filter(void* stream, int tangent, int hidden, int n_pairs, int nu
     return MLFF_ERR_INVALID;
   }
   if (n_pairs == 0) return MLFF_OK;
-  const int RP = num_rbf <= 16 ? 16 : 32;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  hipError_t e;
-  switch (hidden * 2 + (tan ? 1 : 0)) {
-#define MLFF_TF(HH, TT)                                                                      \
-  case HH * 2 + TT:                                                                          \
-    e = launch_train_filter<HH, TT>(s, n_pairs, num_rbf, RP, x_dev, w1_padded_dev, b1_dev, \
-                                    w2_planes_dev, b2_dev, a_dev, a_out_dev, h_out_dev,     \
-                                    w_out_dev);                                              \
-    break;
-    MLFF_TF(32, false)
-    MLFF_TF(32, true)
-    MLFF_TF(64, false)
-    MLFF_TF(64, true)
-    MLFF_TF(128, false)
-    MLFF_TF(128, true)
-#undef MLFF_TF
-    default:
-      e = hipErrorInvalidValue;
+  FilterRows rows = {};
+  FilterRow& q = rows.row[0];
+  q.w1p = w1_padded_dev; q.b1 = b1_dev; q.w2 = w2_planes_dev; q.b2 = b2_dev;
+  if (tan) {
+    q.a = const_cast<float*>(a_dev);   // read only
+    q.da = a_out_dev; q.dh = h_out_dev; q.dw = w_out_dev;
+  } else {
+    q.a = a_out_dev; q.h = h_out_dev; q.w = w_out_dev;
   }
+  hipError_t e = dispatch_train_filter(static_cast<hipStream_t>(stream), hidden, tan, n_pairs,
+                                       num_rbf, x_dev, x_dev, 1, rows);
+  if (e != hipSuccess) {
+    set_error("%s: %s", nm, hipGetErrorString(e));
+    return MLFF_ERR_HIP;
+  }
+  return MLFF_OK;
+}
+
+int mlff_train_filters(void* stream, int hidden, int n_blocks, int n_pairs, int num_rbf,
+                       const float* e_dev, const float* de_dev, const void* const* rows) {
+  const char* nm = "mlff_train_filters";
+  if (hidden != 32 && hidden != 64 && hidden != 128) {
+    set_error("%s: hidden_dim %d not supported (32, 64, 128)", nm, hidden);
+    return MLFF_ERR_UNSUPPORTED;
+  }
+  if (n_blocks < 0 || n_blocks > kTfMaxLayers || n_pairs < 0 || num_rbf < 1 || num_rbf > 32) {
+    set_error("%s: need 0 <= n_blocks <= %d, n_pairs >= 0 and 1 <= num_rbf <= 32", nm,
+              kTfMaxLayers);
+    return MLFF_ERR_INVALID;
+  }
+  if (n_blocks == 0) return MLFF_OK;
+  const int what = de_dev ? 2 : 0;
+  FilterRows t = {};
+  bool null = !e_dev || !rows, odd = false;
+  for (int k = 0; k < n_blocks && !null; ++k) {
+    const void* const* r = rows + 10 * k;
+    for (int i = 0; i < (what ? 10 : 7); ++i) null = null || !r[i];
+    odd = odd || !aligned16(r[0]) || !aligned16(r[2]);
+    auto out = [&](int i) { return static_cast<float*>(const_cast<void*>(r[i])); };
+    t.row[k] = {static_cast<const float*>(r[0]), static_cast<const float*>(r[1]),
+                static_cast<const uint16_t*>(r[2]), static_cast<const float*>(r[3]),
+                out(4), out(5), out(6), out(7), out(8), out(9)};
+  }
+  if (null) {
+    set_error("%s: null buffer", nm);
+    return MLFF_ERR_INVALID;
+  }
+  if (odd) {
+    set_error("%s: padded W1 and the W2 planes must be 16-byte aligned", nm);
+    return MLFF_ERR_INVALID;
+  }
+  if (n_pairs == 0) return MLFF_OK;
+  hipError_t e = dispatch_train_filter(static_cast<hipStream_t>(stream), hidden, what, n_pairs,
+                                       num_rbf, e_dev, de_dev, n_blocks, t);
   if (e != hipSuccess) {
     set_error("%s: %s", nm, hipGetErrorString(e));
     return MLFF_ERR_HIP;

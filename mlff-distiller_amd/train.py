@@ -40,6 +40,7 @@ device; energies are summed in float64.
 
 from __future__ import annotations
 
+import ctypes
 import math
 import weakref
 from dataclasses import dataclass
@@ -437,6 +438,34 @@ def _filter(p: Dict[str, Tensor], pre: str, x: Tensor, a: Optional[Tensor] = Non
     return a_out, h_out, w_out
 
 
+def _filters(p: Dict[str, Tensor], L: int, e: Tensor, de: Optional[Tensor] = None):
+    """The filter MLPs of all L blocks on the basis e and, with de, their
+    tangents, in one launch (mlff_train_filters): a list of (a1, h, W) or
+    (a1, h, W, da1, dh, dW) per block, as _filter gives them."""
+    e = _dense(e)
+    de = None if de is None else _dense(de)
+    P, R = e.shape
+    H = p["interactions.0.message.rbf_to_scalar.0.weight"].shape[0]
+    got, rows, keep = [], [], []
+    for k in range(L):
+        pre = f"interactions.{k}.message.rbf_to_scalar"
+        w1p, planes, _, _ = _filter_weights(p, pre)
+        if w1p.shape[0] != H or planes.numel() != 3 * p[pre + ".2.weight"].numel():
+            raise RuntimeError("prepared filter weights do not match the layer")
+        b1, b2 = _dense(p[pre + ".0.bias"]), _dense(p[pre + ".2.bias"])
+        out = [torch.empty(P, c, dtype=torch.float32, device=e.device)
+               for c in (H, H, 3 * H) * (1 if de is None else 2)]
+        got.append(out)
+        keep += [w1p, planes, b1, b2]
+        rows += [C.ptr(t) for t in (w1p, b1, planes, b2, *out)] + [0] * (6 - len(out))
+    for at in range(0, L, 8):   # at most 8 blocks per launch
+        n = min(8, L - at)
+        table = (ctypes.c_void_p * (10 * n))(*rows[10 * at:10 * (at + n)])
+        C.check("mlff_train_filters", C.lib().mlff_train_filters(
+            C.stream_handle(), H, n, P, R, C.ptr(e), C.ptr(de), table))
+    return got
+
+
 def _filter_adjoint(p: Dict[str, Tensor], pre: str, gW: Tensor, a1: Tensor,
                     dgW: Optional[Tensor] = None, da1: Optional[Tensor] = None):
     """Reverse of the filter's first layer on the fused pair kernel
@@ -602,7 +631,6 @@ _WG_SPLIT: Dict[tuple, tuple] = {}   # (rows per wave, partials) by (K, M, N)
 def _wg_split(K: int, M: int, N: int):
     got = _WG_SPLIT.get((K, M, N))
     if got is None:
-        import ctypes
         rw, S = ctypes.c_int(), ctypes.c_int()
         C.check("mlff_weight_grad_split", C.lib().mlff_weight_grad_split(
             K, M, N, ctypes.byref(rw), ctypes.byref(S)))
@@ -719,14 +747,13 @@ def forward(p: Dict[str, Tensor], Z: Tensor, x: Tensor, g: PairGraph, rc: float,
     layers = []
     cache = dict(H=H, L=L, n=n, x=x, vec=vec, d=d, den=den, u=u, e=e, de=de, layers=layers,
                  Z=Z, rc=rc, lam=None)
-    t = None if lam is None else _Tangent(p, cache, lam)
+    t = None if lam is None else _Tangent(p, cache, lam, g, filters=True)
+    filters = _filters(p, L, e, None if t is None else t.geometry[2])
     for k in range(L):
-        pre = f"interactions.{k}.message.rbf_to_scalar"
-        a1, h, W = _filter(p, pre, e)
-        lay = dict(s=s, v=v, a1=a1, h=h, W=W)
+        lay = dict(zip(("a1", "h", "W", "da1", "dh", "dW"), filters[k]), s=s, v=v)
         layers.append(lay)
         if t is None:
-            s_m, v_m, _, _ = _message(g, H, s, v, W, u)
+            s_m, v_m, _, _ = _message(g, H, s, v, lay["W"], u)
         else:
             s_m, v_m = t.message(k, g)
         # PaiNNUpdate.forward (student_model.py:430-470)
@@ -751,25 +778,26 @@ class _Tangent:
     """Tangent of the forward pass along the position direction lam [N,3], block
     by block behind the primal pass of each; stored in the cache."""
 
-    def __init__(self, p: Dict[str, Tensor], c: dict, lam: Tensor):
-        self.p, self.c, self.lam = p, c, lam
-        self.geometry = None
+    def __init__(self, p: Dict[str, Tensor], c: dict, lam: Tensor, g: PairGraph,
+                 filters: bool = False):
+        self.p, self.c, self.lam, self.filters = p, c, lam, filters
+        self.geometry = _geometry(g, c["x"], p["rbf.centers"], p["rbf.widths"], c["rc"],
+                                  lam.to(torch.float32))
+        f = lambda *shape: torch.zeros(*shape, dtype=torch.float32, device=c["x"].device)
+        self.ds, self.dv = f(c["n"], c["H"]), f(c["n"], 3, c["H"])
 
     def message(self, k: int, g: PairGraph):
-        """Block k's filters and message outputs; returns the primal outputs."""
+        """Block k's message outputs (and its filters' tangent, unless ``filters``:
+        formed with the primal ones); returns the primal outputs."""
         p, c, H = self.p, self.c, self.c["H"]
-        if self.geometry is None:
-            self.geometry = _geometry(g, c["x"], p["rbf.centers"], p["rbf.widths"], c["rc"],
-                                      self.lam.to(torch.float32))
-            f = lambda *shape: torch.zeros(*shape, dtype=torch.float32, device=c["x"].device)
-            self.ds, self.dv = f(c["n"], H), f(c["n"], 3, H)
         _, du, de_t = self.geometry
         lay = c["layers"][k]
         lay["ds"], lay["dv"] = self.ds, self.dv
-        da1, dh, dW = _filter(p, f"interactions.{k}.message.rbf_to_scalar", de_t, lay["a1"])
-        lay["da1"], lay["dh"], lay["dW"] = da1, dh, dW
+        if not self.filters:
+            lay["da1"], lay["dh"], lay["dW"] = _filter(
+                p, f"interactions.{k}.message.rbf_to_scalar", de_t, lay["a1"])
         s_m, v_m, self.dsm, self.dvm = _message(g, H, lay["s"], lay["v"], lay["W"], c["u"],
-                                                self.ds, self.dv, dW, du)
+                                                self.ds, self.dv, lay["dW"], du)
         return s_m, v_m
 
     def moved(self, k: int):
@@ -789,7 +817,7 @@ class _Tangent:
 
 def tangent(p: Dict[str, Tensor], c: dict, g: PairGraph, lam: Tensor):
     """Tangent of a finished forward pass along lam [N,3], stored in the cache."""
-    t = _Tangent(p, c, lam)
+    t = _Tangent(p, c, lam, g)
     for k in range(c["L"]):
         t.message(k, g)
         lay = c["layers"][k]

@@ -329,3 +329,49 @@ def test_partial_sums_are_added_in_chunks_of_eight(gpu, S):
                 chunk = chunk + row
             total = chunk if total is None else total + chunk
         assert torch.equal(o.cpu(), total)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,R,P,L", [(128, 20, 2050, 3), (128, 32, 63, 1), (64, 16, 1000, 2),
+                                     (32, 16, 4099, 9), (32, 20, 1, 2)])
+def test_filters_of_all_blocks_equal_single_launches(gpu, H, R, P, L):
+    """The filters of all blocks in one launch, with and without their tangents,
+    have the bits of one launch each (more blocks than one launch takes, ragged
+    tiles, one pair)."""
+    print(f"[case] train_filters H={H} R={R} P={P} L={L}", flush=True)
+    g = torch.Generator().manual_seed(H + R + P + L)
+    p = {}
+    for k in range(L):
+        pre = f"interactions.{k}.message.rbf_to_scalar"
+        p[pre + ".0.weight"] = (torch.randn(H, R, generator=g) / R ** 0.5).to(gpu)
+        p[pre + ".0.bias"] = (0.1 * torch.randn(H, generator=g)).to(gpu)
+        p[pre + ".2.weight"] = (torch.randn(3 * H, H, generator=g) / H ** 0.5).to(gpu)
+        p[pre + ".2.bias"] = (0.1 * torch.randn(3 * H, generator=g)).to(gpu)
+    e, de = torch.rand(P, R, generator=g).to(gpu), torch.randn(P, R, generator=g).to(gpu)
+    both, alone = train._filters(p, L, e, de), train._filters(p, L, e)
+    for k in range(L):
+        pre = f"interactions.{k}.message.rbf_to_scalar"
+        want = train._filter(p, pre, e)
+        want += train._filter(p, pre, de, want[0])
+        assert all(torch.equal(x, y) for x, y in zip(both[k], want)) and len(both[k]) == 6
+        assert all(torch.equal(x, y) for x, y in zip(alone[k], want)) and len(alone[k]) == 3
+
+
+def test_filters_of_all_blocks_refuse_bad_calls():
+    import ctypes
+    lib = train.C.lib()
+    f = 4096
+    table = lambda *r: (ctypes.c_void_p * len(r))(*r)
+    ok, fwd = table(*[f] * 10), table(*[f] * 7 + [0] * 3)
+    call = lambda H, n, P, R, e, de, t: lib.mlff_train_filters(None, H, n, P, R, e, de, t)
+    assert call(48, 1, 10, 20, f, f, ok) == -2
+    assert call(128, 9, 10, 20, f, f, ok) == -1
+    assert call(128, -1, 10, 20, f, f, ok) == -1
+    assert call(128, 1, -1, 20, f, f, ok) == -1
+    assert call(128, 1, 10, 33, f, f, ok) == -1
+    assert call(128, 1, 10, 20, None, f, ok) == -1
+    assert call(128, 1, 10, 20, f, f, None) == -1
+    assert call(128, 1, 10, 20, f, f, fwd) == -1                       # no tangent outputs
+    assert call(128, 1, 10, 20, f, None, table(f + 4, *[f] * 6, 0, 0, 0)) == -1
+    assert call(128, 0, 10, 20, f, f, None) == 0
+    assert call(128, 1, 0, 20, f, None, fwd) == 0
