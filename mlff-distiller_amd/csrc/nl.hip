@@ -14,7 +14,8 @@
 //           {p_hi - p_lo (+ shift @ cell), d}
 //   link  : per atom (one wave), edges with j < i find their pair in row j
 //           by binary search among row j's sorted upper neighbours.
-// Small lists: count, then fill with scan and link in it (nl_fill_small_kernel).
+// Up to kSmallAtoms atoms: count, then a fill that scans for itself, and where no
+// cells are used links in it too (nl_fill_small_kernel).
 // Every write is guarded by the edge / pair capacity; a run that exceeds a
 // capacity sets counts[MLFF_COUNT_OVERFLOW] and never writes out of bounds.
 //

@@ -1,7 +1,8 @@
 // Elementwise parts of PaiNNUpdate (student_model.py:430-470) in the
 // force-matching training pass: the forward, its tangent along a position
 // direction, and the reverse pass with its tangent, around the update MLP's
-// two products (which run as library GEMMs between these kernels).
+// two products, which the caller runs between these kernels (train_block.hip has
+// the whole block in one launch).
 //
 // Forward of the reference block:
 //   nrm = |v|_xyz,  xin = (s, nrm),  y = MLP(xin) = (ds, g1, g2),
