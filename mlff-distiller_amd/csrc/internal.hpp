@@ -179,15 +179,18 @@ hipError_t launch_reduce(const Buffers& b, hipStream_t s, double* energy, double
                          float* atom_energy);
 
 // MD launches (md.hip).
-// counts (may be null): the step counter is advanced here; launch_vv_second
-// then writes the rows of the step before
+// counts (may be null): the step counter is advanced here, by the steps of the run;
+// launch_vv_second then writes the rows of the step `back` before it and, with turn,
+// starts the next step
 hipError_t launch_vv_first(int N, double* x, double* p, const double* inv_mass, const float* F,
-                           float* pos32, double dt, int32_t* counts, hipStream_t s);
+                           float* pos32, double dt, int32_t* counts, int advance,
+                           hipStream_t s);
 hipError_t launch_vv_second(int N, int B, const int32_t* mol_ptr, double* p,
                             const double* inv_mass, const float* F, double dt,
                             const double* epot, double* ledger, int ledger_len,
-                            const int32_t* counts, const double* x, double* fx, double* fp,
-                            float* fF, int n_frames, hipStream_t s);
+                            const int32_t* counts, int back, bool turn, double* x,
+                            float* pos32, double* fx, double* fp, float* fF, int n_frames,
+                            hipStream_t s);
 
 hipError_t launch_mts_kick(int N, double* p, const float* Fa, const float* Fb, double coef,
                            hipStream_t s);

@@ -19,51 +19,67 @@ namespace {
 __global__ void vv_first_kernel(int N, double* __restrict__ x, double* __restrict__ p,
                                 const double* __restrict__ inv_mass, const float* __restrict__ F,
                                 float* __restrict__ pos32, double dt,
-                                int32_t* __restrict__ counts) {
+                                int32_t* __restrict__ counts, int advance) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   // nothing between here and vv_second_kernel reads the step counter
-  if (i == 0 && counts != nullptr) counts[MLFF_COUNT_STEP] += 1;
+  if (i == 0 && counts != nullptr) counts[MLFF_COUNT_STEP] += advance;
   if (i >= N) return;
   const double im = inv_mass[i];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    const double pa = p[3 * i + a] + 0.5 * dt * (double)F[3 * i + a];
-    const double xa = x[3 * i + a] + dt * pa * im;
+    const double pa = fma(0.5 * dt, (double)F[3 * i + a], p[3 * i + a]);
+    const double xa = fma(dt * pa, im, x[3 * i + a]);
     p[3 * i + a] = pa;
     x[3 * i + a] = xa;
     pos32[3 * i + a] = (float)xa;
   }
 }
 
+// back: steps from this one to the counter, which was advanced at the start of the
+// step or run.  TURN: the first half of the next step too (x and pos32 written), the
+// same operations as vv_first_kernel on values still in registers (the fma of both
+// are written out, so that the bits are the same in any run length): 60 atoms,
+// 4.3 + 3.3 us in two launches.
+template <bool TURN>
 __global__ __launch_bounds__(256) void vv_second_kernel(
     int B, const int32_t* __restrict__ mol_ptr, double* __restrict__ p,
     const double* __restrict__ inv_mass, const float* __restrict__ F, double dt,
     const double* __restrict__ epot, double* __restrict__ ledger, int ledger_len,
-    const int32_t* __restrict__ counts, int N, const double* __restrict__ x,
-    double* __restrict__ fx, double* __restrict__ fp, float* __restrict__ fF, int n_frames) {
+    const int32_t* __restrict__ counts, int back, int N, double* __restrict__ x,
+    float* __restrict__ pos32, double* __restrict__ fx, double* __restrict__ fp,
+    float* __restrict__ fF, int n_frames) {
   __shared__ double sh[256];
   const int b = blockIdx.x;
   if (b >= B) return;
   const int i0 = mol_ptr[b], i1 = mol_ptr[b + 1];
-  // the counter was advanced at the start of the step
-  const int step = counts[MLFF_COUNT_STEP] - 1;
+  const int step = counts[MLFF_COUNT_STEP] - back;
   // frame row of this step (all three frame buffers are bound together)
   const size_t fbase = n_frames > 0 ? (size_t)(step % n_frames) * (size_t)N * 3 : 0;
   double ke = 0.0;
   for (int i = i0 + threadIdx.x; i < i1; i += 256) {
     double s = 0.0;
+    const double im = inv_mass[i];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const double pa = p[3 * i + a] + 0.5 * dt * (double)F[3 * i + a];
-      p[3 * i + a] = pa;
-      s += pa * pa;
+      const float f = F[3 * i + a];
+      const double pa = fma(0.5 * dt, (double)f, p[3 * i + a]);
+      s = fma(pa, pa, s);
       if (n_frames > 0) {
         fx[fbase + 3 * i + a] = x[3 * i + a];
         fp[fbase + 3 * i + a] = pa;
-        fF[fbase + 3 * i + a] = F[3 * i + a];
+        fF[fbase + 3 * i + a] = f;
+      }
+      if (TURN) {
+        const double pn = fma(0.5 * dt, (double)f, pa);
+        const double xa = fma(dt * pn, im, x[3 * i + a]);
+        p[3 * i + a] = pn;
+        x[3 * i + a] = xa;
+        pos32[3 * i + a] = (float)xa;
+      } else {
+        p[3 * i + a] = pa;
       }
     }
-    ke += 0.5 * s * inv_mass[i];
+    ke = fma(0.5 * s, im, ke);
   }
   sh[threadIdx.x] = ke;
   __syncthreads();
@@ -179,20 +195,24 @@ hipError_t launch_mts_ledger(int B, const int32_t* mol_ptr, const double* p,
 }
 
 hipError_t launch_vv_first(int N, double* x, double* p, const double* inv_mass, const float* F,
-                           float* pos32, double dt, int32_t* counts, hipStream_t s) {
+                           float* pos32, double dt, int32_t* counts, int advance,
+                           hipStream_t s) {
   if (N > 0)
-    vv_first_kernel<<<(N + 255) / 256, 256, 0, s>>>(N, x, p, inv_mass, F, pos32, dt, counts);
+    vv_first_kernel<<<(N + 255) / 256, 256, 0, s>>>(N, x, p, inv_mass, F, pos32, dt, counts,
+                                                    advance);
   return hipGetLastError();
 }
 
 hipError_t launch_vv_second(int N, int B, const int32_t* mol_ptr, double* p,
                             const double* inv_mass, const float* F, double dt,
                             const double* epot, double* ledger, int ledger_len,
-                            const int32_t* counts, const double* x, double* fx, double* fp,
-                            float* fF, int n_frames, hipStream_t s) {
+                            const int32_t* counts, int back, bool turn, double* x,
+                            float* pos32, double* fx, double* fp, float* fF, int n_frames,
+                            hipStream_t s) {
   if (B > 0)
-    vv_second_kernel<<<B, 256, 0, s>>>(B, mol_ptr, p, inv_mass, F, dt, epot, ledger, ledger_len,
-                                       counts, N, x, fx, fp, fF, n_frames);
+    (turn ? vv_second_kernel<true> : vv_second_kernel<false>)<<<B, 256, 0, s>>>(
+        B, mol_ptr, p, inv_mass, F, dt, epot, ledger, ledger_len, counts, back, N, x, pos32, fx,
+        fp, fF, n_frames);
   return hipGetLastError();
 }
 

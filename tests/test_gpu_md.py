@@ -182,3 +182,29 @@ def test_edge_count_maximum_is_kept_across_lists(gpu):
     c = plan.read_counts()
     assert int(c[C.MLFF_COUNT_EDGES]) == counts[1]
     assert int(c[C.MLFF_COUNT_EDGES_MAX]) == counts[0]
+
+
+@pytest.mark.parametrize("steps", [1, 2, 13])
+def test_turns_of_a_small_batch_keep_the_bits(gpu, steps):
+    """Up to 1,024 atoms a step's second half and the next one's first are one
+    launch: the trajectory, energies and frames of three molecules have the bits
+    they have among enough others to run the halves apart, eager and captured."""
+    note(f"turns of {steps} steps")
+    synth = pkg_mod("synth")
+    md_mod = pkg_mod("md")
+    model = _model(64, 2, 20)
+    few = synth.molecule_set(3, 10, 40, seed=8)
+    rest = synth.molecule_set(12, 100, 110, seed=9)
+    a = md_mod.BatchedNVE(model, few, seed=3, max_steps=40, record_frames=True)
+    b = md_mod.BatchedNVE(model, few + rest, seed=3, max_steps=40, record_frames=True)
+    n = a.n_atoms
+    assert n <= 1024 < b.n_atoms
+    b.p[:n] = a.p
+    for md in (a, b):
+        md.run(steps, graph=False)
+        md.run(2 * steps, graph=True, steps_per_graph=steps)
+    assert torch.equal(a.x, b.x[:n]) and torch.equal(a.p, b.p[:n])
+    for u, w in zip(a.energies(), b.energies()):
+        assert np.array_equal(u[1:], w[1:, :3])
+    for u, w in zip(a.frames(), b.frames()):
+        assert np.array_equal(u[1:], w[1:, :n])
