@@ -355,8 +355,11 @@ __device__ __forceinline__ float dot3(float a0, float a1, float a2, float b0, fl
 // (mma_tile_k4): on one set they are the largest part of an energy's error
 // (molecules with large biases: 4.7e-5 eV/atom rms with one set, 3.1e-5 with
 // two, 2.3e-5 with four, in the same time).
+// GATES: the vectors too; without, the scalars alone.  Nothing reads the last block's
+// vectors (the energy is a function of its scalars), nor its gates in the adjoint
+// (256 molecules 2032 -> 2011 us, 60 atoms 139.1 -> 137.6 us an MD step).
 // ---------------------------------------------------------------------------
-template <int H, int TM>
+template <int H, int TM, bool GATES>
 __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
     int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ s_mid,
     const float* __restrict__ v_mid, float* __restrict__ s_out, float* __restrict__ v_out,
@@ -364,7 +367,7 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
   constexpr int RT = TM / 16;
   constexpr int LDX = 2 * H + 4, LDH = H + 4;
   constexpr int CT1 = H / 16, NT1 = (CT1 + kUpdWaves - 1) / kUpdWaves;
-  constexpr int NTC = NT1, NT2 = 3 * NTC;
+  constexpr int NTC = NT1, NS = GATES ? 3 : 1, NT2 = NS * NTC;
   __shared__ __align__(16) float x_lds[TM * LDX];
   __shared__ __align__(16) float h_lds[TM * LDH];
   constexpr int PER = TM * H / kUpdBlock;   // tile elements per thread
@@ -423,23 +426,23 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
 #pragma unroll
     for (int q = 0; q < NTC; ++q)
 #pragma unroll
-      for (int sp = 0; sp < 3; ++sp) cb[sp * NTC + q] = sp * H + (wave * NTC + q) * 16;
+      for (int sp = 0; sp < NS; ++sp) cb[sp * NTC + q] = sp * H + (wave * NTC + q) * 16;
     // the epilogue's operands (biases, mixing matrix, the tile's vectors)
     // are loaded before the product, so their latency hides behind it
     const float* b2 = w + lw.u2b;
     const float* U = w + lw.mix;
     float u[9];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) u[k] = U[k];
-    float bias[NTC][3];
+    for (int k = 0; k < 9; ++k) u[k] = GATES ? U[k] : 0.f;
+    float bias[NTC][NS];
     float xv[RT][NTC][4][3];
 #pragma unroll
     for (int q = 0; q < NTC; ++q) {
       const int c = (wave * NTC + q) * 16 + r;
 #pragma unroll
-      for (int sp = 0; sp < 3; ++sp) bias[q][sp] = b2[sp * H + c];
+      for (int sp = 0; sp < NS; ++sp) bias[q][sp] = b2[sp * H + c];
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
+      for (int rt = 0; GATES && rt < RT; ++rt)
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           const int i = min(base + rt * 16 + 4 * g + k, N - 1);
@@ -460,16 +463,18 @@ __global__ __launch_bounds__(kUpdBlock) void update_fwd_kernel(
           const int m = rt * 16 + 4 * g + k, i = base + m;
           if (i >= N) continue;
           const float ds = acc[rt][q][k] + bias[q][0];
-          const float gt1 = acc[rt][NTC + q][k] + bias[q][1];
-          const float gt2 = acc[rt][2 * NTC + q][k] + bias[q][2];
           s_out[(size_t)i * H + c] = x_lds[m * LDX + c] + ds;
-          const float x0 = xv[rt][q][k][0], x1 = xv[rt][q][k][1], x2 = xv[rt][q][k][2];
-          float* vo = v_out + (size_t)i * 3 * H;
-          vo[c] = fma_(dot3(u[0], u[1], u[2], x0, x1, x2), gt2, x0 * gt1);
-          vo[H + c] = fma_(dot3(u[3], u[4], u[5], x0, x1, x2), gt2, x1 * gt1);
-          vo[2 * H + c] = fma_(dot3(u[6], u[7], u[8], x0, x1, x2), gt2, x2 * gt1);
-          g12[(size_t)i * 2 * H + c] = gt1;
-          g12[(size_t)i * 2 * H + H + c] = gt2;
+          if constexpr (GATES) {
+            const float gt1 = acc[rt][NTC + q][k] + bias[q][1];
+            const float gt2 = acc[rt][2 * NTC + q][k] + bias[q][2];
+            const float x0 = xv[rt][q][k][0], x1 = xv[rt][q][k][1], x2 = xv[rt][q][k][2];
+            float* vo = v_out + (size_t)i * 3 * H;
+            vo[c] = fma_(dot3(u[0], u[1], u[2], x0, x1, x2), gt2, x0 * gt1);
+            vo[H + c] = fma_(dot3(u[3], u[4], u[5], x0, x1, x2), gt2, x1 * gt1);
+            vo[2 * H + c] = fma_(dot3(u[6], u[7], u[8], x0, x1, x2), gt2, x2 * gt1);
+            g12[(size_t)i * 2 * H + c] = gt1;
+            g12[(size_t)i * 2 * H + H + c] = gt2;
+          }
         }
       }
   }
@@ -770,14 +775,14 @@ __global__ __launch_bounds__(kUpdBlock) void update_bwd_kernel(
 // against 13.6).  All of a wave's weights are requested first.  Same sums as the
 // whole-tile kernels, bit for bit.  Grid (16-atom tiles, H / 32).
 // ---------------------------------------------------------------------------
-template <int H>
+template <int H, bool GATES>
 __global__ __launch_bounds__(4 * H) void update_fwd_split_kernel(
     int N, const float* __restrict__ w, LayerW lw, const float* __restrict__ s_mid,
     const float* __restrict__ v_mid, float* __restrict__ s_out, float* __restrict__ v_out,
     float* __restrict__ a_upd, float* __restrict__ g12) {
   constexpr int BLK = 4 * H, WAVES = H / 16;
-  constexpr int LDX = 2 * H + 4, LDH = H + 4, LDY = 96 + 4;
-  constexpr int NT = (6 + WAVES - 1) / WAVES;    // second product: 6 column tiles, ds, g1, g2
+  constexpr int LDX = 2 * H + 4, LDH = H + 4, CT = GATES ? 6 : 2, LDY = 16 * CT + 4;
+  constexpr int NT = (CT + WAVES - 1) / WAVES;   // second product: column tiles of ds, g1, g2
   constexpr int PE = 16 * 32 / BLK;              // outputs per thread
   __shared__ __align__(16) float x_lds[16 * LDX];
   __shared__ __align__(16) float h_lds[16 * LDH];
@@ -791,7 +796,7 @@ __global__ __launch_bounds__(4 * H) void update_fwd_split_kernel(
   int col[NT];
 #pragma unroll
   for (int q = 0; q < NT; ++q) {
-    const int t = min(wave + q * WAVES, 5);
+    const int t = min(wave + q * WAVES, CT - 1);
     col[q] = t / 2 * H + slice + 16 * (t % 2);
     const int c2[1] = {col[q]};
     load_weights(w + lw.u2w, H, c2, w2[q]);
@@ -817,10 +822,10 @@ __global__ __launch_bounds__(4 * H) void update_fwd_split_kernel(
     const size_t i = min(base + e / 32, N - 1);
     sm[k] = s_mid[i * H + c];
 #pragma unroll
-    for (int x = 0; x < 3; ++x) xv[k][x] = v_mid[(i * 3 + x) * H + c];
+    for (int x = 0; x < 3; ++x) xv[k][x] = GATES ? v_mid[(i * 3 + x) * H + c] : 0.f;
   }
 #pragma unroll
-  for (int k = 0; k < 9; ++k) u[k] = (w + lw.mix)[k];
+  for (int k = 0; k < 9; ++k) u[k] = GATES ? (w + lw.mix)[k] : 0.f;
   const float b1 = (w + lw.u1b)[cb[0] + r];
   float b2[NT];
 #pragma unroll
@@ -844,7 +849,7 @@ __global__ __launch_bounds__(4 * H) void update_fwd_split_kernel(
 #pragma unroll
   for (int q = 0; q < NT; ++q) {
     const int t = wave + q * WAVES;
-    if (t >= 6) break;
+    if (t >= CT) break;
     f4 acc[1][1];
     zero_acc(acc);
     mma_regs(h_lds, LDH, w2[q], acc);
@@ -857,9 +862,10 @@ __global__ __launch_bounds__(4 * H) void update_fwd_split_kernel(
     const int e = threadIdx.x + k * BLK, m = e / 32, c = slice + e % 32, i = base + m;
     if (i >= N) continue;
     const float* y = y_lds + m * LDY + e % 32;
-    const float ds = y[0], gt1 = y[32], gt2 = y[64];
+    s_out[(size_t)i * H + c] = sm[k] + y[0];
+    if (!GATES) continue;
+    const float gt1 = y[32], gt2 = y[64];
     const float x0 = xv[k][0], x1 = xv[k][1], x2 = xv[k][2];
-    s_out[(size_t)i * H + c] = sm[k] + ds;
     float* vo = v_out + (size_t)i * 3 * H;
     vo[c] = fma_(dot3(u[0], u[1], u[2], x0, x1, x2), gt2, x0 * gt1);
     vo[H + c] = fma_(dot3(u[3], u[4], u[5], x0, x1, x2), gt2, x1 * gt1);
@@ -1473,18 +1479,21 @@ void launch_message(const Buffers& b, hipStream_t st, int l, const float* s_in, 
 // kSmallTileAtoms), 32-atom tiles above.  Same bits.
 template <int H>
 void launch_update_fwd(const Buffers& b, hipStream_t s, const LayerW& lw, const float* s_mid,
-                       const float* v_mid, float* s_out, float* v_out, float* a_upd, float* g12) {
+                       const float* v_mid, float* s_out, float* v_out, float* a_upd, float* g12,
+                       bool gates) {
   if (b.N <= kSplitAtoms) {
     const dim3 grid((b.N + 15) / 16, H / 32);
-    update_fwd_split_kernel<H><<<grid, 4 * H, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, s_out, v_out,
-                                                      a_upd, g12);
+    auto kernel = gates ? update_fwd_split_kernel<H, true> : update_fwd_split_kernel<H, false>;
+    kernel<<<grid, 4 * H, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, s_out, v_out, a_upd, g12);
   } else {
     auto run = [&](auto kernel, int tm) {
       kernel<<<(b.N + tm - 1) / tm, kUpdBlock, 0, s>>>(b.N, b.w, lw, s_mid, v_mid, s_out, v_out,
                                                        a_upd, g12);
     };
-    if (b.N <= kSmallTileAtoms) run(update_fwd_kernel<H, 16>, 16);
-    else run(update_fwd_kernel<H, 32>, 32);
+    if (b.N <= kSmallTileAtoms)
+      run(gates ? update_fwd_kernel<H, 16, true> : update_fwd_kernel<H, 16, false>, 16);
+    else
+      run(gates ? update_fwd_kernel<H, 32, true> : update_fwd_kernel<H, 32, false>, 32);
   }
 }
 
@@ -1582,7 +1591,7 @@ hipError_t forward_impl(const Buffers& b, hipStream_t s) {
     launch_message<H, true>(b, s, l, Sl, Vl, Sm, Vm);
     launch_update_fwd<H>(b, s, lw, Sm, Vm, b.S + (size_t)(l + 1) * nh(b),
                          b.V + (size_t)(l + 1) * 3 * nh(b), b.Aupd + (size_t)l * nh(b),
-                         b.G12 + (size_t)l * 2 * nh(b));
+                         b.G12 + (size_t)l * 2 * nh(b), l + 1 < b.L);
   }
   launch_readout<H>(b, s);
   if (st.err != hipSuccess) return st.err;
@@ -1645,7 +1654,8 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
     case MLFF_STAGE_UPDATE_FWD:
       launch_update_fwd<H>(b, s, lw, b.Smid + (size_t)l * nh(b), b.Vmid + (size_t)l * 3 * nh(b),
                            b.S + (size_t)(l + 1) * nh(b), b.V + (size_t)(l + 1) * 3 * nh(b),
-                           b.Aupd + (size_t)l * nh(b), b.G12 + (size_t)l * 2 * nh(b));
+                           b.Aupd + (size_t)l * nh(b), b.G12 + (size_t)l * 2 * nh(b),
+                           l + 1 < b.L);
       break;
     case MLFF_STAGE_READOUT:
       launch_readout<H>(b, s);

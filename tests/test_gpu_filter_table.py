@@ -154,3 +154,28 @@ def test_runs_of_pairs_keep_a_structures_bits(gpu, H, n):
             one = m.evaluate(Zt[at], Pt[at], np.diff(ptr)[k:k + 1], need_virial=True)
         assert torch.equal(one[0][0], e[k]) and torch.equal(one[1], f[at])
         assert torch.equal(one[2][0], v[k])
+
+
+@pytest.mark.parametrize("H", [32, 64, 128])
+@pytest.mark.parametrize("L", [1, 2])
+def test_last_block_without_its_vectors(gpu, H, L):
+    """The last block's update forms its scalars only: against the float64 model for
+    few atoms, and a structure's bits in the forms of up to 1,024, up to 4,096 and
+    more atoms."""
+    print(f"[case] last block H{H} L{L}", flush=True)
+    synth = pkg_mod("synth")
+    rng = np.random.Generator(np.random.PCG64(H + L))
+    Z, P, ptr = synth.flatten([synth.random_molecule(41, rng) for _ in range(110)])
+    torch.manual_seed(1)
+    m = pkg().StudentForceField(hidden_dim=H, num_interactions=L, num_rbf=20).to(gpu)
+    P32, sizes = P.astype(np.float32), np.diff(ptr)
+    n = int(ptr[3])
+    _check(m, Z[:n], P32[:n], sizes[:3], 5.0)
+    Zt, Pt = torch.tensor(Z, device=gpu), torch.tensor(P32, device=gpu)
+    runs = []
+    for k in (3, 40, 110):
+        for _ in range(3):     # resolve the tables
+            r = m.evaluate(Zt[:ptr[k]], Pt[:ptr[k]], sizes[:k], need_virial=True)
+        runs.append((r[0][:3], r[1][:n], r[2][:3]))
+    for r in runs[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(runs[0], r))
