@@ -385,6 +385,15 @@ int mlff_train_message_adjoint(void* stream, int hidden_dim, int n_atoms,
                                const float* dgv_dev, const float* dw_dev, float* gs_out_dev,
                                float* gv_out_dev, float* dgs_out_dev, float* dgv_out_dev);
 
+/* gs_out and, with dgs, dgs_out of it alone: where the block's input vectors are
+ * constants. */
+int mlff_train_message_adjoint_scalars(void* stream, int hidden_dim, int n_atoms,
+                                       const int32_t* row_ptr_dev, const int32_t* col_dev,
+                                       const int32_t* edge_pair_dev, const float* gs_dev,
+                                       const float* w_dev, const float* dgs_dev,
+                                       const float* dw_dev, float* gs_out_dev,
+                                       float* dgs_out_dev);
+
 /* Gradient w.r.t. each pair's filter output W_p (the backward of
  * student_model.py:351-385 into rbf_to_scalar's output): for p = (a < b),
  *   gW[p] = (gs_a s_b + gs_b s_a,  sum_x gv_a,x v_b,x + gv_b,x v_a,x,

@@ -42,7 +42,8 @@ EXPORTS = (
     "mlff_md_bind_frames", "mlff_md_init_forces", "mlff_md_run", "mlff_md_graph_run",
     "mlff_launch_stage", "mlff_plan_set_blocks", "mlff_plan_set_cell_grid", "mlff_mts_bind", "mlff_mts_init_forces",
     "mlff_mts_run", "mlff_mts_graph_run", "mlff_plan_set_streams", "mlff_energy_forces_static",
-    "mlff_train_message", "mlff_train_message_adjoint", "mlff_train_pair_grad",
+    "mlff_train_message", "mlff_train_message_adjoint", "mlff_train_message_adjoint_scalars",
+    "mlff_train_pair_grad",
     "mlff_segment_sum", "mlff_plan_set_tiles", "mlff_edge_message", "mlff_edge_grad",
     "mlff_edge_csr", "mlff_edge_index",
     "mlff_weight_grad_workspace_bytes", "mlff_weight_grad", "mlff_weight_grad_partial_count",
@@ -155,6 +156,8 @@ def _declare(lib):
     lib.mlff_mts_graph_run.argtypes = [vp, vp, ctypes.c_int, ctypes.c_int]
     lib.mlff_train_message.restype = ctypes.c_int
     lib.mlff_train_message.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 15
+    lib.mlff_train_message_adjoint_scalars.restype = ctypes.c_int
+    lib.mlff_train_message_adjoint_scalars.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 9
     lib.mlff_train_message_adjoint.restype = ctypes.c_int
     lib.mlff_train_message_adjoint.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * 13
     lib.mlff_train_pair_grad.restype = ctypes.c_int

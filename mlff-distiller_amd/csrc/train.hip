@@ -157,7 +157,10 @@ __global__ __launch_bounds__(kTrainBlock) void train_message_kernel(
 //   gv_out[i] = gv[i] + sum_e gv[j] Wv1[p]
 //   dgs_out[i] = dgs[i] + sum_e (dgs[j] Ws + gs[j] dWs)
 //   dgv_out[i] = dgv[i] + sum_e (dgv[j] Wv1 + gv[j] dWv1)
-template <int H, bool TAN>
+// VEC: the vectors' gradients too; without, gs_out and dgs_out alone (the first
+// block's vectors are zeros that nothing differentiates), a third of the reads: 56 and
+// 24 us a block with tangents, 64 molecules at H = 128.
+template <int H, bool TAN, bool VEC>
 __global__ __launch_bounds__(kTrainBlock) void train_message_adjoint_kernel(
     int N, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col,
     const int32_t* __restrict__ edge_pair, const float* __restrict__ gs,
@@ -165,7 +168,8 @@ __global__ __launch_bounds__(kTrainBlock) void train_message_adjoint_kernel(
     const float* __restrict__ dgv, const float* __restrict__ dW, float* __restrict__ gs_out,
     float* __restrict__ gv_out, float* __restrict__ dgs_out, float* __restrict__ dgv_out) {
   constexpr int G = H / 4, RPB = kTrainBlock / (G * kTrainSegs);
-  __shared__ f4 part[kTrainSegs - 1][RPB * G][TAN ? 8 : 4];   // groups 1.. sums, per (row, lane)
+  __shared__ f4 part[kTrainSegs - 1][RPB * G][VEC ? (TAN ? 8 : 4) : (TAN ? 2 : 1)];   // groups 1.. sums, per (row, lane)
+  constexpr int AD = VEC ? 4 : 1;   // the tangent's place
   const int grp = threadIdx.x / G, seg = grp % kTrainSegs;
   const int i = blockIdx.x * RPB + grp / kTrainSegs;
   const int c = 4 * (threadIdx.x % G);
@@ -178,18 +182,18 @@ __global__ __launch_bounds__(kTrainBlock) void train_message_adjoint_kernel(
     if (seg == 0) {
       as = ld4(gs + (size_t)i * H + c);
 #pragma unroll
-      for (int x = 0; x < 3; ++x) av[x] = ld4(gv + ((size_t)i * 3 + x) * H + c);
+      for (int x = 0; VEC && x < 3; ++x) av[x] = ld4(gv + ((size_t)i * 3 + x) * H + c);
       if (TAN) {
         ads = ld4(dgs + (size_t)i * H + c);
 #pragma unroll
-        for (int x = 0; x < 3; ++x) adv[x] = ld4(dgv + ((size_t)i * 3 + x) * H + c);
+        for (int x = 0; VEC && x < 3; ++x) adv[x] = ld4(dgv + ((size_t)i * 3 + x) * H + c);
       }
     }
     const int r0 = row_ptr[i], len = row_ptr[i + 1] - r0;
     e0 = r0 + len * seg / kTrainSegs;
     e1 = r0 + len * (seg + 1) / kTrainSegs;
   }
-  constexpr int U = kTrainUnroll<TAN>;
+  constexpr int U = VEC ? kTrainUnroll<TAN> : 2 * kTrainUnroll<TAN>;
   constexpr int UT = TAN ? U : 1;
   for (int e = e0; e < e1; e += U) {
     int jj[U], pp[U];
@@ -206,17 +210,17 @@ __global__ __launch_bounds__(kTrainBlock) void train_message_adjoint_kernel(
       const int j = jj[k], p = pp[k];
       const float* w = W + (size_t)p * 3 * H + c;
       ws[k] = ld4(w);
-      wv1[k] = ld4(w + H);
+      if (VEC) wv1[k] = ld4(w + H);
       gsj[k] = ld4(gs + (size_t)j * H + c);
 #pragma unroll
-      for (int x = 0; x < 3; ++x) gvj[k][x] = ld4(gv + ((size_t)j * 3 + x) * H + c);
+      for (int x = 0; VEC && x < 3; ++x) gvj[k][x] = ld4(gv + ((size_t)j * 3 + x) * H + c);
       if (TAN) {
         const float* dw = dW + (size_t)p * 3 * H + c;
         dws[k] = ld4(dw);
-        dwv1[k] = ld4(dw + H);
+        if (VEC) dwv1[k] = ld4(dw + H);
         dgsj[k] = ld4(dgs + (size_t)j * H + c);
 #pragma unroll
-        for (int x = 0; x < 3; ++x) dgvj[k][x] = ld4(dgv + ((size_t)j * 3 + x) * H + c);
+        for (int x = 0; VEC && x < 3; ++x) dgvj[k][x] = ld4(dgv + ((size_t)j * 3 + x) * H + c);
       }
     }
 #pragma unroll
@@ -224,11 +228,11 @@ __global__ __launch_bounds__(kTrainBlock) void train_message_adjoint_kernel(
       if (e + k >= e1) break;
       as += gsj[k] * ws[k];
 #pragma unroll
-      for (int x = 0; x < 3; ++x) av[x] += gvj[k][x] * wv1[k];
+      for (int x = 0; VEC && x < 3; ++x) av[x] += gvj[k][x] * wv1[k];
       if (TAN) {
         ads += dgsj[k] * ws[k] + gsj[k] * dws[k];
 #pragma unroll
-        for (int x = 0; x < 3; ++x) adv[x] += dgvj[k][x] * wv1[k] + gvj[k][x] * dwv1[k];
+        for (int x = 0; VEC && x < 3; ++x) adv[x] += dgvj[k][x] * wv1[k] + gvj[k][x] * dwv1[k];
       }
     }
   }
@@ -236,11 +240,11 @@ __global__ __launch_bounds__(kTrainBlock) void train_message_adjoint_kernel(
     f4* q = part[seg - 1][slot];
     q[0] = as;
 #pragma unroll
-    for (int x = 0; x < 3; ++x) q[1 + x] = av[x];
+    for (int x = 0; VEC && x < 3; ++x) q[1 + x] = av[x];
     if (TAN) {
-      q[TAN ? 4 : 0] = ads;
+      q[TAN ? AD : 0] = ads;
 #pragma unroll
-      for (int x = 0; x < 3; ++x) q[TAN ? 5 + x : 0] = adv[x];
+      for (int x = 0; VEC && x < 3; ++x) q[TAN ? 5 + x : 0] = adv[x];
     }
   }
   __syncthreads();
@@ -249,20 +253,20 @@ __global__ __launch_bounds__(kTrainBlock) void train_message_adjoint_kernel(
   for (int k = 0; k < kTrainSegs - 1; ++k) {
     as += part[k][slot][0];
 #pragma unroll
-    for (int x = 0; x < 3; ++x) av[x] += part[k][slot][1 + x];
+    for (int x = 0; VEC && x < 3; ++x) av[x] += part[k][slot][1 + x];
     if (TAN) {
-      ads += part[k][slot][TAN ? 4 : 0];
+      ads += part[k][slot][TAN ? AD : 0];
 #pragma unroll
-      for (int x = 0; x < 3; ++x) adv[x] += part[k][slot][TAN ? 5 + x : 0];
+      for (int x = 0; VEC && x < 3; ++x) adv[x] += part[k][slot][TAN ? 5 + x : 0];
     }
   }
   st4(gs_out + (size_t)i * H + c, as);
 #pragma unroll
-  for (int x = 0; x < 3; ++x) st4(gv_out + ((size_t)i * 3 + x) * H + c, av[x]);
+  for (int x = 0; VEC && x < 3; ++x) st4(gv_out + ((size_t)i * 3 + x) * H + c, av[x]);
   if (TAN) {
     st4(dgs_out + (size_t)i * H + c, ads);
 #pragma unroll
-    for (int x = 0; x < 3; ++x) st4(dgv_out + ((size_t)i * 3 + x) * H + c, adv[x]);
+    for (int x = 0; VEC && x < 3; ++x) st4(dgv_out + ((size_t)i * 3 + x) * H + c, adv[x]);
   }
 }
 
@@ -901,7 +905,7 @@ hipError_t message_impl(hipStream_t st, int N, const int32_t* row_ptr, const int
   return hipGetLastError();
 }
 
-template <int H>
+template <int H, bool VEC>
 hipError_t adjoint_impl(hipStream_t st, int N, const int32_t* row_ptr, const int32_t* col,
                         const int32_t* edge_pair, const float* gs, const float* gv, const float* W,
                         const float* dgs, const float* dgv, const float* dW, float* gs_out,
@@ -909,10 +913,10 @@ hipError_t adjoint_impl(hipStream_t st, int N, const int32_t* row_ptr, const int
   constexpr int RPB = kTrainBlock / (H / 4 * kTrainSegs);
   const int grid = (N + RPB - 1) / RPB;
   if (dgs)
-    train_message_adjoint_kernel<H, true><<<grid, kTrainBlock, 0, st>>>(
+    train_message_adjoint_kernel<H, true, VEC><<<grid, kTrainBlock, 0, st>>>(
         N, row_ptr, col, edge_pair, gs, gv, W, dgs, dgv, dW, gs_out, gv_out, dgs_out, dgv_out);
   else
-    train_message_adjoint_kernel<H, false><<<grid, kTrainBlock, 0, st>>>(
+    train_message_adjoint_kernel<H, false, VEC><<<grid, kTrainBlock, 0, st>>>(
         N, row_ptr, col, edge_pair, gs, gv, W, dgs, dgv, dW, gs_out, gv_out, dgs_out, dgv_out);
   return hipGetLastError();
 }
@@ -1029,9 +1033,9 @@ int mlff_train_message_adjoint(void* stream, int hidden_dim, int n_atoms,
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
   switch (hidden_dim) {
-    case 32: e = adjoint_impl<32>(st, n_atoms, row_ptr_dev, col_dev, edge_pair_dev, gs_dev, gv_dev, w_dev, dgs_dev, dgv_dev, dw_dev, gs_out_dev, gv_out_dev, dgs_out_dev, dgv_out_dev); break;
-    case 64: e = adjoint_impl<64>(st, n_atoms, row_ptr_dev, col_dev, edge_pair_dev, gs_dev, gv_dev, w_dev, dgs_dev, dgv_dev, dw_dev, gs_out_dev, gv_out_dev, dgs_out_dev, dgv_out_dev); break;
-    case 128: e = adjoint_impl<128>(st, n_atoms, row_ptr_dev, col_dev, edge_pair_dev, gs_dev, gv_dev, w_dev, dgs_dev, dgv_dev, dw_dev, gs_out_dev, gv_out_dev, dgs_out_dev, dgv_out_dev); break;
+    case 32: e = adjoint_impl<32, true>(st, n_atoms, row_ptr_dev, col_dev, edge_pair_dev, gs_dev, gv_dev, w_dev, dgs_dev, dgv_dev, dw_dev, gs_out_dev, gv_out_dev, dgs_out_dev, dgv_out_dev); break;
+    case 64: e = adjoint_impl<64, true>(st, n_atoms, row_ptr_dev, col_dev, edge_pair_dev, gs_dev, gv_dev, w_dev, dgs_dev, dgv_dev, dw_dev, gs_out_dev, gv_out_dev, dgs_out_dev, dgv_out_dev); break;
+    case 128: e = adjoint_impl<128, true>(st, n_atoms, row_ptr_dev, col_dev, edge_pair_dev, gs_dev, gv_dev, w_dev, dgs_dev, dgv_dev, dw_dev, gs_out_dev, gv_out_dev, dgs_out_dev, dgv_out_dev); break;
     default:
       set_error("mlff_train_message_adjoint: hidden_dim %d not supported (32, 64, 128)",
                 hidden_dim);
@@ -1039,6 +1043,46 @@ int mlff_train_message_adjoint(void* stream, int hidden_dim, int n_atoms,
   }
   if (e != hipSuccess) {
     set_error("mlff_train_message_adjoint: %s", hipGetErrorString(e));
+    return MLFF_ERR_HIP;
+  }
+  return MLFF_OK;
+}
+
+int mlff_train_message_adjoint_scalars(void* stream, int hidden_dim, int n_atoms,
+                                       const int32_t* row_ptr_dev, const int32_t* col_dev,
+                                       const int32_t* edge_pair_dev, const float* gs_dev,
+                                       const float* w_dev, const float* dgs_dev,
+                                       const float* dw_dev, float* gs_out_dev,
+                                       float* dgs_out_dev) {
+  const char* nm = "mlff_train_message_adjoint_scalars";
+  if (n_atoms < 0) { set_error("%s: negative size", nm); return MLFF_ERR_INVALID; }
+  if (n_atoms == 0) return MLFF_OK;
+  if (!row_ptr_dev || !col_dev || !edge_pair_dev || !gs_dev || !w_dev || !gs_out_dev ||
+      (dgs_dev && (!dw_dev || !dgs_out_dev))) {
+    set_error("%s: null pointer", nm);
+    return MLFF_ERR_INVALID;
+  }
+  if (!aligned16(gs_dev) || !aligned16(w_dev) || !aligned16(gs_out_dev) ||
+      (dgs_dev && (!aligned16(dgs_dev) || !aligned16(dw_dev) || !aligned16(dgs_out_dev)))) {
+    set_error("%s: feature buffers must be 16-byte aligned", nm);
+    return MLFF_ERR_INVALID;
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  auto run = [&](auto impl) {
+    return impl(st, n_atoms, row_ptr_dev, col_dev, edge_pair_dev, gs_dev, nullptr, w_dev, dgs_dev,
+                nullptr, dw_dev, gs_out_dev, nullptr, dgs_out_dev, nullptr);
+  };
+  hipError_t e;
+  switch (hidden_dim) {
+    case 32: e = run(adjoint_impl<32, false>); break;
+    case 64: e = run(adjoint_impl<64, false>); break;
+    case 128: e = run(adjoint_impl<128, false>); break;
+    default:
+      set_error("%s: hidden_dim %d not supported (32, 64, 128)", nm, hidden_dim);
+      return MLFF_ERR_UNSUPPORTED;
+  }
+  if (e != hipSuccess) {
+    set_error("%s: %s", nm, hipGetErrorString(e));
     return MLFF_ERR_HIP;
   }
   return MLFF_OK;

@@ -206,6 +206,20 @@ def _message_adjoint(g: PairGraph, H: int, gs, gv, W, dgs=None, dgv=None, dW=Non
     return go, gvo, dgo, dgvo
 
 
+def _message_adjoint_scalars(g: PairGraph, H: int, gs, W, dgs=None, dW=None):
+    """gs + sum gs_j Ws and, with the tangent inputs, its tangent: _message_adjoint
+    for a block whose input vectors are constants
+    (mlff_train_message_adjoint_scalars)."""
+    gs, W, dgs, dW = _dense(gs), _dense(W), dgs if dgs is None else _dense(dgs), \
+        dW if dW is None else _dense(dW)
+    go = torch.empty_like(gs)
+    dgo = None if dgs is None else torch.empty_like(gs)
+    C.check("mlff_train_message_adjoint_scalars", C.lib().mlff_train_message_adjoint_scalars(
+        C.stream_handle(), H, gs.shape[0], _p(g.row_ptr), _p(g.col), _p(g.edge_pair), _p(gs),
+        _p(W), _p(dgs), _p(dW), _p(go), _p(dgo)))
+    return go, dgo
+
+
 def _pair_grad(g: PairGraph, H: int, u, s, v, gs, gv, du=None, ds=None, dv=None, dgs=None,
                dgv=None):
     """dL/dW per pair from both endpoints and, with the tangents, its tangent
@@ -974,7 +988,10 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
             for name, ek, dek in (("rbf.centers", e_mu, de_mu), ("rbf.widths", e_w, de_w)):
                 direct(name, lambda: (wp(ge) * ek).sum(0),
                        lambda: (dge * ek + ge * dek * dd).sum(0))
-        if T:
+        if k == 0:   # the first vectors are zeros: only the scalars' gradient is used
+            gs, dgs = _message_adjoint_scalars(g, H, gs_m, W, dgs_m if T else None,
+                                               lay["dW"] if T else None)
+        elif T:
             gs, gv, dgs, dgv = _message_adjoint(g, H, gs_m, gv_m, W, dgs_m, dgv_m, lay["dW"])
         else:
             gs, gv, _, _ = _message_adjoint(g, H, gs_m, gv_m, W)

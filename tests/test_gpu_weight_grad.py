@@ -375,3 +375,47 @@ def test_filters_of_all_blocks_refuse_bad_calls():
     assert call(128, 1, 10, 20, f, None, table(f + 4, *[f] * 6, 0, 0, 0)) == -1
     assert call(128, 0, 10, 20, f, f, None) == 0
     assert call(128, 1, 0, 20, f, None, fwd) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [32, 64, 128])
+@pytest.mark.parametrize("n", [1, 9, 70])
+def test_scalar_message_adjoint_has_the_bits_of_the_full_one(gpu, H, n):
+    """The message adjoint for constant vectors gives the scalars' gradient of the
+    full one, with and without its tangent, on rows of 0 to n - 1 edges."""
+    print(f"[case] scalar message adjoint H={H} n={n}", flush=True)
+    g = torch.Generator().manual_seed(H + n)
+    near = torch.rand(n, n, generator=g) < torch.linspace(0, 1, n)[:, None]
+    near = torch.triu(near, 1)
+    lo, hi = near.nonzero(as_tuple=True)
+    pair = torch.full((n, n), -1)
+    pair[lo, hi] = pair[hi, lo] = torch.arange(len(lo))
+    rows, cols = (near | near.T).nonzero(as_tuple=True)
+    ptr = torch.zeros(n + 1, dtype=torch.int32)
+    ptr[1:] = torch.bincount(rows, minlength=n).cumsum(0)
+
+    class Graph:
+        row_ptr = ptr.to(gpu)
+        col = torch.cat([cols, torch.zeros(1, dtype=cols.dtype)]).to(torch.int32).to(gpu)
+        edge_pair = torch.cat([pair[rows, cols], torch.zeros(1, dtype=pair.dtype)]).to(
+            torch.int32).to(gpu)
+    mk = lambda *s: torch.randn(*s, generator=g).to(gpu)
+    gs, gv, dgs, dgv = mk(n, H), mk(n, 3, H), mk(n, H), mk(n, 3, H)
+    W, dW = mk(len(lo) + 1, 3 * H), mk(len(lo) + 1, 3 * H)
+    full = train._message_adjoint(Graph, H, gs, gv, W, dgs, dgv, dW)
+    got = train._message_adjoint_scalars(Graph, H, gs, W, dgs, dW)
+    alone = train._message_adjoint_scalars(Graph, H, gs, W)
+    assert torch.equal(got[0], full[0]) and torch.equal(got[1], full[2])
+    assert torch.equal(alone[0], train._message_adjoint(Graph, H, gs, gv, W)[0])
+    assert alone[1] is None
+
+
+def test_scalar_message_adjoint_refuses_bad_calls():
+    fn = train.C.lib().mlff_train_message_adjoint_scalars
+    f, odd = 4096, 4100
+    assert fn(None, 48, 5, f, f, f, f, f, f, f, f, f) == -2
+    assert fn(None, 64, -1, f, f, f, f, f, f, f, f, f) == -1
+    assert fn(None, 64, 5, f, f, f, None, f, f, f, f, f) == -1
+    assert fn(None, 64, 5, f, f, f, f, f, f, None, f, f) == -1      # a tangent without dW
+    assert fn(None, 64, 5, f, f, f, f, odd, None, None, f, None) == -1
+    assert fn(None, 64, 0, f, f, f, f, f, None, None, f, None) == 0
