@@ -85,9 +85,11 @@ def _edge_csr(src: torch.Tensor, dst: torch.Tensor, n: int, lists: int):
     i32 = lambda *shape: torch.empty(*shape, dtype=torch.int32, device=src.device)
     row_ptr, col, eid, ends = i32(lists, n + 1), i32(lists, E), i32(lists, E), i32(2, E)
     scratch, bad = i32(lists * (n + E) + 1), i32(1)
+    # named: an address does not keep a copy alive
+    src, dst = src.contiguous(), dst.contiguous()
     C.check("mlff_edge_csr", C.lib().mlff_edge_csr(
-        C.stream_handle(), E, n, lists, C.ptr(src.contiguous()), C.ptr(dst.contiguous()),
-        C.ptr(row_ptr), C.ptr(col), C.ptr(eid), C.ptr(ends), C.ptr(scratch), C.ptr(bad)))
+        C.stream_handle(), E, n, lists, C.ptr(src), C.ptr(dst), C.ptr(row_ptr), C.ptr(col),
+        C.ptr(eid), C.ptr(ends), C.ptr(scratch), C.ptr(bad)))
     if E and bad.item():
         raise ValueError("edge_index refers to atoms outside [0, num_atoms)")
     return row_ptr, col, eid, ends

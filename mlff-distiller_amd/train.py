@@ -445,10 +445,10 @@ def _filter(p: Dict[str, Tensor], pre: str, x: Tensor, a: Optional[Tensor] = Non
     tan = a is not None
     b1 = None if tan else _dense(p[pre + ".0.bias"])
     b2 = None if tan else _dense(p[pre + ".2.bias"])
+    a = _dense(a) if tan else None
     C.check("mlff_train_filter", C.lib().mlff_train_filter(
         C.stream_handle(), int(tan), H, P, R, C.ptr(x), C.ptr(w1p), C.ptr(b1), C.ptr(planes),
-        C.ptr(b2), C.ptr(_dense(a) if tan else None), C.ptr(a_out), C.ptr(h_out),
-        C.ptr(w_out)))
+        C.ptr(b2), C.ptr(a), C.ptr(a_out), C.ptr(h_out), C.ptr(w_out)))
     return a_out, h_out, w_out
 
 
@@ -494,15 +494,15 @@ def _filter_adjoint(p: Dict[str, Tensor], pre: str, gW: Tensor, a1: Tensor,
     tan = dgW is not None
     ga = torch.empty(P, H, dtype=torch.float32, device=a1.device)
     dga = torch.empty_like(ga) if tan else None
+    dgW, da1 = (_dense(dgW), _dense(da1)) if tan else (None, None)
     if H > 32:
         C.check("mlff_train_filter_adjoint_x6", C.lib().mlff_train_filter_adjoint_x6(
-            C.stream_handle(), H, P, C.ptr(gW), C.ptr(_dense(dgW) if tan else None),
-            C.ptr(planes_t), C.ptr(a1), C.ptr(_dense(da1) if tan else None), C.ptr(ga),
-            C.ptr(dga)))
+            C.stream_handle(), H, P, C.ptr(gW), C.ptr(dgW), C.ptr(planes_t), C.ptr(a1),
+            C.ptr(da1), C.ptr(ga), C.ptr(dga)))
         return ga, dga
     C.check("mlff_train_filter_adjoint", C.lib().mlff_train_filter_adjoint(
-        C.stream_handle(), int(tan), H, P, C.ptr(gW), C.ptr(_dense(dgW) if tan else None),
-        C.ptr(w2t), C.ptr(a1), C.ptr(_dense(da1) if tan else None), C.ptr(ga), C.ptr(dga)))
+        C.stream_handle(), int(tan), H, P, C.ptr(gW), C.ptr(dgW), C.ptr(w2t), C.ptr(a1),
+        C.ptr(da1), C.ptr(ga), C.ptr(dga)))
     return ga, dga
 
 
@@ -530,6 +530,8 @@ def _geometry(g: PairGraph, x: Tensor, centers: Tensor, widths: Tensor, rc: floa
     dev = x.device
     f = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=dev)
     shift = None if g.shift is None else _dense(g.shift.to(torch.float32))
+    x, centers, widths = _dense(x), _dense(centers), _dense(widths)
+    lam = None if lam is None else _dense(lam)
     if lam is None:
         outs = (f(P, 3), f(P), f(P), f(P, 3), f(P, R), f(P, R))
         ptrs = [C.ptr(t) for t in outs] + [None] * 3
@@ -537,9 +539,8 @@ def _geometry(g: PairGraph, x: Tensor, centers: Tensor, widths: Tensor, rc: floa
         outs = (f(P), f(P, 3), f(P, R))
         ptrs = [None] * 6 + [C.ptr(t) for t in outs]
     C.check("mlff_train_geometry", C.lib().mlff_train_geometry(
-        C.stream_handle(), P, R, C.ptr(_dense(x)), C.ptr(None if lam is None else _dense(lam)),
-        C.ptr(g.lo32), C.ptr(g.hi32), C.ptr(shift), C.ptr(_dense(centers)),
-        C.ptr(_dense(widths)), float(rc), EPS, *ptrs))
+        C.stream_handle(), P, R, C.ptr(x), C.ptr(lam), C.ptr(g.lo32), C.ptr(g.hi32),
+        C.ptr(shift), C.ptr(centers), C.ptr(widths), float(rc), EPS, *ptrs))
     return outs
 
 
@@ -728,11 +729,12 @@ def _xyz_outer(a, b, a1=None, b1=None, w=None, group: Optional[_WgGroup] = None,
     S = int(lib.mlff_xyz_outer_partial_count(n))
     buf = torch.empty(12 * S + 12, dtype=torch.float32, device=a.device)
     opt = lambda t: None if t is None else _dense(t)
+    a, b, a1, b1 = _dense(a), _dense(b), opt(a1), opt(b1)
     wv = None if w is None else _dense(w.to(torch.float32))
     fn = "mlff_xyz_outer_diff_partials" if diff else "mlff_xyz_outer_partials"
     C.check(fn, getattr(lib, fn)(
-        C.stream_handle(), n, H, C.ptr(_dense(a)), C.ptr(_dense(b)), C.ptr(opt(a1)),
-        C.ptr(opt(b1)), C.ptr(wv), buf.data_ptr()))
+        C.stream_handle(), n, H, C.ptr(a), C.ptr(b), C.ptr(a1), C.ptr(b1), C.ptr(wv),
+        buf.data_ptr()))
     out = buf[12 * S:]
     grp = group if group is not None else _WgGroup()
     grp.add(S, 3, buf.data_ptr(), out.data_ptr(), buf)

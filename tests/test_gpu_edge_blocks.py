@@ -70,3 +70,27 @@ def test_blocks_equal_the_module_path(gpu, H, R, n, E):
     assert not type(blk.update(ins[0], ins[1])[0].grad_fn).__name__.startswith("_UpdateBlock")
     for k, (a, b) in enumerate(zip(fused, plain)):
         assert (a - b).norm() <= 2e-5 * b.norm() + 1e-30, k
+
+
+def test_blocks_take_a_strided_edge_list(gpu):
+    """The rows of an [E, 2] list's transpose are strided: the lists, outputs and
+    gradients of the contiguous edge list, bit for bit."""
+    print("[case] strided edge list", flush=True)
+    model = pkg_mod("model")
+    gen = torch.Generator().manual_seed(2)
+    H, R, n, E = 64, 20, 50, 3000
+    pairs = torch.randint(0, n, (E, 2), generator=gen).to(gpu)
+    torch.manual_seed(3)
+    blk = model.PaiNNInteraction(H, R).to(gpu)
+    ins = [torch.randn(*sh, generator=gen).to(gpu).requires_grad_(True)
+           for sh in ((n, H), (n, 3, H), (E, R), (E, 3))]
+
+    def run(edges):
+        out = blk(ins[0], ins[1], edges, ins[2], ins[3])
+        grads = torch.autograd.grad(out[0].square().sum() + out[1].square().sum(),
+                                    ins + list(blk.parameters()))
+        return list(model._edge_csr(edges[0], edges[1], n, 2)) + list(out) + list(grads)
+
+    assert not pairs.t()[0].is_contiguous()
+    for k, (a, b) in enumerate(zip(run(pairs.t()), run(pairs.t().contiguous()))):
+        assert torch.equal(a, b), k
