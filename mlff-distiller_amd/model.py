@@ -151,7 +151,8 @@ def _fused_mlp(seq, *tensors) -> bool:
     """Whether an MLP block on ``tensors`` may run as one autograd function with
     its own weight-gradient kernels.  Everything else takes the module path:
     replaced, hooked or parametrized layers, other types, devices and empty
-    inputs, autocast, tracing, function transforms and forward-mode AD."""
+    inputs, autocast, tracing, function transforms and forward-mode AD.  The
+    layers' sizes are the caller's to check."""
     if type(seq) is not nn.Sequential or tuple(type(m) for m in seq) != _MLP_TYPES:
         return False
     m = nn.modules.module
@@ -315,8 +316,11 @@ class PaiNNUpdate(nn.Module):
         _device_f32(scalar_features, vector_features)
         H = self.hidden_dim
         n, mlp, mix = scalar_features.shape[0], self.update_mlp, self.mixing_matrix
+        # the kernel takes the layers' sizes from H: any others run as modules
         if (H in (32, 64, 128) and scalar_features.shape == (n, H) and vector_features.shape == (n, 3, H)
-                and mix.shape == (3, 3) and _fused_mlp(mlp, scalar_features, vector_features, mix)):
+                and mix.shape == (3, 3) and _fused_mlp(mlp, scalar_features, vector_features, mix)
+                and mlp[0].weight.shape == (H, 2 * H) and mlp[0].bias.shape == (H,)
+                and mlp[2].weight.shape == (3 * H, H) and mlp[2].bias.shape == (3 * H,)):
             return _UpdateBlock.apply(scalar_features, vector_features, mlp[0].weight,
                                       mlp[0].bias, mlp[2].weight, mlp[2].bias, mix)
         norms = torch.linalg.vector_norm(vector_features, dim=1)

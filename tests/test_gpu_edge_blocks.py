@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from conftest import pkg_mod
+from oracle import painn_ref as R_
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +95,41 @@ def test_blocks_take_a_strided_edge_list(gpu):
     assert not pairs.t()[0].is_contiguous()
     for k, (a, b) in enumerate(zip(run(pairs.t()), run(pairs.t().contiguous()))):
         assert torch.equal(a, b), k
+
+
+@pytest.mark.parametrize("H,K", [(32, 64), (64, 256), (64, 32), (128, 16)])
+def test_layers_of_another_width_take_the_module_path(gpu, H, K):
+    """update_mlp and rbf_to_scalar with K hidden channels: the block's outputs and
+    gradients in float64 (2e-5 of the norm, as above)."""
+    print(f"[case] other widths H{H} K{K}", flush=True)
+    nn, model = torch.nn, pkg_mod("model")
+    torch.manual_seed(7)
+    n, E, R = 30, 400, 12
+    blk = model.PaiNNInteraction(H, R).to(gpu)
+    blk.update.update_mlp = nn.Sequential(nn.Linear(2 * H, K), nn.SiLU(), nn.Linear(K, 3 * H)).to(gpu)
+    blk.message.rbf_to_scalar = nn.Sequential(nn.Linear(R, K), nn.SiLU(),
+                                              nn.Linear(K, 3 * H)).to(gpu)
+    ins = [torch.randn(*sh, device=gpu).requires_grad_(True)
+           for sh in ((n, H), (n, 3, H), (E, R), (E, 3))]
+    edges = torch.randint(0, n, (2, E), device=gpu)
+    leaves = ins + list(blk.parameters())
+    out = blk(ins[0], ins[1], edges, ins[2], ins[3])
+    got = list(out) + list(torch.autograd.grad(out[0].square().sum() + out[1].square().sum(), leaves))
+    sd = {f"interactions.0.{k}": p.detach().cpu().double().requires_grad_(True)
+          for k, p in blk.named_parameters()}
+    s, v, rbf, ev = rins = [t.detach().cpu().double().requires_grad_(True) for t in ins]
+    ei = edges.cpu()
+    want = R_.update(sd, 0, H, *R_.message(sd, 0, H, s, v, ei[0], ei[1], rbf, ev))
+    want = list(want) + list(torch.autograd.grad(
+        want[0].square().sum() + want[1].square().sum(), rins + list(sd.values())))
+    for k, (a, b) in enumerate(zip(got, want)):
+        assert (a.detach().cpu().double() - b.detach()).norm() <= 2e-5 * b.norm() + 1e-30, k
+
+
+def test_an_update_of_the_wrong_output_width_is_refused(gpu):
+    print("[case] wrong output width", flush=True)
+    nn, model = torch.nn, pkg_mod("model")
+    blk = model.PaiNNUpdate(64).to(gpu)
+    blk.update_mlp[2] = nn.Linear(64, 256).to(gpu)
+    with pytest.raises(RuntimeError):
+        blk(torch.randn(5, 64, device=gpu), torch.randn(5, 3, 64, device=gpu))
