@@ -312,10 +312,24 @@ def _update_adjoint(w, lay: dict, gs, gv, dgs=None, dgv=None):
     return out, dout
 
 
+def _fit(t: Tensor, *shape) -> Tensor:
+    """t as a dense buffer of the shape that the kernels assume: a layer with fewer
+    hidden channels is filled up with zeros, as in the weight blob.  A zero channel
+    has silu(0) = 0 and zero weights behind it, so it changes no other value."""
+    if tuple(t.shape) != shape:
+        if t.dim() != len(shape) or any(a > b for a, b in zip(t.shape, shape)):
+            raise ValueError(f"layer of shape {tuple(t.shape)} in place of {shape}")
+        pad = [q for a, b in zip(reversed(t.shape), reversed(shape)) for q in (0, b - a)]
+        t = torch.nn.functional.pad(t, pad)
+    return _dense(t)
+
+
 def _update_weights(p: Dict[str, Tensor], upre: str):
-    return tuple(_dense(p[upre + k]) for k in (".update_mlp.0.weight", ".update_mlp.0.bias",
-                                               ".update_mlp.2.weight", ".update_mlp.2.bias",
-                                               ".mixing_matrix"))
+    H = p["embedding.weight"].shape[1]
+    shapes = ((".update_mlp.0.weight", H, 2 * H), (".update_mlp.0.bias", H),
+              (".update_mlp.2.weight", 3 * H, H), (".update_mlp.2.bias", 3 * H),
+              (".mixing_matrix", 3, 3))
+    return tuple(_fit(p[upre + k], *shape) for k, *shape in shapes)
 
 
 def _readout(w, s, c: Optional[dict] = None, ds=None, primal: bool = True):
@@ -357,8 +371,10 @@ def _readout_adjoint(w, c: dict, seed, batch, T: bool):
 
 
 def _readout_weights(p: Dict[str, Tensor]):
-    return tuple(_dense(p["energy_head." + k]) for k in ("0.weight", "0.bias", "2.weight",
-                                                         "2.bias", "4.weight", "4.bias"))
+    H = p["embedding.weight"].shape[1]
+    shapes = (("0.weight", H // 2, H), ("0.bias", H // 2), ("2.weight", H // 4, H // 2),
+              ("2.bias", H // 4), ("4.weight", 1, H // 4), ("4.bias", 1))
+    return tuple(_fit(p["energy_head." + k], *shape) for k, *shape in shapes)
 
 
 def _silu_call(a, da=None, g=None, dg=None, h=False, dh=False, dga=False):
@@ -903,6 +919,9 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
         """Weight and bias gradients of a Linear with adjoint ga and input b."""
         def put(store, *a, **kw):
             gw_, gb_ = _wgrad(*a, bias=True, group=grp, short=short, **kw)
+            m, k = p[name + ".weight"].shape
+            if gw_.shape != (m, k):   # channels that the layer has not (_fit, the seeds)
+                gw_, gb_ = gw_[:m, :k], gb_[:m]
             acc(store, name + ".weight", gw_)
             acc(store, name + ".bias", gb_)
 
@@ -942,10 +961,6 @@ def reverse(p: Dict[str, Tensor], c: dict, g: PairGraph, gE: Tensor,
     linear("energy_head.4", g4, c["h4"], torch.zeros_like(g4) if T else None, d("dh4"), w_atom)
     linear("energy_head.2", gr2, c["h3"], dgr2, d("dh3"), w_atom)
     linear("energy_head.0", gr1, c["sL"], dgr1, d("dsL"), w_atom)
-    for store in (grads, tg):
-        for k, rows in (("energy_head.4.weight", slice(0, 1)), ("energy_head.4.bias", slice(0, 1))):
-            if k in store:
-                store[k] = store[k][rows]
     gv = torch.zeros(n, 3, H, dtype=torch.float32, device=dev)
     if T:
         dgv = torch.zeros_like(gv)

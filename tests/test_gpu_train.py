@@ -362,3 +362,41 @@ def test_pair_graph_from_the_neighbour_kernels_equals_the_csr_form(gpu):
         a, b = getattr(g, name), getattr(ref, name)
         assert a.dtype == b.dtype and torch.equal(a, b), name
     assert g.shift is None and g.n_structures == ref.n_structures
+
+
+@pytest.mark.parametrize("H,K,K1,K2", [(32, 24, 12, 4), (64, 64, 32, 8), (128, 20, 64, 32)])
+def test_training_of_narrower_layers(gpu, H, K, K1, K2):
+    """update_mlp and energy_head with fewer hidden channels than the model's own
+    layers: the trainer's loss and gradients against float64 autograd, and through
+    the autograd interface."""
+    note(f"narrower layers H{H}: {K}, {K1}, {K2}")
+    nn, synth = torch.nn, pkg_mod("synth")
+    torch.manual_seed(1)
+    teacher = pkg().StudentForceField(hidden_dim=32, num_interactions=2)
+    torch.manual_seed(0)
+    student = pkg().StudentForceField(hidden_dim=H, num_interactions=2)
+    for b in student.interactions:
+        b.update.update_mlp = nn.Sequential(nn.Linear(2 * H, K), nn.SiLU(), nn.Linear(K, 3 * H))
+    student.energy_head = nn.Sequential(nn.Linear(H, K1), nn.SiLU(), nn.Linear(K1, K2), nn.SiLU(),
+                                        nn.Linear(K2, 1))
+    student = student.to(gpu)
+    Z, P, sizes, b, El, Fl = _labels({k: v.double() for k, v in teacher.state_dict().items()},
+                                     synth.molecule_set(4, 10, 30, seed=4))
+    Zt, Pt = torch.tensor(Z, device=gpu), torch.tensor(P, device=gpu)
+    El32, Fl32 = El.float().to(gpu), Fl.float().to(gpu)
+    tr = pkg_mod("train").ForceMatchingTrainer(student)
+    loss, _, _, grads = tr.loss_and_grads(Zt, Pt, sizes, El32, Fl32)
+    sd = {k: v.detach().cpu() for k, v in student.state_dict().items()}
+    loss_ref, ref = _ref_grads(sd, Z, P, b, El, Fl, 1.0, 100.0)
+    assert abs(float(loss) - loss_ref) < 1e-4 * abs(loss_ref)
+    pos = Pt.clone().requires_grad_(True)
+    E = student(Zt, pos, batch=torch.tensor(b, device=gpu))
+    F = -torch.autograd.grad(E.sum(), pos, create_graph=True)[0]
+    student.zero_grad()
+    (((E - El32) ** 2).mean() + 100.0 * ((F - Fl32) ** 2).mean()).backward()
+    shapes = {k: prm.shape for k, prm in student.named_parameters()}
+    for k in ref:
+        for g in (grads[k], dict(student.named_parameters())[k].grad):
+            assert g.shape == shapes[k]
+            rel = ((g.double().cpu() - ref[k]).norm() / (ref[k].norm() + 1e-30)).item()
+            assert rel < 2e-3, (k, rel)
