@@ -175,16 +175,24 @@ def _fused_mlp(seq, *tensors) -> bool:
                 or torch.autograd.forward_ad._current_level >= 0)
 
 
-def _plain_grads(ctx, outputs, inputs, grads):
+def _plain_grads(ctx, plain, inputs, grads):
     """Gradients of a block that can be differentiated again, from its plain
-    formula (create_graph)."""
+    formula (create_graph).  The formula takes views of the inputs: where one
+    input was formed from another, the gradient of that one must not pass
+    through here as well."""
+    views = [t.view_as(t) for t in inputs]
     need = [k for k, on in enumerate(ctx.needs_input_grad) if on]
-    got = torch.autograd.grad(outputs, [inputs[k] for k in need], grads, create_graph=True,
+    got = torch.autograd.grad(plain(*views), [views[k] for k in need], grads, create_graph=True,
                               allow_unused=True)
     out = [None] * len(inputs)
     for k, g in zip(need, got):
         out[k] = g
     return tuple(out)
+
+
+def _filter_plain(x, w1, b1, w2, b2):
+    F = nn.functional
+    return F.linear(F.silu(F.linear(x, w1, b1)), w2, b2)
 
 
 class _EdgeFilter(torch.autograd.Function):
@@ -205,9 +213,7 @@ class _EdgeFilter(torch.autograd.Function):
         from . import train
         x, w1, b1, w2, b2, a, h = ctx.saved_tensors
         if torch.is_grad_enabled():
-            F = nn.functional
-            return _plain_grads(ctx, F.linear(F.silu(F.linear(x, w1, b1)), w2, b2),
-                                (x, w1, b1, w2, b2), g)
+            return _plain_grads(ctx, _filter_plain, (x, w1, b1, w2, b2), g)
         need = ctx.needs_input_grad
         g = g.contiguous()
         grp = train._WgGroup()
@@ -253,8 +259,7 @@ class _UpdateBlock(torch.autograd.Function):
         from . import train
         s, v, w1, b1, w2, b2, mix, xin, a, h, y, mv = ctx.saved_tensors
         if torch.is_grad_enabled():
-            ins = (s, v, w1, b1, w2, b2, mix)
-            return _plain_grads(ctx, _update_plain(*ins), ins, (gs, gv))
+            return _plain_grads(ctx, _update_plain, (s, v, w1, b1, w2, b2, mix), (gs, gv))
         need = ctx.needs_input_grad
         w = tuple(train._dense(t) for t in (w1, b1, w2, b2, mix))
         lay = dict(v_m=train._dense(v), Mv=mv, y=y, a2=a, xin=xin)

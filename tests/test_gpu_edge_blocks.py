@@ -133,3 +133,33 @@ def test_an_update_of_the_wrong_output_width_is_refused(gpu):
     blk.update_mlp[2] = nn.Linear(64, 256).to(gpu)
     with pytest.raises(RuntimeError):
         blk(torch.randn(5, 64, device=gpu), torch.randn(5, 3, 64, device=gpu))
+
+
+def test_second_derivatives_where_one_input_depends_on_another(gpu):
+    """v = f(s), and a bias that s was formed from: the gradient of a gradient norm
+    equals the module path's (2e-5 of the norm, as above)."""
+    print("[case] dependent inputs, second derivatives", flush=True)
+    model = pkg_mod("model")
+    torch.manual_seed(8)
+    n, H, E, R = 20, 64, 200, 12
+    upd, msg = model.PaiNNUpdate(H).to(gpu), model.PaiNNMessage(H, R).to(gpu)
+    x = torch.randn(n, H, device=gpu).requires_grad_(True)
+    y = torch.randn(E, R, device=gpu).requires_grad_(True)
+
+    def run(apply):
+        s = x * torch.sigmoid(upd.update_mlp[0].bias)
+        v = torch.stack([s.sin(), s.cos(), s * s], dim=1)
+        so, vo = upd(s, v)
+        w = msg.rbf_to_scalar
+        x2 = y * w[2].bias[:R]
+        filt = apply(x2, w[0].weight, w[0].bias, w[2].weight, w[2].bias)
+        leaves = [x, y] + list(upd.parameters()) + list(w.parameters())
+        g = torch.autograd.grad(so.square().sum() + vo.square().sum() + filt.square().sum(), leaves,
+                                create_graph=True)
+        return list(g) + list(torch.autograd.grad(sum(t.square().sum() for t in g), leaves))
+
+    fused = run(model._EdgeFilter.apply)
+    upd.update_mlp.register_forward_hook(lambda *a: None)
+    plain = run(lambda t, *w: msg.rbf_to_scalar(t))
+    for k, (a, b) in enumerate(zip(fused, plain)):
+        assert (a - b).norm() <= 2e-5 * b.norm() + 1e-30, k
