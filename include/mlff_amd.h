@@ -201,10 +201,16 @@ int mlff_plan_set_cell_grid(mlff_plan* plan, const int32_t* grid_host, int n_str
 /* Rebind a bound plan to a new weight blob of the same layout (a training
  * step's updated weights) without the host synchronisation of
  * mlff_plan_bind: what the plan derives from the weights (bf16 planes and
- * distance tables of the filters) is remade by the next evaluation, on its
- * stream, which the caller orders after the blob's writes.  Drops the plan's
- * captured graphs.  (The reference's modules read their parameters in place,
- * student_model.py:585-605.) */
+ * distance tables of the filters) is remade on `stream`, ordered after the
+ * blob's writes when those are on the same stream.  Evaluations on another
+ * stream must be ordered after it by the caller.  Drops the plan's captured
+ * graphs.  (The reference's modules read their parameters in place,
+ * student_model.py:585-605.)
+ *
+ * Inside a caller's graph the remaking is part of every replay.  A caller's
+ * graph of mlff_energy_forces reads what the plan's workspace holds when it is
+ * replayed: after the blob that it was captured with has been rewritten and
+ * bound again it gives the new weights' results. */
 int mlff_plan_set_weights(mlff_plan* plan, void* stream, const float* weights_dev);
 
 /* Device pointer to the plan's int32 counts[MLFF_COUNT_SLOTS]. */

@@ -121,11 +121,12 @@ struct mlff_plan {
   int stream_dev;
   hipStream_t aux;
   hipEvent_t ev[2 * 8 + 2];
-  // filter tables: what the host knows of the guard's flag, whether the
-  // weights changed since they were made, and the evaluations since then
+  // filter tables: what the host knows of the guard's flag, the evaluations
+  // since they were made, whether a caller's graph remakes them at its replays,
+  // and whether a graph of the plan's own is being captured
   enum { kTabNone, kTabGood, kTabBad, kTabUnknown } tab_state;
-  bool tab_stale;
   int tab_runs;
+  bool tab_replayed, own_capture;
   // workspace carve-up (byte offsets); core_bytes: without the tables
   struct { int64_t off, bytes; } seg[48];
   int nseg;
@@ -271,11 +272,16 @@ bool capturing(hipStream_t s) {
   return st != hipStreamCaptureStatusNone;
 }
 
-// How the pair kernels of the next evaluation run, from what is known of the tables.
-void choose_filter_form(mlff_plan* pl) {
-  Buffers& b = pl->buf;
-  b.use_table = pl->tab_state == mlff_plan::kTabGood || pl->tab_state == mlff_plan::kTabUnknown;
-  b.gate = pl->tab_state == mlff_plan::kTabUnknown ? b.tab_bad : nullptr;
+// Make the planes and tables of the bound weights on stream s.
+hipError_t remake_filters(mlff_plan* pl, hipStream_t s) {
+  hipError_t e = prepare_filters(pl->buf, s);
+  if (e != hipSuccess) return e;
+  pl->tab_state = pl->buf.tab != nullptr ? mlff_plan::kTabUnknown : mlff_plan::kTabNone;
+  pl->tab_runs = 0;
+  // inside a caller's capture: every replay makes them again, from the weights as
+  // they are then, so nothing that the host reads of the flag stays true
+  if (capturing(s)) pl->tab_replayed = true;
+  return hipSuccess;
 }
 
 // Read the guard's flag on the host (waits for stream s).
@@ -285,31 +291,29 @@ hipError_t resolve_tables(mlff_plan* pl, hipStream_t s) {
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return e;
   pl->tab_state = bad ? mlff_plan::kTabBad : mlff_plan::kTabGood;
-  choose_filter_form(pl);
   return hipSuccess;
 }
 
-// Bring the planes and tables up to the bound weights on stream s.  They are
-// remade by the first evaluation after a weight change (a training loop over
-// changing batch shapes keeps several plans and uses one of them per step).
-// That evaluation launches both forms of the pair kernels behind the flag, so
-// nothing waits for it; when a second one follows on the same weights the
-// host reads the flag once and the idle launches go (never under capture).
-// now: read the flag at once.
-hipError_t refresh_filters(mlff_plan* pl, hipStream_t s, bool now) {
-  const bool known = pl->tab_state != mlff_plan::kTabUnknown;
-  if (!pl->tab_stale && known) return hipSuccess;
-  if (pl->tab_stale) {
-    hipError_t e = prepare_filters(pl->buf, s);
-    if (e != hipSuccess) return e;
-    pl->tab_stale = false;
-    pl->tab_runs = 0;
-    pl->tab_state = pl->buf.tab != nullptr ? mlff_plan::kTabUnknown : mlff_plan::kTabNone;
-    choose_filter_form(pl);
-    if (pl->tab_state == mlff_plan::kTabNone) return hipSuccess;
+// Choose the form of the next evaluation's pair kernels on stream s.  The first
+// evaluation of new tables launches both forms behind the flag, so nothing waits
+// for it; when a second one follows on the same weights the host reads the flag
+// once and the idle launches go (now: at once).  A caller's graph holds both forms
+// or, after tables that failed, the direct one: the caller may replay it after
+// mlff_plan_set_weights.  The plan's own graphs are dropped there and hold one form.
+hipError_t choose_filters(mlff_plan* pl, hipStream_t s, bool now) {
+  const bool caller_graph = !pl->own_capture && capturing(s);
+  if (pl->tab_state == mlff_plan::kTabUnknown && !pl->tab_replayed && !caller_graph &&
+      !pl->own_capture) {
+    if (now || pl->tab_runs > 0) {
+      hipError_t e = resolve_tables(pl, s);
+      if (e != hipSuccess) return e;
+    }
+    ++pl->tab_runs;
   }
-  if ((now || pl->tab_runs > 0) && !capturing(s)) return resolve_tables(pl, s);
-  ++pl->tab_runs;
+  Buffers& b = pl->buf;
+  b.use_table = pl->tab_state == mlff_plan::kTabGood || pl->tab_state == mlff_plan::kTabUnknown;
+  b.gate = b.use_table && (pl->tab_state == mlff_plan::kTabUnknown || caller_graph) ? b.tab_bad
+                                                                                   : nullptr;
   return hipSuccess;
 }
 
@@ -560,9 +564,10 @@ int mlff_plan_bind(mlff_plan* pl, void* ws, int64_t ws_bytes, const float* weigh
   // the weights may have just been written on another stream
   e = hipDeviceSynchronize();
   if (e == hipSuccess) {
-    pl->tab_stale = true;
-    e = refresh_filters(pl, nullptr, true);
+    pl->tab_replayed = false;
+    e = remake_filters(pl, nullptr);
   }
+  if (e == hipSuccess) e = choose_filters(pl, nullptr, true);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   if (e != hipSuccess) return hip_fail(e, "mlff_plan_bind: filter planes and tables");
   pl->bound = true;
@@ -581,9 +586,10 @@ int mlff_plan_set_weights(mlff_plan* pl, void* stream, const float* weights_dev)
     set_error("mlff_plan_set_weights: weights must be non-null and 16-byte aligned");
     return MLFF_ERR_INVALID;
   }
-  (void)stream;
   pl->buf.w = weights_dev;
-  pl->tab_stale = true;   // planes and tables follow with the next evaluation, on its stream
+  // the planes and tables follow the new weights in stream order on the caller's stream
+  hipError_t e = remake_filters(pl, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "mlff_plan_set_weights: filter planes and tables");
   // captured graphs hold the old weights
   if (pl->mts_exec) { (void)hipGraphExecDestroy(pl->mts_exec); pl->mts_exec = nullptr; }
   if (pl->mts_graph) { (void)hipGraphDestroy(pl->mts_graph); pl->mts_graph = nullptr; }
@@ -597,7 +603,7 @@ int32_t* mlff_plan_counts(mlff_plan* pl) { return (pl && pl->bound) ? pl->buf.co
 static int run_ef(mlff_plan* pl, hipStream_t s, const float* pos, double* energy, float* forces,
                   double* virial, float* atom_energy) {
   pl->nl.pos = pos;
-  hipError_t e = refresh_filters(pl, s, false);
+  hipError_t e = choose_filters(pl, s, false);
   if (e != hipSuccess) return hip_fail(e, "filter tables");
   e = launch_neighbor_list(pl->nl, s, true);
   if (e != hipSuccess) return hip_fail(e, "neighbour list");
@@ -631,7 +637,7 @@ int mlff_launch_stage(mlff_plan* pl, void* stream, int stage, int layer) {
     if (!pl->nl.pos) { set_error("mlff_launch_stage: no evaluation yet"); return MLFF_ERR_STATE; }
     e = launch_neighbor_list(pl->nl, s, true);
   } else {
-    e = refresh_filters(pl, s, true);
+    e = choose_filters(pl, s, true);
     if (e != hipSuccess) return hip_fail(e, "mlff_launch_stage: filter tables");
     e = launch_stage(pl->buf, s, stage, layer);
   }
@@ -825,11 +831,13 @@ int mlff_md_graph_run(mlff_plan* pl, void* stream, int steps_per_graph, int n_la
   if (!pl->graph_exec || pl->graph_steps != steps_per_graph) {
     if (pl->graph_exec) { (void)hipGraphExecDestroy(pl->graph_exec); pl->graph_exec = nullptr; }
     if (pl->graph) { (void)hipGraphDestroy(pl->graph); pl->graph = nullptr; }
-    hipError_t e = refresh_filters(pl, s, true);   // the graph holds one form only
+    hipError_t e = choose_filters(pl, s, true);   // the graph holds one form only
     if (e != hipSuccess) return hip_fail(e, "mlff_md_graph_run: filter tables");
     e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
+    pl->own_capture = true;
     int rc = md_steps(pl, s, steps_per_graph);
+    pl->own_capture = false;
     hipGraph_t g = nullptr;
     e = hipStreamEndCapture(s, &g);
     if (rc != MLFF_OK) { if (g) (void)hipGraphDestroy(g); return rc; }
@@ -852,7 +860,7 @@ int mlff_md_graph_run(mlff_plan* pl, void* stream, int steps_per_graph, int n_la
 // positions, same cutoff, equal capacities).
 static int run_ef_on(mlff_plan* pl, hipStream_t s, double* energy, float* forces,
                      const Buffers& src) {
-  hipError_t e = refresh_filters(pl, s, false);
+  hipError_t e = choose_filters(pl, s, false);
   if (e != hipSuccess) return hip_fail(e, "outer filter tables");
   Buffers b = pl->buf;
   b.counts = src.counts;
@@ -970,13 +978,15 @@ int mlff_mts_graph_run(mlff_plan* pl, void* stream, int outer_per_graph, int n_l
   if (!pl->mts_exec || pl->mts_graph_steps != outer_per_graph) {
     if (pl->mts_exec) { (void)hipGraphExecDestroy(pl->mts_exec); pl->mts_exec = nullptr; }
     if (pl->mts_graph) { (void)hipGraphDestroy(pl->mts_graph); pl->mts_graph = nullptr; }
-    hipError_t e = refresh_filters(pl, s, true);
-    if (e == hipSuccess) e = refresh_filters(pl->mts_inner, s, true);
+    hipError_t e = choose_filters(pl, s, true);
+    if (e == hipSuccess) e = choose_filters(pl->mts_inner, s, true);
     if (e != hipSuccess) return hip_fail(e, "mlff_mts_graph_run: filter tables");
     e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
     int rc = MLFF_OK;
+    pl->own_capture = pl->mts_inner->own_capture = true;
     for (int k = 0; k < outer_per_graph && rc == MLFF_OK; ++k) rc = mts_outer_step(pl, s, false);
+    pl->own_capture = pl->mts_inner->own_capture = false;
     hipGraph_t g = nullptr;
     e = hipStreamEndCapture(s, &g);
     if (rc != MLFF_OK) { if (g) (void)hipGraphDestroy(g); return rc; }
@@ -1121,6 +1131,7 @@ extern "C" int mlff_energy_forces_static(void* stream, const mlff_config* cfg,
   fill_i32_kernel<<<1, 64, 0, s>>>(counts_dev, MLFF_COUNT_SLOTS, 0);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, who);
-  pl.tab_stale = true;   // planes and tables of this call's weights, made by run_ef
+  e = remake_filters(&pl, s);
+  if (e != hipSuccess) return hip_fail(e, "mlff_energy_forces_static: filter planes and tables");
   return run_ef(&pl, s, pos_dev, energy_dev, forces_dev, virial_dev, atom_energy_dev);
 }

@@ -565,8 +565,6 @@ class StudentForceField(nn.Module):
             # were bound with, consistent with their split bf16 copies
             self._packed = engine.pack_weights(sd, device)
             self._packed_sig = sig
-            for entry in self._plans.values():
-                entry["plan"].set_weights(self._packed)
         return self._packed
 
     def _plan_for(self, sizes: np.ndarray, device, periodic: bool, cells, pbc,
@@ -664,6 +662,11 @@ class StudentForceField(nn.Module):
     def _launch(self, entry, pos, B, need_forces, need_virial):
         device = pos.device
         plan = entry["plan"]
+        # a training loop over changing batch shapes keeps several plans and uses one
+        # of them per step: only that one takes the new weights
+        weights = self.packed_weights(device)
+        if plan.weights is not weights:
+            plan.set_weights(weights)
         N = pos.shape[0]
         energy = torch.empty(B, dtype=torch.float64, device=device)
         forces = torch.empty(N, 3, dtype=torch.float32, device=device) if need_forces else None
@@ -685,7 +688,6 @@ class StudentForceField(nn.Module):
             return self._empty_results(sizes, device, need_forces, need_virial)
         pos = positions.detach().to(torch.float32).contiguous()
         entry = self._plan_for(sizes, device, periodic, cells, pbc, pos)
-        self.packed_weights(device)
         entry["numbers"].copy_(atomic_numbers.to(torch.int64))
         for _attempt in range(2):
             out = self._launch(entry, pos, len(sizes), need_forces, need_virial)
@@ -722,7 +724,6 @@ class StudentForceField(nn.Module):
             return done
         pos = positions.detach().to(torch.float32).contiguous()
         entry = self._plan_for(sizes, device, periodic, cells, pbc, pos)
-        self.packed_weights(device)
         entry["numbers"].copy_(atomic_numbers.to(torch.int64))
         out = self._launch(entry, pos, len(sizes), need_forces, need_virial)
         # pinned (torch caches the pages): the copy stays asynchronous

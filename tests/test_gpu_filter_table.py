@@ -179,3 +179,115 @@ def test_last_block_without_its_vectors(gpu, H, L):
         runs.append((r[0][:3], r[1][:n], r[2][:3]))
     for r in runs[1:]:
         assert all(torch.equal(a, b) for a, b in zip(runs[0], r))
+
+
+def _plans(blobs, H=64, L=2, R_=20):
+    """A batch, and for every weight blob the results of a plan bound to it."""
+    synth, engine = pkg_mod("synth"), pkg_mod("engine")
+    dev = torch.device("cuda:0")
+    Z, P, ptr = synth.flatten(synth.molecule_set(5, 10, 40, seed=4))
+    pos = torch.tensor(P.astype(np.float32), device=dev)
+    lay = engine.make_layout(np.diff(ptr), dev)
+    numbers = torch.tensor(Z, dtype=torch.int64, device=dev)
+    cap = engine.edge_capacity_bound(np.diff(ptr), False)
+    new = lambda w: engine.Plan(H, L, R_, 118, 5.0, lay, numbers, w, cap)
+    outs = lambda: (torch.empty(len(ptr) - 1, dtype=torch.float64, device=dev),
+                    torch.empty(len(Z), 3, dtype=torch.float32, device=dev))
+
+    def run(plan):
+        o = outs()
+        plan.energy_forces(pos, *o)
+        return o
+    return pos, new, outs, run, [run(new(w)) for w in blobs]
+
+
+def _blobs():
+    """Two sets of weights that the tables follow and one that they cannot."""
+    models = [_model(64, 2, 20, 5.0, bias) for bias in (0.05, 0.3, 0.3)]
+    with torch.no_grad():
+        models[2].rbf.widths.mul_(0.02)
+    return [m.packed_weights("cuda:0") for m in models]
+
+
+def _equal(a, b):
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+def _captured(plan, pos, o):
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        plan.energy_forces(pos, *o)
+    return g
+
+
+@pytest.mark.parametrize("new", [1, 2])
+def test_capture_right_after_a_weight_change(gpu, new):
+    """New weights, a capture, then eager evaluations before and between the
+    graph's replays: all with the new weights, and after another change too."""
+    note(f"capture after set_weights, blob {new}")
+    blobs = _blobs()
+    pos, make, outs, run, want = _plans(blobs)
+    plan = make(blobs[0])
+    for _ in range(3):
+        _equal(run(plan), want[0])
+    plan.set_weights(blobs[new])
+    o = outs()
+    g = _captured(plan, pos, o)
+    _equal(run(plan), want[new])
+    for _ in range(3):
+        for t in o:
+            t.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        _equal(o, want[new])
+        _equal(run(plan), want[new])
+    plan.set_weights(blobs[0])
+    for _ in range(3):
+        _equal(run(plan), want[0])
+
+
+def test_replays_follow_weights_written_in_place(gpu):
+    """A captured evaluation, its blob rewritten and bound again: replays and eager
+    evaluations give the new weights' results, with tables and without."""
+    note("replays after in-place weight changes")
+    blobs = _blobs()
+    pos, make, outs, run, want = _plans(blobs)
+    w = blobs[0].clone()
+    plan = make(w)
+    for _ in range(3):
+        _equal(run(plan), want[0])
+    o = outs()
+    g = _captured(plan, pos, o)
+    for k in (0, 1, 2, 1, 2, 0):
+        w.copy_(blobs[k])
+        plan.set_weights(w)
+        for _ in range(2):
+            for t in o:
+                t.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            _equal(o, want[k])
+            _equal(run(plan), want[k])
+
+
+def test_weights_bound_inside_a_capture(gpu):
+    """set_weights and an evaluation in one graph: every replay takes the blob as it
+    is then, and eager evaluations follow what the last replay bound."""
+    note("set_weights inside a capture")
+    blobs = _blobs()
+    pos, make, outs, run, want = _plans(blobs)
+    w = blobs[0].clone()
+    plan = make(w)
+    run(plan)
+    o = outs()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        plan.set_weights(w)
+        plan.energy_forces(pos, *o)
+    for k in (0, 1, 2, 1, 0):
+        w.copy_(blobs[k])
+        g.replay()
+        torch.cuda.synchronize()
+        _equal(o, want[k])
+        for _ in range(3):
+            _equal(run(plan), want[k])
