@@ -116,6 +116,8 @@ struct mlff_plan {
   float* f_outer; float* f_inner; float* f_mix; double* e_outer; double* e_inner;
   const uint8_t* flag; float* dis_max; int n_inner;
   hipGraph_t mts_graph; hipGraphExec_t mts_exec; int mts_graph_steps;
+  // weights bound so far, and those of the inner plan that the graph was captured with
+  int64_t weights_bound, mts_weights;
   // filter stream (created at bind on the current device) and its fork/join events
   int n_streams;
   int stream_dev;
@@ -278,6 +280,7 @@ hipError_t remake_filters(mlff_plan* pl, hipStream_t s) {
   if (e != hipSuccess) return e;
   pl->tab_state = pl->buf.tab != nullptr ? mlff_plan::kTabUnknown : mlff_plan::kTabNone;
   pl->tab_runs = 0;
+  ++pl->weights_bound;
   // inside a caller's capture: every replay makes them again, from the weights as
   // they are then, so nothing that the host reads of the flag stays true
   if (capturing(s)) pl->tab_replayed = true;
@@ -975,7 +978,9 @@ int mlff_mts_graph_run(mlff_plan* pl, void* stream, int outer_per_graph, int n_l
     set_error("mlff_mts_graph_run: needs a non-default stream and positive counts");
     return MLFF_ERR_INVALID;
   }
-  if (!pl->mts_exec || pl->mts_graph_steps != outer_per_graph) {
+  // the graph holds the inner plan's launches in the form that its weights had
+  if (!pl->mts_exec || pl->mts_graph_steps != outer_per_graph ||
+      pl->mts_weights != pl->mts_inner->weights_bound) {
     if (pl->mts_exec) { (void)hipGraphExecDestroy(pl->mts_exec); pl->mts_exec = nullptr; }
     if (pl->mts_graph) { (void)hipGraphDestroy(pl->mts_graph); pl->mts_graph = nullptr; }
     hipError_t e = choose_filters(pl, s, true);
@@ -997,6 +1002,7 @@ int mlff_mts_graph_run(mlff_plan* pl, void* stream, int outer_per_graph, int n_l
     pl->mts_graph = g;
     pl->mts_exec = ge;
     pl->mts_graph_steps = outer_per_graph;
+    pl->mts_weights = pl->mts_inner->weights_bound;
   }
   for (int k = 0; k < n_launches; ++k) {
     hipError_t e = hipGraphLaunch(pl->mts_exec, s);

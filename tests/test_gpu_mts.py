@@ -156,3 +156,29 @@ def test_mts_full_seed5_workload_graph_equals_eager(gpu):
     assert torch.equal(a.x, b.x) and torch.equal(a.p, b.p)
     ea, ka = a.energies()
     assert np.array_equal(ea, b.energies()[0]) and np.isfinite(ea).all() and np.isfinite(ka).all()
+
+
+@pytest.mark.parametrize("narrow", [False, True])
+def test_graph_follows_new_inner_weights(gpu, narrow):
+    """The inner model's blob rewritten and bound again between two runs of the same
+    graph: the steps of eager runs with the same change, for weights that the filter
+    tables follow and (narrow) for some that they cannot."""
+    note(f"MTS graph, inner weights changed, narrow {narrow}")
+    synth, mts = pkg_mod("synth"), pkg_mod("mts")
+    mols = synth.molecule_set(8, 10, 60, seed=14)
+    new = _model(32, 2, 16, seed=4)
+    if narrow:
+        with torch.no_grad():
+            new.rbf.widths.mul_(0.02)
+    runs = []
+    for graph in (True, False):
+        a = mts.MTSNVE(_model(), _model(32, 2, 16, seed=3), mols, seed=7, threshold=1e9, max_outer=40)
+        a.run(10, chunk=10, graph=graph)
+        w = a.plan_fast.weights
+        w.copy_(new.packed_weights("cuda:0"))
+        a.plan_fast.set_weights(w)
+        torch.cuda.synchronize()
+        a.run(10, chunk=10, graph=graph)
+        runs.append((a.x, a.p))
+    assert torch.isfinite(runs[0][0]).all()
+    assert torch.equal(runs[0][0], runs[1][0]) and torch.equal(runs[0][1], runs[1][1])
