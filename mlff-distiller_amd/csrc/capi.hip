@@ -287,11 +287,17 @@ hipError_t remake_filters(mlff_plan* pl, hipStream_t s) {
   return hipSuccess;
 }
 
-// Read the guard's flag on the host (waits for stream s).
+// Read the guard's flag on the host (waits for stream s, which is not being
+// captured).  In the relaxed mode: the copy and the wait are refused otherwise, and
+// end the capture, while another stream is captured by this or another thread.
 hipError_t resolve_tables(mlff_plan* pl, hipStream_t s) {
   int32_t bad = 1;
-  hipError_t e = hipMemcpyAsync(&bad, pl->buf.tab_bad, 4, hipMemcpyDeviceToHost, s);
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+  if (e != hipSuccess) return e;
+  e = hipMemcpyAsync(&bad, pl->buf.tab_bad, 4, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
   if (e != hipSuccess) return e;
   pl->tab_state = bad ? mlff_plan::kTabBad : mlff_plan::kTabGood;
   return hipSuccess;

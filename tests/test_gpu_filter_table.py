@@ -291,3 +291,26 @@ def test_weights_bound_inside_a_capture(gpu):
         _equal(o, want[k])
         for _ in range(3):
             _equal(run(plan), want[k])
+
+
+def test_evaluations_beside_a_capture_of_another_stream(gpu):
+    """While one stream is being captured, evaluations on another one run (the
+    second one after a weight change is the one that reads the tables' flag)."""
+    note("evaluations beside a capture")
+    blobs = _blobs()
+    pos, make, outs, run, want = _plans(blobs)
+    plan, side = make(blobs[0]), torch.cuda.Stream()
+    x = torch.zeros(64, device=gpu)
+    plan.set_weights(blobs[1])
+    o = [outs() for _ in range(3)]
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        x.add_(1.0)
+        for q in o:
+            plan.energy_forces(pos, *q, stream=side)
+    g.replay()
+    torch.cuda.synchronize()
+    assert float(x[0]) == 1.0
+    for q in o:
+        _equal(q, want[1])
