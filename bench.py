@@ -220,6 +220,8 @@ def stage_times(md, reps=20):
     for sid, name in enumerate(STAGES):
         per_layer = sid in (1, 2, 3, 5, 6, 7)
         layers = range(L) if per_layer else [0]
+        if name == "message_bwd" and L > 1:
+            layers = range(1, L)     # a step has no use for the first block's
         tot = 0.0
         for l in layers:
             C.check("stage", lib.mlff_launch_stage(md.plan.handle, stream.cuda_stream, sid, l))

@@ -450,14 +450,15 @@ hipError_t build_tables(const Buffers& b, hipStream_t s) {
 }
 
 template <int H>
-void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1, bool embed) {
+void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1, bool embed,
+                             bool all) {
   constexpr int Q = 3 * H / 4;
   int64_t units = ((int64_t)b.pcap * Q + kTabBlock * kTabUnroll - 1) / (kTabBlock * kTabUnroll);
   if (embed) units = std::max(units, ((int64_t)b.N * (H / 4) + kTabBlock - 1) / kTabBlock);
   filter_table_fwd_kernel<H><<<dim3(table_grid(b, units), l1 - l0 + embed), kTabBlock, 0, s>>>(
       b.geom, b.counts, b.pcap, table_view(b.ts, b.tab, l0, 3 * H), b.ts.layer_floats, b.gate,
       b.Wf + (size_t)l0 * b.pcap * 3 * H, l1 - l0, b.N, b.numbers, b.w + b.mw->emb, b.S, b.V,
-      l0 == 0 && zero_vectors(b));
+      l0 == 0 && zero_vectors(b) && !all);
 }
 
 template <int H>
@@ -473,7 +474,7 @@ void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l0, int l1) {
 }
 
 #define MLFF_TABLE_INST(HH)                                                         \
-  template void launch_filter_table_fwd<HH>(const Buffers&, hipStream_t, int, int, bool); \
+  template void launch_filter_table_fwd<HH>(const Buffers&, hipStream_t, int, int, bool, bool); \
   template void launch_filter_table_bwd<HH>(const Buffers&, hipStream_t, int, int);
 MLFF_TABLE_INST(32)
 MLFF_TABLE_INST(64)

@@ -163,9 +163,11 @@ int alternative_shape(int H, int which);
 hipError_t prepare_filters(const Buffers& b, hipStream_t s);
 // Fill and check every block's table (tab_bad must be 0 before).
 hipError_t build_tables(const Buffers& b, hipStream_t s);
-// Blocks l0 ... l1 - 1 in one launch; embed: the atoms' first features too.
+// Blocks l0 ... l1 - 1 in one launch; embed: the atoms' first features too; all: the
+// columns too that the first block has no use for (zero_vectors).
 template <int H>
-void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1, bool embed);
+void launch_filter_table_fwd(const Buffers& b, hipStream_t s, int l0, int l1, bool embed,
+                             bool all = false);
 template <int H>
 void launch_filter_table_bwd(const Buffers& b, hipStream_t s, int l0, int l1);
 hipError_t launch_forward(const Buffers& b, hipStream_t s);

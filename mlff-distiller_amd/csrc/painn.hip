@@ -1669,6 +1669,8 @@ hipError_t stage_impl(const Buffers& b, hipStream_t s, int stage, int l) {
       if (direct_filters(b)) launch_filter_bwd<H>(b, s, l);
       break;
     case MLFF_STAGE_MESSAGE_BWD:
+      // no evaluation runs block 0's, so its Wv1 columns may not be there
+      if (l == 0 && zero_vectors(b)) launch_filter_table_fwd<H>(b, s, 0, 1, false, true);
       launch_message<H, false>(b, s, l, b.gS1 + (size_t)l * nh(b),
                                b.gV1 + (size_t)l * 3 * nh(b), b.gS0, b.gV0);
       break;

@@ -314,3 +314,28 @@ def test_evaluations_beside_a_capture_of_another_stream(gpu):
     assert float(x[0]) == 1.0
     for q in o:
         _equal(q, want[1])
+
+
+def test_stage_of_the_first_blocks_message_adjoint(gpu, monkeypatch):
+    """Block 0's message adjoint as a stage reads filter columns that the evaluation
+    itself does not need: in a workspace of NaN bytes, what the stage writes is
+    finite, and the same twice."""
+    note("stage: message adjoint of block 0")
+    engine, C = pkg_mod("engine"), pkg_mod("_capi")
+    empty = torch.empty
+    monkeypatch.setattr(engine.torch, "empty",
+                        lambda *a, **k: empty(*a, **k).fill_(255) if k.get("dtype") == torch.uint8
+                        else empty(*a, **k))
+    pos, make, outs, run, want = _plans([_model(64, 2, 20, 5.0).packed_weights("cuda:0")])
+    plan = make(_model(64, 2, 20, 5.0).packed_weights("cuda:0"))
+    for _ in range(3):
+        _equal(run(plan), want[0])
+    written = []
+    before = plan.workspace.view(torch.int32).clone()
+    for _ in range(2):
+        C.check("stage", C.lib().mlff_launch_stage(plan.handle, C.stream_handle(), 7, 0))
+        after = plan.workspace.view(torch.int32).clone()
+        new = after != before
+        assert new.any() and torch.isfinite(after[new].view(torch.float32)).all()
+        written.append(after)
+    assert torch.equal(*written)
