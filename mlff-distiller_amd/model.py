@@ -175,15 +175,29 @@ def _fused_mlp(seq, *tensors) -> bool:
                 or torch.autograd.forward_ad._current_level >= 0)
 
 
+def _storage(*grads) -> bool:
+    """Whether the gradients have addresses for a kernel: batches of them
+    (is_grads_batched, vectorized Jacobians) have not."""
+    try:
+        for g in grads:
+            g.data_ptr()
+    except RuntimeError:
+        return False
+    return True
+
+
 def _plain_grads(ctx, plain, inputs, grads):
-    """Gradients of a block that can be differentiated again, from its plain
-    formula (create_graph).  The formula takes views of the inputs: where one
-    input was formed from another, the gradient of that one must not pass
+    """Gradients of a block from its plain formula: where they are differentiated
+    again (create_graph) or come in batches.  The formula takes tensors of its own:
+    where one input was formed from another, the gradient of that one must not pass
     through here as well."""
-    views = [t.view_as(t) for t in inputs]
+    again = torch.is_grad_enabled()
     need = [k for k, on in enumerate(ctx.needs_input_grad) if on]
-    got = torch.autograd.grad(plain(*views), [views[k] for k in need], grads, create_graph=True,
-                              allow_unused=True)
+    with torch.enable_grad():
+        own = [t.view_as(t) if again else t.detach().requires_grad_(k in need)
+               for k, t in enumerate(inputs)]
+        got = torch.autograd.grad(plain(*own), [own[k] for k in need], grads, create_graph=again,
+                                  allow_unused=True)
     out = [None] * len(inputs)
     for k, g in zip(need, got):
         out[k] = g
@@ -212,7 +226,7 @@ class _EdgeFilter(torch.autograd.Function):
     def backward(ctx, g):
         from . import train
         x, w1, b1, w2, b2, a, h = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not _storage(g):
             return _plain_grads(ctx, _filter_plain, (x, w1, b1, w2, b2), g)
         need = ctx.needs_input_grad
         g = g.contiguous()
@@ -258,7 +272,7 @@ class _UpdateBlock(torch.autograd.Function):
     def backward(ctx, gs, gv):
         from . import train
         s, v, w1, b1, w2, b2, mix, xin, a, h, y, mv = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not _storage(gs, gv):
             return _plain_grads(ctx, _update_plain, (s, v, w1, b1, w2, b2, mix), (gs, gv))
         need = ctx.needs_input_grad
         w = tuple(train._dense(t) for t in (w1, b1, w2, b2, mix))

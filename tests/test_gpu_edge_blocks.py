@@ -163,3 +163,24 @@ def test_second_derivatives_where_one_input_depends_on_another(gpu):
     plain = run(lambda t, *w: msg.rbf_to_scalar(t))
     for k, (a, b) in enumerate(zip(fused, plain)):
         assert (a - b).norm() <= 2e-5 * b.norm() + 1e-30, k
+
+
+def test_batched_gradients(gpu):
+    """is_grads_batched and vectorized Jacobians, one gradient after the other."""
+    print("[case] batched gradients", flush=True)
+    model = pkg_mod("model")
+    torch.manual_seed(9)
+    n, H, R = 7, 32, 12
+    upd, mlp = model.PaiNNUpdate(H).to(gpu), model.PaiNNMessage(H, R).to(gpu).rbf_to_scalar
+    s = torch.randn(n, H, device=gpu).requires_grad_(True)
+    v = torch.randn(n, 3, H, device=gpu).requires_grad_(True)
+    x = torch.randn(n, R, device=gpu).requires_grad_(True)
+    filt = model._EdgeFilter.apply(x, mlp[0].weight, mlp[0].bias, mlp[2].weight, mlp[2].bias)
+    for out, leaves in ((upd(s, v), [s, v] + list(upd.parameters())),
+                        ((filt,), [x] + list(mlp.parameters()))):
+        gs = [torch.randn(4, *t.shape, device=gpu) for t in out]
+        got = torch.autograd.grad(out, leaves, gs, is_grads_batched=True, retain_graph=True)
+        for k in range(4):
+            one = torch.autograd.grad(out, leaves, [g[k] for g in gs], retain_graph=True)
+            for q, (a, b) in enumerate(zip(got, one)):
+                assert (a[k] - b).norm() <= 2e-5 * b.norm() + 1e-30, (k, q)
