@@ -151,8 +151,8 @@ def _fused_mlp(seq, *tensors) -> bool:
     """Whether an MLP block on ``tensors`` may run as one autograd function with
     its own weight-gradient kernels.  Everything else takes the module path:
     replaced, hooked or parametrized layers, other types, devices and empty
-    inputs, autocast, tracing, function transforms and forward-mode AD.  The
-    layers' sizes are the caller's to check."""
+    inputs, autocast, tracing, graph capture, function transforms and forward-mode
+    AD.  The layers' sizes are the caller's to check."""
     if type(seq) is not nn.Sequential or tuple(type(m) for m in seq) != _MLP_TYPES:
         return False
     m = nn.modules.module
@@ -170,27 +170,30 @@ def _fused_mlp(seq, *tensors) -> bool:
                 or t.dtype != torch.float32):
             return False
     return not (torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
+                or torch.cuda.is_current_stream_capturing()
                 or torch.compiler.is_compiling()
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.autograd.forward_ad._current_level >= 0)
 
 
-def _storage(*grads) -> bool:
-    """Whether the gradients have addresses for a kernel: batches of them
-    (is_grads_batched, vectorized Jacobians) have not."""
+def _kernels_take(*grads) -> bool:
+    """Whether a backward pass may run on the kernels: not where it is
+    differentiated again; nor where the gradients have no addresses, as batches of
+    them (is_grads_batched, vectorized Jacobians); nor inside a graph capture,
+    whose replays would copy the weight gradients' table of addresses from host
+    memory that is long used for something else."""
     try:
         for g in grads:
             g.data_ptr()
     except RuntimeError:
         return False
-    return True
+    return not (torch.is_grad_enabled() or torch.cuda.is_current_stream_capturing())
 
 
 def _plain_grads(ctx, plain, inputs, grads):
-    """Gradients of a block from its plain formula: where they are differentiated
-    again (create_graph) or come in batches.  The formula takes tensors of its own:
-    where one input was formed from another, the gradient of that one must not pass
-    through here as well."""
+    """Gradients of a block from its plain formula, where _kernels_take says no.  The
+    formula takes tensors of its own: where one input was formed from another, the
+    gradient of that one must not pass through here as well."""
     again = torch.is_grad_enabled()
     need = [k for k, on in enumerate(ctx.needs_input_grad) if on]
     with torch.enable_grad():
@@ -226,7 +229,7 @@ class _EdgeFilter(torch.autograd.Function):
     def backward(ctx, g):
         from . import train
         x, w1, b1, w2, b2, a, h = ctx.saved_tensors
-        if torch.is_grad_enabled() or not _storage(g):
+        if not _kernels_take(g):
             return _plain_grads(ctx, _filter_plain, (x, w1, b1, w2, b2), g)
         need = ctx.needs_input_grad
         g = g.contiguous()
@@ -272,7 +275,7 @@ class _UpdateBlock(torch.autograd.Function):
     def backward(ctx, gs, gv):
         from . import train
         s, v, w1, b1, w2, b2, mix, xin, a, h, y, mv = ctx.saved_tensors
-        if torch.is_grad_enabled() or not _storage(gs, gv):
+        if not _kernels_take(gs, gv):
             return _plain_grads(ctx, _update_plain, (s, v, w1, b1, w2, b2, mix), (gs, gv))
         need = ctx.needs_input_grad
         w = tuple(train._dense(t) for t in (w1, b1, w2, b2, mix))

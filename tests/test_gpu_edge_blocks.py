@@ -184,3 +184,41 @@ def test_batched_gradients(gpu):
             one = torch.autograd.grad(out, leaves, [g[k] for g in gs], retain_graph=True)
             for q, (a, b) in enumerate(zip(got, one)):
                 assert (a[k] - b).norm() <= 2e-5 * b.norm() + 1e-30, (k, q)
+
+
+@pytest.mark.parametrize("whole", [True, False])
+def test_captured_update_block(gpu, whole):
+    """The update block's forward and backward, or its backward alone, in a graph:
+    every replay gives the eager gradients of the inputs as they are then (2e-5 of
+    the norm, as above), with other work and other pinned memory in between."""
+    print(f"[case] captured update block, forward too: {whole}", flush=True)
+    model = pkg_mod("model")
+    torch.manual_seed(10)
+    n, H = 16, 64
+    upd = model.PaiNNUpdate(H).to(gpu)
+    s = torch.randn(n, H, device=gpu).requires_grad_(True)
+    v = torch.randn(n, 3, H, device=gpu).requires_grad_(True)
+    gs = [torch.randn(n, H, device=gpu), torch.randn(n, 3, H, device=gpu)]
+    leaves = [s, v] + list(upd.parameters())
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        for _ in range(3):
+            out = upd(s, v)
+            torch.autograd.grad(out, leaves, gs, retain_graph=True)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        if whole:
+            out = upd(s, v)
+        got = torch.autograd.grad(out, leaves, gs)
+    for k in range(4):
+        with torch.no_grad():
+            for t in gs + ([s, v] if whole else []):
+                t.normal_()
+        torch.ones(1 << 14, dtype=torch.int64, pin_memory=True)
+        g.replay()
+        torch.cuda.synchronize()
+        want = torch.autograd.grad(upd(s, v), leaves, gs)
+        for q, (a, b) in enumerate(zip(got, want)):
+            assert (a - b).norm() <= 2e-5 * b.norm() + 1e-30, (k, q)
