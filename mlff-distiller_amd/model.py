@@ -167,7 +167,7 @@ def _fused_mlp(seq, *tensors) -> bool:
         return False
     for t in (*tensors, seq[0].weight, seq[0].bias, seq[2].weight, seq[2].bias):
         if (type(t) not in (torch.Tensor, nn.Parameter) or not t.is_cuda or t.numel() == 0
-                or t.dtype != torch.float32):
+                or t.dtype != torch.float32 or t.device != tensors[0].device):
             return False
     return not (torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
                 or torch.cuda.is_current_stream_capturing()
@@ -312,13 +312,14 @@ class PaiNNMessage(nn.Module):
         """s_i + sum_{j->i} s_j Ws, v_i + sum_{j->i} (v_j Wv1 + e_ji (x) Wv2)
         with (Ws, Wv1, Wv2) = rbf_to_scalar(edge_rbf) per edge."""
         mlp = self.rbf_to_scalar
-        if edge_rbf.dim() == 2 and _fused_mlp(mlp, edge_rbf):
-            filt = _EdgeFilter.apply(edge_rbf, mlp[0].weight, mlp[0].bias, mlp[2].weight,
-                                     mlp[2].bias)
-        else:
-            filt = mlp(edge_rbf)
-        return _EdgeMessage.apply(scalar_features, vector_features, filt, edge_vector,
-                                  edge_index[0], edge_index[1])
+        with torch.cuda.device_of(scalar_features):   # kernels go to the current device
+            if edge_rbf.dim() == 2 and _fused_mlp(mlp, edge_rbf):
+                filt = _EdgeFilter.apply(edge_rbf, mlp[0].weight, mlp[0].bias, mlp[2].weight,
+                                         mlp[2].bias)
+            else:
+                filt = mlp(edge_rbf)
+            return _EdgeMessage.apply(scalar_features, vector_features, filt, edge_vector,
+                                      edge_index[0], edge_index[1])
 
 
 class PaiNNUpdate(nn.Module):
@@ -343,8 +344,9 @@ class PaiNNUpdate(nn.Module):
                 and mix.shape == (3, 3) and _fused_mlp(mlp, scalar_features, vector_features, mix)
                 and mlp[0].weight.shape == (H, 2 * H) and mlp[0].bias.shape == (H,)
                 and mlp[2].weight.shape == (3 * H, H) and mlp[2].bias.shape == (3 * H,)):
-            return _UpdateBlock.apply(scalar_features, vector_features, mlp[0].weight,
-                                      mlp[0].bias, mlp[2].weight, mlp[2].bias, mix)
+            with torch.cuda.device_of(scalar_features):   # kernels go to the current device
+                return _UpdateBlock.apply(scalar_features, vector_features, mlp[0].weight,
+                                          mlp[0].bias, mlp[2].weight, mlp[2].bias, mix)
         norms = torch.linalg.vector_norm(vector_features, dim=1)
         upd = self.update_mlp(torch.cat([scalar_features, norms], dim=-1))
         ds, g1, g2 = upd[:, :H], upd[:, H:2 * H], upd[:, 2 * H:]

@@ -222,3 +222,44 @@ def test_captured_update_block(gpu, whole):
         want = torch.autograd.grad(upd(s, v), leaves, gs)
         for q, (a, b) in enumerate(zip(got, want)):
             assert (a - b).norm() <= 2e-5 * b.norm() + 1e-30, (k, q)
+
+
+def test_blocks_run_on_their_tensors_device(gpu, monkeypatch):
+    """The blocks' kernels are launched with their tensors' device made current, as
+    torch's operations are (one device here: the guard is seen to be around them);
+    tensors of two devices are refused."""
+    print("[case] device of the blocks", flush=True)
+    model, C = pkg_mod("model"), pkg_mod("_capi")
+    H, n, E = 32, 6, 20
+    blk = model.PaiNNInteraction(H, 12).to(gpu)
+    s, v = torch.randn(n, H, device=gpu), torch.randn(n, 3, H, device=gpu)
+    inside, launches = [], []
+    guard, handle = torch.cuda.device_of, C.stream_handle
+
+    class Guard(guard):
+        def __init__(self, t):
+            super().__init__(t)
+            self.seen = t.device
+
+        def __enter__(self):
+            inside.append(self.seen)
+            return super().__enter__()
+
+        def __exit__(self, *a):
+            inside.pop()
+            return super().__exit__(*a)
+
+    def record(stream=None):
+        launches.append(list(inside))
+        return handle(stream)
+
+    monkeypatch.setattr(torch.cuda, "device_of", Guard)
+    monkeypatch.setattr(C, "stream_handle", record)
+    with torch.no_grad():
+        blk(s, v, torch.randint(0, n, (2, E), device=gpu), torch.randn(E, 12, device=gpu),
+            torch.randn(E, 3, device=gpu))
+    assert len(launches) == 3 and all(got == [s.device] for got in launches), launches
+    monkeypatch.undo()
+    blk.update.update_mlp[2].cpu()
+    with pytest.raises(RuntimeError):
+        blk.update(s, v)
