@@ -761,6 +761,7 @@ __global__ void nl_fill_kernel(const float* __restrict__ pos, int N,
     // a row longer than the LDS list: lane 0 collects in cell order, sorts by
     // neighbour index, then emits
     const int e0 = e;
+    int p1 = p + udeg;
     for_each_cell_candidate(cl, i, b, [&](int j) {
       if (j == i) return;
       float vx, vy, vz, d;
@@ -812,6 +813,13 @@ __global__ void nl_fill_kernel(const float* __restrict__ pos, int N,
         if (edge_pair != nullptr) edge_pair[k] = (p < pcap) ? p : -1;
         ++p;
       }
+    }
+    // A row that the edge capacity cuts off: the pair kernels read the pairs that
+    // were counted for it all the same, so they get a place and a distance.
+    for (p1 = min(p1, pcap); pair_lo != nullptr && p < p1; ++p) {
+      pair_lo[p] = pair_hi[p] = i;
+      if (pair_shift) pair_shift[3 * p] = pair_shift[3 * p + 1] = pair_shift[3 * p + 2] = 0;
+      store_pair(geom, unit, p, 0.f, 0.f, 0.f, 0.f);
     }
     return;
   }

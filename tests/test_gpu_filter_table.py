@@ -339,3 +339,43 @@ def test_stage_of_the_first_blocks_message_adjoint(gpu, monkeypatch):
         assert new.any() and torch.isfinite(after[new].view(torch.float32)).all()
         written.append(after)
     assert torch.equal(*written)
+
+
+@pytest.mark.parametrize("n,ecap", [(2000, 100000), (2000, 3), (4200, 400000)])
+def test_long_rows_cut_off_by_the_edge_capacity(gpu, monkeypatch, n, ecap):
+    """Rows of more than 256 neighbours from the cell list, more edges than their
+    capacity and room for every pair: the pairs of the rows that are cut off are read
+    by the pair kernels.  In a workspace of NaN bytes the overflow is flagged and the
+    results are finite; with the capacity that the counters ask for they are those
+    of a plan that was large enough."""
+    note(f"long rows cut off, {n} atoms, {ecap} edges")
+    engine, C = pkg_mod("engine"), pkg_mod("_capi")
+    empty = torch.empty
+    monkeypatch.setattr(engine.torch, "empty",
+                        lambda *a, **k: empty(*a, **k).fill_(255) if k.get("dtype") == torch.uint8
+                        else empty(*a, **k))
+    dev = torch.device("cuda:0")
+    rng = np.random.Generator(np.random.PCG64(n))
+    box = 15.1 * (n / 2000) ** (1 / 3)
+    pos = torch.tensor((rng.random((n, 3)) * box).astype(np.float32), device=dev)
+    lay = engine.make_layout([n], dev, np.eye(3)[None] * box, np.ones((1, 3)))
+    numbers = torch.ones(n, dtype=torch.int64, device=dev)
+    m = _model(32, 1, 16, 5.0)
+    edges = engine.count_edges(pos, lay, 5.0)
+    assert edges > 256 * n
+
+    def run(cap):
+        plan = engine.Plan(32, 1, 16, m.max_z, 5.0, lay, numbers, m.packed_weights(dev), cap,
+                           pair_capacity=edges // 2 + 64)
+        assert plan.cell_grid[0, 0] >= 3
+        o = (empty(1, dtype=torch.float64, device=dev), empty(n, 3, device=dev))
+        for _ in range(2):
+            plan.energy_forces(pos, *o)
+        c = plan.read_counts()
+        assert c[C.MLFF_COUNT_EDGES] == edges and bool(c[C.MLFF_COUNT_OVERFLOW]) == (cap < edges)
+        assert all(torch.isfinite(t).all() for t in o)
+        return o
+
+    run(ecap)
+    a, b = run(edges), run(edges + 1000)
+    _equal(a, b)
