@@ -129,10 +129,11 @@ struct mlff_plan {
   enum { kTabNone, kTabGood, kTabBad, kTabUnknown } tab_state;
   int tab_runs;
   bool tab_replayed, own_capture;
-  // workspace carve-up (byte offsets); core_bytes: without the tables
+  // workspace carve-up (byte offsets); core_bytes: without the tables; limit_bytes:
+  // what MLFF_STATIC_SCRATCH_BYTES bounds
   struct { int64_t off, bytes; } seg[48];
   int nseg;
-  int64_t core_bytes;
+  int64_t core_bytes, limit_bytes;
 };
 
 namespace {
@@ -195,13 +196,22 @@ void carve(mlff_plan* pl) {
   pl->buf.ts = table_shape((int)H, c.num_rbf, (int)L, c.cutoff);
   sz[S_TABBAD] = pl->buf.ts.bytes ? 4 : 0;
   sz[S_TAB] = pl->buf.ts.bytes;
-  int64_t off = 0;
+  // The static entry's limit leaves out the segments of the faster kernels (hit
+  // masks, unit vectors, split adjoint, kept cell rows, tables) and counts two rows
+  // per pair for the gradients, whatever L: a batch that was small enough without
+  // them stays so.  They lie in kStaticReserve.
+  auto padded = [](int64_t bytes) { return (bytes + 255) & ~(int64_t)255; };
+  int64_t off = 0, limit = 2 * padded(16 * P);
   for (int k = 0; k < S_COUNT_; ++k) {
     if (k == S_TAB) pl->core_bytes = off;
     pl->seg[k].off = off;
     pl->seg[k].bytes = sz[k];
-    off += (sz[k] + 255) & ~(int64_t)255;
+    off += padded(sz[k]);
+    if (k != S_MASK && k != S_UNIT && k != S_PACC && k != S_GA && k != S_HITS && k != S_TABBAD &&
+        k != S_TAB)
+      limit += padded(sz[k]);
   }
+  pl->limit_bytes = limit;
   pl->nseg = S_COUNT_;
   pl->ws_bytes = off;
 }
@@ -1026,7 +1036,13 @@ int mlff_mts_graph_run(mlff_plan* pl, void* stream, int outer_per_graph, int n_l
 
 namespace {
 
-static __device__ __align__(256) unsigned char scratch[MLFF_STATIC_SCRATCH_BYTES];
+// The reserve holds what the limit does not count (no cells here): 16 (L + 1) bytes per
+// pair less the 32 counted, against the 12 H L and more that are counted; 4 H per
+// atom against 92 H; the hit masks.  With H >= 32 and L <= 8 under 4.5 % of the limit,
+// 2 MiB and padding.
+constexpr int64_t kStaticReserve = 6ll << 20;
+static __device__ __align__(256) unsigned char scratch[MLFF_STATIC_SCRATCH_BYTES +
+                                                       kStaticReserve];
 // filter tables of the calls' weights, beside the workspace (kTableMaxBytes
 // bounds them, so every configuration that has tables fits)
 static __device__ __align__(256) unsigned char table_scratch[kTableMaxBytes];
@@ -1115,7 +1131,8 @@ extern "C" int mlff_energy_forces_static(void* stream, const mlff_config* cfg,
                         &pl.mw, nullptr, 0, nullptr);
   if (rc != MLFF_OK) return rc;
   carve(&pl);
-  if (pl.core_bytes > (int64_t)MLFF_STATIC_SCRATCH_BYTES) {
+  if (pl.limit_bytes > (int64_t)MLFF_STATIC_SCRATCH_BYTES ||
+      pl.core_bytes > (int64_t)MLFF_STATIC_SCRATCH_BYTES + kStaticReserve) {
     set_error("%s: this batch needs %lld bytes of scratch, filter tables included; the static "
               "scratch holds %lld beside the tables (use mlff_energy_forces with a workspace)",
               who, (long long)pl.ws_bytes, (long long)MLFF_STATIC_SCRATCH_BYTES);

@@ -159,6 +159,24 @@ def test_static_entry_rejects_before_touching_the_device():
     bad = C.Config(128, 3, 20, 118, 5.0, 0, 1, 10, 10, 0, 0, 0)
     assert lib.mlff_energy_forces_static(None, ctypes.byref(bad), *([fake] * 12)) == -1
 
+@pytest.mark.parametrize("H,L,R_,N,E", [
+    (128, 3, 20, 60, 27602), (128, 3, 20, 500, 22490), (128, 3, 20, 2000, 5058),
+    (32, 1, 16, 60, 293460), (32, 1, 16, 500, 287672), (32, 1, 16, 2000, 267930),
+    (64, 8, 20, 60, 20768), (64, 8, 20, 500, 16120), (64, 8, 20, 2000, 278)])
+def test_static_entry_takes_the_batches_that_its_limit_counts(H, L, R_, N, E):
+    """The largest edge capacities that 64 MiB held before the evaluation kept
+    anything beside its features, filters and gradients: accepted, and one more
+    refused (without weights, so that nothing is launched)."""
+    lib = C.lib()
+    fake = ctypes.c_void_p(1 << 20)
+
+    def refused(edges):
+        cfg = C.Config(H, L, R_, 118, 5.0, N, 1, edges, (edges + 1) // 2, 0, 0, 0)
+        rc = lib.mlff_energy_forces_static(None, ctypes.byref(cfg), None, *([fake] * 11))
+        assert rc != 0
+        return rc == -4
+    assert not refused(E) and refused(E + 1)
+
 
 @pytest.mark.parametrize("H", [32, 64, 128])
 def test_launch_shape_defaults_are_the_first_values(H):

@@ -104,3 +104,18 @@ def test_static_entry_rejects_oversized_batch(gpu):
     rc = C.lib().mlff_energy_forces_static(C.stream_handle(), ctypes.byref(cfg), *([fake] * 12))
     assert rc == -4
     assert b"static scratch" in C.lib().mlff_last_error()
+
+
+@pytest.mark.parametrize("H,L,N,ecap", [(128, 3, 500, 22490), (32, 1, 2000, 267930),
+                                        (64, 8, 500, 16120)])
+def test_static_entry_at_its_limit(gpu, monkeypatch, H, L, N, ecap):
+    """The largest capacities that the scratch takes (the batch's edges are fewer):
+    the plan's results."""
+    synth, engine = pkg_mod("synth"), pkg_mod("engine")
+    rng = np.random.Generator(np.random.PCG64(N))
+    n = N // 20
+    mols = [synth.random_molecule(20, rng) for _ in range(n)]
+    note(f"no-alloc: at the limit, H{H}/L{L}, {n} molecules")
+    # _both takes a quarter more than the count, and 64
+    monkeypatch.setattr(engine, "count_edges", lambda *a: (ecap - 63.5) / 1.25)
+    _same(*_both(_model(H, L, 20), mols))
