@@ -247,8 +247,7 @@ int mlff_energy_forces(mlff_plan* plan, void* stream, const float* pos_dev,
  * cleared by the call and receives the edge and pair counts and the overflow
  * flag of this evaluation.  The filters' bf16 planes and distance tables are
  * remade from weights_dev on every call, inside a captured graph at every
- * replay (one molecule of 12 atoms at hidden_dim 128: 212 us a call, 267 us on
- * the direct products alone that the tables replace).
+ * replay; a plan makes them once.
  * ------------------------------------------------------------------------- */
 #define MLFF_STATIC_SCRATCH_BYTES (64ll << 20)
 int mlff_energy_forces_static(void* stream, const mlff_config* cfg, const float* weights_dev,

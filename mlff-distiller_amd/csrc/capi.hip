@@ -1160,6 +1160,10 @@ extern "C" int mlff_energy_forces_static(void* stream, const mlff_config* cfg,
   fill_i32_kernel<<<1, 64, 0, s>>>(counts_dev, MLFF_COUNT_SLOTS, 0);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, who);
+  // The plan's bits need the plan's tables, also where a batch has fewer pairs than
+  // they have knots: 12 atoms, H = 128, three blocks, 2560 intervals 213 us a call
+  // against 206 us on the direct products alone (6 molecules of 10-60 atoms 242 and
+  // 225 us); two blocks of 6349 intervals (R = 32, cutoff 6.2) 253 and 144 us.
   e = remake_filters(&pl, s);
   if (e != hipSuccess) return hip_fail(e, "mlff_energy_forces_static: filter planes and tables");
   return run_ef(&pl, s, pos_dev, energy_dev, forces_dev, virial_dev, atom_energy_dev);
