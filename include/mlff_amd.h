@@ -294,6 +294,12 @@ int mlff_plan_set_blocks(mlff_plan* plan, int blocks);
 int mlff_plan_set_tiles(mlff_plan* plan, int fwd_pairs, int bwd_pairs, int msg_unroll_fwd,
                         int msg_unroll_bwd, int bwd_variant);
 
+/* Which of these five kinds the plan's launches read, as its last evaluation ran:
+ * bit k for argument k.  The filter kinds are read by the direct kernels, which do
+ * not run where the filters come from their distance tables; the message kinds
+ * above 1,024 atoms.  -1 for a null plan. */
+int mlff_plan_shapes_used(const mlff_plan* plan);
+
 /* Number of streams one evaluation uses: 1 (default) keeps every kernel on the
  * caller's stream; 2 runs the pair filter kernels on a stream of the plan's
  * own, forked from and joined back into the caller's stream with events, so

@@ -44,7 +44,7 @@ EXPORTS = (
     "mlff_mts_run", "mlff_mts_graph_run", "mlff_plan_set_streams", "mlff_energy_forces_static",
     "mlff_train_message", "mlff_train_message_adjoint", "mlff_train_message_adjoint_scalars",
     "mlff_train_pair_grad",
-    "mlff_segment_sum", "mlff_plan_set_tiles", "mlff_edge_message", "mlff_edge_grad",
+    "mlff_segment_sum", "mlff_plan_set_tiles", "mlff_plan_shapes_used", "mlff_edge_message", "mlff_edge_grad",
     "mlff_edge_csr", "mlff_edge_index",
     "mlff_weight_grad_workspace_bytes", "mlff_weight_grad", "mlff_weight_grad_partial_count",
     "mlff_weight_grad_partials", "mlff_weight_grad_diff_partials",
@@ -219,6 +219,8 @@ def _declare(lib):
         fn = getattr(lib, name)
         fn.restype = ctypes.c_int
         fn.argtypes = [vp, ctypes.c_int, ctypes.c_int] + [vp] * n_ptrs
+    lib.mlff_plan_shapes_used.restype = ctypes.c_int
+    lib.mlff_plan_shapes_used.argtypes = [vp]
     lib.mlff_plan_set_weights.restype = ctypes.c_int
     lib.mlff_plan_set_weights.argtypes = [vp, vp, vp]
     lib.mlff_train_filter.restype = ctypes.c_int

@@ -16,8 +16,10 @@ caller repeats):
 
 The grid is searched first with the default shapes, then each shape kind in
 turn is switched to its alternative and kept when the evaluation gets
-faster (coordinate descent).  The choice is remembered per (device, hidden
-size, streams, pair-count bucket).
+faster (coordinate descent).  A kind that no launch of the workload reads (the
+direct filter kernels' where the filters come from their tables, the message
+rows' on few atoms) keeps its default: its timings would be noise.  The choice is
+remembered per (device, hidden size, streams, kinds in use, pair-count bucket).
 """
 
 from __future__ import annotations
@@ -39,7 +41,8 @@ def _key(plan) -> str:
     counts = plan.read_counts()
     pairs = max(int(counts[C.MLFF_COUNT_PAIRS]), 1)
     streams = getattr(plan, "streams", 1)
-    return f"{name}|H{plan.H}|L{plan.L}|S{streams}|P2^{int(math.log2(pairs))}"
+    used = "".join(str(int(u)) for u in plan.shapes_used())
+    return f"{name}|H{plan.H}|L{plan.L}|S{streams}|K{used}|P2^{int(math.log2(pairs))}"
 
 
 def default_candidates(cus: Optional[int] = None) -> Iterable[int]:
@@ -84,7 +87,8 @@ def tune(plan, positions: torch.Tensor, candidates: Optional[Iterable[int]] = No
     B = plan.layout.n_structures
     e = torch.empty(B, dtype=torch.float64, device=positions.device)
     f = torch.empty(plan.layout.n_atoms, 3, dtype=torch.float32, device=positions.device)
-    plan.energy_forces(positions, e, f)
+    for _ in range(2):   # the second one after a weight change is the one that repeats
+        plan.energy_forces(positions, e, f)
     key = _key(plan) + ("" if shapes else "|grid")
     if cache_file and os.path.exists(cache_file):
         with open(cache_file) as fh:
@@ -110,7 +114,10 @@ def tune(plan, positions: torch.Tensor, candidates: Optional[Iterable[int]] = No
         best_us = time_evaluation(plan, positions, e, f, reps) * 1e6
         shape_timings["default"] = best_us
         shapes_h = launch_shapes(plan.H)
+        used = plan.shapes_used()
         for k, values in enumerate(shapes_h):
+            if not used[k]:
+                continue
             best_k = list(tiles)
             for v in values:
                 if v == tiles[k]:

@@ -765,6 +765,8 @@ int mlff_plan_set_tiles(mlff_plan* pl, int fwd_pairs, int bwd_pairs, int msg_unr
   return MLFF_OK;
 }
 
+int mlff_plan_shapes_used(const mlff_plan* pl) { return pl ? shapes_used(pl->buf) : -1; }
+
 int mlff_md_bind(mlff_plan* pl, double* x_dev, double* p_dev, const double* inv_mass_dev,
                  float* pos32_dev, float* forces_dev, double* energy_dev, double* ledger_dev,
                  int32_t ledger_len, double dt) {

@@ -158,6 +158,8 @@ __host__ __device__ inline int64_t wbf_elems(int H, int L) { return (int64_t)L *
 // variant number; every value up to it exists).
 int default_shape(int H, int which);
 int alternative_shape(int H, int which);
+// bit k: the launches of an evaluation read the shape of kind k
+int shapes_used(const Buffers& b);
 // What the pair kernels read beside the weight blob, remade on stream s for
 // new weights: the filters' bf16 planes and their tables with the guard's flag.
 hipError_t prepare_filters(const Buffers& b, hipStream_t s);

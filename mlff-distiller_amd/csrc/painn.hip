@@ -1707,6 +1707,11 @@ int alternative_shape(int H, int which) {
   }
 }
 
+int shapes_used(const Buffers& b) {
+  return (direct_filters(b) ? 1 << 0 | 1 << 1 | 1 << 4 : 0) |
+         (b.N > kMsgSplitAtoms ? 1 << 2 | 1 << 3 : 0);
+}
+
 hipError_t prepare_filters(const Buffers& b, hipStream_t s) {
   if (b.wbf == nullptr || b.L < 1) return hipSuccess;
   split_filter_weights_kernel<<<256, 256, 0, s>>>(b.w, *b.mw, b.wbf, b.tab_bad);

@@ -304,6 +304,12 @@ class Plan:
         want = (fwd_pairs, bwd_pairs, msg_unroll_fwd, msg_unroll_bwd, bwd_variant)
         self.tiles = tuple(int(w) if w else d for w, d in zip(want, default_tiles(self.H)))
 
+    def shapes_used(self) -> Tuple[bool, ...]:
+        """Whether the last evaluation's launches read each launch-shape kind
+        (mlff_plan_shapes_used)."""
+        mask = self.lib.mlff_plan_shapes_used(self.handle)
+        return tuple(bool(mask >> k & 1) for k in range(len(self.tiles)))
+
     def _apply_cell_grid(self):
         if int(self.cell_grid[:, 0].max(initial=0)) > 0:
             g = np.ascontiguousarray(self.cell_grid, dtype=np.int32)

@@ -379,3 +379,35 @@ def test_long_rows_cut_off_by_the_edge_capacity(gpu, monkeypatch, n, ecap):
     run(ecap)
     a, b = run(edges), run(edges + 1000)
     _equal(a, b)
+
+
+@pytest.mark.parametrize("narrow,n", [(False, 3), (False, 40), (True, 3), (True, 40)])
+def test_tuner_leaves_shapes_alone_that_nothing_reads(gpu, narrow, n):
+    """With tables the direct filter kernels do not run, up to 1,024 atoms the message
+    rows take one form: the tuner times the kinds that are read, and the others keep
+    their defaults.  Same bits after it."""
+    note(f"tuner, narrow {narrow}, {n} molecules")
+    synth, engine, tuner = pkg_mod("synth"), pkg_mod("engine"), pkg_mod("autotune")
+    dev = torch.device("cuda:0")
+    Z, P, ptr = synth.flatten(synth.molecule_set(n, 30, 50, seed=n))
+    pos = torch.tensor(P.astype(np.float32), device=dev)
+    lay = engine.make_layout(np.diff(ptr), dev)
+    m = _model(64, 2, 20, 5.0)
+    if narrow:
+        with torch.no_grad():
+            m.rbf.widths.mul_(0.02)
+    plan = engine.Plan(64, 2, 20, 118, 5.0, lay, torch.tensor(Z, device=dev),
+                       m.packed_weights(dev), engine.edge_capacity_bound(np.diff(ptr), False))
+    o = (torch.empty(n, dtype=torch.float64, device=dev), torch.empty(len(Z), 3, device=dev))
+    plan.energy_forces(pos, *o)
+    before = [t.clone() for t in o]
+    tuner._CACHE.clear()
+    got = tuner.tune(plan, pos, candidates=[512], reps=2)
+    used = {k: (narrow if k.startswith("filter") else len(Z) > 1024) for k in tuner.SHAPE_NAMES}
+    assert plan.shapes_used() == tuple(used[k] for k in tuner.SHAPE_NAMES)
+    timed = {k.split("=")[0] for k in got["shape_timings_us"]} - {"default"}
+    assert timed <= {k for k in used if used[k]} and (not any(used.values()) or timed)
+    for k, shape, default in zip(tuner.SHAPE_NAMES, got["tiles"], engine.default_tiles(64)):
+        assert used[k] or shape == default
+    plan.energy_forces(pos, *o)
+    _equal(o, before)
