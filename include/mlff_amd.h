@@ -642,7 +642,8 @@ int mlff_split_bf16x3(void* stream, int64_t n, const float* src_dev, uint16_t* p
  * training pass, around the update MLP's two products.  s [N][H],
  * v [N][3][H], xin [N][2H], y = MLP(xin) = (ds, g1, g2) [N][3H], M the 3x3
  * mixing matrix (row-major, device); hidden a multiple of 4, buffers
- * 16-byte aligned float32.
+ * 16-byte aligned float32.  For hidden sizes and products that mlff_train_update
+ * does not cover; this library's own training pass takes that one.
  *   update_norm:          xin = (s, |v|_xyz)
  *   update_apply:         s' = s + ds, Mv = M v, v' = v g1 + Mv g2
  *   update_norm_tangent:  dxin = (ds, dnrm), dnrm = sum_x v dv / |v| (0 at |v| = 0)

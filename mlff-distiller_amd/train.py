@@ -255,19 +255,6 @@ def _segment_sum(seg_ptr: Tensor, src: Tensor, perm: Optional[Tensor] = None,
 # elementwise pieces and dense products
 # ---------------------------------------------------------------------------
 
-def _glue(name: str, *args):
-    """Call one of the update-block kernels (mlff_update_*): leading ints,
-    then tensors (made dense float32) or None."""
-    conv = []
-    for a in args:
-        if isinstance(a, Tensor):
-            a = _p(_dense(a))
-        elif a is None:
-            a = None
-        conv.append(a)
-    C.check(name, getattr(C.lib(), name)(C.stream_handle(), *conv))
-
-
 def _update(w, s, v, lay: Optional[dict] = None, ds=None, dv=None, primal: bool = True):
     """The update block on inputs (s, v) and, with (ds, dv), its tangent, in one
     launch (mlff_train_update); ``primal`` False: the tangent of the pass stored

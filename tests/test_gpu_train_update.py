@@ -126,3 +126,58 @@ def test_readout_and_its_derivatives(gpu, n, H):
         assert torch.equal(o[0][:, 0].cpu(), seed[batch]) and not o[0][:, 1:].any()
         close(o[3], gs, "gs")
     close(tan[2], dgs, "dgs")
+
+
+@pytest.mark.parametrize("n,H", [(1, 4), (300, 20), (65, 128)])
+def test_elementwise_parts_for_other_products(gpu, n, H):
+    """The update block's elementwise entry points against their formulas in float64
+    (1e-6 of the norm: a few roundings of each element), with a zero vector."""
+    print(f"[case] update parts n{n} H{H}", flush=True)
+    C = pkg_mod("_capi")
+    g = torch.Generator().manual_seed(n + H)
+    r = lambda *sh: torch.randn(*sh, generator=g)
+    s, v, ds, dv = r(n, H), r(n, 3, H), r(n, H), r(n, 3, H)
+    y, dy, gx, dgx = r(n, 3 * H), r(n, 3 * H), r(n, 2 * H), r(n, 2 * H)
+    gs, gv, dgs, dgv, M = r(n, H), r(n, 3, H), r(n, H), r(n, 3, H), r(3, 3)
+    v[0, :, 1] = 0.0
+    D = lambda t: t.double()
+    S, V, dS, dV, Y, dY, GX, dGX, GS, GV, dGS, dGV, Md = map(D, (s, v, ds, dv, y, dy, gx, dgx, gs, gv,
+                                                                 dgs, dgv, M))
+    part = lambda t, k: t[:, k * H:(k + 1) * H]
+    up = lambda t: t[:, None]
+    nrm = V.pow(2).sum(1).sqrt()
+    over = torch.where(nrm > 0, 1 / nrm, torch.zeros_like(nrm))
+    dn = (V * dV).sum(1) * over
+    MV, dMV, g1, g2, dg1, dg2 = Md @ V, Md @ dV, part(Y, 1), part(Y, 2), part(dY, 1), part(dY, 2)
+    want = {
+        "xin": torch.cat([S, nrm], 1), "s": S + part(Y, 0), "v": V * up(g1) + MV * up(g2), "mv": MV,
+        "dxin": torch.cat([dS, dn], 1), "ds": dS + part(dY, 0), "dmv": dMV,
+        "dv": dV * up(g1) + V * up(dg1) + dMV * up(g2) + MV * up(dg2),
+        "gy": torch.cat([GS, (GV * V).sum(1), (GV * MV).sum(1)], 1),
+        "dgy": torch.cat([dGS, (dGV * V + GV * dV).sum(1), (dGV * MV + GV * dMV).sum(1)], 1),
+        "gvg2": GV * up(g2), "dgvg2": dGV * up(g2) + GV * up(dg2),
+    }
+    gn, dgn, unit = part(GX, 1), part(dGX, 1), V * up(over)
+    dunit = dV * up(over) - V * up(dn * over * over)
+    want.update(gs=GS + part(GX, 0), dgs=dGS + part(dGX, 0),
+                gv=GV * up(g1) + Md.T @ want["gvg2"] + up(gn) * unit,
+                dgv=dGV * up(g1) + GV * up(dg1) + Md.T @ want["dgvg2"] + up(dgn) * unit
+                + up(gn) * dunit)
+    ins = {k: t.to(gpu) for k, t in dict(s=s, v=v, ds=ds, dv=dv, y=y, dy=dy, gx=gx, dgx=dgx, gs=gs,
+                                         gv=gv, dgs=dgs, dgv=dgv, M=M).items()}
+    out = {k: torch.full(t.shape, float("nan"), dtype=torch.float32, device=gpu)
+           for k, t in want.items()}
+
+    def call(name, *args):
+        ptrs = [C.ptr(ins[a] if kind == "i" else out[a]) for kind, a in (q.split(".") for q in args)]
+        C.check(name, getattr(C.lib(), "mlff_update_" + name)(C.stream_handle(), n, H, *ptrs))
+
+    call("norm", "i.s", "i.v", "o.xin")
+    call("apply", "i.M", "i.y", "i.s", "i.v", "o.s", "o.v", "o.mv")
+    call("norm_tangent", "i.v", "o.xin", "i.ds", "i.dv", "o.dxin")
+    call("apply_tangent", "i.M", "i.y", "i.dy", "i.ds", "i.v", "i.dv", "o.mv", "o.ds", "o.dv", "o.dmv")
+    call("gate_adjoint", "i.gs", "i.gv", "i.v", "o.mv", "i.dgs", "i.dgv", "i.dv", "o.dmv", "o.gy", "o.dgy")
+    call("input_adjoint", "i.M", "i.gx", "i.gs", "i.gv", "i.y", "i.v", "o.xin", "i.dgx", "i.dgs", "i.dgv",
+         "i.dy", "i.dv", "o.dxin", "o.gs", "o.gv", "o.gvg2", "o.dgs", "o.dgv", "o.dgvg2")
+    for k, ref in want.items():
+        assert (out[k].cpu().double() - ref).norm() <= 1e-6 * ref.norm(), k
