@@ -147,33 +147,38 @@ class _EdgeMessage(torch.autograd.Function):
 _MLP_TYPES = (nn.Linear, nn.SiLU, nn.Linear)
 
 
-def _fused_mlp(seq, *tensors) -> bool:
-    """Whether an MLP block on ``tensors`` may run as one autograd function with
-    its own weight-gradient kernels.  Everything else takes the module path:
-    replaced, hooked or parametrized layers, other types, devices and empty
-    inputs, autocast, tracing, graph capture, function transforms and forward-mode
-    AD.  The layers' sizes are the caller's to check."""
-    if type(seq) is not nn.Sequential or tuple(type(m) for m in seq) != _MLP_TYPES:
-        return False
+def _fused_mlp(seq, *tensors):
+    """(w1, b1, w2, b2) of an MLP block that may run on ``tensors`` as one autograd
+    function with its own weight-gradient kernels, or None.  Everything else takes
+    the module path: replaced, hooked or parametrized layers, other types, devices
+    and empty inputs, autocast, tracing, graph capture, function transforms and
+    forward-mode AD.  The layers' sizes are the caller's to check."""
+    if type(seq) is not nn.Sequential:
+        return None
+    mods = tuple(seq)
+    if tuple(type(m) for m in mods) != _MLP_TYPES:
+        return None
     m = nn.modules.module
     if (m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
             or m._global_backward_pre_hooks):
-        return False
-    for mod in (seq, *seq):
+        return None
+    for mod in (seq, *mods):
         if (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks
                 or mod._backward_pre_hooks or "forward" in mod.__dict__):
-            return False
-    if seq[0].bias is None or seq[2].bias is None:
-        return False
-    for t in (*tensors, seq[0].weight, seq[0].bias, seq[2].weight, seq[2].bias):
+            return None
+    weights = (mods[0].weight, mods[0].bias, mods[2].weight, mods[2].bias)
+    device = tensors[0].device
+    for t in (*tensors, *weights):
         if (type(t) not in (torch.Tensor, nn.Parameter) or not t.is_cuda or t.numel() == 0
-                or t.dtype != torch.float32 or t.device != tensors[0].device):
-            return False
-    return not (torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
-                or torch.cuda.is_current_stream_capturing()
-                or torch.compiler.is_compiling()
-                or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0)
+                or t.dtype != torch.float32 or t.device != device):
+            return None
+    if (torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
+            or torch.cuda.is_current_stream_capturing()
+            or torch.compiler.is_compiling()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0):
+        return None
+    return weights
 
 
 def _kernels_take(*grads) -> bool:
@@ -313,11 +318,8 @@ class PaiNNMessage(nn.Module):
         with (Ws, Wv1, Wv2) = rbf_to_scalar(edge_rbf) per edge."""
         mlp = self.rbf_to_scalar
         with torch.cuda.device_of(scalar_features):   # kernels go to the current device
-            if edge_rbf.dim() == 2 and _fused_mlp(mlp, edge_rbf):
-                filt = _EdgeFilter.apply(edge_rbf, mlp[0].weight, mlp[0].bias, mlp[2].weight,
-                                         mlp[2].bias)
-            else:
-                filt = mlp(edge_rbf)
+            w = _fused_mlp(mlp, edge_rbf) if edge_rbf.dim() == 2 else None
+            filt = mlp(edge_rbf) if w is None else _EdgeFilter.apply(edge_rbf, *w)
             return _EdgeMessage.apply(scalar_features, vector_features, filt, edge_vector,
                                       edge_index[0], edge_index[1])
 
@@ -339,14 +341,15 @@ class PaiNNUpdate(nn.Module):
         _device_f32(scalar_features, vector_features)
         H = self.hidden_dim
         n, mlp, mix = scalar_features.shape[0], self.update_mlp, self.mixing_matrix
+        w = None
+        if (H in (32, 64, 128) and scalar_features.shape == (n, H)
+                and vector_features.shape == (n, 3, H) and mix.shape == (3, 3)):
+            w = _fused_mlp(mlp, scalar_features, vector_features, mix)
         # the kernel takes the layers' sizes from H: any others run as modules
-        if (H in (32, 64, 128) and scalar_features.shape == (n, H) and vector_features.shape == (n, 3, H)
-                and mix.shape == (3, 3) and _fused_mlp(mlp, scalar_features, vector_features, mix)
-                and mlp[0].weight.shape == (H, 2 * H) and mlp[0].bias.shape == (H,)
-                and mlp[2].weight.shape == (3 * H, H) and mlp[2].bias.shape == (3 * H,)):
+        if w is not None and (w[0].shape == (H, 2 * H) and w[1].shape == (H,)
+                              and w[2].shape == (3 * H, H) and w[3].shape == (3 * H,)):
             with torch.cuda.device_of(scalar_features):   # kernels go to the current device
-                return _UpdateBlock.apply(scalar_features, vector_features, mlp[0].weight,
-                                          mlp[0].bias, mlp[2].weight, mlp[2].bias, mix)
+                return _UpdateBlock.apply(scalar_features, vector_features, *w, mix)
         norms = torch.linalg.vector_norm(vector_features, dim=1)
         upd = self.update_mlp(torch.cat([scalar_features, norms], dim=-1))
         ds, g1, g2 = upd[:, :H], upd[:, H:2 * H], upd[:, 2 * H:]

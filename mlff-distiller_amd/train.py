@@ -41,6 +41,7 @@ device; energies are summed in float64.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import weakref
 from dataclasses import dataclass
@@ -299,11 +300,11 @@ def _update_adjoint(w, lay: dict, gs, gv, dgs=None, dgv=None):
     return out, dout
 
 
-def _fit(t: Tensor, *shape) -> Tensor:
+def _fit(t: Tensor, shape: tuple) -> Tensor:
     """t as a dense buffer of the shape that the kernels assume: a layer with fewer
     hidden channels is filled up with zeros, as in the weight blob.  A zero channel
     has silu(0) = 0 and zero weights behind it, so it changes no other value."""
-    if tuple(t.shape) != shape:
+    if t.shape != shape:
         if t.dim() != len(shape) or any(a > b for a, b in zip(t.shape, shape)):
             raise ValueError(f"layer of shape {tuple(t.shape)} in place of {shape}")
         pad = [q for a, b in zip(reversed(t.shape), reversed(shape)) for q in (0, b - a)]
@@ -311,12 +312,28 @@ def _fit(t: Tensor, *shape) -> Tensor:
     return _dense(t)
 
 
+@functools.lru_cache(maxsize=None)
+def _update_shapes(H: int):
+    return ((".update_mlp.0.weight", (H, 2 * H)), (".update_mlp.0.bias", (H,)),
+            (".update_mlp.2.weight", (3 * H, H)), (".update_mlp.2.bias", (3 * H,)),
+            (".mixing_matrix", (3, 3)))
+
+
+@functools.lru_cache(maxsize=None)
+def _readout_shapes(H: int):
+    return (("energy_head.0.weight", (H // 2, H)), ("energy_head.0.bias", (H // 2,)),
+            ("energy_head.2.weight", (H // 4, H // 2)), ("energy_head.2.bias", (H // 4,)),
+            ("energy_head.4.weight", (1, H // 4)), ("energy_head.4.bias", (1,)))
+
+
 def _update_weights(p: Dict[str, Tensor], upre: str):
     H = p["embedding.weight"].shape[1]
-    shapes = ((".update_mlp.0.weight", H, 2 * H), (".update_mlp.0.bias", H),
-              (".update_mlp.2.weight", 3 * H, H), (".update_mlp.2.bias", 3 * H),
-              (".mixing_matrix", 3, 3))
-    return tuple(_fit(p[upre + k], *shape) for k, *shape in shapes)
+    return tuple([_fit(p[upre + k], shape) for k, shape in _update_shapes(H)])
+
+
+def _readout_weights(p: Dict[str, Tensor]):
+    H = p["embedding.weight"].shape[1]
+    return tuple([_fit(p[k], shape) for k, shape in _readout_shapes(H)])
 
 
 def _readout(w, s, c: Optional[dict] = None, ds=None, primal: bool = True):
@@ -355,13 +372,6 @@ def _readout_adjoint(w, c: dict, seed, batch, T: bool):
         C.ptr(c["dr1"] if T else None), C.ptr(c["dr2"] if T else None), C.ptr(w[0]), C.ptr(w[2]),
         C.ptr(w[4]), C.ptr(g4), *[C.ptr(t) for t in out + dout]))
     return (g4, *out), dout
-
-
-def _readout_weights(p: Dict[str, Tensor]):
-    H = p["embedding.weight"].shape[1]
-    shapes = (("0.weight", H // 2, H), ("0.bias", H // 2), ("2.weight", H // 4, H // 2),
-              ("2.bias", H // 4), ("4.weight", 1, H // 4), ("4.bias", 1))
-    return tuple(_fit(p["energy_head." + k], *shape) for k, *shape in shapes)
 
 
 def _silu_call(a, da=None, g=None, dg=None, h=False, dh=False, dga=False):
