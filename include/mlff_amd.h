@@ -181,9 +181,9 @@ int64_t mlff_plan_workspace_bytes(const mlff_plan* plan);
  * cells_dev [B,3,3] (rows = lattice vectors) and pbc_dev [B,3] may be NULL
  * for non-periodic batches.  weights_dev is the packed blob.  The workspace
  * and the weights must be 16-byte aligned (MLFF_ERR_INVALID otherwise).  Binding is
- * synchronous: it clears the plan's counters and splits the filter weights
- * into their bf16 planes inside the workspace, then waits for the device;
- * it also creates the plan's second stream on the current device. */
+ * synchronous: it clears the plan's counters and makes the filters' bf16 planes
+ * and distance tables inside the workspace, then waits for the device; where the
+ * plan has a second stream it is created on the current device. */
 int mlff_plan_bind(mlff_plan* plan, void* workspace_dev, int64_t workspace_bytes,
                    const float* weights_dev, const int64_t* numbers_dev,
                    const int32_t* mol_ptr_dev, const int32_t* atom_mol_dev,

@@ -455,8 +455,8 @@ int mlff_plan_create(mlff_plan** out, const mlff_config* cfg) {
   set_default_shapes(pl);
   // one stream: with the filter tables the pair kernels are short and bound by
   // memory like the atom-side ones, and the fork and join events cost more than
-  // the overlap gives (256 molecules 2.41 ms on two streams, 2.30 on one; an MD
-  // step of one 60-atom molecule 298 and 245 us)
+  // the overlap gives (256 molecules 2.04 ms on two streams, 1.93 on one; an MD
+  // step of one 60-atom molecule 172 and 110 us)
   pl->n_streams = 1;
   pl->stream_dev = -1;
   *out = pl;

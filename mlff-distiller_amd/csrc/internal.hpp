@@ -96,7 +96,7 @@ __device__ __forceinline__ T hermite(const TableAt& a, const T& f0, const T& g0,
   return f0 + fma_(a.h01, f1 - f0, fma_(a.h10, g0, a.h11 * g1));
 }
 
-// Model launches (painn_fwd.hip / painn_bwd.hip).
+// Model launches (painn.hip).
 struct Buffers {
   int N, B, H, L, R;
   float rc;

@@ -12,14 +12,18 @@
 // output W_p [3H] = (W_s | W_v1 | W_v2) of each block.
 //
 // Kernels and what bounds them:
-//   filter_fwd   pairs, MFMA (R->H, SiLU, H->3H; the H->3H product on the bf16
-//                matrix cores with three-way split operands); 2(RH + 3H^2) flop/pair
+//   filter_table_fwd, filter_table_bwd (filter_table.hip)  pairs, the filters and their
+//                adjoint from distance tables: HBM writes, table rows from beyond the L2
+//   filter_fwd, filter_bwd  the same by the MLP per pair, where no table can stand and
+//                behind the guard's flag until the host has read it:
+//     forward    MFMA (R->H, SiLU, H->3H; the H->3H product on the bf16 matrix cores
+//                with three-way split operands); 2(RH + 3H^2) flop/pair
+//     adjoint    gathers both endpoints' features and gradients, MFMA (3H->H, H->R)
+//                back to dE/dd and dE/du
 //   message      receiver rows, gather of s_j, v_j, W_p (HBM/L2)
 //   update_fwd   atoms, MFMA (2H->H, SiLU, H->3H) + gated vector epilogue
 //   readout      atoms, MFMA head and its input gradient in one pass
 //   update_bwd   atoms, MFMA (3H->H, H->2H) transposed products
-//   filter_bwd   pairs, gathers both endpoints' features and gradients, MFMA
-//                (3H->H, H->R) back to dE/dd and dE/du
 //   force_gather receiver rows, forces and per-atom virial from dE/dvec
 //   reduce       per structure FP64 sums (energy, virial)
 
@@ -52,9 +56,16 @@ constexpr int kUpdBlock = 64 * kUpdWaves;
 // CUs in either, half the products per CU); 14,000 atoms 89 us in 32-atom and
 // 109 us in 16-atom tiles, which read the weights twice as often.
 // Readout: 14 -> 7 us at 60 atoms, 15 -> 9 us at 3000.
+// Where the lines lie, whole evaluations of 40-atom molecules, three blocks at H = 128
+// (two at H = 32): split against 16-atom tiles 191 / 204 us at 720 atoms, 221 / 235 at
+// 1000, 274 / 248 at 1240 (H = 32: 4 us behind from 240 atoms on); 16-atom against
+// 32-atom tiles 533 / 556 us at 4000 atoms, 653 / 633 at 5000 (H = 32: ahead by 5 % up to
+// 10,000).
 constexpr int kSplitAtoms = 1024;
 constexpr int kSmallTileAtoms = 4096;
-// Message rows: sums per row, and the atoms up to which each has threads of its own
+// Message rows: sums per row, and the atoms up to which each has threads of its own.
+// The same evaluations, split against whole rows: 143 / 151 us at 240 atoms, 166 / 166 at
+// 480, 221 / 209 at 1000 (H = 32: 62 / 73, 69 / 79, 79 / 85, 98 / 96 at 2000).
 constexpr int kMsgSums = 4;
 constexpr int kMsgSplitAtoms = 1024;
 // edges in flight per row in the message kernels (forward, adjoint)
